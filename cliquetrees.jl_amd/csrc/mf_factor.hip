@@ -500,135 +500,182 @@ __device__ __forceinline__ void ea_columns(const DevPlan& P, const DevFactor<T>&
     }
 }
 
-constexpr int PB = 16;                          // block size inside the diagonal tile
-constexpr int PTILE = NB * LDS + 3 * PB * PB + 2 * NB + PB;  // LDS elements of potrf_blocked
+constexpr int PB = 16;            // block size inside the diagonal tile
+constexpr int LDP = PB + 1;       // leading dimension of the tile's inverse diagonal blocks
+constexpr int PTILE = NB * LDS + (NB / PB) * PB * LDP + 3 * NB;  // LDS elements of potrf_blocked
 
-// Value of v held by lane l of the wavefront (l wave-uniform).
-__device__ __forceinline__ double bcast(double v, int l) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, l);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), l);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+// Column operations with the multiplier broadcast inside each row of sixteen
+// lanes (DPP row_newbcast): a(q) += (lane L0 + q of s) * m for q < N.  One
+// instruction per element, where a readlane pair and a multiply-add take
+// 20 cycles against 9.5 (FP64, one wavefront).  The leading s_nop covers the
+// two wait states between a vector write of s and its first DPP read.
+template <int L0>
+__device__ __forceinline__ void dpp_fma1(double& a0, double s, double m) {
+    asm("s_nop 1\n\t"
+        "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+        : "+v"(a0) : "v"(s), "v"(m), "n"(L0));
 }
-__device__ __forceinline__ float bcast(float v, int l) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+template <int L0>
+__device__ __forceinline__ void dpp_fma4(double& a0, double& a1, double& a2, double& a3, double s, double m) {
+    asm("s_nop 1\n\t"
+        "v_fmac_f64_dpp %0, %4, %5 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %1, %4, %5 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %2, %4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %3, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3)
+        : "v"(s), "v"(m), "n"(L0), "n"(L0 + 1), "n"(L0 + 2), "n"(L0 + 3));
+}
+template <int L0>
+__device__ __forceinline__ void dpp_fma1(float& a0, float s, float m) {
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+        : "+v"(a0) : "v"(s), "v"(m), "n"(L0));
+}
+template <int L0>
+__device__ __forceinline__ void dpp_fma4(float& a0, float& a1, float& a2, float& a3, float s, float m) {
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %4, %5 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %4, %5 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %2, %4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3)
+        : "v"(s), "v"(m), "n"(L0), "n"(L0 + 1), "n"(L0 + 2), "n"(L0 + 3));
+}
+// a[j] += (lane j of s) * m for K < j < 16
+template <int K, typename T>
+__device__ __forceinline__ void dpp_cols(T (&a)[PB], T s, T m) {
+    constexpr int G = (K + 4) / 4 * 4;  // first whole group of four columns
+    if constexpr (K + 1 < G) dpp_fma1<K + 1>(a[K + 1], s, m);
+    if constexpr (K + 2 < G) dpp_fma1<K + 2>(a[K + 2], s, m);
+    if constexpr (K + 3 < G) dpp_fma1<K + 3>(a[K + 3], s, m);
+    if constexpr (G <= 4) dpp_fma4<4>(a[4], a[5], a[6], a[7], s, m);
+    if constexpr (G <= 8) dpp_fma4<8>(a[8], a[9], a[10], a[11], s, m);
+    if constexpr (G <= 12) dpp_fma4<12>(a[12], a[13], a[14], a[15], s, m);
+}
+// Lane K of every row of sixteen lanes, to all its lanes.
+template <int K>
+__device__ __forceinline__ double dpp_bcast(double s) {
+    double v;
+    asm("s_nop 1\n\tv_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "=v"(v) : "v"(s), "n"(K));
+    return v;
+}
+template <int K>
+__device__ __forceinline__ float dpp_bcast(float s) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0x150 + K, 0xf, 0xf, true));
 }
 
-// 16 x 16 block product on the matrix cores: acc += sum over the K = 16 * kt
-// columns of  opA(i, k) * opB(k, j), with opA(i, k) = X[(ra + i) + (ca + k) * LDS]
-// (times sc[ca + k] when sc is given) and opB(k, j) = Y[(rb + k) + (cb + j) * ldy].
-template <typename T>
-__device__ __forceinline__ void blk_mma(const T* X, int ra, int ca, const T* Y, int rb, int cb, int ldy,
-                                        int kt, const T* sc, typename Mfma<T>::v4& acc) {
-    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-    for (int s = 0; s < 4 * kt; ++s) {
-        const int k = 4 * s + lk;
-        T av = X[(ra + li) + (ca + k) * LDS];
-        if (sc) av *= sc[ca + k];
-        acc = Mfma<T>::op(av, Y[(rb + k) + (cb + li) * ldy], acc);
-    }
+// 1 / sqrt(d) and 1 / d to full double precision: the hardware estimate
+// (about 24 bits) and one step of third order, a chain of five and three
+// operations.
+__device__ __forceinline__ double rsqrt_full(double d) {
+    const double y = __builtin_amdgcn_rsq(d);
+    const double e = __builtin_fma(-(d * y), y, 1.0);
+    return __builtin_fma(y, e * __builtin_fma(e, 0.375, 0.5), y);
+}
+__device__ __forceinline__ double rcp_full(double d) {
+    const double y = __builtin_amdgcn_rcp(d);
+    const double e = __builtin_fma(-d, y, 1.0);
+    return __builtin_fma(y, __builtin_fma(e, e, e), y);
 }
 
-// Factors the 16 x 16 diagonal block held by lanes 0..15 of one wavefront
-// (lane i: row i in x[0..15]; the other lanes compute alongside and are
-// ignored), nk <= 16 columns.  Per pivot the pivot itself comes by readlane
-// (a short chain to the next pivot), and column k reaches every lane through
-// LDS (cb) for the rank-1 update.  pv/rd receive the pivots and the
-// reciprocals of L's diagonal (Cholesky) or of the pivots (LDLt).  RULE 0: the general pivot rule (signs,
-// regularization: regularize per pivot); RULE 1: Cholesky with the default
-// signs (fails unless the pivot is positive); RULE 2: LDLt with the default
-// signs (fails on a zero pivot only).
-template <typename T, int RULE>
-__device__ __forceinline__ void pivot_block(T (&x)[PB], const DevFactor<T>& F, const int gcol0, const int nk,
-                                            const bool chol, T* cb, T* pv, T* rd, const int lane) {
-    // the pivot of the next step, as it will stand after this step's update:
-    // lane k+1 forms it from its own entries (x[k+1] - ar * ark is the same
-    // fused multiply-add as the rank-1 update below applies to its x[k+1],
-    // since the broadcast column entry of row k+1 is its own x[k]), so the
-    // chain from pivot to pivot skips the LDS round trip of the column
-    T dnext = bcast(x[0], 0);
-#pragma unroll
-    for (int k = 0; k < PB; ++k) {
-        if (k >= nk) continue;  // uniform
-        // the lane id is re-read per step so that the compiler does not keep
-        // sixteen steps' worth of lane masks live in scalar registers
-        int ln = lane;
-        asm volatile("" : "+v"(ln));
-        // column k as it stands to every lane through LDS: one write, then
-        // uniform reads (a wavefront's LDS operations complete in order)
-        if (ln < PB) cb[ln] = x[k];
-        __builtin_amdgcn_wave_barrier();
-        const T akk = dnext;
-        double piv;
-        bool bad;
-        if (RULE == 0) {
-            piv = regularize(F, sign_of(F, gcol0 + k), (double)akk);
-            bad = (piv == 0.0);
+// Pivot rules of the diagonal tile.  PR_RULE: signs and regularization, one
+// call of regularize per pivot; PR_CHOL / PR_LDLT: the default signs (fails
+// unless the pivot is positive / on a zero pivot only); PR_INV / PR_INV_UNIT:
+// the block is factored already (Cholesky / LDLt) and only carries the other
+// rows along.
+enum { PR_RULE = 0, PR_CHOL = 1, PR_LDLT = 2, PR_INV = 3, PR_INV_UNIT = 4 };
+
+// Columns K..15 of a 16-column block by one wavefront.  x: row (lane & 15) of
+// the diagonal block, repeated in each row of sixteen lanes (so that DPP can
+// broadcast its column); y: one other row per lane.  Per pivot k with s =
+// 1 / l_kk (Cholesky) or 1 / d_k (LDLt): l = x_k s, and every later column
+// takes x_j -= l_jk m, y_j -= l_jk m_y, with m, m_y the finished x_k, y_k:
+// l for Cholesky, the unscaled column a_ik for LDLt (the caller multiplies
+// by s where it needs l).  The rows below the block (a panel solve) and rows
+// of the identity (which become rows of L^-T) are the same operation.
+// Finished columns go to LDS at once (xw, yw: this lane's rows, column
+// strides LDS and ys; what lands above the diagonal is not read).  pv / sc
+// (LDS): the pivots and s for LDLt.  fails: bit k for a failed pivot.
+template <typename T, int RULE, int K>
+__device__ __forceinline__ void pivot_cols(T (&x)[PB], T (&y)[PB], const DevFactor<T>& F, const int gcol0,
+                                           const int nk, const bool chol, T* pv, T* sc, T* xw, T* yw,
+                                           const int ys, unsigned& fails, const int lane) {
+    if constexpr (K < PB) {
+        T l, m, my;
+        if constexpr (RULE == PR_INV_UNIT) {
+            l = x[K];
+            my = y[K];
+        } else if constexpr (RULE == PR_INV) {
+            l = x[K];
+            my = y[K] * (T)rcp_full((double)dpp_bcast<K>(x[K]));
         } else {
-            piv = (double)akk;
-            bad = RULE == 1 ? !(piv > 0.0) : (piv == 0.0);
-        }
-        if (bad) piv = 1.0;  // keeps the rest finite after a failure
-        // 1/sqrt(piv) and 1/piv from the hardware estimates plus two Newton
-        // steps each (full double precision, a short dependency chain)
-        T ip, sq = (T)1, isq = (T)1;
-        if (chol) {
-            double y = __builtin_amdgcn_rsq(piv);
-            const double h = 0.5 * piv;
-            y = y * __builtin_fma(-h * y, y, 1.5);
-            y = y * __builtin_fma(-h * y, y, 1.5);
-            isq = (T)y;
-            sq = (T)(piv * y);
-            ip = (T)(y * y);
-        } else {
-            double y = __builtin_amdgcn_rcp(piv);
-            y = __builtin_fma(__builtin_fma(-piv, y, 1.0), y, y);
-            y = __builtin_fma(__builtin_fma(-piv, y, 1.0), y, y);
-            ip = (T)y;
-        }
-        T colv[PB];
-#pragma unroll
-        for (int j = k + 1; j < PB; ++j) colv[j] = cb[j];
-        const T ark = x[k], ar = ark * ip;
-        if (k + 1 < PB) dnext = bcast(x[k + 1] - ar * ark, k + 1);
-        if (ln == 0) {
-            if (bad) atomicMin(F.info, (unsigned long long)(gcol0 + k + 1));
-            else if (!chol) stc(F.d + gcol0 + k, (T)piv);
-            pv[k] = (T)piv;
-            rd[k] = chol ? isq : ip;
-        }
-#pragma unroll
-        for (int j = k + 1; j < PB; ++j) x[j] -= ar * colv[j];
-        if (ln >= k) {
-            if (chol) {
-                x[k] = (ln == k) ? sq : ark * isq;
-            } else if (ln > k) {
-                x[k] = ar;  // LDLt keeps the unregularized pivot on the diagonal
+            double piv = (double)dpp_bcast<K>(x[K]);
+            const bool ch = RULE == PR_CHOL || (RULE == PR_RULE && chol);
+            bool bad = false;
+            if constexpr (RULE == PR_RULE) {
+                // padding columns (K >= nk) keep their pivot 1: no sign is read
+                if (K < nk) piv = regularize(F, sign_of(F, gcol0 + K), piv);
+                bad = piv == 0.0;
+            } else {
+                bad = RULE == PR_CHOL ? !(piv > 0.0) : piv == 0.0;
             }
+            fails |= bad ? 1u << K : 0u;
+            if constexpr (RULE == PR_RULE) {
+                if (bad) piv = 1.0;
+            }
+            const double s = ch ? rsqrt_full(piv) : rcp_full(piv);
+            l = x[K] * (T)s;
+            if constexpr (RULE == PR_RULE) {
+                // the (possibly replaced) pivot on the diagonal
+                if ((lane & (PB - 1)) == K && ch) l = (T)(piv * s);
+            }
+            m = ch ? l : x[K];
+            my = ch ? y[K] * (T)s : y[K];
+            if (!ch && lane == 0) {
+                pv[K] = (T)piv;
+                sc[K] = (T)s;
+            }
+            dpp_cols<K>(x, l, -m);
+            if (lane < PB) xw[K * LDS] = m;
         }
+        dpp_cols<K>(y, l, -my);
+        yw[K * ys] = my;
+        pivot_cols<T, RULE, K + 1>(x, y, F, gcol0, nk, chol, pv, sc, xw, yw, ys, fails, lane);
     }
 }
 
-// Diagonal tile, blocked: the 64 x 64 tile lives in LDS and is factored in
-// four 16-column block steps (potrf2!'s right-looking recursion cut at 16):
-// (1) one wavefront factors the 16 x 16 diagonal block in registers with the
-// pivot rule (columns broadcast with readlane, no LDS round trip) and keeps
-// the reciprocals of the diagonal, (2) one lane per row solves the rows below
-// against it, (3) the rank-16 update of the trailing lower triangle runs on
-// the matrix cores, one 16 x 16 block per wavefront.  Then W = L^-1 in place:
-// the four diagonal blocks are inverted one per wavefront, and the block rows
-// below follow in three stages of W_ij = -W_ii (sum_k L_ik W_kj), again on the
-// matrix cores.  L goes to the panel and W (ld = nn, zeros above the
-// diagonal) to the W pool.  LDS: PTILE elements.
+// Diagonal tile, blocked by 16 columns: the 64 x 64 tile A lives in LDS.  The
+// factor and its inverse come out of one pass over [A; I]: the column
+// operations that turn A into L turn the identity into L^-T.  Rows of A use
+// the tile's lower blocks and rows of the identity its upper blocks, which A
+// does not use; the identity's diagonal blocks have a place of their own
+// (WD).  So "row block w" is rows [16w, 16w + 16) of A for w > b and of the
+// identity for w <= b, 64 rows beside the diagonal block in every block step
+// b.  A block step:
+// (1) wavefront 0 takes the diagonal block and all 64 other rows through the
+//     block's 16 pivots in registers (pivot_cols), while the other
+//     wavefronts finish the previous step's update;
+// (2) the rank-16 update X_wc -= X_wb (s L_cb)' on the matrix cores, first
+//     the next block column (wavefront w its row block), then, beside the
+//     next step's pivots, the later ones (c <= w for rows of A).
+// Bound: wavefront 0's instruction issue in the chain of 64 pivots (FP64
+// operations issue every 8 cycles on one wavefront).  A full tile on an idle
+// CU, load to last store: FP64 13.6 us, FP32 12.4 us (19.0 and
+// 16.0 us with the pivot row broadcast by readlane, one wavefront per row
+// block; 40 us with the rows below and the inverse in passes of their own).
+// L goes to the panel and W = L^-1 (ld = nn, zeros above the diagonal) to the
+// W pool.  invert_only: the tile already holds L and only W is formed.  LDS:
+// PTILE elements.
 template <typename T>
 __device__ __forceinline__ void potrf_blocked(const DevFactor<T>& F, const Front& f, int k0, bool invert_only,
                               T* lds, const int tid) {
     typedef typename Mfma<T>::v4 v4;
-    T* A = lds;                       // 64 x LDS, column-major
-    T* Tm = lds + NB * LDS;           // 3 blocks of 16 x 16 (stage products, ld 16)
-    T* pv = Tm + 3 * PB * PB;         // pivots of the tile (LDLt scaling)
-    T* rd = pv + NB;                  // reciprocals of L's diagonal (Cholesky)
-    T* cb = rd + NB;                  // the pivot column of the 16 x 16 block (broadcast)
+    constexpr int NBLK = NB / PB;
+    T* A = lds;                          // 64 x LDS, column-major
+    T* WD = lds + NB * LDS;              // diagonal blocks of L^-T, PB x LDP each
+    T* sc = WD + NBLK * PB * LDP;        // 1 (Cholesky) or the reciprocal pivots (LDLt)
+    T* pv = sc + NB;                     // the pivots (LDLt)
     const int nj = f.nn + f.na, kb = min(NB, f.nn - k0), gc0 = f.c0 + k0;
     T* blk = F.panel + f.poff + k0 + (int64_t)k0 * nj;
     const int r = tid & 63, cg = tid >> 6, lane = tid & 63, wave = tid >> 6;
@@ -643,145 +690,109 @@ __device__ __forceinline__ void potrf_blocked(const DevFactor<T>& F, const Front
             const int c = cg + 4 * i;
             tv[i] = ldc(blk + ((r < kb && c < kb && c <= r) ? r + (int64_t)c * nj : 0));
         }
+        // the identity's diagonal blocks: block = wave, four elements per thread
+#pragma unroll
+        for (int q = 0; q < 4; ++q) WD[wave * PB * LDP + li + (lk + 4 * q) * LDP] = li == lk + 4 * q ? (T)1 : (T)0;
+        if (tid < NB) sc[tid] = (T)1;
 #pragma unroll
         for (int i = 0; i < NB / 4; ++i) {
             const int c = cg + 4 * i;
             A[r + c * LDS] = (r < kb && c < kb && c <= r) ? tv[i] : (r == c ? (T)1 : (T)0);
         }
     }
-    if (tid < NB) {
-        pv[tid] = (T)1;
-        rd[tid] = (T)1;
-    }
     __syncthreads();
+    // X_wc -= X_wb (s L_cb)' for row block w of block step b
+    auto update = [&](int w, int b, int c) {
+        const T* xa = w == b ? WD + b * PB * LDP : A + PB * w + PB * b * LDS;
+        const int xs = w == b ? LDP : LDS;
+        T av[4], bv[4], xv[4];
+        v4 acc = v4{0, 0, 0, 0};
+        T* xc = A + PB * w + (PB * c + li) * LDS;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            av[s] = xa[li + (4 * s + lk) * xs];
+            bv[s] = A[(PB * c + li) + (PB * b + 4 * s + lk) * LDS] * sc[PB * b + 4 * s + lk];
+            xv[s] = xc[Mfma<T>::row(lk, s)];
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc = Mfma<T>::op(av[s], bv[s], acc);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) xc[Mfma<T>::row(lk, v)] = xv[v] - acc[v];
+    };
+#pragma unroll 1
+    for (int b = 0; b < NBLK; ++b) {
+        const int c0 = b * PB;
+        if (c0 >= kb) break;  // uniform
+        if (wave == 0) {
+            T x[PB], y[PB];
+            T* xw = A + (c0 + li) + c0 * LDS;
+            T* yw = lk == b ? WD + b * PB * LDP + li : A + lane + c0 * LDS;  // this lane's other row
+            const int ys = lk == b ? LDP : LDS;
+#pragma unroll
+            for (int j = 0; j < PB; ++j) x[j] = xw[j * LDS];
+#pragma unroll
+            for (int j = 0; j < PB; ++j) y[j] = yw[j * ys];
+            const int nk = min(PB, kb - c0), g0 = gc0 + c0;
+            T *pb = pv + c0, *sb = sc + c0;
+            unsigned fails = 0;
+            if (invert_only) {
+                // rows of A below the block are final: their results go to a spare place
+                if (lk > b) yw = pv + NB + lane;
+                const int yi = lk > b ? 0 : ys;
+                if (chol) pivot_cols<T, PR_INV, 0>(x, y, F, g0, nk, true, pb, sb, xw, yw, yi, fails, lane);
+                else pivot_cols<T, PR_INV_UNIT, 0>(x, y, F, g0, nk, false, pb, sb, xw, yw, yi, fails, lane);
+            } else if (F.signs != nullptr || F.reg_kind != 0) {
+                // signs or a regularization take the general form
+                pivot_cols<T, PR_RULE, 0>(x, y, F, g0, nk, chol, pb, sb, xw, yw, ys, fails, lane);
+            } else if (chol) {
+                pivot_cols<T, PR_CHOL, 0>(x, y, F, g0, nk, true, pb, sb, xw, yw, ys, fails, lane);
+            } else {
+                pivot_cols<T, PR_LDLT, 0>(x, y, F, g0, nk, false, pb, sb, xw, yw, ys, fails, lane);
+            }
+            if (fails != 0 && lane == 0)
+                atomicMin(F.info, (unsigned long long)(g0 + __builtin_ctz(fails) + 1));
+        } else if (b > 0) {
+            // the later block columns of the previous step, beside the pivots
+            int q = 0;
+            for (int w = 0; w < NBLK; ++w)
+                for (int c = b + 1; c <= (w > b - 1 ? w : NBLK - 1); ++c, ++q)
+                    if (q % 3 == wave - 1 && !(invert_only && w > b - 1)) update(w, b - 1, c);
+        }
+        __syncthreads();
+        // the next block column
+        if (b + 1 < NBLK && c0 + PB < kb && !(invert_only && wave > b)) update(wave, b, b + 1);
+        __syncthreads();
+    }
+    // all of a thread's LDS reads first, then its stores
     if (!invert_only) {
-        for (int b = 0; b < NB / PB; ++b) {
-            const int c0 = b * PB;
-            if (c0 >= kb) break;  // uniform
-            // (1) diagonal block by wavefront 0: lane i < 16 holds row c0 + i
-            if (tid < 64) {
-                T x[PB];
+        T v[NB / 4];
 #pragma unroll
-                for (int j = 0; j < PB; ++j) x[j] = lane < PB ? A[(c0 + lane) + (c0 + j) * LDS] : (T)0;
-                const int nk = min(PB, kb - c0);
-                // the default pivot rule (no signs, no regularization) without
-                // per-pivot branches; signs or a regularization take the general form
-                if (F.signs != nullptr || F.reg_kind != 0)
-                    pivot_block<T, 0>(x, F, gc0 + c0, nk, chol, cb, pv + c0, rd + c0, lane);
-                else if (chol)
-                    pivot_block<T, 1>(x, F, gc0 + c0, nk, true, cb, pv + c0, rd + c0, lane);
-                else
-                    pivot_block<T, 2>(x, F, gc0 + c0, nk, false, cb, pv + c0, rd + c0, lane);
-                if (lane < PB)
-#pragma unroll
-                    for (int j = 0; j < PB; ++j)
-                        if (j <= lane) A[(c0 + lane) + (c0 + j) * LDS] = x[j];
-            }
-            __syncthreads();
-            // (2) rows below: y L_D' = a (unit L_D for LDLt), then l = y / d for LDLt
-            // (the reciprocals rd loaded unconditionally and applied by selects:
-            // a load under a branch would be waited for inside it)
-            const int rb = c0 + PB;
-            if (tid < 64 && rb + lane < NB) {
-                const int i = rb + lane;
-                T y[PB], rv[PB];
-#pragma unroll
-                for (int j = 0; j < PB; ++j) {
-                    y[j] = A[i + (c0 + j) * LDS];
-                    rv[j] = rd[c0 + j];
-                }
-#pragma unroll
-                for (int k = 0; k < PB; ++k) {
-                    y[k] *= chol ? rv[k] : (T)1;
-#pragma unroll
-                    for (int j = k + 1; j < PB; ++j) y[j] -= y[k] * A[(c0 + j) + (c0 + k) * LDS];
-                }
-#pragma unroll
-                for (int k = 0; k < PB; ++k) A[i + (c0 + k) * LDS] = chol ? y[k] : y[k] * rv[k];
-            }
-            __syncthreads();
-            // (3) trailing update of the lower triangle, A_ij -= sum_k L_ik s_k L_jk,
-            // one 16 x 16 block (ti >= tj > b) per wavefront on the matrix cores
-            {
-                int q = 0;
-                for (int ti = b + 1; ti < NB / PB; ++ti)
-                    for (int tj = b + 1; tj <= ti; ++tj, ++q) {
-                        if ((q & 3) != wave) continue;
-                        v4 acc = v4{0, 0, 0, 0};
-#pragma unroll
-                        for (int s4 = 0; s4 < PB / 4; ++s4) {
-                            const int k = 4 * s4 + lk;
-                            T av = A[(PB * ti + li) + (c0 + k) * LDS];
-                            const T sv = pv[c0 + k];
-                            av *= chol ? (T)1 : sv;
-                            acc = Mfma<T>::op(av, A[(PB * tj + li) + (c0 + k) * LDS], acc);
-                        }
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) {
-                            const int row = PB * ti + Mfma<T>::row(lk, v), col = PB * tj + li;
-                            if (row >= col) A[row + col * LDS] -= acc[v];
-                        }
-                    }
-            }
-            __syncthreads();
+        for (int i = 0; i < NB / 4; ++i) {
+            const int c = cg + 4 * i;
+            v[i] = A[r + c * LDS] * (r > c ? sc[c] : (T)1);
         }
-        for (int c = cg; c < kb; c += 4) {
-            T* colp = blk + (int64_t)c * nj;
-            if (r < kb && c <= r) stc(colp + r, A[r + c * LDS]);
+#pragma unroll
+        for (int i = 0; i < NB / 4; ++i) {
+            const int c = cg + 4 * i;
+            if (r < kb && c <= r) stc(blk + r + (int64_t)c * nj, v[i]);
         }
-        __syncthreads();  // L is read out before the inverse overwrites it
-    } else if (tid < NB) {
-        rd[tid] = chol ? (T)1 / A[tid + tid * LDS] : (T)1;
+        if (!chol && tid < kb) stc(F.d + gc0 + tid, pv[tid]);
     }
-    if (invert_only) __syncthreads();
-    // W = L^-1 in place.  Diagonal blocks: wavefront w inverts block w; lane
-    // c < 16 keeps column c of W_ww (forward substitution, unit for LDLt).
-    {
-        const int bw = cg, c0 = bw * PB;
-        T w[PB];
-        if (lane < PB) {
-#pragma unroll
-            for (int i = 0; i < PB; ++i) w[i] = (i == lane) ? (T)1 : (T)0;
-#pragma unroll
-            for (int k = 0; k < PB; ++k) {
-                const T rk = rd[c0 + k];
-                w[k] *= chol ? rk : (T)1;
-#pragma unroll
-                for (int i = k + 1; i < PB; ++i) w[i] -= A[(c0 + i) + (c0 + k) * LDS] * w[k];
-            }
-        }
-        // a wavefront's LDS reads complete before its writes: only this
-        // wavefront touches block (bw, bw) here
-        if (lane < PB)
-#pragma unroll
-            for (int i = 0; i < PB; ++i) A[(c0 + i) + (c0 + lane) * LDS] = (i >= lane) ? w[i] : (T)0;
-    }
-    __syncthreads();
-    for (int bi = 1; bi < NB / PB; ++bi) {
-        // T_ij = sum_{k=j}^{i-1} L_ik W_kj for j < i (W_kj rows done, L_ik intact):
-        // block bj by wavefront bj
-        if (wave < bi) {
-            const int bj = wave;
-            v4 acc = v4{0, 0, 0, 0};
-            blk_mma<T>(A, PB * bi, PB * bj, A, PB * bj, PB * bj, LDS, bi - bj, nullptr, acc);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) Tm[bj * PB * PB + Mfma<T>::row(lk, v) + li * PB] = acc[v];
-        }
-        __syncthreads();
-        // W_ij = -W_ii T_ij
-        if (wave < bi) {
-            const int bj = wave;
-            v4 acc = v4{0, 0, 0, 0};
-            blk_mma<T>(A, PB * bi, PB * bi, Tm + bj * PB * PB, 0, 0, PB, 1, nullptr, acc);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) A[(PB * bi + Mfma<T>::row(lk, v)) + (PB * bj + li) * LDS] = -acc[v];
-        }
-        __syncthreads();
-    }
+    // W(r, c) = L^-T(c, r)
     T* W = F.W + f.woff + k0;
-    for (int c = cg; c < kb; c += 4) {
-        T* colp = W + (int64_t)c * f.nn;
-        if (r < kb) stc(colp + r, (c <= r) ? A[r + c * LDS] : (T)0);
+    {
+        T v[NB / 4];
+#pragma unroll
+        for (int i = 0; i < NB / 4; ++i) {
+            const int c = cg + 4 * i, bc = i / 4, br = r / PB;
+            const T* src = bc == br ? WD + bc * PB * LDP + (c & (PB - 1)) + (r & (PB - 1)) * LDP : A + c + r * LDS;
+            v[i] = *src;
+        }
+#pragma unroll
+        for (int i = 0; i < NB / 4; ++i) {
+            const int c = cg + 4 * i;
+            if (r < kb && c < kb) stc(W + r + (int64_t)c * f.nn, (c <= r) ? v[i] : (T)0);
+        }
     }
 }
 
