@@ -37,7 +37,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 TABLE = os.path.join(HERE, "tuning.json")
 
 DEFAULTS = {"upd_group": 8, "ea_rows": 16384, "wide_k": 128, "sim_workers": 512, "zero_ppm": 50000,
-            "prio": 0, "fuse": 0, "wg_per_cu": 0}
+            "prio": 0, "fuse": 1, "wg_per_cu": 0}
 CANDIDATES = {
     "upd_group": [4, 8, 12, 16],
     "ea_rows": [8192, 16384, 32768],

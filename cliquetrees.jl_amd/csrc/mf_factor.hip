@@ -664,9 +664,9 @@ __device__ __forceinline__ void pivot_cols(T (&x)[PB], T (&y)[PB], const DevFact
 // CU, load to last store: FP64 13.6 us, FP32 12.4 us (19.0 and
 // 16.0 us with the pivot row broadcast by readlane, one wavefront per row
 // block; 40 us with the rows below and the inverse in passes of their own).
-// L goes to the panel and W = L^-1 (ld = nn, zeros above the diagonal) to the
-// W pool.  invert_only: the tile already holds L and only W is formed.  LDS:
-// PTILE elements.
+// W = L^-1 (ld = nn, zeros above the diagonal) goes to the W pool; L stays in
+// LDS for store_diag.  invert_only: the tile already holds L and only W is
+// formed.  LDS: PTILE elements.
 template <typename T>
 __device__ __forceinline__ void potrf_blocked(const DevFactor<T>& F, const Front& f, int k0, bool invert_only,
                               T* lds, const int tid) {
@@ -763,37 +763,161 @@ __device__ __forceinline__ void potrf_blocked(const DevFactor<T>& F, const Front
         if (b + 1 < NBLK && c0 + PB < kb && !(invert_only && wave > b)) update(wave, b, b + 1);
         __syncthreads();
     }
-    // all of a thread's LDS reads first, then its stores
-    if (!invert_only) {
-        T v[NB / 4];
-#pragma unroll
-        for (int i = 0; i < NB / 4; ++i) {
-            const int c = cg + 4 * i;
-            v[i] = A[r + c * LDS] * (r > c ? sc[c] : (T)1);
-        }
-#pragma unroll
-        for (int i = 0; i < NB / 4; ++i) {
-            const int c = cg + 4 * i;
-            if (r < kb && c <= r) stc(blk + r + (int64_t)c * nj, v[i]);
-        }
-        if (!chol && tid < kb) stc(F.d + gc0 + tid, pv[tid]);
-    }
-    // W(r, c) = L^-T(c, r)
+    // W(r, c) = L^-T(c, r): the panel solves wait for it.  All of a thread's
+    // LDS reads first, then its stores.
     T* W = F.W + f.woff + k0;
-    {
-        T v[NB / 4];
+    T v[NB / 4];
 #pragma unroll
-        for (int i = 0; i < NB / 4; ++i) {
-            const int c = cg + 4 * i, bc = i / 4, br = r / PB;
-            const T* src = bc == br ? WD + bc * PB * LDP + (c & (PB - 1)) + (r & (PB - 1)) * LDP : A + c + r * LDS;
-            v[i] = *src;
-        }
-#pragma unroll
-        for (int i = 0; i < NB / 4; ++i) {
-            const int c = cg + 4 * i;
-            if (r < kb && c < kb) stc(W + r + (int64_t)c * f.nn, (c <= r) ? v[i] : (T)0);
-        }
+    for (int i = 0; i < NB / 4; ++i) {
+        const int c = cg + 4 * i, bc = i / 4, br = r / PB;
+        const T* src = bc == br ? WD + bc * PB * LDP + (c & (PB - 1)) + (r & (PB - 1)) * LDP : A + c + r * LDS;
+        v[i] = *src;
     }
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) {
+        const int c = cg + 4 * i;
+        if (r < kb && c < kb) stc(W + r + (int64_t)c * f.nn, (c <= r) ? v[i] : (T)0);
+    }
+    if (!invert_only && !chol && tid < kb) stc(F.d + gc0 + tid, pv[tid]);
+}
+
+// The factored tile, from LDS (as potrf_blocked leaves it) to the panel.
+template <typename T>
+__device__ __forceinline__ void store_diag(const DevFactor<T>& F, const Front& f, int k0, const T* lds, const int tid) {
+    const T* sc = lds + NB * LDS + (NB / PB) * PB * LDP;
+    const int nj = f.nn + f.na, kb = min(NB, f.nn - k0), r = tid & 63, cg = tid >> 6;
+    T* blk = F.panel + f.poff + k0 + (int64_t)k0 * nj;
+    T v[NB / 4];
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) {
+        const int c = cg + 4 * i;
+        v[i] = lds[r + c * LDS] * (r > c ? sc[c] : (T)1);
+    }
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) {
+        const int c = cg + 4 * i;
+        if (r < kb && c <= r) stc(blk + r + (int64_t)c * nj, v[i]);
+    }
+}
+
+// A 64 x 64 tile of C in the row-contiguous layout of memory: thread (r, g)
+// holds C(r, g + 4i).  The matrix cores' output registers hold 16 columns by
+// 4 rows per instruction, 32-byte pieces of 16 cache lines; read and written
+// like that a tile cost 2 us in loads and 3 us in stores, in this layout
+// about 1 us each.  Products therefore leave through LDS (Cs, leading
+// dimension LDS, complete on entry).
+template <typename T>
+__device__ __forceinline__ void fetch_c(const T* C, int64_t ldc_, int m, int n, T (&c)[NB / 4], const int tid) {
+    const int r = min(tid & 63, m - 1), g = tid >> 6;
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) c[i] = ldc(C + r + min(g + 4 * i, n - 1) * ldc_);
+}
+// C = c - Cs (sub) or Cs
+template <typename T, bool SUB>
+__device__ __forceinline__ void write_c(T* C, int64_t ldc_, int m, int n, bool lower, const T (&c)[NB / 4],
+                                        const T* Cs, const int tid) {
+    const int r = tid & 63, g = tid >> 6;
+    T x[NB / 4];
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) x[i] = Cs[r + (g + 4 * i) * LDS];
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) {
+        const int col = g + 4 * i;
+        if (r < m && col < n && (!lower || r >= col)) stc(C + r + col * ldc_, SUB ? c[i] - x[i] : x[i]);
+    }
+}
+
+// The two products that follow a diagonal tile on the critical chain, by the
+// workgroup that factored it (potrf_blocked has just returned: lds still
+// holds L, W' = L^-T and the pivots): the panel solve of the tile below,
+// L1 = A1 W' (/ D), and the update of the next diagonal tile,
+// C -= L1 (D) L1'.  t: the panel solve's product, u: the update's.  W' is
+// read from LDS (its zero blocks skipped), A1 goes straight from memory into
+// the matrix cores' operand registers, and L1 takes the diagonal tile's place
+// in LDS for the update.  The diagonal tile's own L leaves here, behind the
+// loads, since no task waits for it.  The caller has seen A1 and C final
+// through the previous block column.  LDS: PTILE + NB * LDS elements.
+template <typename T>
+__device__ __forceinline__ void chain_step(const DevFactor<T>& F, const Front& f, int k0, const GemmTask& t,
+                                           const GemmTask& u, T* lds, const int tid) {
+    typedef typename Mfma<T>::v4 v4;
+    constexpr int NBLK = NB / PB;
+    T* A = lds;
+    const T* WD = lds + NB * LDS;
+    const T* pv = WD + NBLK * PB * LDP + NB;
+    T* Cs = lds + PTILE;
+    const int lane = tid & 63, wave = tid >> 6, li = lane & 15, lk = lane >> 4;
+    const bool chol = F.diag == 0;
+    const int m = t.m, nj = t.lda;
+    T* A1 = F.panel + t.a_off;
+    T* C = F.panel + u.c_off;
+    // rows 16 wave + li of A1 (t.k = 64 columns)
+    T a[NB / 4], c[NB / 4];
+    {
+        const int row = min(PB * wave + li, m - 1);
+#pragma unroll
+        for (int s = 0; s < NB / 4; ++s) a[s] = ldc(A1 + row + (int64_t)(4 * s + lk) * nj);
+    }
+    fetch_c(C, nj, m, m, c, tid);
+    store_diag<T>(F, f, k0, lds, tid);
+    v4 acc[NBLK];
+#pragma unroll
+    for (int j = 0; j < NBLK; ++j) acc[j] = v4{0, 0, 0, 0};
+#pragma unroll
+    for (int kb = 0; kb < NBLK; ++kb)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int k = 4 * s + lk;
+#pragma unroll
+            for (int j = kb; j < NBLK; ++j) {
+                const T b = j == kb ? WD[j * PB * LDP + k + li * LDP] : A[(PB * kb + k) + (PB * j + li) * LDS];
+                acc[j] = Mfma<T>::op(a[4 * kb + s], b, acc[j]);
+            }
+        }
+    if (!chol)
+#pragma unroll
+        for (int j = 0; j < NBLK; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[j][v] /= pv[PB * j + li];
+    __syncthreads();  // every wavefront has read L and W'
+    // L1 (rows past m are zero) takes the tile's place
+#pragma unroll
+    for (int j = 0; j < NBLK; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int row = PB * wave + Mfma<T>::row(lk, v);
+            A[row + (PB * j + li) * LDS] = row < m ? acc[j][v] : (T)0;
+        }
+    __syncthreads();
+    write_c<T, false>(A1, nj, m, NB, false, c, A, tid);
+    // the ten 16 x 16 blocks (br, bc) of C's lower triangle: block q to
+    // wavefront q % 4 (blocks past the tenth repeat block 0 and are dropped)
+    const T *pa[3], *pb[3];
+    int dst[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const int e = wave + 4 * q;
+        int br = e < 1 ? 0 : e < 3 ? 1 : e < 6 ? 2 : 3;
+        int bc = e - br * (br + 1) / 2;
+        if (e >= 10) br = bc = 0;
+        pa[q] = A + PB * br + li + lk * LDS;
+        pb[q] = A + PB * bc + li + lk * LDS;
+        dst[q] = PB * br + (PB * bc + li) * LDS;
+        acc[q] = v4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int s = 0; s < NB / 4; ++s) {
+        const T sc = chol ? (T)1 : pv[4 * s + lk];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) acc[q] = Mfma<T>::op(pa[q][4 * s * LDS] * sc, pb[q][4 * s * LDS], acc[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+        if (wave + 4 * q < 10)  // uniform
+#pragma unroll
+            for (int v = 0; v < 4; ++v) Cs[dst[q] + Mfma<T>::row(lk, v)] = acc[q][v];
+    __syncthreads();
+    write_c<T, true>(C, nj, m, m, true, c, Cs, tid);
 }
 
 // Diagonal tile under GMW81 (chol_factor! GMW81 specialization,
@@ -916,6 +1040,7 @@ __global__ __launch_bounds__(256) void k_diag(DevPlan P, DevFactor<T> F, int t0,
     __shared__ T lds[PTILE];
     const DiagTask dt = P.diag[t0 + blockIdx.x];
     potrf_blocked<T>(F, P.fronts[dt.front], dt.k0, invert_only != 0, lds, (int)threadIdx.x);
+    if (!invert_only) store_diag<T>(F, P.fronts[dt.front], dt.k0, lds, (int)threadIdx.x);
 }
 
 template <typename T>
@@ -923,14 +1048,15 @@ __device__ __forceinline__ T* arr_base(const DevFactor<T>& F, int a) {
     return a == ARR_PANEL ? F.panel : (a == ARR_U ? F.U : F.W);
 }
 
-// One 64x64 output tile; wave w owns a 32x32 quarter as 2x2 blocks of 16x16
-// MFMA tiles (v_mfma_*_16x16x4: lane l holds A[l%16][l/16] and B[l/16][l%16];
-// the row of output register v is Mfma<T>::row).  The k-loop is software
-// pipelined: the next KC-chunk of A and B is loaded into registers while the
-// MFMAs consume the current chunk from LDS (As/Bs: KC x LDT each).  For
-// C -= A B' the C tile is fetched before the k-loop.
+// One 64x64 output tile C -= A diag(s) B'; wave w owns a 32x32 quarter as 2x2
+// blocks of 16x16 MFMA tiles (v_mfma_*_16x16x4: lane l holds A[l%16][l/16]
+// and B[l/16][l%16]; the row of output register v is Mfma<T>::row).  The
+// k-loop is software pipelined: the next KC-chunk of A and B is loaded into
+// registers while the MFMAs consume the current chunk from LDS (As/Bs: KC x
+// LDT each).  C is fetched before the k-loop; the product leaves through Cs
+// (64 x LDS).
 template <typename T>
-__device__ __forceinline__ void gemm_tile(const DevFactor<T>& F, const GemmTask& g, T* As, T* Bs, const int tid) {
+__device__ __forceinline__ void gemm_tile(const DevFactor<T>& F, const GemmTask& g, T* As, T* Bs, T* Cs, const int tid) {
     typedef typename Mfma<T>::v4 v4;
     constexpr int PER = KC * 64 / 256;  // elements of A (and of B) per thread and chunk
     const T* A = arr_base(F, g.arrA) + g.a_off;
@@ -939,21 +1065,9 @@ __device__ __forceinline__ void gemm_tile(const DevFactor<T>& F, const GemmTask&
     const int wave = tid >> 6, lane = tid & 63;
     const int wr = (wave & 1) * 32, wc = (wave >> 1) * 32;
     const int li = lane & 15, lk = lane >> 4;
-    const bool sub = g.mode == G_SUB;
-    const T* s = (F.diag != 0 && sub && g.s_col >= 0) ? F.d + g.s_col : nullptr;
-    T cv[2][2][4];
-    if (sub) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int row = wr + i * 16 + Mfma<T>::row(lk, v), col = wc + j * 16 + li;
-                    cv[i][j][v] = (row < g.m && col < g.n && (!g.lower || row >= col))
-                                      ? ldc(C + row + (int64_t)col * g.ldc) : (T)0;
-                }
-    }
+    const T* s = (F.diag != 0 && g.s_col >= 0) ? F.d + g.s_col : nullptr;
+    T cv[NB / 4];
+    fetch_c(C, g.ldc, g.m, g.n, cv, tid);
     v4 acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -998,34 +1112,79 @@ __device__ __forceinline__ void gemm_tile(const DevFactor<T>& F, const GemmTask&
         }
         __syncthreads();
     }
-    const bool scale = (g.mode == G_TRSM) && F.diag != 0;
-    // the LDLt pivots of this thread's two columns, loaded before the stores
-    // (unconditionally, column clamped) rather than one wait per element
-    T dcol[2] = {(T)1, (T)1};
-    if (scale)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) dcol[j] = ldc(F.d + g.s_col + min(wc + j * 16 + li, g.n - 1));
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+            for (int v = 0; v < 4; ++v)
+                Cs[(wr + i * 16 + Mfma<T>::row(lk, v)) + (wc + j * 16 + li) * LDS] = acc[i][j][v];
+    __syncthreads();
+    write_c<T, true>(C, g.ldc, g.m, g.n, g.lower != 0, cv, Cs, tid);
+}
+
+// 64 x 64 output tile with k <= 64 (every panel solve and the single-step
+// trailing updates of the critical chain).  Wave w owns the rows
+// [16w, 16w + 16): its A operand goes from memory straight into the matrix
+// cores' operand registers, B is staged whole in LDS (Bs: 64 x LDT), so the
+// tile costs one load round trip and one barrier.  The product is summed on
+// its own and subtracted from C once (FP32 accuracy).  All loads are unconditional from clamped addresses.
+// TRSM: B = W = L^-1 is lower triangular, the zero blocks are skipped.  Bound:
+// the load round trip from the other XCDs' writes plus 40 (panel solve) or 64
+// matrix-core operations of 64 cycles per wavefront; a full panel-solve tile
+// on an idle chip takes 5.3 us (10.4 in two 32-wide chunks), a
+// single-step update 6.2 us (7.4).
+template <typename T, bool TRSM>
+__device__ __forceinline__ void gemm_tile64(const DevFactor<T>& F, const GemmTask& g, T* Bs, T* Cs, const int tid) {
+    typedef typename Mfma<T>::v4 v4;
+    constexpr int NBLK = NB / PB;
+    const T* A = arr_base(F, g.arrA) + g.a_off;
+    const T* B = arr_base(F, g.arrB) + g.b_off;
+    T* C = arr_base(F, g.arrC) + g.c_off;
+    const int wave = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    const T* s = (!TRSM && F.diag != 0 && g.s_col >= 0) ? F.d + g.s_col : nullptr;
+    T b[NB / 4], a[NB / 4], cv[NB / 4];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int row = wr + i * 16 + Mfma<T>::row(lk, v);
-                const int col = wc + j * 16 + li;
-                if (row < g.m && col < g.n && (!g.lower || row >= col)) {
-                    T* cp = C + row + (int64_t)col * g.ldc;
-                    if (sub) {
-                        stc(cp, cv[i][j][v] - acc[i][j][v]);
-                    } else {
-                        T x = acc[i][j][v];
-                        if (scale) x /= dcol[j];
-                        stc(cp, x);
-                    }
-                }
-            }
-        }
+    for (int i = 0; i < NB / 4; ++i)
+        b[i] = ldc(B + min(lane, g.n - 1) + (int64_t)min(wave + 4 * i, g.k - 1) * g.ldb);
+    const int row = PB * wave + li;
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) a[i] = ldc(A + min(row, g.m - 1) + (int64_t)min(4 * i + lk, g.k - 1) * g.lda);
+    if constexpr (!TRSM) fetch_c(C, g.ldc, g.m, g.n, cv, tid);
+    if (s) {
+#pragma unroll
+        for (int i = 0; i < NB / 4; ++i) a[i] *= ldc(s + min(4 * i + lk, g.k - 1));
     }
+    // the LDLt pivots of this thread's columns
+    T dcol[NBLK];
+    if (TRSM && F.diag != 0)
+#pragma unroll
+        for (int j = 0; j < NBLK; ++j) dcol[j] = ldc(F.d + g.s_col + min(PB * j + li, g.n - 1));
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) {
+        const int k = wave + 4 * i;
+        Bs[k * LDT + lane] = (k < g.k && lane < g.n) ? b[i] : (T)0;
+        a[i] = 4 * i + lk < g.k ? a[i] : (T)0;
+    }
+    v4 acc[NBLK];
+#pragma unroll
+    for (int j = 0; j < NBLK; ++j) acc[j] = v4{0, 0, 0, 0};
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i)
+#pragma unroll
+        for (int j = TRSM ? i / 4 : 0; j < NBLK; ++j)
+            acc[j] = Mfma<T>::op(a[i], Bs[(4 * i + lk) * LDT + PB * j + li], acc[j]);
+#pragma unroll
+    for (int j = 0; j < NBLK; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            T x = acc[j][v];
+            if (TRSM && F.diag != 0) x /= dcol[j];
+            Cs[(PB * wave + Mfma<T>::row(lk, v)) + (PB * j + li) * LDS] = x;
+        }
+    __syncthreads();
+    write_c<T, !TRSM>(C, g.ldc, g.m, g.n, g.lower != 0, cv, Cs, tid);
 }
 
 constexpr int KW = 16;        // k-chunk of the wide tile
@@ -1039,7 +1198,7 @@ constexpr int LDW = 128 + 4;  // leading dimension of its LDS stages
 // and B through two LDS buffers (As/Bs: 2 x KW x LDW each): while the waves
 // multiply out of one buffer, the next chunk, prefetched into registers one
 // chunk ahead, is written to the other, so each chunk costs one barrier.  C
-// is updated after the k-loop in four row-block rounds.
+// is updated after the k-loop in four rounds of 32 columns.
 template <typename T>
 __device__ __forceinline__ void gemm_tile128(const DevFactor<T>& F, const GemmTask& g, T* As, T* Bs, const int tid) {
     typedef typename Mfma<T>::v4 v4;
@@ -1111,26 +1270,41 @@ __device__ __forceinline__ void gemm_tile128(const DevFactor<T>& F, const GemmTa
         if (more) stage(buf ^ 1);
         __syncthreads();
     }
-    if (idle) return;
+    // C in four rounds of 32 columns: the two wavefronts that own them put
+    // their products in LDS (Cs: 128 x 32, over the stages), then every thread
+    // updates row-contiguous pieces; the next round's C is fetched meanwhile
+    constexpr int LDC = 128 + 1, CPER = 128 * 32 / 256;
+    T* Cs = As;
+    T cv[CPER];
+    auto fetch_round = [&](int q) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        T cv[4][4];
+        for (int i = 0; i < CPER; ++i)
+            cv[i] = ldc(C + min(r, g.m - 1) + (int64_t)min(32 * q + kq + 2 * i, g.n - 1) * g.ldc);
+    };
+    fetch_round(0);
+    for (int q = 0; q < 4; ++q) {
+        if (32 * q >= g.n) break;  // uniform
+        if ((wave >> 1) == (q >> 1) && !idle) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < 4; ++j)
+                if ((j >> 1) == (q & 1))
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int row = wr + 16 * i + Mfma<T>::row(lk, v), col = wc + 16 * j + li;
-                cv[j][v] = (row < g.m && col < g.n && (!g.lower || row >= col))
-                               ? ldc(C + row + (int64_t)col * g.ldc) : (T)0;
-            }
+                    for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+                        for (int v = 0; v < 4; ++v)
+                            Cs[(wr + 16 * i + Mfma<T>::row(lk, v)) + (16 * (j & 1) + li) * LDC] = acc[i][j][v];
+        }
+        __syncthreads();
+        T x[CPER];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int row = wr + 16 * i + Mfma<T>::row(lk, v), col = wc + 16 * j + li;
-                if (row < g.m && col < g.n && (!g.lower || row >= col))
-                    stc(C + row + (int64_t)col * g.ldc, cv[j][v] - acc[i][j][v]);
-            }
+        for (int i = 0; i < CPER; ++i) x[i] = cv[i] - Cs[r + (kq + 2 * i) * LDC];
+        if (q < 3) fetch_round(q + 1);
+#pragma unroll
+        for (int i = 0; i < CPER; ++i) {
+            const int col = 32 * q + kq + 2 * i;
+            if (r < g.m && col < g.n && (!g.lower || r >= col)) stc(C + r + (int64_t)col * g.ldc, x[i]);
+        }
+        __syncthreads();
     }
 }
 
@@ -1235,8 +1409,9 @@ constexpr unsigned long long WMASK = WDEP == 64 ? ~0ull : (1ull << (WDEP & 63)) 
 // GMW: the GMW81 instance (diagonal tiles by potrf_gmw, block-column waits);
 // the other regularizations run the instance without it.
 template <typename T, bool GMW>
-__global__ __launch_bounds__(256, 2) void k_dag(DevPlan P, DevFactor<T> F, DevDag D) {
-    constexpr int S1 = PTILE, S2 = 2 * KC * LDT, S3 = 4 * KW * LDW;
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, DevFactor<T> F, DevDag D) {
+    constexpr int S1 = PTILE + NB * LDS, S2 = NB * LDT + NB * LDS, S3 = 4 * KW * LDW;
+    static_assert(2 * KC * LDT <= NB * LDT && 32 * 129 <= 4 * KW * LDW, "stages");
     constexpr int SMEM = S1 > S2 ? (S1 > S3 ? S1 : S3) : (S2 > S3 ? S2 : S3);
     static_assert(SMEM >= 2 * NB * LDS + NB + 6 * (int)(sizeof(double) / sizeof(T)), "potrf_gmw LDS");
     __shared__ __align__(16) T smem[SMEM];
@@ -1352,44 +1527,41 @@ __global__ __launch_bounds__(256, 2) void k_dag(DevPlan P, DevFactor<T> F, DevDa
             case DT_POTRF:
                 if constexpr (GMW) potrf_gmw<T>(F, P.fronts[J], d.a * NB, smem, tid);
                 else potrf_blocked<T>(F, P.fronts[J], d.a * NB, false, smem, tid);
-                if (d.b >= 0) {
+                if (d.b < 0) {
+                    if constexpr (!GMW) store_diag<T>(F, P.fronts[J], d.a * NB, smem, tid);
+                } else {
                     // publish the diagonal tile (the other panel solves of column a
-                    // need only it), then the fused panel solve of tile (a+1, a)
+                    // need only it), then the fused panel solve of tile (a+1, a) and
+                    // the update of the next diagonal tile, once both tiles are
+                    // updated through column a - 1: set by tasks with smaller tickets
+                    // (the planner checks), so the waits end
                     drain_stores();
                     __syncthreads();
                     if (tid == 0) {
                         __builtin_amdgcn_s_waitcnt(0);
                         __hip_atomic_store(cnt + d.a * g.R + d.a, d.a + 1, __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
-                        // tile (a+1, a) updated through column a - 1: set by a
-                        // task with a smaller ticket (the planner checks), so
-                        // the wait ends
                         (void)bounded_wait(cnt + d.a * g.R + d.a + 1, d.a, F.hang, F.ticket, F.stall, 1);
+                        (void)bounded_wait(cnt + (d.a + 1) * g.R + d.a + 1, d.a, F.hang, F.ticket, F.stall, 1);
                     }
                     __syncthreads();
-                    gemm_tile<T>(F, P.gemm[d.b], smem, smem + KC * LDT, tid);
-                    if (d.c >= 0) {
-                        // publish tile (a+1, a), then the fused look-ahead update of
-                        // the next diagonal tile, which reads it back
+                    if constexpr (GMW) {
+                        gemm_tile64<T, true>(F, P.gemm[d.b], smem, smem + NB * LDT, tid);
+                        // the update reads the panel solve's tile back from memory
                         drain_stores();
                         __syncthreads();
-                        if (tid == 0) {
-                            __builtin_amdgcn_s_waitcnt(0);
-                            __hip_atomic_store(cnt + d.a * g.R + d.a + 1, d.a + 1, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
-                            // tile (a+1, a+1) updated through column a - 1 (as above)
-                            (void)bounded_wait(cnt + (d.a + 1) * g.R + d.a + 1, d.a, F.hang, F.ticket,
-                                               F.stall, 1);
-                        }
-                        __syncthreads();
-                        gemm_tile<T>(F, P.gemm[d.c], smem, smem + KC * LDT, tid);
+                        gemm_tile64<T, false>(F, P.gemm[d.c], smem, smem + NB * LDT, tid);
+                    } else {
+                        chain_step<T>(F, P.fronts[J], d.a * NB, P.gemm[d.b], P.gemm[d.c], smem, tid);
                     }
                 }
                 break;
             default: {
                 const GemmTask gt = P.gemm[d.a];
                 if (gt.wide) gemm_tile128<T>(F, gt, smem, smem + 2 * KW * LDW, tid);
-                else gemm_tile<T>(F, gt, smem, smem + KC * LDT, tid);
+                else if (gt.mode == G_TRSM) gemm_tile64<T, true>(F, gt, smem, smem + NB * LDT, tid);
+                else if (gt.k <= NB) gemm_tile64<T, false>(F, gt, smem, smem + NB * LDT, tid);
+                else gemm_tile<T>(F, gt, smem, smem + KC * LDT, smem + NB * LDT, tid);
                 break;
             }
         }

@@ -71,6 +71,8 @@ struct Allocator {
     }
 };
 
+constexpr int32_t NEAR = 3;  // tile distance from the diagonal of the finer trailing updates
+
 inline int64_t rup(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 
 // The planner's stages.  Each stage reads what the earlier ones left in the
@@ -623,29 +625,39 @@ std::string Planner::factor_tasks() {
                 }
                 // trailing updates grouped by UPD_GROUP panel steps: tile
                 // (I, Jc) receives the columns [K0, K1) in one product once
-                // block column K1 - 1 is final.  The last step before Jc (the
-                // look-ahead column, which carries the next diagonal tile) is
-                // a product of its own, so the critical chain POTRF -> TRSM ->
-                // update -> POTRF runs a single-step update; the steps before
-                // it go in a partial group one step earlier.  Per step K:
-                //   pass 0: Jc = K + 1, columns [K, K + 1)
-                //   pass 1: Jc = K + 2, columns [K0, K + 1) (partial group)
-                //   pass 2: Jc >= K + 2, columns [K0, K + 1) (complete group)
-                const int32_t K0g = (K / UPD_GROUP) * UPD_GROUP;
-                const bool full = (K + 1) % UPD_GROUP == 0;
-                for (int pass = 0; pass < 3; ++pass)
+                // block column K1 - 1 is final.  The products of a tile end at
+                // the multiples of UPD_GROUP below Jc, then at Jc - 1 and Jc, so
+                // that the last step before Jc is a single-step product.  Tiles
+                // near the diagonal (I - Jc <= NEAR) carry the critical chain
+                // POTRF -> panel solve -> update -> POTRF: their last products
+                // end at Jc - 4, Jc - 2, Jc - 1 and Jc, since an eight-step
+                // product (28 us) takes longer than a panel step (with Jc - 1
+                // and Jc alone the chain waited for it: 33 us per step of the
+                // 31 x 29 x 27 grid's root front against 29).
+                const int32_t K1 = K + 1;
+                auto ends_at = [&](int32_t I, int32_t Jc, int32_t e) {
+                    if (e == Jc || e == Jc - 1 || e % UPD_GROUP == 0) return true;
+                    return I - Jc <= NEAR && (e == Jc - 2 || e == Jc - 4);
+                };
+                for (int pass = 0; pass < 2; ++pass)
                     for (int32_t J : L.big_list) {
                         const Front& F = P.fronts[J];
                         const DagFront& D = P.dagf[J];
                         if (K >= D.p) continue;
-                        if (pass == 1 && full) continue;   // a complete group: pass 2
-                        if (pass == 2 && !full) continue;  // group not complete yet
-                        const int32_t K1 = K + 1, K0 = pass == 0 ? K : K0g;
-                        const int32_t nj = F.nn + F.na, k0 = K0 * NB, kk = (K1 - K0) * NB;
+                        const int32_t nj = F.nn + F.na;
+                        // pass 0: the next block column; pass 1: the later ones
                         const int32_t jc0 = pass == 0 ? K + 1 : K + 2;
-                        const int32_t jc1 = pass == 2 ? D.p : std::min(jc0 + 1, D.p);
+                        const bool full = K1 % UPD_GROUP == 0;
+                        const int32_t jc1 = pass == 0 ? std::min(K + 2, D.p) : full ? D.p : std::min(K + 6, D.p);
                         for (int32_t Jc = jc0; Jc < jc1; ++Jc)
                             for (int32_t I = Jc; I < D.R; ++I) {
+                                if (!ends_at(I, Jc, K1)) {
+                                    if (I - Jc > NEAR) break;
+                                    continue;
+                                }
+                                int32_t K0 = K;
+                                while (K0 > 0 && !ends_at(I, Jc, K0)) --K0;
+                                const int32_t k0 = K0 * NB, kk = (K1 - K0) * NB;
                                 if (FUSE && pass == 0 && I == Jc && Jc == K + 1 && Jc < D.p)
                                     P.dag[potrf_at[J]].c = (int32_t)P.gemm.size();
                                 else
@@ -1365,12 +1377,8 @@ std::string Planner::schedule() {
                 }
                 case DT_SMALL: c += 20.0; break;
                 case DT_POTRF:
-                    c += 26.0;
-                    for (int32_t gi : {d.b, d.c})
-                        if (gi >= 0) {
-                            const GemmTask& g = P.gemm[gi];
-                            c += 2.0 * g.m * g.n * (double)g.k / 7.5e4;
-                        }
+                    c += 9.0;
+                    if (d.b >= 0) c += 6.0;  // the fused panel solve and update
                     break;
                 default: {
                     const GemmTask& g = P.gemm[d.a];
