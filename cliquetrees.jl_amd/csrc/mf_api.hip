@@ -646,7 +646,8 @@ static std::vector<std::pair<void**, size_t>> factor_buffers(mf_factor* f, const
                                                             bool refs) {
     const size_t nf = H.fronts.size() + 1, n1 = (size_t)(H.n + 1);
     std::vector<std::pair<void**, size_t>> v = {
-        {&f->panel, es * (size_t)H.panel_elems}, {&f->U, es * (size_t)H.u_elems},
+        {&f->panel, es * (size_t)(H.panel_elems + 2 * NB)}, {&f->U,  // (the long products read past the last tile)
+        es * (size_t)H.u_elems},
         {&f->W, es * (size_t)H.w_elems},         {&f->d, es * n1}};
     if (refs) {
         v.push_back({(void**)&f->Dref, 8 * (size_t)H.ndz});

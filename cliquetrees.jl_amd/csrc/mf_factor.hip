@@ -95,8 +95,8 @@ __device__ __forceinline__ void stc(T* p, T v) {
 }
 
 constexpr int LDS = SMALL_NJ + 1;  // leading dimension of LDS fronts and tiles
-constexpr int KC = 32;             // k-chunk of the GEMM tile
-constexpr int LDT = 64 + 4;        // leading dimension of the GEMM LDS stages
+constexpr int LDT = 64 + 4;        // leading dimension of the 64-wide tile's LDS operand
+constexpr int GEMM_LDS = 4 * 16 * 128;  // two stages of two operands of a long product
 
 // Right-looking partial factorization of the first nn columns of the
 // nj x nj front M (lower triangle, leading dimension LDS) in LDS.
@@ -1048,79 +1048,150 @@ __device__ __forceinline__ T* arr_base(const DevFactor<T>& F, int a) {
     return a == ARR_PANEL ? F.panel : (a == ARR_U ? F.U : F.W);
 }
 
-// One 64x64 output tile C -= A diag(s) B'; wave w owns a 32x32 quarter as 2x2
-// blocks of 16x16 MFMA tiles (v_mfma_*_16x16x4: lane l holds A[l%16][l/16]
-// and B[l/16][l%16]; the row of output register v is Mfma<T>::row).  The
-// k-loop is software pipelined: the next KC-chunk of A and B is loaded into
-// registers while the MFMAs consume the current chunk from LDS (As/Bs: KC x
-// LDT each).  C is fetched before the k-loop; the product leaves through Cs
-// (64 x LDS).
-template <typename T>
-__device__ __forceinline__ void gemm_tile(const DevFactor<T>& F, const GemmTask& g, T* As, T* Bs, T* Cs, const int tid) {
+// Sixteen bytes per lane from memory straight into LDS (lds: the wavefront's
+// first lane's place, the lanes follow contiguously), device-coherent like
+// ldc.  Only the global address's dword alignment is needed, so any row
+// offset and leading dimension will do.
+__device__ __forceinline__ void load_lds16(const void* g, void* lds) {
+    typedef __attribute__((address_space(1))) const void gptr;
+    typedef __attribute__((address_space(3))) void lptr;
+    constexpr int SC1 = 16;  // device scope
+    __builtin_amdgcn_global_load_lds((gptr*)g, (lptr*)lds, 16, 0, SC1);
+}
+
+// E x E output tile C -= A diag(s) B' (lower part only on the diagonal): the
+// update-matrix tiles (E = 128 for long k) and the multi-step trailing
+// updates (E = 64).  Wave w owns the (E/2) x (E/2) quarter (w & 1, w >> 1) as
+// MFMA blocks (v_mfma_*_16x16x4: lane l holds A[l%16][l/16] and
+// B[l/16][l%16]; the row of output register v is Mfma<T>::row); the strictly
+// upper quarter of a diagonal tile does no MFMA work.  The k-loop runs on two
+// LDS stages of KW columns of A and B (leading dimension E, no padding: every
+// load instruction writes whole 128-byte lines): while the waves multiply out
+// of one stage, the next chunk goes from memory straight into the other
+// (load_lds16), one barrier per chunk.  Rows past the tile are loaded too
+// (the panel pool has 2 NB elements of slack behind its end) and only reach
+// rows and columns of C that are not stored.  C leaves through LDS in rounds
+// (fetch_c's reason).  Bound: the matrix cores, which reach 75 TFLOP/s from
+// LDS alone; FP64, 1,176 tiles of 128 x 128 x 512 on 512 workgroups: 52.7
+// TFLOP/s (34.9 with the chunks staged through registers), 4,656 tiles of
+// 64 x 64 x 512: 45.8 (39.4).
+template <typename T, int E>
+__device__ __forceinline__ void gemm_tile(const DevFactor<T>& F, const GemmTask& g, T* S, const int tid) {
     typedef typename Mfma<T>::v4 v4;
-    constexpr int PER = KC * 64 / 256;  // elements of A (and of B) per thread and chunk
+    constexpr int KW = E == 128 ? 16 : 32;           // columns per stage
+    constexpr int EPL = 16 / (int)sizeof(T);         // elements per lane and load
+    constexpr int LPC = E / EPL, CPI = 64 / LPC;     // lanes per column, columns per load
+    constexpr int ST = KW * E, M = E / 32, Q = E / 2;
+    static_assert(4 * ST <= GEMM_LDS, "stages");
     const T* A = arr_base(F, g.arrA) + g.a_off;
     const T* B = arr_base(F, g.arrB) + g.b_off;
     T* C = arr_base(F, g.arrC) + g.c_off;
-    const int wave = tid >> 6, lane = tid & 63;
-    const int wr = (wave & 1) * 32, wc = (wave >> 1) * 32;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = (wave & 1) * Q, wc = (wave >> 1) * Q;
     const int li = lane & 15, lk = lane >> 4;
+    const bool idle = g.lower && wc > wr;  // strictly above the diagonal
     const T* s = (F.diag != 0 && g.s_col >= 0) ? F.d + g.s_col : nullptr;
-    T cv[NB / 4];
-    fetch_c(C, g.ldc, g.m, g.n, cv, tid);
-    v4 acc[2][2];
+    v4 acc[M][M];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < M; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = v4{0, 0, 0, 0};
-    T ra[PER], rb[PER], rs[PER];
-    const int r = tid & 63, kq = tid >> 6;  // element (r, kq + 4i) of each chunk
-    auto fetch = [&](int k0) {
+        for (int j = 0; j < M; ++j) acc[i][j] = v4{0, 0, 0, 0};
+    T sv[KW / 4];  // the LDLt pivots of the chunk in flight
+    auto load = [&](int k0, T* st) {
+        if (k0 + KW <= g.k) {
+            const T* a = A + EPL * (lane % LPC) + (int64_t)(k0 + lane / LPC) * g.lda;
+            const T* b = B + EPL * (lane % LPC) + (int64_t)(k0 + lane / LPC) * g.ldb;
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int gk = k0 + kq + 4 * i;
-            T av = (T)0, bv = (T)0, sv = (T)1;
-            if (gk < g.k) {
-                if (r < g.m) av = ldc(A + r + (int64_t)gk * g.lda);
-                if (s) sv = ldc(s + gk);  // applied when staged: no wait here
-                if (r < g.n) bv = ldc(B + r + (int64_t)gk * g.ldb);
+            for (int i = 0; i < KW / CPI / 4; ++i) {
+                const int k = (wave + 4 * i) * CPI;
+                load_lds16(a + (int64_t)k * g.lda, st + k * E);
+                load_lds16(b + (int64_t)k * g.ldb, st + ST + k * E);
             }
-            ra[i] = av;
-            rb[i] = bv;
-            rs[i] = sv;
+        } else {
+            // the last, shorter chunk: its missing columns are zero
+            for (int e = tid; e < ST; e += 256) {
+                const int r = e % E, k = k0 + e / E;
+                const T x = ldc(A + min(r, g.m - 1) + (int64_t)min(k, g.k - 1) * g.lda);
+                const T y = ldc(B + min(r, g.n - 1) + (int64_t)min(k, g.k - 1) * g.ldb);
+                st[e] = k < g.k ? x : (T)0;
+                st[ST + e] = k < g.k ? y : (T)0;
+            }
         }
-    };
-    fetch(0);
-    for (int k0 = 0; k0 < g.k; k0 += KC) {
+        if (s)
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            As[(kq + 4 * i) * LDT + r] = s ? ra[i] * rs[i] : ra[i];
-            Bs[(kq + 4 * i) * LDT + r] = rb[i];
+            for (int i = 0; i < KW / 4; ++i) sv[i] = ldc(s + min(k0 + 4 * i + lk, g.k - 1));
+    };
+    load(0, S);
+    int buf = 0;
+    for (int k0 = 0; k0 < g.k; k0 += KW, buf ^= 1) {
+        // the chunk has arrived (each wave waits for its own loads, then the
+        // barrier) and the other stage is no longer read
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        T cs[KW / 4];
+        if (s)
+#pragma unroll
+            for (int i = 0; i < KW / 4; ++i) cs[i] = sv[i];
+        if (k0 + KW < g.k) load(k0 + KW, S + (buf ^ 1) * 2 * ST);
+        if (!idle) {
+            const T* a0 = S + buf * 2 * ST;
+            const T* b0 = a0 + ST;
+#pragma unroll
+            for (int kk = 0; kk < KW; kk += 4) {
+                T a[M], b[M];
+#pragma unroll
+                for (int i = 0; i < M; ++i) {
+                    a[i] = a0[(kk + lk) * E + wr + 16 * i + li];
+                    b[i] = b0[(kk + lk) * E + wc + 16 * i + li];
+                }
+                if (s)
+#pragma unroll
+                    for (int i = 0; i < M; ++i) a[i] *= cs[kk / 4];
+#pragma unroll
+                for (int i = 0; i < M; ++i)
+#pragma unroll
+                    for (int j = 0; j < M; ++j) acc[i][j] = Mfma<T>::op(a[i], b[j], acc[i][j]);
+            }
+        }
+    }
+    __syncthreads();  // every wave is done with the stages
+    // C in rounds of NC columns: the wavefronts that own them put their
+    // products in LDS (Cs: E x NC, over the stages), then every thread updates
+    // row-contiguous pieces; the next round's C is fetched meanwhile
+    constexpr int NC = 32, LDC = E + 1, CPER = E * NC / 256, CS = 256 / E;
+    T* Cs = S;
+    const int r = tid % E, kq = tid / E;
+    T cv[CPER];
+    auto fetch_round = [&](int q) {
+#pragma unroll
+        for (int i = 0; i < CPER; ++i)
+            cv[i] = ldc(C + min(r, g.m - 1) + (int64_t)min(NC * q + kq + CS * i, g.n - 1) * g.ldc);
+    };
+    fetch_round(0);
+#pragma unroll
+    for (int q = 0; q < E / NC; ++q) {
+        if (NC * q >= g.n) break;  // uniform
+        if (NC * q / Q == wave >> 1 && !idle) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int i = 0; i < M; ++i)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        Cs[(wr + 16 * i + Mfma<T>::row(lk, v)) + (16 * j + li) * LDC] = acc[i][(2 * q + j) % M][v];
         }
         __syncthreads();
-        if (k0 + KC < g.k) fetch(k0 + KC);
+        T x[CPER];
 #pragma unroll
-        for (int kk = 0; kk < KC; kk += 4) {
-            const T a0 = As[(kk + lk) * LDT + wr + li];
-            const T a1 = As[(kk + lk) * LDT + wr + 16 + li];
-            const T b0 = Bs[(kk + lk) * LDT + wc + li];
-            const T b1 = Bs[(kk + lk) * LDT + wc + 16 + li];
-            acc[0][0] = Mfma<T>::op(a0, b0, acc[0][0]);
-            acc[0][1] = Mfma<T>::op(a0, b1, acc[0][1]);
-            acc[1][0] = Mfma<T>::op(a1, b0, acc[1][0]);
-            acc[1][1] = Mfma<T>::op(a1, b1, acc[1][1]);
+        for (int i = 0; i < CPER; ++i) x[i] = cv[i] - Cs[r + (kq + CS * i) * LDC];
+        if (q + 1 < E / NC) fetch_round(q + 1);
+#pragma unroll
+        for (int i = 0; i < CPER; ++i) {
+            const int col = NC * q + kq + CS * i;
+            if (r < g.m && col < g.n && (!g.lower || r >= col)) stc(C + r + (int64_t)col * g.ldc, x[i]);
         }
         __syncthreads();
     }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-                Cs[(wr + i * 16 + Mfma<T>::row(lk, v)) + (wc + j * 16 + li) * LDS] = acc[i][j][v];
-    __syncthreads();
-    write_c<T, true>(C, g.ldc, g.m, g.n, g.lower != 0, cv, Cs, tid);
 }
 
 // 64 x 64 output tile with k <= 64 (every panel solve and the single-step
@@ -1185,127 +1256,6 @@ __device__ __forceinline__ void gemm_tile64(const DevFactor<T>& F, const GemmTas
         }
     __syncthreads();
     write_c<T, !TRSM>(C, g.ldc, g.m, g.n, g.lower != 0, cv, Cs, tid);
-}
-
-constexpr int KW = 16;        // k-chunk of the wide tile
-constexpr int LDW = 128 + 4;  // leading dimension of its LDS stages
-
-// 128 x 128 update-matrix tile, C -= A diag(s) B' (lower part only on the
-// diagonal): twice the flops per byte of the 64 x 64 tile, for the long-k
-// update matrices that carry most of the flops.  Wave w owns the 64 x 64
-// quarter (w & 1, w >> 1) as 4 x 4 MFMA blocks (the strictly upper quarter
-// of a diagonal tile does no MFMA work).  The k-loop stages KW columns of A
-// and B through two LDS buffers (As/Bs: 2 x KW x LDW each): while the waves
-// multiply out of one buffer, the next chunk, prefetched into registers one
-// chunk ahead, is written to the other, so each chunk costs one barrier.  C
-// is updated after the k-loop in four rounds of 32 columns.
-template <typename T>
-__device__ __forceinline__ void gemm_tile128(const DevFactor<T>& F, const GemmTask& g, T* As, T* Bs, const int tid) {
-    typedef typename Mfma<T>::v4 v4;
-    constexpr int PER = KW * 128 / 256;
-    const T* A = arr_base(F, g.arrA) + g.a_off;
-    const T* B = arr_base(F, g.arrB) + g.b_off;
-    T* C = arr_base(F, g.arrC) + g.c_off;
-    const int wave = tid >> 6, lane = tid & 63;
-    const int wr = (wave & 1) * 64, wc = (wave >> 1) * 64;
-    const int li = lane & 15, lk = lane >> 4;
-    const bool idle = g.lower && wc > wr;  // strictly above the diagonal
-    const T* s = (F.diag != 0 && g.s_col >= 0) ? F.d + g.s_col : nullptr;
-    v4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = v4{0, 0, 0, 0};
-    T ra[PER], rb[PER], rs[PER];
-    const int r = tid & 127, kq = tid >> 7;  // element (r, kq + 2i) of each chunk
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int gk = k0 + kq + 2 * i;
-            T av = (T)0, bv = (T)0, sv = (T)1;
-            if (gk < g.k) {
-                if (r < g.m) av = ldc(A + r + (int64_t)gk * g.lda);
-                if (s) sv = ldc(s + gk);  // applied when staged: no wait here
-                if (r < g.n) bv = ldc(B + r + (int64_t)gk * g.ldb);
-            }
-            ra[i] = av;
-            rb[i] = bv;
-            rs[i] = sv;
-        }
-    };
-    auto stage = [&](int buf) {
-        T* a = As + buf * KW * LDW;
-        T* b = Bs + buf * KW * LDW;
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            a[(kq + 2 * i) * LDW + r] = s ? ra[i] * rs[i] : ra[i];
-            b[(kq + 2 * i) * LDW + r] = rb[i];
-        }
-    };
-    fetch(0);
-    stage(0);
-    __syncthreads();
-    int buf = 0;
-    for (int k0 = 0; k0 < g.k; k0 += KW, buf ^= 1) {
-        const bool more = k0 + KW < g.k;
-        if (more) fetch(k0 + KW);
-        if (!idle) {
-            const T* a0 = As + buf * KW * LDW;
-            const T* b0 = Bs + buf * KW * LDW;
-#pragma unroll
-            for (int kk = 0; kk < KW; kk += 4) {
-                T a[4], b[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    a[i] = a0[(kk + lk) * LDW + wr + 16 * i + li];
-                    b[i] = b0[(kk + lk) * LDW + wc + 16 * i + li];
-                }
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[i][j] = Mfma<T>::op(a[i], b[j], acc[i][j]);
-            }
-        }
-        // the other buffer was last read in the previous chunk, before its barrier
-        if (more) stage(buf ^ 1);
-        __syncthreads();
-    }
-    // C in four rounds of 32 columns: the two wavefronts that own them put
-    // their products in LDS (Cs: 128 x 32, over the stages), then every thread
-    // updates row-contiguous pieces; the next round's C is fetched meanwhile
-    constexpr int LDC = 128 + 1, CPER = 128 * 32 / 256;
-    T* Cs = As;
-    T cv[CPER];
-    auto fetch_round = [&](int q) {
-#pragma unroll
-        for (int i = 0; i < CPER; ++i)
-            cv[i] = ldc(C + min(r, g.m - 1) + (int64_t)min(32 * q + kq + 2 * i, g.n - 1) * g.ldc);
-    };
-    fetch_round(0);
-    for (int q = 0; q < 4; ++q) {
-        if (32 * q >= g.n) break;  // uniform
-        if ((wave >> 1) == (q >> 1) && !idle) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if ((j >> 1) == (q & 1))
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v)
-                            Cs[(wr + 16 * i + Mfma<T>::row(lk, v)) + (16 * (j & 1) + li) * LDC] = acc[i][j][v];
-        }
-        __syncthreads();
-        T x[CPER];
-#pragma unroll
-        for (int i = 0; i < CPER; ++i) x[i] = cv[i] - Cs[r + (kq + 2 * i) * LDC];
-        if (q < 3) fetch_round(q + 1);
-#pragma unroll
-        for (int i = 0; i < CPER; ++i) {
-            const int col = 32 * q + kq + 2 * i;
-            if (r < g.m && col < g.n && (!g.lower || r >= col)) stc(C + r + (int64_t)col * g.ldc, x[i]);
-        }
-        __syncthreads();
-    }
 }
 
 // Dependency q of DAG task d: the counter w that must reach target.  Returns
@@ -1410,9 +1360,9 @@ constexpr unsigned long long WMASK = WDEP == 64 ? ~0ull : (1ull << (WDEP & 63)) 
 // the other regularizations run the instance without it.
 template <typename T, bool GMW>
 __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, DevFactor<T> F, DevDag D) {
-    constexpr int S1 = PTILE + NB * LDS, S2 = NB * LDT + NB * LDS, S3 = 4 * KW * LDW;
-    static_assert(2 * KC * LDT <= NB * LDT && 32 * 129 <= 4 * KW * LDW, "stages");
+    constexpr int S1 = PTILE + NB * LDS, S2 = NB * LDT + NB * LDS, S3 = GEMM_LDS;
     constexpr int SMEM = S1 > S2 ? (S1 > S3 ? S1 : S3) : (S2 > S3 ? S2 : S3);
+    static_assert(4 * EA_WIN <= SMEM && SMALL_NJ * LDS <= SMEM && 32 * 129 <= SMEM, "LDS");
     static_assert(SMEM >= 2 * NB * LDS + NB + 6 * (int)(sizeof(double) / sizeof(T)), "potrf_gmw LDS");
     __shared__ __align__(16) T smem[SMEM];
     __shared__ T s_piv, s_inv;
@@ -1558,10 +1508,10 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
                 break;
             default: {
                 const GemmTask gt = P.gemm[d.a];
-                if (gt.wide) gemm_tile128<T>(F, gt, smem, smem + 2 * KW * LDW, tid);
+                if (gt.wide) gemm_tile<T, 128>(F, gt, smem, tid);
                 else if (gt.mode == G_TRSM) gemm_tile64<T, true>(F, gt, smem, smem + NB * LDT, tid);
                 else if (gt.k <= NB) gemm_tile64<T, false>(F, gt, smem, smem + NB * LDT, tid);
-                else gemm_tile<T>(F, gt, smem, smem + KC * LDT, smem + NB * LDT, tid);
+                else gemm_tile<T, 64>(F, gt, smem, tid);
                 break;
             }
         }
