@@ -96,6 +96,7 @@ struct mf_plan {
     DagFront* d_dagf = nullptr;
     int32_t* d_uwait_ptr = nullptr;
     int32_t* d_uwait = nullptr;
+    int32_t* d_cnt0 = nullptr;     // initial tile counters
     double ea_bytes = 0, small_flops = 0, diag_flops = 0;
     // reference flops (sum nn^3/3 + na nn^2 + na^2 nn over the reference's own
     // fronts) of the fronts each launch factors: the small region, the DAG
@@ -138,7 +139,7 @@ struct mf_factor {
     int32_t* hang = nullptr;
     double* gmw = nullptr;      // GMW81: reduction scratch, then beta (gmw[2])
     int32_t* cnt = nullptr;     // tile-DAG counters
-    int32_t* eacnt = nullptr;   // 2 (fronts + 1): all extend-add tasks, then panel ones
+    int32_t* eacnt = nullptr;   // finished extend-add tasks per front
     unsigned long long* prof = nullptr;  // task-kind profile of the tile-DAG (NULL: off)
     // FP64 matrix of the refinement residual (full symmetric CSC, original order)
     int64_t A_n = -1, A_nnz = 0;
@@ -378,12 +379,11 @@ void enqueue_factor(mf_factor* f) {
         launch_small<T>(P, F, P.small_order, P.small_units, (int)H.small_units.size(), s);
     });
     if (!H.dag.empty()) {
-        launch_fill<int32_t>(f->cnt, H.dag_counters, 0, s);
-        const size_t nfr1 = H.fronts.size() + 1;
-        launch_fill<int32_t>(f->eacnt, 2 * nfr1, 0, s);
+        launch_copy_i32(pl->d_cnt0, f->cnt, H.dag_counters, s);
+        launch_fill<int32_t>(f->eacnt, (int64_t)H.fronts.size() + 1, 0, s);
         launch_fill<uint32_t>(f->ticket, 1, 0u, s);
         // GMW81: the ticket order where a diagonal tile follows every update of its block column
-        DevDag D{f->reg_kind == MF_REG_GMW81 ? pl->d_dag_gmw : pl->d_dag, pl->d_dagf, pl->d_uwait_ptr, pl->d_uwait, f->cnt, f->eacnt, f->eacnt + nfr1,
+        DevDag D{f->reg_kind == MF_REG_GMW81 ? pl->d_dag_gmw : pl->d_dag, pl->d_dagf, pl->d_uwait_ptr, pl->d_uwait, f->cnt, f->eacnt,
                  f->prof, f->prof ? f->trace_buf : nullptr,
                  (int32_t)H.dag.size(), H.tune.prio, H.tune.wg_per_cu};
         timed(f, MF_KC_DAG, pl->ref_flops_dag, 1, [&] { launch_dag<T>(P, F, D, s); });
@@ -448,7 +448,7 @@ std::string hang_message(const mf_factor* f, const int32_t* h) {
     } bufs[] = {{"front flag/done", f->flags, nf1},
                 {"solve progress", f->prog, nf1},
                 {"tile counter", f->cnt, (size_t)H.dag_counters + 1},
-                {"extend-add counter", f->eacnt, 2 * nf1}};
+                {"extend-add counter", f->eacnt, nf1}};
     std::string where = "an unknown counter";
     for (const Buf& b : bufs) {
         const unsigned long long b0 = (unsigned long long)b.base;
@@ -500,36 +500,7 @@ static int plan_create(int64_t n, int64_t nfr, const int64_t* resptr, const int6
     for (int64_t j = 0; j < H.nfr; ++j)
         for (int64_t g = H.resptr[j]; g < H.resptr[j + 1]; ++g) pl->col2ref[g] = (int32_t)j;
     for (int32_t J : H.small_order) pl->in_small[J] = 1;
-    std::vector<int32_t> ea_src = H.ea_src;
-    std::vector<EaDst> ea_dst(H.ea.size());
-    for (size_t e = 0; e < H.ea.size(); ++e) {
-        const Front& F = H.fronts[H.ea[e].front];
-        const int32_t pc = H.ea[e].col;
-        const bool to_u = pc >= F.nn;
-        ea_dst[e].off = to_u ? F.uoff + (int64_t)(pc - F.nn) * F.na - F.nn
-                             : F.poff + (int64_t)pc * (F.nn + F.na);
-        ea_dst[e].to_u = to_u ? 1 : 0;
-        ea_dst[e].pad = 0;
-    }
-    std::vector<EaSrc> ea_srcx(H.ea_src.size() / 2);
-    for (const EaTask& e : H.ea) {
-        const int32_t w = e.row0 / EA_WIN;
-        for (int32_t q = e.src0; q < e.src1; ++q) {
-            const int32_t K = H.ea_src[2 * q], tcol = H.ea_src[2 * q + 1];
-            const Front& Kf = H.fronts[K];
-            EaSrc& x = ea_srcx[q];
-            x.u_off = Kf.uoff + (int64_t)tcol * Kf.na;
-            x.rel_off = Kf.reloff;
-            x.ws_off = H.wsoff[K];
-            x.tcol = tcol;
-            x.i0 = std::max(H.wstart[H.wsoff[K] + w], tcol);
-            x.i1 = H.wstart[H.wsoff[K] + w + 1];
-            x.pad = 0;
-        }
-    }
     if ((rc = upload(H.fronts, (Front**)&D.fronts, pl->allocs)) ||
-        (rc = upload(ea_dst, (EaDst**)&D.ea_dst, pl->allocs)) ||
-        (rc = upload(ea_srcx, (EaSrc**)&D.ea_srcx, pl->allocs)) ||
         (rc = upload(H.rows, (int32_t**)&D.rows, pl->allocs)) ||
         (rc = upload(H.chd, (int32_t**)&D.chd, pl->allocs)) ||
         (rc = upload(H.rel, (int32_t**)&D.rel, pl->allocs)) ||
@@ -538,9 +509,8 @@ static int plan_create(int64_t n, int64_t nfr, const int64_t* resptr, const int6
         (rc = upload(H.level_small, (int32_t**)&D.level_small, pl->allocs)) ||
         (rc = upload(H.level_big, (int32_t**)&D.level_big, pl->allocs)) ||
         (rc = upload(H.ea, (EaTask**)&D.ea, pl->allocs)) ||
-        (rc = upload(ea_src, (int32_t**)&D.ea_src, pl->allocs)) ||
-        (rc = upload(H.wstart, (int32_t**)&D.wstart, pl->allocs)) ||
-        (rc = upload(H.wsoff, (int32_t**)&D.wsoff, pl->allocs)) ||
+        (rc = upload(H.ea_src, (EaSrc**)&D.ea_src, pl->allocs)) ||
+        (rc = upload(H.cnt0, &pl->d_cnt0, pl->allocs)) ||
         (rc = upload(H.sgstart, (int32_t**)&D.sgstart, pl->allocs)) ||
         (rc = upload(H.sgoff, (int32_t**)&D.sgoff, pl->allocs)) ||
         (rc = upload(H.gemm, (GemmTask**)&D.gemm, pl->allocs)) ||
@@ -657,7 +627,7 @@ static std::vector<std::pair<void**, size_t>> factor_buffers(mf_factor* f, const
         {(void**)&f->dref, 8 * n1},   {(void**)&f->adiag, 8 * n1},  {(void**)&f->signs, 8 * n1},
         {(void**)&f->info, 64},       {(void**)&f->flags, 4 * nf},  {(void**)&f->prog, 4 * nf},
         {(void**)&f->ticket, 64},     {(void**)&f->hang, 64},       {(void**)&f->gmw, 64},
-        {(void**)&f->cnt, 4 * (size_t)(H.dag_counters + 1)},        {(void**)&f->eacnt, 8 * nf},
+        {(void**)&f->cnt, 4 * (size_t)(H.dag_counters + 1)},        {(void**)&f->eacnt, 4 * nf},
         {(void**)&f->perm_dev, 8 * n1}};
     v.insert(v.end(), std::begin(rest), std::end(rest));
     return v;

@@ -8,8 +8,8 @@
 //               the children's completion flags (bounded wait).
 //               Reference: chol_loop_snd!/nod! cholesky.jl:434-692,
 //               chol_send! cholesky.jl:950-983, potrf2! blas/potrf.jl:3-41.
-//   k_dag       persistent tile-DAG over all big fronts: extend-add column
-//               groups (F11/F21 += F, cholesky.jl:520-521; M22 <- F22,
+//   k_dag       persistent tile-DAG over all big fronts: extend-add
+//               tiles (F11/F21 += F, cholesky.jl:520-521; M22 <- F22,
 //               cholesky.jl:542), small fronts above the small region,
 //               diagonal-tile factor + inverse (potrf2!), panel solve tiles
 //               (trsm!, blas/trsx.jl:156-159, as a product with the inverted
@@ -97,6 +97,32 @@ __device__ __forceinline__ void stc(T* p, T v) {
 constexpr int LDS = SMALL_NJ + 1;  // leading dimension of LDS fronts and tiles
 constexpr int LDT = 64 + 4;        // leading dimension of the 64-wide tile's LDS operand
 constexpr int GEMM_LDS = 4 * 16 * 128;  // two stages of two operands of a long product
+
+// A plan record that every lane of the workgroup has loaded from the same
+// place, into scalar registers: sizes, strides and offsets then cost no vector
+// registers or vector arithmetic.
+template <typename S>
+__device__ __forceinline__ S uniform(const S& v) {
+    static_assert(sizeof(S) % 4 == 0, "whole words");
+    struct Words {
+        int w[sizeof(S) / 4];
+    };
+    Words x = __builtin_bit_cast(Words, v);
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(S) / 4); ++i) x.w[i] = __builtin_amdgcn_readfirstlane(x.w[i]);
+    return __builtin_bit_cast(S, x);
+}
+
+// Computes v here, before the stores that follow.  A store under a per-lane
+// predicate is a branch; arithmetic left to that branch waits there for its
+// operands' loads, and on this hardware that wait covers the stores already
+// issued, so a run of predicated stores would take one memory round trip each
+// (660 cycles per store in the extend-add, 16 stores per tile).
+template <typename T, int N>
+__device__ __forceinline__ void pin(T (&v)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
+}
 
 // Right-looking partial factorization of the first nn columns of the
 // nj x nj front M (lower triangle, leading dimension LDS) in LDS.
@@ -357,147 +383,120 @@ __global__ __launch_bounds__(256, 4) void k_small(DevPlan P, DevFactor<T> F, con
     }
 }
 
-// Extend-add of one parent column by one wavefront: for each window of
-// EA_WIN parent rows the children's contributions (in the reference's
-// reverse child order) are accumulated in a wave-private LDS window, then
-// added to the panel (F11/F21 += F, cholesky.jl:520-521) or written to U
-// (M22 <- F22, cholesky.jl:542).  The child rows that land in window w are
-// [wstart[w], wstart[w+1]) (rel is increasing), so no search is needed; a
-// wavefront's LDS operations complete in order, so no barrier is needed.
-// The column's destination and its sources' addresses come precomputed
-// (EaDst, EaSrc; source s in lane s % 64), the panel values of the window
-// are fetched together with the window bounds, and the next source's rows
-// are fetched while the current source's are added.  A wavefront takes the
-// columns e_first, e_first + 4, ... < e_end; the records of the next column
-// are fetched while the current one is processed.
-// acc[i] += v in LDS without returning the old value: no wait for a read
-// before the add (a read-add-write per element is one LDS round trip each,
-// since the compiler cannot tell the indices apart).  A wavefront's LDS
-// operations complete in order, so the additions happen in program order.
-template <typename T>
-__device__ __forceinline__ void lds_add(T* p, T v) {
-    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-}
+constexpr int EA_LDS = 17 * LDS;  // LDS elements of a wavefront's extend-add columns
 
+// Extend-add of one 64 x 64 tile (F11/F21 += F, cholesky.jl:520-521, or
+// M22 <- F22, cholesky.jl:542).  Wavefront w takes the tile's columns
+// [16w, 16w + 16) in an LDS accumulator of its own (acc, 16 columns of LDS),
+// so no barrier is needed.  Per child (in the reference's reverse order) lane
+// l is the child's row ra + l, which lands in one row of the tile; the
+// child's columns landing in the wavefront's (at most sixteen) are all in
+// flight at once, the next child's while this one's are added, eight
+// independent read-add-writes in LDS at a time (a wavefront's LDS operations
+// complete in order, so children add up in their order).  The finished columns are added to the panel or written to
+// U row-contiguously.  Bound: the load round trips (source record and rel
+// map, then U); one tile takes 5.2 us of a workgroup on an idle chip (about 22
+// us per 4,096 elements when each wavefront took one parent column at a time
+// through a 1,024-row window).
 template <typename T>
-__device__ __forceinline__ void ea_columns(const DevPlan& P, const DevFactor<T>& F, int e_first, int e_end,
-                                           T* acc, int lane) {
-    EaTask e_nx = P.ea[e_first];
-    EaDst d_nx = P.ea_dst[e_first];
-    EaSrc s_nx{};
-    if (e_nx.src1 - e_nx.src0 <= 64 && lane < e_nx.src1 - e_nx.src0) s_nx = P.ea_srcx[e_nx.src0 + lane];
-    for (int ei = e_first; ei < e_end; ei += 4) {
-        const EaTask e = e_nx;
-        const EaDst ed = d_nx;
-        int64_t my_u = s_nx.u_off;
-        int my_rel = s_nx.rel_off, my_ws = s_nx.ws_off, my_tcol = s_nx.tcol, my_f0 = s_nx.i0, my_f1 = s_nx.i1;
-        if (ei + 4 < e_end) {
-            e_nx = P.ea[ei + 4];
-            d_nx = P.ea_dst[ei + 4];
-            const int nsn = e_nx.src1 - e_nx.src0;
-            if (nsn <= 64 && lane < nsn) s_nx = P.ea_srcx[e_nx.src0 + lane];
-        }
-        T* dst = (ed.to_u ? F.U : F.panel) + ed.off;  // dst[p]: parent row p
-        const bool to_u = ed.to_u != 0;
-        const int ns = e.src1 - e.src0;
-        auto load_meta = [&](int sb) {
-            if (sb + lane < ns) {
-                const EaSrc x = P.ea_srcx[e.src0 + sb + lane];
-                my_u = x.u_off;
-                my_rel = x.rel_off;
-                my_ws = x.ws_off;
-                my_tcol = x.tcol;
-                my_f0 = x.i0;
-                my_f1 = x.i1;
+__device__ __forceinline__ void ea_tile(const DevPlan& P, const DevFactor<T>& F, const EaTask e, T* lds, const int tid) {
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), cw = 16 * wave;
+    const Front f = uniform(P.fronts[e.front]);
+    const int p = (f.nn + NB - 1) / NB, nj = f.nn + f.na;
+    const int r0 = e.I < p ? e.I * NB : f.nn + (e.I - p) * NB, c0 = e.J < p ? e.J * NB : f.nn + (e.J - p) * NB;
+    const int m = min(NB, (e.I < p ? f.nn : nj) - r0), n = min(NB, (e.J < p ? f.nn : nj) - c0);
+    if (cw >= n) return;
+    const bool to_u = e.J >= p;
+    const int64_t ld = to_u ? f.na : nj;
+    T* dst = to_u ? F.U + f.uoff + (r0 - f.nn) + (int64_t)(c0 - f.nn) * ld : F.panel + f.poff + r0 + (int64_t)c0 * ld;
+    T* acc = lds + wave * EA_LDS;  // sixteen columns and a spare one
+    const bool diag = e.I == e.J;
+    T pre[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        // the assembled A entries (an earlier launch wrote them)
+        pre[j] = to_u ? (T)0 : dst[min(lane, m - 1) + (int64_t)min(cw + j, n - 1) * ld];
+        acc[lane + j * LDS] = (T)0;
+    }
+    // One source in flight: its rel maps, then its part of U (up to sixteen
+    // columns of the tile's)
+    struct Src {
+        int rr, rc, i, rb, t0, t1, ta;
+        T v[16];
+    };
+    for (int sb = e.src0; sb < e.src1; sb += 64) {
+        const int ns = min(64, e.src1 - sb);
+        // the source records, one per lane
+        const EaSrc x = P.ea_src[sb + min(lane, ns - 1)];
+        auto get = [&](int32_t v, int q) { return __builtin_amdgcn_readlane(v, q); };
+        auto rels = [&](int q, Src& s) {
+            const int32_t* rel = P.rel + get(x.rel_off, q);
+            const int ra = get(x.ra, q), tb = get(x.tb, q);
+            s.ta = get(x.ta, q);
+            s.rb = get(x.rb, q);
+            s.i = ra + lane;
+            s.rr = rel[min(s.i, s.rb - 1)] - r0;            // this lane's row of the tile
+            s.rc = rel[min(s.ta + lane, tb - 1)] - c0;      // column of the tile of child column ta + lane
+            s.t1 = tb;
+        };
+        auto cols = [&](int q, Src& s) {
+            const bool has = lane < s.t1 - s.ta;
+            s.t0 = s.ta + (int)__popcll(__ballot(has && s.rc < cw));
+            s.t1 = s.ta + (int)__popcll(__ballot(has && s.rc < cw + 16));
+            const uint64_t uo = (uint32_t)get((int32_t)(uint64_t)x.u_off, q) |
+                                (uint64_t)(uint32_t)get((int32_t)((uint64_t)x.u_off >> 32), q) << 32;
+            const int ma = get(x.ma, q);
+            const T* u = F.U + uo + min(s.i, s.rb - 1);
+#pragma unroll
+            for (int h = 0; h < 16; h += 8) {
+                if (s.t0 + h >= s.t1) break;  // uniform
+#pragma unroll
+                for (int j = h; j < h + 8; ++j) s.v[j] = ldc(u + (int64_t)min(s.t0 + j, s.t1 - 1) * ma);
             }
         };
-        const int wfirst = e.row0 / EA_WIN;
-        for (int w0 = (e.row0 / EA_WIN) * EA_WIN; w0 < e.row1; w0 += EA_WIN) {
-            const int w = w0 / EA_WIN;
-            T pre[EA_WIN / 64];
+        // columns past the child's last go to the spare column
+        auto add = [&](const Src& s) {
+            if (s.i >= s.rb) return;
 #pragma unroll
-            for (int j = 0; j < EA_WIN / 64; ++j) {
-                const int p = w0 + lane + 64 * j;
-                pre[j] = (!to_u && p >= e.row0 && p < e.row1) ? dst[p] : (T)0;
-                acc[lane + 64 * j] = (T)0;
-            }
-            for (int sb = 0; sb < ns; sb += 64) {
-                if (ns > 64) load_meta(sb);
-                const int nsb = min(64, ns - sb);
-                int my_i0 = my_f0, my_i1 = my_f1;  // the first window's bounds come with the record
-                if (lane < nsb && w != wfirst) {
-                    const int32_t* ws = P.wstart + my_ws;
-                    my_i0 = max(ws[w], my_tcol);
-                    my_i1 = ws[w + 1];
+            for (int h = 0; h < 16; h += 8) {
+                if (s.t0 + h >= s.t1) break;  // uniform
+                T o[8];
+                int pc[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int t = s.t0 + h + j;
+                    const int c = t < s.t1 ? get(s.rc, t - s.ta) - cw : 16;
+                    pc[j] = c * LDS + s.rr;
+                    o[j] = acc[pc[j]];
                 }
-                // rows i0 + lane + 64 j (j < 4) of source q.  The loads are
-                // unconditional (rows past the source's end read its row 0,
-                // always in bounds, and are flagged in ok), so the eight loads
-                // of a fetch are in flight together; a load under a per-lane
-                // branch would be waited for inside that branch.
-                int rr[4];
-                T vv[4];
-                unsigned ok = 0;
-                auto fetch = [&](int q, int i) {
-                    const int i1 = __builtin_amdgcn_readlane(my_i1, q);
-                    const int relo = __builtin_amdgcn_readlane(my_rel, q);
-                    const unsigned ulo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(uint64_t)my_u, q);
-                    const unsigned uhi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)((uint64_t)my_u >> 32), q);
-                    const int64_t uo = (int64_t)(((uint64_t)uhi << 32) | ulo);
-                    ok = 0;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int ii = i + lane + 64 * j;
-                        const int ic = ii < i1 ? ii : 0;
-                        ok |= (ii < i1 ? 1u : 0u) << j;
-                        rr[j] = P.rel[relo + ic];
-                        vv[j] = ldc(F.U + uo + ic);
-                    }
-                };
-                if (nsb > 0) fetch(0, __builtin_amdgcn_readlane(my_i0, 0));
-                for (int q = 0; q < nsb; ++q) {
-                    const int i0 = __builtin_amdgcn_readlane(my_i0, q), i1 = __builtin_amdgcn_readlane(my_i1, q);
-                    int cr[4];
-                    T cv[4];
-                    const unsigned cok = ok;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        cr[j] = rr[j];
-                        cv[j] = vv[j];
-                    }
-                    if (q + 1 < nsb) fetch(q + 1, __builtin_amdgcn_readlane(my_i0, q + 1));
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if ((cok >> j) & 1u) lds_add(acc + (cr[j] - w0), cv[j]);
-                    // rows beyond the first 256 of this source in the window
-                    for (int i = i0 + 256; i < i1; i += 256) {
-                        const int relo = __builtin_amdgcn_readlane(my_rel, q);
-                        const unsigned ulo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(uint64_t)my_u, q);
-                        const unsigned uhi =
-                            (unsigned)__builtin_amdgcn_readlane((int)(unsigned)((uint64_t)my_u >> 32), q);
-                        const int64_t uo = (int64_t)(((uint64_t)uhi << 32) | ulo);
-                        int r2[4];
-                        T v2[4];
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const int ii = i + lane + 64 * j;
-                            const int ic = ii < i1 ? ii : 0;
-                            r2[j] = P.rel[relo + ic];
-                            v2[j] = ldc(F.U + uo + ic);
-                        }
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            if (i + lane + 64 * j < i1) lds_add(acc + (r2[j] - w0), v2[j]);
-                    }
-                }
+                for (int j = 0; j < 8; ++j)
+                    acc[pc[j]] = o[j] + (!diag || s.i >= s.t0 + h + j ? s.v[h + j] : (T)0);
             }
-#pragma unroll
-            for (int j = 0; j < EA_WIN / 64; ++j) {
-                const int p = w0 + lane + 64 * j;
-                if (p >= e.row0 && p < e.row1) stc(dst + p, to_u ? acc[lane + 64 * j] : pre[j] + acc[lane + 64 * j]);
-            }
+        };
+        Src s0, s1;
+        rels(0, s0);
+        if (ns > 1) rels(1, s1);
+        cols(0, s0);
+        for (int q = 0; q < ns; q += 2) {
+            if (q + 1 < ns) cols(q + 1, s1);
+            add(s0);
+            if (q + 2 < ns) rels(q + 2, s0);
+            if (q + 1 < ns) add(s1);
+            if (q + 3 < ns) rels(q + 3, s1);
+            if (q + 2 < ns) cols(q + 2, s0);
         }
     }
+    // all LDS reads first, then the stores
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const T a = acc[lane + j * LDS];
+        pre[j] = to_u ? a : pre[j] + a;
+    }
+    pin(pre);
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+        if (lane < m && cw + j < n && (!diag || lane >= cw + j)) stc(dst + lane + (int64_t)(cw + j) * ld, pre[j]);
 }
 
 constexpr int PB = 16;            // block size inside the diagonal tile
@@ -668,7 +667,7 @@ __device__ __forceinline__ void pivot_cols(T (&x)[PB], T (&y)[PB], const DevFact
 // LDS for store_diag.  invert_only: the tile already holds L and only W is
 // formed.  LDS: PTILE elements.
 template <typename T>
-__device__ __forceinline__ void potrf_blocked(const DevFactor<T>& F, const Front& f, int k0, bool invert_only,
+__device__ __forceinline__ void potrf_blocked(const DevFactor<T>& F, const Front f, int k0, bool invert_only,
                               T* lds, const int tid) {
     typedef typename Mfma<T>::v4 v4;
     constexpr int NBLK = NB / PB;
@@ -771,19 +770,20 @@ __device__ __forceinline__ void potrf_blocked(const DevFactor<T>& F, const Front
     for (int i = 0; i < NB / 4; ++i) {
         const int c = cg + 4 * i, bc = i / 4, br = r / PB;
         const T* src = bc == br ? WD + bc * PB * LDP + (c & (PB - 1)) + (r & (PB - 1)) * LDP : A + c + r * LDS;
-        v[i] = *src;
+        v[i] = (c <= r) ? *src : (T)0;
     }
+    pin(v);
 #pragma unroll
     for (int i = 0; i < NB / 4; ++i) {
         const int c = cg + 4 * i;
-        if (r < kb && c < kb) stc(W + r + (int64_t)c * f.nn, (c <= r) ? v[i] : (T)0);
+        if (r < kb && c < kb) stc(W + r + (int64_t)c * f.nn, v[i]);
     }
     if (!invert_only && !chol && tid < kb) stc(F.d + gc0 + tid, pv[tid]);
 }
 
 // The factored tile, from LDS (as potrf_blocked leaves it) to the panel.
 template <typename T>
-__device__ __forceinline__ void store_diag(const DevFactor<T>& F, const Front& f, int k0, const T* lds, const int tid) {
+__device__ __forceinline__ void store_diag(const DevFactor<T>& F, const Front f, int k0, const T* lds, const int tid) {
     const T* sc = lds + NB * LDS + (NB / PB) * PB * LDP;
     const int nj = f.nn + f.na, kb = min(NB, f.nn - k0), r = tid & 63, cg = tid >> 6;
     T* blk = F.panel + f.poff + k0 + (int64_t)k0 * nj;
@@ -793,6 +793,7 @@ __device__ __forceinline__ void store_diag(const DevFactor<T>& F, const Front& f
         const int c = cg + 4 * i;
         v[i] = lds[r + c * LDS] * (r > c ? sc[c] : (T)1);
     }
+    pin(v);
 #pragma unroll
     for (int i = 0; i < NB / 4; ++i) {
         const int c = cg + 4 * i;
@@ -819,11 +820,15 @@ __device__ __forceinline__ void write_c(T* C, int64_t ldc_, int m, int n, bool l
     const int r = tid & 63, g = tid >> 6;
     T x[NB / 4];
 #pragma unroll
-    for (int i = 0; i < NB / 4; ++i) x[i] = Cs[r + (g + 4 * i) * LDS];
+    for (int i = 0; i < NB / 4; ++i) {
+        const T y = Cs[r + (g + 4 * i) * LDS];
+        x[i] = SUB ? c[i] - y : y;
+    }
+    pin(x);
 #pragma unroll
     for (int i = 0; i < NB / 4; ++i) {
         const int col = g + 4 * i;
-        if (r < m && col < n && (!lower || r >= col)) stc(C + r + col * ldc_, SUB ? c[i] - x[i] : x[i]);
+        if (r < m && col < n && (!lower || r >= col)) stc(C + r + col * ldc_, x[i]);
     }
 }
 
@@ -838,8 +843,8 @@ __device__ __forceinline__ void write_c(T* C, int64_t ldc_, int m, int n, bool l
 // loads, since no task waits for it.  The caller has seen A1 and C final
 // through the previous block column.  LDS: PTILE + NB * LDS elements.
 template <typename T>
-__device__ __forceinline__ void chain_step(const DevFactor<T>& F, const Front& f, int k0, const GemmTask& t,
-                                           const GemmTask& u, T* lds, const int tid) {
+__device__ __forceinline__ void chain_step(const DevFactor<T>& F, const Front f, int k0, const GemmTask t,
+                                           const GemmTask u, T* lds, const int tid) {
     typedef typename Mfma<T>::v4 v4;
     constexpr int NBLK = NB / PB;
     T* A = lds;
@@ -1076,7 +1081,7 @@ __device__ __forceinline__ void load_lds16(const void* g, void* lds) {
 // TFLOP/s (34.9 with the chunks staged through registers), 4,656 tiles of
 // 64 x 64 x 512: 45.8 (39.4).
 template <typename T, int E>
-__device__ __forceinline__ void gemm_tile(const DevFactor<T>& F, const GemmTask& g, T* S, const int tid) {
+__device__ __forceinline__ void gemm_tile(const DevFactor<T>& F, const GemmTask g, T* S, const int tid) {
     typedef typename Mfma<T>::v4 v4;
     constexpr int KW = E == 128 ? 16 : 32;           // columns per stage
     constexpr int EPL = 16 / (int)sizeof(T);         // elements per lane and load
@@ -1184,6 +1189,7 @@ __device__ __forceinline__ void gemm_tile(const DevFactor<T>& F, const GemmTask&
         T x[CPER];
 #pragma unroll
         for (int i = 0; i < CPER; ++i) x[i] = cv[i] - Cs[r + (kq + CS * i) * LDC];
+        pin(x);
         if (q + 1 < E / NC) fetch_round(q + 1);
 #pragma unroll
         for (int i = 0; i < CPER; ++i) {
@@ -1206,7 +1212,7 @@ __device__ __forceinline__ void gemm_tile(const DevFactor<T>& F, const GemmTask&
 // on an idle chip takes 5.3 us (10.4 in two 32-wide chunks), a
 // single-step update 6.2 us (7.4).
 template <typename T, bool TRSM>
-__device__ __forceinline__ void gemm_tile64(const DevFactor<T>& F, const GemmTask& g, T* Bs, T* Cs, const int tid) {
+__device__ __forceinline__ void gemm_tile64(const DevFactor<T>& F, const GemmTask g, T* Bs, T* Cs, const int tid) {
     typedef typename Mfma<T>::v4 v4;
     constexpr int NBLK = NB / PB;
     const T* A = arr_base(F, g.arrA) + g.a_off;
@@ -1288,23 +1294,23 @@ __device__ __forceinline__ bool dag_dep(const DevPlan& P, const DevFactor<T>& F,
             // the diagonal tile (the fused products wait for their own tiles
             // inside the task, after the factorization); under GMW81 every
             // tile of the block column, updated through the previous column
-            *nw = (GMW && d.a > 0) ? g.R - d.a : 1;
+            *nw = GMW ? g.R - d.a : 1;
             if (q >= *nw) return false;
-            *w = d.a == 0 ? D.eapcnt + J : cnt + d.a * g.R + d.a + q;
-            *target = d.a == 0 ? g.n_eap : d.a;
+            *w = cnt + d.a * g.R + d.a + q;
+            *target = d.a + 1;
             return true;
         case DT_TRSM:
-            *nw = d.c > 0 ? 2 : 1;
+            *nw = 2;
             if (q >= *nw) return false;
             *w = cnt + d.c * g.R + (q == 0 ? d.c : d.b);
-            *target = q == 0 ? d.c + 1 : d.c;
+            *target = q == 0 ? d.c + 2 : d.c + 1;
             return true;
         case DT_UPD: {  // columns [K0, K1): rows I, Jc final through K1 - 1
             const int K0 = d.d & 0xffff, K1 = d.d >> 16;
-            *nw = K0 > 0 ? 3 : 2;
+            *nw = 3;
             if (q >= *nw) return false;
             *w = q == 2 ? cnt + d.c * g.R + d.b : cnt + (K1 - 1) * g.R + (q == 0 ? d.b : d.c);
-            *target = q == 2 ? K0 : K1;
+            *target = q == 2 ? K0 + 1 : K1 + 1;
             return true;
         }
         default: {  // DT_SYRK: the tile's row blocks of the panel are final, and
@@ -1318,7 +1324,7 @@ __device__ __forceinline__ bool dag_dep(const DevPlan& P, const DevFactor<T>& F,
             }
             const int blk = q == 0 ? d.b : q == 1 ? d.c : (q == 2 && (d.d & 1)) ? d.b + 1 : d.c + 1;
             *w = cnt + (g.p - 1) * g.R + blk;
-            *target = g.p;
+            *target = g.p + 1;
             return true;
         }
     }
@@ -1343,11 +1349,9 @@ constexpr unsigned long long WMASK = WDEP == 64 ? ~0ull : (1ull << (WDEP & 63)) 
 // resident workgroups.  Counters:
 //   F.flags[J]   finished update-matrix tiles of front J (1 for a small front)
 //   D.eacnt[J]   finished extend-add tasks of J (1 for a small front)
-//   D.eapcnt[J]  finished extend-add tasks of J into panel columns (the
-//                first diagonal tile waits only for these; the update-matrix
-//                tiles wait for all of them)
-//   D.cnt[toff_J + K*R_J + I]  panel columns applied to tile (I, K); K+1
-//                once the tile is final
+//   D.cnt[toff_J + K*R_J + I]  tile (I, K) of the panel: 0 until its
+//                extend-add is done (1 at the start where no child reaches the
+//                tile), 1 + the panel columns applied, K+2 once it is final
 // Synchronization per task: lanes of wave 0 poll the dependencies of the
 // held tickets with relaxed loads (WDEP lanes per ticket).  Every value a
 // task reads that another task of this launch wrote is loaded with a
@@ -1362,7 +1366,7 @@ template <typename T, bool GMW>
 __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, DevFactor<T> F, DevDag D) {
     constexpr int S1 = PTILE + NB * LDS, S2 = NB * LDT + NB * LDS, S3 = GEMM_LDS;
     constexpr int SMEM = S1 > S2 ? (S1 > S3 ? S1 : S3) : (S2 > S3 ? S2 : S3);
-    static_assert(4 * EA_WIN <= SMEM && SMALL_NJ * LDS <= SMEM && 32 * 129 <= SMEM, "LDS");
+    static_assert(SMALL_NJ * LDS <= SMEM && 4 * EA_LDS <= SMEM && 32 * 129 <= SMEM, "LDS");
     static_assert(SMEM >= 2 * NB * LDS + NB + 6 * (int)(sizeof(double) / sizeof(T)), "potrf_gmw LDS");
     __shared__ __align__(16) T smem[SMEM];
     __shared__ T s_piv, s_inv;
@@ -1453,10 +1457,10 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
         __syncthreads();
         const int sel = s_sel;
         if (sel < 0) break;
-        const int t = s_win[sel];
-        const DagTask d = D.task[t];
+        const int t = __builtin_amdgcn_readfirstlane(s_win[sel]);
+        const DagTask d = uniform(D.task[t]);
         const int J = d.front;
-        const DagFront g = D.df[J];
+        const DagFront g = uniform(D.df[J]);
         int32_t* cnt = D.cnt + g.toff;
         unsigned long long t_begin = 0;
         if (D.prof && tid == 0) t_begin = wall_clock64();
@@ -1467,18 +1471,17 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
         if (raise) __builtin_amdgcn_s_setprio(3);
         switch (d.kind) {
             case DT_EA: {
-                const int wave = tid >> 6, lane = tid & 63;
-                if (d.a + wave < d.b) ea_columns<T>(P, F, d.a + wave, d.b, smem + wave * EA_WIN, lane);
+                for (int e = d.a; e < d.b; ++e) ea_tile<T>(P, F, uniform(P.ea[e]), smem, tid);
                 break;
             }
             case DT_SMALL:
                 small_front<T>(P, F, J, smem, &s_piv, &s_inv, &s_fail, tid);
                 break;
             case DT_POTRF:
-                if constexpr (GMW) potrf_gmw<T>(F, P.fronts[J], d.a * NB, smem, tid);
-                else potrf_blocked<T>(F, P.fronts[J], d.a * NB, false, smem, tid);
+                if constexpr (GMW) potrf_gmw<T>(F, uniform(P.fronts[J]), d.a * NB, smem, tid);
+                else potrf_blocked<T>(F, uniform(P.fronts[J]), d.a * NB, false, smem, tid);
                 if (d.b < 0) {
-                    if constexpr (!GMW) store_diag<T>(F, P.fronts[J], d.a * NB, smem, tid);
+                    if constexpr (!GMW) store_diag<T>(F, uniform(P.fronts[J]), d.a * NB, smem, tid);
                 } else {
                     // publish the diagonal tile (the other panel solves of column a
                     // need only it), then the fused panel solve of tile (a+1, a) and
@@ -1489,25 +1492,26 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
                     __syncthreads();
                     if (tid == 0) {
                         __builtin_amdgcn_s_waitcnt(0);
-                        __hip_atomic_store(cnt + d.a * g.R + d.a, d.a + 1, __ATOMIC_RELAXED,
+                        __hip_atomic_store(cnt + d.a * g.R + d.a, d.a + 2, __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
-                        (void)bounded_wait(cnt + d.a * g.R + d.a + 1, d.a, F.hang, F.ticket, F.stall, 1);
-                        (void)bounded_wait(cnt + (d.a + 1) * g.R + d.a + 1, d.a, F.hang, F.ticket, F.stall, 1);
+                        (void)bounded_wait(cnt + d.a * g.R + d.a + 1, d.a + 1, F.hang, F.ticket, F.stall, 1);
+                        (void)bounded_wait(cnt + (d.a + 1) * g.R + d.a + 1, d.a + 1, F.hang, F.ticket, F.stall, 1);
                     }
                     __syncthreads();
                     if constexpr (GMW) {
-                        gemm_tile64<T, true>(F, P.gemm[d.b], smem, smem + NB * LDT, tid);
+                        gemm_tile64<T, true>(F, uniform(P.gemm[d.b]), smem, smem + NB * LDT, tid);
                         // the update reads the panel solve's tile back from memory
                         drain_stores();
                         __syncthreads();
-                        gemm_tile64<T, false>(F, P.gemm[d.c], smem, smem + NB * LDT, tid);
+                        gemm_tile64<T, false>(F, uniform(P.gemm[d.c]), smem, smem + NB * LDT, tid);
                     } else {
-                        chain_step<T>(F, P.fronts[J], d.a * NB, P.gemm[d.b], P.gemm[d.c], smem, tid);
+                        chain_step<T>(F, uniform(P.fronts[J]), d.a * NB, uniform(P.gemm[d.b]),
+                                      uniform(P.gemm[d.c]), smem, tid);
                     }
                 }
                 break;
             default: {
-                const GemmTask gt = P.gemm[d.a];
+                const GemmTask gt = uniform(P.gemm[d.a]);
                 if (gt.wide) gemm_tile<T, 128>(F, gt, smem, tid);
                 else if (gt.mode == G_TRSM) gemm_tile64<T, true>(F, gt, smem, smem + NB * LDT, tid);
                 else if (gt.k <= NB) gemm_tile64<T, false>(F, gt, smem, smem + NB * LDT, tid);
@@ -1537,7 +1541,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
             constexpr int R = __ATOMIC_RELAXED, S = __HIP_MEMORY_SCOPE_AGENT;
             switch (d.kind) {
                 case DT_EA:
-                    if (d.c) __hip_atomic_fetch_add(D.eapcnt + J, 1, R, S);
+                    for (int e = d.a; d.c && e < d.b; ++e)
+                        __hip_atomic_store(cnt + P.ea[e].J * g.R + P.ea[e].I, 1, R, S);
                     __hip_atomic_fetch_add(D.eacnt + J, 1, R, S);
                     break;
                 case DT_SMALL:
@@ -1545,12 +1550,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
                     __hip_atomic_store(F.flags + J, 1, R, S);
                     break;
                 case DT_POTRF:
-                    __hip_atomic_store(cnt + d.a * g.R + d.a, d.a + 1, R, S);
-                    if (d.b >= 0) __hip_atomic_store(cnt + d.a * g.R + d.a + 1, d.a + 1, R, S);
-                    if (d.c >= 0) __hip_atomic_store(cnt + (d.a + 1) * g.R + d.a + 1, d.a + 1, R, S);
+                    __hip_atomic_store(cnt + d.a * g.R + d.a, d.a + 2, R, S);
+                    if (d.b >= 0) __hip_atomic_store(cnt + d.a * g.R + d.a + 1, d.a + 2, R, S);
+                    if (d.c >= 0) __hip_atomic_store(cnt + (d.a + 1) * g.R + d.a + 1, d.a + 2, R, S);
                     break;
-                case DT_TRSM: __hip_atomic_store(cnt + d.c * g.R + d.b, d.c + 1, R, S); break;
-                case DT_UPD: __hip_atomic_store(cnt + d.c * g.R + d.b, d.d >> 16, R, S); break;
+                case DT_TRSM: __hip_atomic_store(cnt + d.c * g.R + d.b, d.c + 2, R, S); break;
+                case DT_UPD: __hip_atomic_store(cnt + d.c * g.R + d.b, (d.d >> 16) + 1, R, S); break;
                 default: __hip_atomic_fetch_add(F.flags + J, 1, R, S); break;
             }
             const unsigned long long r1 = D.prof ? wall_clock64() : 0;
@@ -1564,6 +1569,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
         // closes the thread-0 block before the back-edge
         __syncthreads();
     }
+}
+
+__global__ void k_copy_i32(const int32_t* src, int32_t* dst, int64_t count) {
+    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (; i < count; i += stride) dst[i] = src[i];
 }
 
 template <typename T>
@@ -1669,6 +1680,11 @@ template <typename T>
 void launch_fill(T* p, int64_t count, T value, hipStream_t s) {
     if (count <= 0) return;
     hipLaunchKernelGGL(k_fill<T>, dim3(grid_for(count, 256)), dim3(256), 0, s, p, count, value);
+}
+
+void launch_copy_i32(const int32_t* src, int32_t* dst, int64_t count, hipStream_t s) {
+    if (count <= 0) return;
+    hipLaunchKernelGGL(k_copy_i32, dim3(grid_for(count, 256)), dim3(256), 0, s, src, dst, count);
 }
 
 template <typename T>

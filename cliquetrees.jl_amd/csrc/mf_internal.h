@@ -24,8 +24,8 @@ namespace mf {
 constexpr int NB = 64;          // panel width and GEMM tile edge of big fronts
 constexpr int SMALL_NJ = 64;    // fronts with nJ <= SMALL_NJ use the fused LDS kernel
 constexpr int TINY_NJ = 32;     // small fronts that one wavefront factors (four per ticket)
-constexpr int EA_WIN = 1024;    // parent rows per extend-add window (one wave)
-constexpr int EA_ROWS = 16384;  // parent rows per extend-add task (about)
+constexpr int EA_TILE = 4096;   // elements of an extend-add tile (64 x 64)
+constexpr int EA_ROWS = 16384;  // elements per extend-add task (at most, where that fills the chip)
 constexpr int WIDE_K = 128;     // update-matrix tiles are 128 x 128 when nn >= WIDE_K
 constexpr int UPD_GROUP = 8;    // panel steps applied by one trailing-update tile
 constexpr int SIM_WORKERS = 512;  // resident workgroups assumed when ordering the DAG tickets
@@ -47,31 +47,22 @@ struct Front {
     int32_t parent;  // internal parent, -1 for roots
 };
 
-// Extend-add task: parent front, parent column, parent row range.
+// One extend-add tile: row block I by column block J of a big front's row
+// blocks (panel blocks [64b, 64b + 64) for b < p, then update rows
+// [nn + 64 (b - p), ...)), I >= J, and its sources: the children with rows in
+// both blocks, in accumulation order.
 struct EaTask {
     int32_t front;
-    int32_t col;
-    int32_t row0;
-    int32_t row1;
-    int32_t src0;   // sources [src0, src1) in ea_src (child, child column)
+    int32_t I, J;
+    int32_t src0;   // sources [src0, src1) in ea_src
     int32_t src1;
 };
-
-// Device form of an extend-add column: destination (panel or U element of
-// parent row 0, so dst[p] is parent row p) and, per source, the child's U
-// column, rel map and window table, so the kernel reads them in one step.
-struct EaDst {
-    int64_t off;
-    int32_t to_u;
-    int32_t pad;
-};
 struct EaSrc {
-    int64_t u_off;    // U element (0, tcol) of the child
-    int32_t rel_off;  // child's rel map in rel[]
-    int32_t ws_off;   // child's window table in wstart[]
-    int32_t tcol;     // child column (its first row)
-    int32_t i0, i1;   // child rows landing in the column's first window
-    int32_t pad;
+    int64_t u_off;    // the child's U
+    int32_t rel_off;  // its rel map in rel[]
+    int32_t ma;       // its leading dimension (rows)
+    int32_t ra, rb;   // its rows landing in row block I
+    int32_t ta, tb;   // its rows (columns of U) landing in column block J
 };
 
 enum : int8_t { ARR_PANEL = 0, ARR_U = 1, ARR_W = 2 };
@@ -116,12 +107,13 @@ struct DagTask {
 
 // Per-front constants of the DAG.
 struct DagFront {
-    int32_t toff;    // offset of the front's tile counters (K * R + I)
+    int32_t toff;    // offset of the front's tile counters (K * R + I): 0 until the tile's
+                     // extend-add is done, 1 + c with c panel columns applied, K + 2 when final
     int32_t R;       // row blocks (panel blocks p, then update-row blocks)
     int32_t p;       // panel (column) blocks
     int32_t n_ea;    // extend-add tasks (all; 1 for a small front)
     int32_t n_done;  // tasks whose completion makes U final (SYRK tiles, or 1 for small)
-    int32_t n_eap;   // extend-add tasks into panel columns: the panel waits only for these
+    int32_t pad;
 };
 
 // Copy-out of one reference front from its internal panel.

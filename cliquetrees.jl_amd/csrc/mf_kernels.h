@@ -22,12 +22,8 @@ struct DevPlan {
     const int32_t* level_small;
     const int32_t* level_big;
     const EaTask* ea;
-    const int32_t* ea_src;
-    const EaDst* ea_dst;        // per extend-add column
-    const EaSrc* ea_srcx;       // per extend-add source (parallel to ea_src pairs)
-    const int32_t* wstart;       // extend-add window tables
-    const int32_t* wsoff;
-    const int32_t* sgstart;      // solve gather tables: sgstart[sgoff[K] + b] = first row of
+    const EaSrc* ea_src;
+    const int32_t* sgstart;      // gather tables: sgstart[sgoff[K] + b] = first row of
     const int32_t* sgoff;        // child K landing in or after row block b of its parent
     const GemmTask* gemm;
     const DiagTask* diag;
@@ -71,7 +67,6 @@ struct DevDag {
     const int32_t* uwait;
     int32_t* cnt;      // tile counters
     int32_t* eacnt;    // finished extend-add tasks per front
-    int32_t* eapcnt;   // finished extend-add tasks into panel columns per front
     unsigned long long* prof;  // NULL, or per task kind: wait, body (wall-clock ticks), count
     unsigned long long* trace; // NULL, or per ticket: start | workgroup << 48, end (wall clock)
     int32_t ntask;
@@ -83,6 +78,7 @@ struct DevDag {
 // ---- factorization (mf_factor.hip) ----
 template <typename T>
 void launch_fill(T* p, int64_t count, T value, hipStream_t s);
+void launch_copy_i32(const int32_t* src, int32_t* dst, int64_t count, hipStream_t s);
 // uplo: 0 = :L, 1 = :U layout of Dval/Lval; adiag: assembled diagonal per
 // permuted column (written by assembly and refresh, read by the copy-out).
 template <typename T>

@@ -92,8 +92,9 @@ class Planner {
     std::string amalgamate();     // 1. internal fronts, children, rel maps, copy-out map
     std::string classify();       // 2. small region, levels of the big region
     std::string layout_memory();  // 3. panel, U (slot reuse), W pools, solve workspaces
+    std::string gather_tables();  // children's rows per row block of a big front
     std::string factor_tasks();   // 4. extend-add, diagonal and tile-DAG tasks
-    std::string solve_tasks();    // gather tables and persistent solve task lists
+    std::string solve_tasks();    // persistent solve task lists
     std::string check_bounds();   // every task's accesses inside its pools
     std::string dataflow();       // predecessor counts and successor lists of the DAG
     std::string schedule();       // tickets by list scheduling (and the GMW81 order)
@@ -246,6 +247,7 @@ std::string Planner::amalgamate() {
                 int32_t v = P.rows[F.rowoff + F.nn + t];
                 const int32_t* it = std::lower_bound(prow, prow + pn, v);
                 if (it == prow + pn || *it != v) return "separator row missing in parent";
+                if (t > 0 && P.rel.back() >= (int32_t)(it - prow)) return "rel map not increasing";
                 P.rel.push_back((int32_t)(it - prow));
             }
         }
@@ -442,14 +444,55 @@ std::string Planner::layout_memory() {
     return std::string();
 }
 
+std::string Planner::gather_tables() {
+    // ---- gather tables ------------------------------------------------------------
+    // An extend-add tile and a solve task of a big front J cover row blocks b of J (panel
+    // blocks [64b, 64b + 64) for b < p, then update rows [nn + 64(b-p), ...)).
+    // For each child K of J, sgstart[sgoff[K] + b] is the first row i of K
+    // with rel_K[i] >= the first row of block b (rel is increasing), b = 0..R,
+    // so the rows of K landing in block b are [tab[b], tab[b+1]).
+    P.sgoff.assign(NJ, -1);
+    P.sgstart.clear();
+    for (int32_t J = 0; J < NJ; ++J) {
+        if (P.is_small[J]) continue;
+        const Front& F = P.fronts[J];
+        const int32_t p = (F.nn + NB - 1) / NB, R = p + (F.na + NB - 1) / NB;
+        auto brow = [&](int32_t b) { return b < p ? std::min(b * NB, F.nn) : std::min(F.nn + (b - p) * NB, F.nn + F.na); };
+        for (int32_t q = F.chd0; q < F.chd1; ++q) {
+            const int32_t K = P.chd[q];
+            const Front& Kf = P.fronts[K];
+            P.sgoff[K] = (int32_t)P.sgstart.size();
+            int32_t i = 0;
+            for (int32_t b = 0; b <= R; ++b) {
+                const int32_t r0 = b < R ? brow(b) : F.nn + F.na;
+                while (i < Kf.na && P.rel[Kf.reloff + i] < r0) ++i;
+                P.sgstart.push_back(i);
+            }
+        }
+    }
+
+    for (int32_t J = 0; J < NJ; ++J) {
+        if (P.is_small[J]) continue;
+        const Front& F = P.fronts[J];
+        const int32_t R = (F.nn + NB - 1) / NB + (F.na + NB - 1) / NB;
+        for (int32_t q = F.chd0; q < F.chd1; ++q) {
+            const int32_t K = P.chd[q], o = P.sgoff[K];
+            if (o < 0 || (size_t)o + R + 1 > P.sgstart.size()) return "gather table";
+            for (int32_t b = 0; b <= R; ++b)
+                if (P.sgstart[o + b] < 0 || P.sgstart[o + b] > P.fronts[K].na ||
+                    (b > 0 && P.sgstart[o + b] < P.sgstart[o + b - 1]))
+                    return "gather table range";
+        }
+    }
+    return std::string();
+}
+
 std::string Planner::factor_tasks() {
     // ---- 4. task lists ---------------------------------------------------------
     P.level_small.clear();
     P.level_big.clear();
     P.ea.clear();
     P.ea_src.clear();
-    P.wstart.clear();
-    P.wsoff.assign(NJ, -1);
     P.gemm.clear();
     P.diag.clear();
 
@@ -486,49 +529,46 @@ std::string Planner::factor_tasks() {
         L.bigL1 = (int32_t)P.level_big.size();
         // extend-add tasks
         L.ea0 = (int32_t)P.ea.size();
+        // extend-add tiles: every tile of the update matrix, and the panel
+        // tiles that a child reaches
         for (int32_t J : L.big_list) {
             const Front& F = P.fronts[J];
-            int32_t nj = F.nn + F.na;
-            std::vector<std::vector<int32_t>> src(nj);
+            const int32_t p = (F.nn + NB - 1) / NB, R = p + (F.na + NB - 1) / NB;
+            std::vector<std::vector<std::pair<int32_t, int32_t>>> hit(R);  // per row block: (child's place, child)
+            std::vector<std::vector<int32_t>> blocks;                      // per child: its row blocks
             for (int32_t q = F.chd0; q < F.chd1; ++q) {
-                int32_t K = P.chd[q];
-                const Front& Kf = P.fronts[K];
-                for (int32_t t = 0; t < Kf.na; ++t) {
-                    int32_t pc = P.rel[Kf.reloff + t];
-                    src[pc].push_back(K);
-                    src[pc].push_back(t);
-                }
+                const int32_t* tb = P.sgstart.data() + P.sgoff[P.chd[q]];
+                std::vector<int32_t> bl;
+                for (int32_t b = 0; b < R; ++b)
+                    if (tb[b + 1] > tb[b]) bl.push_back(b);
+                for (int32_t b : bl) hit[b].push_back({q - F.chd0, P.chd[q]});
+                blocks.push_back(std::move(bl));
             }
-            for (int32_t pc = 0; pc < nj; ++pc) {
-                if (pc < F.nn && src[pc].empty()) continue;
-                EaTask e{};
-                e.front = J;
-                e.col = pc;
-                e.row0 = pc;
-                e.row1 = nj;
-                e.src0 = (int32_t)(P.ea_src.size() / 2);
-                P.ea_src.insert(P.ea_src.end(), src[pc].begin(), src[pc].end());
-                e.src1 = (int32_t)(P.ea_src.size() / 2);
-                P.ea.push_back(e);
+            for (int32_t Jc = 0; Jc < R; ++Jc) {
+                // sources per row block I >= Jc, children in accumulation order
+                std::vector<std::vector<int32_t>> src(R - Jc);
+                for (auto& h : hit[Jc])
+                    for (int32_t I : blocks[h.first])
+                        if (I >= Jc) src[I - Jc].push_back(h.second);
+                for (int32_t I = Jc; I < R; ++I) {
+                    if (Jc < p && src[I - Jc].empty()) continue;
+                    EaTask e{};
+                    e.front = J;
+                    e.I = I;
+                    e.J = Jc;
+                    e.src0 = (int32_t)P.ea_src.size();
+                    for (int32_t K : src[I - Jc]) {
+                        const Front& Kf = P.fronts[K];
+                        const int32_t* tb = P.sgstart.data() + P.sgoff[K];
+                        P.ea_src.push_back(EaSrc{Kf.uoff, Kf.reloff, Kf.na, tb[I], tb[I + 1], tb[Jc], tb[Jc + 1]});
+                    }
+                    e.src1 = (int32_t)P.ea_src.size();
+                    P.ea.push_back(e);
+                }
             }
         }
         L.ea1 = (int32_t)P.ea.size();
-        // window tables of the children read by this level's extend-add:
-        // wstart[wsoff[K] + w] = first row i of child K with rel_K[i] >= EA_WIN*w
-        for (int32_t J : L.big_list) {
-            const Front& F = P.fronts[J];
-            int32_t nw = (F.nn + F.na + EA_WIN - 1) / EA_WIN;
-            for (int32_t q = F.chd0; q < F.chd1; ++q) {
-                int32_t K = P.chd[q];
-                const Front& Kf = P.fronts[K];
-                P.wsoff[K] = (int32_t)P.wstart.size();
-                int32_t i = 0;
-                for (int32_t w = 0; w <= nw; ++w) {
-                    while (i < Kf.na && P.rel[Kf.reloff + i] < w * EA_WIN) ++i;
-                    P.wstart.push_back(i);
-                }
-            }
-        }
+        if (P.ea_src.size() > (size_t)INT32_MAX) return "too many extend-add sources";
         // diagonal tiles (the inverse-only pass of solves on given factors)
         for (int32_t J : L.big_list) {
             const Front& F = P.fronts[J];
@@ -544,9 +584,9 @@ std::string Planner::factor_tasks() {
 
     // ---- tile-DAG factorization of the big region -----------------------------
     // Row blocks of a big front: panel blocks [64K, 64K+kb_K) for K < p, then
-    // update rows [nn + 64m, ...).  Tile (I, K) of the panel carries a counter
-    // = number of panel columns applied; K+1 once it is final (factored or
-    // solved).  Order per level: small fronts, extend-add, then per panel step
+    // update rows [nn + 64m, ...).  Tile (I, K) of the panel carries a counter:
+    // 0 until its extend-add is done, 1 + the number of panel columns applied,
+    // K+2 once it is final (factored or solved).  Order per level: small fronts, extend-add, then per panel step
     // K: POTRF(K), TRSM(., K), the look-ahead column updates (., K+1, K), the
     // other updates; finally the update-matrix tiles (SYRK, K = nn).
     {
@@ -574,23 +614,20 @@ std::string Planner::factor_tasks() {
                 toff += (int64_t)D.R * D.p;
                 D.n_done = 0;  // counted with the update-matrix tiles below
             }
-            // extend-add groups: consecutive columns of one front, about
-            // EA_ROWS parent rows (each wave of the task takes every fourth
-            // column).  A group holds panel columns or update-matrix columns,
-            // never both: the panel's first diagonal tile waits only for the
-            // panel groups, the update-matrix tiles for all of them.
+            // extend-add tasks: consecutive tiles of one front, panel tiles or
+            // update-matrix tiles, never both (a panel task waits for its own
+            // tiles, an update-matrix tile's product for all of the front's
+            // tasks).  As many tiles per task as EA_ROWS allows where the level
+            // fills the chip, else one: a level's extend-add is on the critical
+            // path, and a tile takes 5.2 us of a workgroup
+            const int32_t gt = std::max(1, std::min(EA_ROWS / EA_TILE, (L.ea1 - L.ea0) / (2 * SIM_WORKERS)));
             for (int32_t e = L.ea0; e < L.ea1;) {
                 int32_t J = P.ea[e].front, e1 = e + 1;
-                const bool pan = P.ea[e].col < P.fronts[J].nn;
-                int64_t rows = P.ea[e].row1 - P.ea[e].row0;
-                while (e1 < L.ea1 && e1 - e < 64 && P.ea[e1].front == J && rows < EA_ROWS &&
-                       (P.ea[e1].col < P.fronts[J].nn) == pan) {
-                    rows += P.ea[e1].row1 - P.ea[e1].row0;
-                    ++e1;
-                }
+                const int32_t p = P.dagf[J].p;
+                const bool pan = P.ea[e].J < p;
+                while (e1 < L.ea1 && e1 - e < gt && P.ea[e1].front == J && (P.ea[e1].J < p) == pan) ++e1;
                 P.dag.push_back(DagTask{DT_EA, J, e, e1, pan ? 1 : 0, 0});
                 P.dagf[J].n_ea++;
-                if (pan) P.dagf[J].n_eap++;
                 e = e1;
             }
             int32_t maxp = 0;
@@ -691,52 +728,16 @@ std::string Planner::factor_tasks() {
                     }
             }
         }
+        if (toff > INT32_MAX) return "too many tiles";
         P.dag_counters = toff + 1;
+        P.cnt0.assign(P.dag_counters, 1);
+        for (const EaTask& e : P.ea)
+            if (e.J < P.dagf[e.front].p) P.cnt0[P.dagf[e.front].toff + e.J * P.dagf[e.front].R + e.I] = 0;
     }
     return std::string();
 }
 
 std::string Planner::solve_tasks() {
-    // ---- solve gather tables ----------------------------------------------------
-    // A solve task of a big front J covers one row block b of J (diagonal
-    // blocks [64b, 64b + 64) for b < p, then update rows [nn + 64(b-p), ...)).
-    // For each child K of J, sgstart[sgoff[K] + b] is the first row i of K
-    // with rel_K[i] >= the first row of block b (rel is increasing), b = 0..R,
-    // so the rows of K landing in block b are [tab[b], tab[b+1]).
-    P.sgoff.assign(NJ, -1);
-    P.sgstart.clear();
-    for (int32_t J = 0; J < NJ; ++J) {
-        if (P.is_small[J]) continue;
-        const Front& F = P.fronts[J];
-        const int32_t p = (F.nn + NB - 1) / NB, R = p + (F.na + NB - 1) / NB;
-        auto brow = [&](int32_t b) { return b < p ? std::min(b * NB, F.nn) : std::min(F.nn + (b - p) * NB, F.nn + F.na); };
-        for (int32_t q = F.chd0; q < F.chd1; ++q) {
-            const int32_t K = P.chd[q];
-            const Front& Kf = P.fronts[K];
-            P.sgoff[K] = (int32_t)P.sgstart.size();
-            int32_t i = 0;
-            for (int32_t b = 0; b <= R; ++b) {
-                const int32_t r0 = b < R ? brow(b) : F.nn + F.na;
-                while (i < Kf.na && P.rel[Kf.reloff + i] < r0) ++i;
-                P.sgstart.push_back(i);
-            }
-        }
-    }
-
-    for (int32_t J = 0; J < NJ; ++J) {
-        if (P.is_small[J]) continue;
-        const Front& F = P.fronts[J];
-        const int32_t R = (F.nn + NB - 1) / NB + (F.na + NB - 1) / NB;
-        for (int32_t q = F.chd0; q < F.chd1; ++q) {
-            const int32_t K = P.chd[q], o = P.sgoff[K];
-            if (o < 0 || (size_t)o + R + 1 > P.sgstart.size()) return "solve gather table";
-            for (int32_t b = 0; b <= R; ++b)
-                if (P.sgstart[o + b] < 0 || P.sgstart[o + b] > P.fronts[K].na ||
-                    (b > 0 && P.sgstart[o + b] < P.sgstart[o + b - 1]))
-                    return "solve gather table range";
-        }
-    }
-
     // ---- persistent solve task lists ------------------------------------------
     // Each direction is one ticket list.  Forward tickets are ordered by a
     // host list schedule (SIM_WORKERS workgroups, longest remaining path
@@ -1001,26 +1002,22 @@ std::string Planner::check_bounds() {
         }
         for (const EaTask& e : P.ea) {
             const Front& F = P.fronts[e.front];
-            int32_t nj = F.nn + F.na;
-            if (e.col < 0 || e.col >= nj || e.row0 != e.col || e.row1 != nj) return "ea task";
-            if (e.col >= F.nn && (F.uoff < 0 || F.uoff + (int64_t)F.na * F.na > P.u_elems))
-                return "ea U out of bounds";
-            for (int32_t s = e.src0; s < e.src1; ++s) {
-                int32_t K = P.ea_src[2 * s], tc = P.ea_src[2 * s + 1];
-                const Front& Kf = P.fronts[K];
-                if (Kf.parent != e.front || tc < 0 || tc >= Kf.na) return "ea source";
-                if (Kf.uoff < 0 || Kf.uoff + (int64_t)Kf.na * Kf.na > P.u_elems) return "ea child U";
-                int32_t nw = (nj + EA_WIN - 1) / EA_WIN;
-                if (P.wsoff[K] < 0 || (int64_t)P.wsoff[K] + nw >= (int64_t)P.wstart.size())
-                    return "ea window table";
-                for (int32_t w = 0; w < nw; ++w) {
-                    int32_t i0 = P.wstart[P.wsoff[K] + w], i1 = P.wstart[P.wsoff[K] + w + 1];
-                    if (i0 < 0 || i1 < i0 || i1 > Kf.na) return "ea window range";
-                    for (int32_t i = i0; i < i1; ++i) {
-                        int32_t pr = P.rel[Kf.reloff + i];
-                        if (pr < w * EA_WIN || pr >= (w + 1) * EA_WIN || pr >= nj) return "ea window row";
-                    }
-                }
+            const int32_t p = (F.nn + NB - 1) / NB, R = p + (F.na + NB - 1) / NB;
+            if (e.J < 0 || e.I < e.J || e.I >= R || P.is_small[e.front]) return "ea tile";
+            if (e.J >= p && (F.uoff < 0 || F.uoff + (int64_t)F.na * F.na > P.u_elems)) return "ea U out of bounds";
+            auto first = [&](int32_t b) { return b < p ? b * NB : F.nn + (b - p) * NB; };
+            auto last = [&](int32_t b) { return b < p ? std::min(F.nn, b * NB + NB) : std::min(F.nn + F.na, first(b) + NB); };
+            for (int32_t q = e.src0; q < e.src1; ++q) {
+                const EaSrc& x = P.ea_src[q];
+                if (x.ma <= 0 || x.u_off < 0 || x.u_off + (int64_t)x.ma * x.ma > P.u_elems) return "ea child U";
+                if (x.rel_off < 0 || (size_t)x.rel_off + x.ma > P.rel.size()) return "ea rel map";
+                if (x.ra < 0 || x.rb <= x.ra || x.rb > x.ma || x.rb - x.ra > NB || x.ta < 0 || x.tb <= x.ta ||
+                    x.tb > x.ma || x.tb - x.ta > NB)
+                    return "ea source range";
+                for (int32_t i : {x.ra, x.rb - 1})
+                    if (P.rel[x.rel_off + i] < first(e.I) || P.rel[x.rel_off + i] >= last(e.I)) return "ea source row";
+                for (int32_t i : {x.ta, x.tb - 1})
+                    if (P.rel[x.rel_off + i] < first(e.J) || P.rel[x.rel_off + i] >= last(e.J)) return "ea source column";
             }
         }
         for (size_t J = 0; J < P.fronts.size(); ++J) {
@@ -1138,10 +1135,10 @@ std::string Planner::check_bounds() {
 
 std::string Planner::dataflow() {
     // ---- dataflow form of the DAG ------------------------------------------------
-    // Predecessor edges per tile: POTRF(K) <- last update of (K,K) (or every
-    // extend-add task of the front for K = 0); TRSM(I,K) <- POTRF(K), last
-    // update of (I,K); UPD(I,Jc,K) <- the final tiles (I,K), (Jc,K) and the
-    // previous update of (I,Jc); SYRK <- the final last-column tiles of its row
+    // Predecessor edges per tile, its extend-add being its first update:
+    // POTRF(K) <- last update of (K,K); TRSM(I,K) <- POTRF(K), last update of
+    // (I,K); UPD(I,Jc,K) <- the final tiles (I,K), (Jc,K) and the previous
+    // update of (I,Jc); SYRK <- the final last-column tiles of its row
     // blocks.  A host run of the dataflow checks that every task executes.
     {
         const int32_t NT = (int32_t)P.dag.size();
@@ -1171,43 +1168,44 @@ std::string Planner::dataflow() {
         for (int32_t t = 0; t < NT; ++t) {
             const DagTask& d = P.dag[t];
             const int32_t J = d.front;
+            // the previous update of tile (I, K); none is needed before the
+            // first panel column when no child reaches the tile
+            auto after = [&](int32_t I, int32_t K, bool must) {
+                const int32_t w = lastw[tile(J, I, K)];
+                return w < 0 ? !must : edge(w, t);
+            };
             switch (d.kind) {
+                case DT_EA:
+                    for (int32_t e = d.a; d.c && e < d.b; ++e) lastw[tile(J, P.ea[e].I, P.ea[e].J)] = t;
+                    break;
                 case DT_POTRF:
-                    if (d.a == 0) {
-                        for (int32_t e = P.gtask0[J]; e < P.gtask1[J]; ++e)
-                            if (P.dag[e].kind != DT_EA || P.dag[e].c)
-                                if (!edge(e, t)) return "dataflow: potrf edge";
-                    } else if (!edge(lastw[tile(J, d.a, d.a)], t)) {
-                        return "dataflow: potrf without its update";
-                    }
-                    for (int32_t I = d.a + 1; d.a > 0 && I < P.dagf[J].R; ++I) {
+                    if (!after(d.a, d.a, d.a > 0)) return "dataflow: potrf without its update";
+                    for (int32_t I = d.a + 1; I < P.dagf[J].R; ++I) {
                         const int32_t pr = lastw[tile(J, I, d.a)];
-                        if (pr < 0 || pr >= t) return "dataflow: block column update after its diagonal tile";
-                        gmw_edges.push_back({t, pr});
+                        if ((pr < 0 && d.a > 0) || pr >= t) return "dataflow: block column update after its diagonal tile";
+                        if (pr >= 0) gmw_edges.push_back({t, pr});
                     }
                     fin[tile(J, d.a, d.a)] = t;
                     if (d.b >= 0) {  // fused panel solve of (a+1, a)
-                        if (d.a > 0 && !edge(lastw[tile(J, d.a + 1, d.a)], t))
-                            return "dataflow: fused trsm without its update";
+                        if (!after(d.a + 1, d.a, d.a > 0)) return "dataflow: fused trsm without its update";
                         fin[tile(J, d.a + 1, d.a)] = t;
                     }
                     if (d.c >= 0) {  // fused look-ahead update of (a+1, a+1)
                         if (d.b < 0) return "dataflow: fused update without the fused trsm";
-                        if (d.a > 0 && !edge(lastw[tile(J, d.a + 1, d.a + 1)], t))
-                            return "dataflow: fused update order";
+                        if (!after(d.a + 1, d.a + 1, d.a > 0)) return "dataflow: fused update order";
                         lastw[tile(J, d.a + 1, d.a + 1)] = t;
                     }
                     break;
                 case DT_TRSM:
                     if (!edge(fin[tile(J, d.c, d.c)], t)) return "dataflow: trsm without potrf";
-                    if (d.c > 0 && !edge(lastw[tile(J, d.b, d.c)], t)) return "dataflow: trsm without its update";
+                    if (!after(d.b, d.c, d.c > 0)) return "dataflow: trsm without its update";
                     fin[tile(J, d.b, d.c)] = t;
                     break;
                 case DT_UPD: {
                     const int32_t K0 = d.d & 0xffff, K1 = d.d >> 16;
                     if (!edge(fin[tile(J, d.b, K1 - 1)], t) || !edge(fin[tile(J, d.c, K1 - 1)], t))
                         return "dataflow: update without its operands";
-                    if (K0 > 0 && !edge(lastw[tile(J, d.b, d.c)], t)) return "dataflow: update order";
+                    if (!after(d.b, d.c, K0 > 0)) return "dataflow: update order";
                     lastw[tile(J, d.b, d.c)] = t;
                     break;
                 }
@@ -1364,27 +1362,25 @@ std::string Planner::schedule() {
         std::vector<double> cost(NT), bl(NT, 0.0), bgate(NJ, 0.0), bsyrk(NJ, 0.0);
         for (int32_t t = 0; t < NT; ++t) {
             const DagTask& d = P.dag[t];
-            // microseconds per task on one workgroup (measured on MI355X with
-            // two workgroups per CU): dispatch + extend-add rows / panel tile /
-            // MFMA work at the rate each tile shape reaches
-            double c = 5.0;
+            // microseconds per task on one workgroup, hand-off included (task
+            // trace of the 64^3 Laplacian in FP64, two workgroups per CU):
+            // extend-add tiles, the diagonal tile by its width, products by
+            // their k-extent in 64-column steps
+            double c = 2.0;
+            auto product = [&](const GemmTask& g) {
+                const double k = (double)g.k / NB;
+                return g.mode == G_TRSM ? 6.5 : g.wide ? 15.0 + 16.0 * k : 4.5 + 4.4 * k;
+            };
             switch (d.kind) {
-                case DT_EA: {
-                    double rows = 0;
-                    for (int32_t e = d.a; e < d.b; ++e) rows += P.ea[e].row1 - P.ea[e].row0;
-                    c += rows * 0.0053;
+                case DT_EA:
+                    for (int32_t e = d.a; e < d.b; ++e) c += 4.0 + 0.8 * (P.ea[e].src1 - P.ea[e].src0);
                     break;
-                }
                 case DT_SMALL: c += 20.0; break;
                 case DT_POTRF:
-                    c += 9.0;
-                    if (d.b >= 0) c += 6.0;  // the fused panel solve and update
+                    c += 4.0 + 0.2 * std::min(NB, P.fronts[d.front].nn - d.a * NB);
+                    if (d.b >= 0) c += 8.0;  // the fused panel solve and update
                     break;
-                default: {
-                    const GemmTask& g = P.gemm[d.a];
-                    c += 2.0 * g.m * g.n * (double)g.k / (g.wide ? 1.3e5 : 7.5e4);
-                    break;
-                }
+                default: c += product(P.gemm[d.a]); break;
             }
             cost[t] = c;
         }
@@ -1510,8 +1506,8 @@ std::string Planner::check_order() {
     // tile of its block column is updated through the previous column).
     auto validate_dag = [&](const std::vector<DagTask>& dg, bool gmw) -> const char* {
         const int32_t NT = (int32_t)dg.size();
-        std::vector<int32_t> last_ea(NJ, -1), last_pea(NJ, -1), first_panel(NJ, INT32_MAX), last_done(NJ, -1);
-        std::vector<int32_t> n_ea(NJ, 0), n_eap(NJ, 0);
+        std::vector<int32_t> last_ea(NJ, -1), last_done(NJ, -1), n_ea(NJ, 0);
+        std::vector<int32_t> ea_at(P.dag_counters + 1, -1);   // ticket of the tile's extend-add
         std::vector<int32_t> setter(P.dag_counters + 1, -1);  // ticket that finalizes (I, K) at value K+1
         std::map<int64_t, int32_t> upd_at;                      // (tile, K) -> ticket of UPD
         auto cnt_id = [&](int32_t J, int32_t I, int32_t K) {
@@ -1524,15 +1520,14 @@ std::string Planner::check_order() {
                 case DT_EA:
                     last_ea[d.front] = t;
                     n_ea[d.front]++;
-                    if (d.c) {
-                        last_pea[d.front] = t;
-                        n_eap[d.front]++;
+                    for (int32_t e = d.a; e < d.b; ++e) {
+                        if (P.ea[e].front != d.front || (P.ea[e].J < D.p) != (d.c != 0)) return "dag: extend-add task";
+                        if (d.c) ea_at[cnt_id(d.front, P.ea[e].I, P.ea[e].J)] = t;
                     }
                     break;
                 case DT_SMALL: last_done[d.front] = t; break;
                 case DT_POTRF:
                     setter[cnt_id(d.front, d.a, d.a)] = t;
-                    first_panel[d.front] = std::min(first_panel[d.front], t);
                     if (d.b >= 0) setter[cnt_id(d.front, d.a + 1, d.a)] = t;
                     if (d.c >= 0) upd_at[cnt_id(d.front, d.a + 1, d.a + 1) * 4096 + d.a] = t;
                     break;
@@ -1544,8 +1539,10 @@ std::string Planner::check_order() {
             if (d.kind >= DT_POTRF && (d.front < 0 || D.p <= 0)) return "dag task on a front without panel";
         }
         for (int32_t J = 0; J < NJ; ++J)
-            if (n_ea[J] > 0 && (n_ea[J] != P.dagf[J].n_ea || n_eap[J] != P.dagf[J].n_eap))
+            if (n_ea[J] > 0 && n_ea[J] != P.dagf[J].n_ea)
                 return "dag: extend-add counts";
+        for (int64_t q = 0; q < P.dag_counters; ++q)
+            if ((ea_at[q] >= 0) != (P.cnt0[q] == 0)) return "dag: tile counters and extend-add tiles disagree";
         std::vector<int32_t> last_consume(NJ, -1);
         for (int32_t t = 0; t < NT; ++t)
             if (dg[t].kind == DT_EA || dg[t].kind == DT_SMALL) last_consume[dg[t].front] = t;
@@ -1565,7 +1562,15 @@ std::string Planner::check_order() {
                 }
                 continue;
             }
-            if (last_pea[d.front] >= t) return "dag: panel task before extend-add";
+            // the tiles a panel task takes over from the extend-add
+            auto ea_done = [&](int32_t I, int32_t K) { return ea_at[cnt_id(d.front, I, K)] < t; };
+            if (d.kind == DT_POTRF) {
+                if (!ea_done(d.a, d.a) || (d.b >= 0 && !ea_done(d.a + 1, d.a)) || (d.c >= 0 && !ea_done(d.a + 1, d.a + 1)))
+                    return "dag: potrf before extend-add";
+                for (int32_t I = d.a + 1; gmw && I < P.dagf[d.front].R; ++I)
+                    if (!ea_done(I, d.a)) return "dag: potrf before its block column's extend-add";
+            }
+            if ((d.kind == DT_TRSM || d.kind == DT_UPD) && !ea_done(d.b, d.c)) return "dag: panel task before extend-add";
             if (d.kind == DT_SYRK && last_ea[d.front] >= t) return "dag: update-matrix tile before extend-add";
             auto need = [&](int32_t I, int32_t K) { return setter[cnt_id(d.front, I, K)]; };
             if (d.kind == DT_POTRF && d.a > 0) {
@@ -1645,6 +1650,7 @@ std::string build_plan(HostPlan& P, int64_t n, int64_t nfr, const int64_t* respt
     if (e.empty()) e = pl.amalgamate();
     if (e.empty()) e = pl.classify();
     if (e.empty()) e = pl.layout_memory();
+    if (e.empty()) e = pl.gather_tables();
     if (e.empty()) e = pl.factor_tasks();
     if (e.empty() && !tune.factor_only) e = pl.solve_tasks();
     if (e.empty()) e = pl.check_bounds();
@@ -1663,7 +1669,7 @@ std::string tuning_from(const int64_t* v, int64_t nv, PlanTuning* t) {
     const int64_t fu = (v && nv > 6 && v[6] >= 0) ? v[6] : t->fuse;
     const int64_t wc = (v && nv > 7 && v[7] >= 0) ? v[7] : t->wg_per_cu;
     if (ug < 1 || ug > 64) return "upd_group out of range (1..64)";
-    if (er < EA_WIN || er > (1 << 24)) return "ea_rows out of range";
+    if (er < 1024 || er > (1 << 24)) return "ea_rows out of range";
     if (wk < 1 || wk > (1 << 20)) return "wide_k out of range";
     if (sw < 1 || sw > 65536) return "sim_workers out of range";
     if (zf > 1000000) return "zero fraction above 1";
@@ -1697,12 +1703,10 @@ extern "C" int mf_plan_check(int64_t n, int64_t nfr, const int64_t* resptr, cons
         std::copy(err.begin(), err.begin() + k, msg);
         msg[k] = 0;
     }
-    int64_t ea_u = 0, ea_p = 0, ea_src_rows = 0;
+    int64_t ea_u = 0, ea_p = 0, ea_src_rows = 0;  // extend-add tiles (update matrix, panel), source rows
     for (const mf::EaTask& e : P.ea) {
-        const mf::Front& F = P.fronts[e.front];
-        (e.col >= F.nn ? ea_u : ea_p) += e.row1 - e.row0;
-        for (int32_t q = e.src0; q < e.src1; ++q)
-            ea_src_rows += P.fronts[P.ea_src[2 * q]].na - P.ea_src[2 * q + 1];
+        (e.J >= P.dagf[e.front].p ? ea_u : ea_p)++;
+        for (int32_t q = e.src0; q < e.src1; ++q) ea_src_rows += P.ea_src[q].rb - P.ea_src[q].ra;
     }
     int64_t v[] = {(int64_t)P.fronts.size(), P.n_small_region, P.n_big, (int64_t)P.levels.size(),
                    P.panel_elems, P.u_elems, P.w_elems, (int64_t)P.gemm.size(),

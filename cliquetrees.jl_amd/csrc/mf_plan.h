@@ -15,7 +15,7 @@ namespace mf {
 // 7-point Laplacian in FP64).
 struct PlanTuning {
     int32_t upd_group = UPD_GROUP;      // panel steps per trailing-update tile (1..64)
-    int32_t ea_rows = EA_ROWS;          // parent rows per extend-add task (>= EA_WIN)
+    int32_t ea_rows = EA_ROWS;          // elements per extend-add task (at most)
     int32_t wide_k = WIDE_K;            // 128 x 128 update-matrix tiles when nn >= wide_k
     int32_t sim_workers = SIM_WORKERS;  // resident workgroups of the ticket simulation
     double zero_frac = 0.05;            // explicit zeros allowed by a chain merge
@@ -65,9 +65,8 @@ struct HostPlan {
     std::vector<int32_t> level_small, level_big;
     std::vector<Level> levels;
     std::vector<EaTask> ea;
-    std::vector<int32_t> ea_src;       // pairs (child, child column)
-    std::vector<int32_t> wstart, wsoff;  // extend-add window tables per child (-1: none)
-    std::vector<int32_t> sgstart, sgoff;  // solve gather tables per child of a big front (-1: none)
+    std::vector<EaSrc> ea_src;
+    std::vector<int32_t> sgstart, sgoff;  // gather tables per child of a big front (-1: none)
     std::vector<GemmTask> gemm;
     std::vector<DiagTask> diag;
     std::vector<PTask> ftask, btask;   // forward / backward solve tasks, ticket order
@@ -76,6 +75,7 @@ struct HostPlan {
                                        // tile waits for its whole block column)
     std::vector<DagFront> dagf;        // per internal front (small region: n_done = 1)
     int64_t dag_counters = 0;          // tile counters
+    std::vector<int32_t> cnt0;         // their initial values
     std::vector<int32_t> uwait_ptr, uwait;  // per front: fronts whose extend-add must end
                                             // before the front's U slot is written
     // dataflow form of the DAG: a task runs once its predecessors are done;

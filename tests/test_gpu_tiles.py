@@ -61,3 +61,27 @@ def test_tile_edges(ct, oracle, nb, ns, kind):
     B = np.random.default_rng(5).standard_normal((A.shape[0], 3))
     X = ct.solve(F, B)
     assert np.linalg.norm(A @ X - B) <= rtol * np.linalg.norm(B)
+
+
+@pytest.mark.parametrize("kids,rows,ns", [(80, 20, 150), (70, 150, 150), (3, 65, 129), (130, 5, 66)])
+def test_extend_add_many_children(ct, oracle, kids, rows, ns):
+    """A root front whose tiles take from one child up to more children than a wavefront has
+    lanes, with scattered and with complete row sets."""
+    rng = np.random.default_rng(kids + rows)
+    nb = 3
+    n = nb * kids + ns
+    A = np.zeros((n, n))
+    for k in range(kids):
+        r = np.sort(rng.choice(ns, size=min(rows, ns), replace=False)) + nb * kids
+        A[np.ix_(r, range(nb * k, nb * k + nb))] = rng.uniform(-1, 1, (len(r), nb))
+        A[nb * k:nb * k + nb, nb * k:nb * k + nb] = rng.uniform(-1, 1, (nb, nb))
+    A[nb * kids:, nb * kids:] = rng.uniform(-1, 1, (ns, ns))
+    A = np.tril(A, -1)
+    A = A + A.T
+    A = sp.csc_matrix(A + np.diag(np.abs(A).sum(1) + 1.0))
+    P, S = ct.symbolic(A)
+    print(kids, rows, ns, S.nfr, flush=True)
+    Dv, Lv = oracle.assemble(S, P, A)
+    D, L, d, info = oracle.chol_impl(S, Dv, Lv)
+    F = ct.cholesky_(ct.ChordalCholesky(A, P, S))
+    assert info == 0 and _rel(F.Dval, D) <= 1e-12 and _rel(F.Lval, L) <= 1e-12
