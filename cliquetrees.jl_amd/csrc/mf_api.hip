@@ -89,6 +89,7 @@ struct mf_plan {
     std::vector<int32_t> col2ref;
     PTask* d_ftask = nullptr;
     PTask* d_btask = nullptr;
+    DevVPlan V;
     int32_t* d_ntf = nullptr;
     int32_t* d_ntb = nullptr;
     DagTask* d_dag = nullptr;
@@ -135,6 +136,7 @@ struct mf_factor {
     unsigned long long* info = nullptr;
     int32_t* flags = nullptr;
     int32_t* prog = nullptr;
+    void* xf = nullptr;         // forward solution of a solve of few columns
     uint32_t* ticket = nullptr;
     int32_t* hang = nullptr;
     double* gmw = nullptr;      // GMW81: reduction scratch, then beta (gmw[2])
@@ -426,6 +428,11 @@ void enqueue_solve(mf_factor* f, T* B, int64_t ldb, int nrhs, void* mv = nullptr
     DevSolve<T> S{B, ldb, (T*)(mv ? mv : f->Mv), nrhs};
     double bytes = (double)sizeof(T) * (2.0 * (double)(H.ndz + H.nlz) + 4.0 * H.n * nrhs);
     timed(f, MF_KC_SOLVE, bytes, 1, [&] {
+        if (nrhs <= VT_COLS) {
+            launch_solve1<T>(P, F, B, ldb, nrhs, (T*)f->xf, S.Mv, H.mv_elems1, pl->V, (int)H.n,
+                             f->prof ? f->strace_buf : nullptr, (int64_t)H.ftask.size(), f->stream);
+            return;
+        }
         launch_solve<T>(P, F, S, P.nJ, f->flags, f->prog, pl->d_ntf, pl->d_ntb, pl->d_ftask,
                         (int)H.ftask.size(), pl->d_btask, (int)H.btask.size(), (int)H.n,
                         f->prof ? f->strace_buf : nullptr, f->stream);
@@ -448,7 +455,11 @@ std::string hang_message(const mf_factor* f, const int32_t* h) {
     } bufs[] = {{"front flag/done", f->flags, nf1},
                 {"solve progress", f->prog, nf1},
                 {"tile counter", f->cnt, (size_t)H.dag_counters + 1},
-                {"extend-add counter", f->eacnt, nf1}};
+                {"extend-add counter", f->eacnt, nf1},
+                // (the single-column solves wait for the values themselves)
+                {"forward solution word", f->xf, 2 * VT_COLS * (size_t)(H.n + 1)},
+                {"solution word", f->Bws, f->Bws_bytes / 4},
+                {"update vector word", f->Mv, f->Mv_bytes / 4}};
     std::string where = "an unknown counter";
     for (const Buf& b : bufs) {
         const unsigned long long b0 = (unsigned long long)b.base;
@@ -517,6 +528,11 @@ static int plan_create(int64_t n, int64_t nfr, const int64_t* resptr, const int6
         (rc = upload(H.diag, (DiagTask**)&D.diag, pl->allocs)) ||
         (rc = upload(H.ftask, &pl->d_ftask, pl->allocs)) ||
         (rc = upload(H.btask, &pl->d_btask, pl->allocs)) ||
+        (rc = upload(H.vftask, (VTask**)&pl->V.ftask, pl->allocs)) ||
+        (rc = upload(H.vbtask, (VTask**)&pl->V.btask, pl->allocs)) ||
+        (rc = upload(H.vfunit, (int32_t**)&pl->V.funit, pl->allocs)) ||
+        (rc = upload(H.vbunit, (int32_t**)&pl->V.bunit, pl->allocs)) ||
+        (rc = upload(H.vchd, (VChild**)&pl->V.chd, pl->allocs)) ||
         (rc = upload(H.ntf, &pl->d_ntf, pl->allocs)) ||
         (rc = upload(H.ntb, &pl->d_ntb, pl->allocs)) ||
         (rc = upload(H.dag, &pl->d_dag, pl->allocs)) ||
@@ -534,6 +550,8 @@ static int plan_create(int64_t n, int64_t nfr, const int64_t* resptr, const int6
         return rc;
     }
     D.nJ = (int32_t)H.fronts.size();
+    pl->V.nfu = std::max<int32_t>(0, (int32_t)H.vfunit.size() - 1);
+    pl->V.nbu = std::max<int32_t>(0, (int32_t)H.vbunit.size() - 1);
     D.n = (int32_t)H.n;
     D.nfr = (int32_t)H.nfr;
     D.n_small_region = (int32_t)H.n_small_region;
@@ -628,7 +646,7 @@ static std::vector<std::pair<void**, size_t>> factor_buffers(mf_factor* f, const
         {(void**)&f->info, 64},       {(void**)&f->flags, 4 * nf},  {(void**)&f->prog, 4 * nf},
         {(void**)&f->ticket, 64},     {(void**)&f->hang, 64},       {(void**)&f->gmw, 64},
         {(void**)&f->cnt, 4 * (size_t)(H.dag_counters + 1)},        {(void**)&f->eacnt, 4 * nf},
-        {(void**)&f->perm_dev, 8 * n1}};
+        {(void**)&f->perm_dev, 8 * n1}, {&f->xf, 8 * n1 * VT_COLS}};
     v.insert(v.end(), std::begin(rest), std::end(rest));
     return v;
 }

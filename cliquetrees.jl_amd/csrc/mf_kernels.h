@@ -121,6 +121,36 @@ void launch_solve(const DevPlan& P, const DevFactor<T>& F, const DevSolve<T>& S,
                   int32_t* done, int32_t* prog, const int32_t* ntf, const int32_t* ntb,
                   const PTask* ftask, int nf, const PTask* btask, int nb, int n,
                   unsigned long long* trace, hipStream_t s);
+// One right-hand side (mf_solve1.hip): task lists of the plan, and the
+// arguments of one direction.
+struct DevVPlan {
+    const VTask* ftask = nullptr;
+    const VTask* btask = nullptr;
+    const int32_t* funit = nullptr;
+    const int32_t* bunit = nullptr;
+    const VChild* chd = nullptr;
+    int32_t nfu = 0, nbu = 0;
+};
+template <typename T>
+struct DevVSolve {
+    const T* in;
+    T* out;
+    T* Mv;
+    T* wipe;                 // forward: the input, unset once read
+    int64_t ldin, ldout, mvs;  // column strides of in (and wipe), out, Mv
+    const VTask* task;
+    const int32_t* unit;
+    int32_t nunit, cols;
+    const VChild* chd;
+    uint32_t* ticket;
+    unsigned long long* trace;
+};
+// B: the permuted right-hand sides, overwritten by the solutions; X: n x cols
+// elements of scratch (the forward solutions); Mv: mvs x cols update-vector
+// elements; F.ticket: two tickets.
+template <typename T>
+void launch_solve1(const DevPlan& P, const DevFactor<T>& F, T* B, int64_t ldb, int cols, T* X, T* Mv, int64_t mvs,
+                   const DevVPlan& D, int n, unsigned long long* trace, int64_t ntrace_f, hipStream_t s);
 template <typename TB>
 void launch_permute(const double* src, int64_t lds, TB* dst, int64_t ldd, const int64_t* perm,
                     int n, int nrhs, bool inverse, hipStream_t s);

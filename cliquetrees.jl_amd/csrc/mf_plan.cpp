@@ -95,6 +95,7 @@ class Planner {
     std::string gather_tables();  // children's rows per row block of a big front
     std::string factor_tasks();   // 4. extend-add, diagonal and tile-DAG tasks
     std::string solve_tasks();    // persistent solve task lists
+    std::string vector_tasks();   // those of one right-hand side
     std::string check_bounds();   // every task's accesses inside its pools
     std::string dataflow();       // predecessor counts and successor lists of the DAG
     std::string schedule();       // tickets by list scheduling (and the GMW81 order)
@@ -937,18 +938,23 @@ std::string Planner::solve_tasks() {
         }
     }
 
+    std::string err = vector_tasks();
+    if (!err.empty()) return err;
+
     // consecutive tickets of tiny fronts share one ticket, one wavefront each
     // (a front may wait for another front of the same ticket: that one runs
     // on another wavefront of the workgroup, so it makes progress)
     for (std::vector<PTask>* tl : {&P.ftask, &P.btask}) {
         std::vector<PTask> out;
         out.reserve(tl->size());
+        std::vector<int32_t> at(tl->size());  // ticket of every task
         auto tiny = [&](const PTask& t) {
             const Front& F = P.fronts[t.front];
             return t.kind == PT_SMALL && F.nn + F.na <= TINY_NJ;
         };
         for (size_t i = 0; i < tl->size();) {
             if (!tiny((*tl)[i])) {
+                at[i] = (int32_t)out.size();
                 out.push_back((*tl)[i]);
                 if (out.back().kind != PT_SEPB) out.back().c = 0;
                 ++i;
@@ -956,10 +962,122 @@ std::string Planner::solve_tasks() {
             }
             int32_t fr[4] = {-1, -1, -1, -1};
             int n = 0;
-            while (n < 4 && i < tl->size() && tiny((*tl)[i])) fr[n++] = (*tl)[i++].front;
+            while (n < 4 && i < tl->size() && tiny((*tl)[i])) {
+                at[i] = (int32_t)out.size();
+                fr[n++] = (*tl)[i++].front;
+            }
             out.push_back(PTask{PT_TINY, fr[0], fr[1], fr[2], fr[3]});
         }
         tl->swap(out);
+        for (VTask& t : tl == &P.ftask ? P.vftask : P.vbtask) t.t0 = at[t.t0];
+    }
+    return std::string();
+}
+
+// The task lists of the single-column solves, from the ungrouped ftask and
+// btask: small fronts in groups of up to four (a front joins the open group,
+// which keeps the place of its first member, when what it waits for is at or
+// before that place), one-block fronts with few row blocks in one forward
+// task.  Every wait still points to an earlier task or an earlier member of
+// the same group (another wavefront of the same workgroup).
+std::string Planner::vector_tasks() {
+    P.vchd.resize(P.chd.size());
+    for (size_t q = 0; q < P.chd.size(); ++q) {
+        const int32_t K = P.chd[q];
+        P.vchd[q] = VChild{P.mvoff1[K], P.fronts[K].na, P.fronts[K].reloff, P.sgoff[K], 0};
+    }
+    for (int dir = 0; dir < 2; ++dir) {
+        const std::vector<PTask>& in = dir ? P.btask : P.ftask;
+        std::vector<VTask>& out = dir ? P.vbtask : P.vftask;
+        out.clear();
+        std::vector<int32_t> pos(NJ, -1);  // last task of each front so far
+        int32_t open = -1, members = 0, used = 0;
+        for (size_t i = 0; i < in.size(); ++i) {
+            const PTask& t = in[i];
+            const int32_t J = t.front, t0 = (int32_t)i;
+            const Front& F = P.fronts[J];
+            if (t.kind == PT_SMALL) {
+                const int32_t size = ((F.nn + F.na) | 1) * F.nn;
+                bool join = open >= 0 && members < 4 && used + size <= VT_PANELS;
+                if (dir) join = join && (F.parent < 0 || pos[F.parent] <= open);
+                else
+                    for (int32_t q = F.chd0; q < F.chd1 && join; ++q) join = pos[P.chd[q]] <= open;
+                if (!join) {
+                    open = (int32_t)out.size();
+                    members = used = 0;
+                    out.push_back(VTask{VT_SMALL, -1, -1, -1, -1, 0, 0, t0});
+                }
+                VTask& v = out[open];
+                if (members == 0) v.a = J;
+                else if (members == 1) v.b = J, v.o12 |= used;
+                else if (members == 2) v.c = J, v.o12 |= used << 16;
+                else v.d = J, v.o3 = used;
+                ++members;
+                used += size;
+                pos[J] = open;
+                continue;
+            }
+            const bool one = dir == 0 && F.nn <= NB && F.na <= VT_ROWBLOCKS * NB;
+            if (one && t.kind == PT_ROWS) continue;  // part of the front's task
+            if (one) out.push_back(VTask{VT_FRONT, J, 0, 0, 0, 0, 0, t0});
+            else if (t.kind == PT_DIAG) out.push_back(VTask{VT_DIAG, J, t.a, t.b, 0, 0, 0, t0});
+            else if (t.kind == PT_ROWS) out.push_back(VTask{VT_ROWS, J, t.a, t.b, 0, 0, 0, t0});
+            else out.push_back(VTask{VT_SEPB, J, t.a, t.b, t.c, 0, 0, t0});
+            pos[J] = (int32_t)out.size() - 1;
+        }
+        // tasks per ticket: one near both ends of the list (the root path),
+        // up to four in between, where many more tasks are ready than
+        // workgroups run and the ticket counter would set the pace
+        std::vector<int32_t>& unit = dir ? P.vbunit : P.vfunit;
+        unit.assign(1, 0);
+        const int32_t N = (int32_t)out.size();
+        for (int32_t i = 0; i < N;) {
+            i = std::min(N, i + std::min(4, 1 + std::min(i, N - i) / 2048));
+            unit.push_back(i);
+        }
+        // every wait points to an earlier task, or an earlier member of a group
+        std::vector<int64_t> first(NJ, -1), last(NJ, -1);
+        std::vector<int32_t> done(NJ, 0);  // diagonal blocks seen, in chain order
+        for (int32_t i = 0; i < N; ++i) {
+            const VTask& v = out[i];
+            if (v.kind == VT_SMALL) {
+                const int32_t fr[4] = {v.a, v.b, v.c, v.d}, at[4] = {0, v.o12 & 0xffff, (v.o12 >> 16) & 0xffff, v.o3};
+                int32_t end = 0;
+                for (int32_t s = 0; s < 4; ++s) {
+                    const int32_t J = fr[s];
+                    if (J < 0) continue;
+                    if (!P.is_small[J] || first[J] >= 0 || at[s] != end) return "vector solve group";
+                    end += ((P.fronts[J].nn + P.fronts[J].na) | 1) * P.fronts[J].nn;
+                    first[J] = last[J] = 4 * (int64_t)i + s;
+                }
+                if (end > VT_PANELS) return "vector solve group size";
+                continue;
+            }
+            const Front& F = P.fronts[v.a];
+            const int32_t p = (F.nn + NB - 1) / NB;
+            if (P.is_small[v.a] || F.woff < 0) return "vector solve front";
+            if (first[v.a] < 0) first[v.a] = 4 * (int64_t)i;
+            last[v.a] = 4 * (int64_t)i;
+            if (v.kind == VT_FRONT) {
+                if (dir || p != 1 || F.na > VT_ROWBLOCKS * NB) return "vector solve one-task front";
+                done[v.a] = p;
+            } else if (v.kind == VT_DIAG) {
+                if (v.b / NB != (dir ? p - 1 - done[v.a] : done[v.a]) || v.c != std::min(NB, F.nn - v.b)) return "vector solve chain";
+                done[v.a]++;
+            } else if (v.kind == VT_ROWS) {
+                if (dir || done[v.a] != p || v.b < F.nn || v.c > F.nn + F.na || v.c - v.b > NB || (v.b - F.nn) % NB)
+                    return "vector solve rows";
+            } else if (!dir || done[v.a] != 0 || P.sboff1[v.a] < 0) {
+                return "vector solve separator task";
+            }
+        }
+        for (int32_t J = 0; J < NJ; ++J) {
+            const Front& F = P.fronts[J];
+            if (first[J] < 0 || (!P.is_small[J] && done[J] != (F.nn + NB - 1) / NB)) return "vector solve task missing";
+            if (F.parent < 0) continue;
+            const bool ok = dir ? last[F.parent] < first[J] : last[J] < first[F.parent];
+            if (!ok) return "vector solve order";
+        }
     }
     return std::string();
 }

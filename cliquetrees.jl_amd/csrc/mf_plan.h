@@ -40,6 +40,27 @@ struct PTask {
     int32_t c;
 };
 
+// Task of the solves of one right-hand side, and the runs of tasks that one
+// ticket covers.  VT_SMALL: up to four small fronts a, b, c, d (-1: absent),
+// one wavefront each, their panels (leading dimension nJ | 1) in LDS from 0,
+// o12 & 0xffff, o12 >> 16 and o3; VT_FRONT (forward): the front a, one
+// diagonal block and at most VT_ROWBLOCKS row blocks; VT_DIAG: diagonal block
+// [b, b + c) of front a; VT_ROWS: update rows [b, c) of front a; VT_SEPB
+// (backward): separator tiles [c, d) of diagonal block b of front a.  t0: the
+// ticket of the same work in ftask / btask (its first, when merged).
+enum : int32_t { VT_SMALL = 0, VT_FRONT = 1, VT_DIAG = 2, VT_ROWS = 3, VT_SEPB = 4 };
+struct VTask {
+    int32_t kind, a, b, c, d;
+    int32_t o12, o3;
+    int32_t t0;
+};
+// A child in chd[] order: update vector, rel map and gather table.
+struct VChild {
+    int64_t mv;
+    int32_t ma, rel, sg;
+    int32_t pad;
+};
+
 struct Level {
     std::vector<int32_t> small_list;   // small fronts living in the big region
     std::vector<int32_t> big_list;
@@ -70,6 +91,9 @@ struct HostPlan {
     std::vector<GemmTask> gemm;
     std::vector<DiagTask> diag;
     std::vector<PTask> ftask, btask;   // forward / backward solve tasks, ticket order
+    std::vector<VTask> vftask, vbtask; // the same for one right-hand side
+    std::vector<int32_t> vfunit, vbunit;  // ticket u covers tasks [unit[u], unit[u + 1])
+    std::vector<VChild> vchd;          // per entry of chd
     std::vector<DagTask> dag;          // tile-DAG factorization of the big region
     std::vector<DagTask> dag_gmw;      // the same tasks in creation order (GMW81: a diagonal
                                        // tile waits for its whole block column)

@@ -1,4 +1,5 @@
-// mf_solve.hip — gfx950 kernels of the supernodal triangular solves.
+// mf_solve.hip — gfx950 kernels of the supernodal triangular solves, right-hand
+// sides in blocks of 16 (mf_solve1.hip: up to VT_COLS, column by column).
 //
 // Forward  C <- L^-1 C  (div_impl! forward, divide.jl:417-450; per front:
 //   F <- sum_i R_i M_i (div_fwd_update!, divide.jl:1206-1248), C1 += F1,
