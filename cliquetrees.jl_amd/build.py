@@ -16,7 +16,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 ARCH = os.environ.get("MF_OFFLOAD_ARCH", "gfx950")
 
-HIP_SOURCES = ["mf_api.hip", "mf_factor.hip", "mf_solve.hip", "mf_solve1.hip", "mf_refine.hip", "mf_selinv.hip",
+HIP_SOURCES = ["mf_api.hip", "mf_factor.hip", "mf_solve.hip", "mf_solve1.hip", "mf_solve16.hip", "mf_refine.hip", "mf_selinv.hip",
                "mf_complete.hip", "mf_plan.cpp", "mf_selinv_plan.cpp"]
 SYM_SOURCES = ["symbolic.cpp", "mmd.cpp", "mf_plan.cpp", "mf_selinv_plan.cpp"]
 

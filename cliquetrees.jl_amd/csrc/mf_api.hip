@@ -87,11 +87,7 @@ struct mf_plan {
     std::vector<void*> allocs;
     std::vector<uint8_t> in_small;
     std::vector<int32_t> col2ref;
-    PTask* d_ftask = nullptr;
-    PTask* d_btask = nullptr;
     DevVPlan V;
-    int32_t* d_ntf = nullptr;
-    int32_t* d_ntb = nullptr;
     DagTask* d_dag = nullptr;
     DagTask* d_dag_gmw = nullptr;  // the same tasks in creation order (GMW81 factorizations)
     DagFront* d_dagf = nullptr;
@@ -135,7 +131,6 @@ struct mf_factor {
     double* signs = nullptr;
     unsigned long long* info = nullptr;
     int32_t* flags = nullptr;
-    int32_t* prog = nullptr;
     void* xf = nullptr;         // forward solution of a solve of few columns
     uint32_t* ticket = nullptr;
     int32_t* hang = nullptr;
@@ -160,6 +155,8 @@ struct mf_factor {
     size_t stage_bytes = 0;
     void* Mv = nullptr;
     size_t Mv_bytes = 0;
+    void* sw = nullptr;         // solutions of the blocked solves, row by row
+    size_t sw_bytes = 0;
     void* Bws = nullptr;
     size_t Bws_bytes = 0;
     bool solve64 = false;       // FP32 factor: solves in FP64 arithmetic on a widened copy
@@ -198,6 +195,7 @@ struct mf_factor {
         if (A_colptr) (void)hipFree(A_colptr);
         if (A_rowval) (void)hipFree(A_rowval);
         if (A_val) (void)hipFree(A_val);
+        if (sw) (void)hipFree(sw);
         if (Bws) (void)hipFree(Bws);
         if (stage) (void)hipFree(stage);
         if (tgt_panel) (void)hipFree(tgt_panel);
@@ -414,10 +412,29 @@ void sync_ref(mf_factor* f) {
     f->ref_stale = false;
 }
 
-// mv: the update-vector workspace (mv_elems1 x nrhs elements); NULL takes
-// the factor's own.
+// Columns of the blocked solves: blocks of sixteen.
+size_t padded(size_t nrhs) { return (nrhs + 15) & ~(size_t)15; }
+
+// Workspaces of the solves of nrhs columns: update vectors, and for the
+// blocked solves the solutions in their row-by-row form.  Without memory for
+// these the columns are solved VT_COLS at a time.
+int ensure_solve(mf_factor* f, size_t es, size_t nrhs) {
+    const HostPlan& H = f->plan->H;
+    if (nrhs > (size_t)VT_COLS) {
+        const size_t c = padded(nrhs);
+        if (ensure(&f->Mv, &f->Mv_bytes, es * (size_t)H.mv_elems1 * c) == MF_OK &&
+            ensure(&f->sw, &f->sw_bytes, es * 2 * (size_t)H.n * c) == MF_OK)
+            return MF_OK;
+        (void)hipGetLastError();
+        nrhs = VT_COLS;
+    }
+    return ensure(&f->Mv, &f->Mv_bytes, es * (size_t)H.mv_elems1 * nrhs);
+}
+
+// mv, sw: the update-vector and solution workspaces (ensure_solve) instead of
+// the factor's own; blocked: they hold the blocked form.
 template <typename T>
-void enqueue_solve(mf_factor* f, T* B, int64_t ldb, int nrhs, void* mv = nullptr) {
+void enqueue_solve(mf_factor* f, T* B, int64_t ldb, int nrhs, void* mv = nullptr, void* sw = nullptr, bool blocked = false) {
     mf_plan* pl = f->plan;
     const HostPlan& H = pl->H;
     const DevPlan& P = pl->D;
@@ -425,17 +442,23 @@ void enqueue_solve(mf_factor* f, T* B, int64_t ldb, int nrhs, void* mv = nullptr
     if constexpr (sizeof(T) == 8) {
         if (solves64(f)) F = dev_factor_solve64(f);
     }
-    DevSolve<T> S{B, ldb, (T*)(mv ? mv : f->Mv), nrhs};
+    if (!mv) {
+        mv = f->Mv;
+        sw = f->sw;
+        const size_t c = padded(nrhs);
+        blocked = f->Mv_bytes >= sizeof(T) * (size_t)H.mv_elems1 * c && f->sw_bytes >= sizeof(T) * 2 * (size_t)H.n * c;
+    }
     double bytes = (double)sizeof(T) * (2.0 * (double)(H.ndz + H.nlz) + 4.0 * H.n * nrhs);
     timed(f, MF_KC_SOLVE, bytes, 1, [&] {
-        if (nrhs <= VT_COLS) {
-            launch_solve1<T>(P, F, B, ldb, nrhs, (T*)f->xf, S.Mv, H.mv_elems1, pl->V, (int)H.n,
-                             f->prof ? f->strace_buf : nullptr, (int64_t)H.ftask.size(), f->stream);
+        unsigned long long* trace = f->prof ? f->strace_buf : nullptr;
+        if (nrhs > VT_COLS && blocked) {
+            launch_solve16<T>(P, F, B, ldb, nrhs, (T*)sw, (T*)mv, H.mv_elems1, pl->V, trace, (int64_t)H.ftask.size(),
+                              f->stream);
             return;
         }
-        launch_solve<T>(P, F, S, P.nJ, f->flags, f->prog, pl->d_ntf, pl->d_ntb, pl->d_ftask,
-                        (int)H.ftask.size(), pl->d_btask, (int)H.btask.size(), (int)H.n,
-                        f->prof ? f->strace_buf : nullptr, f->stream);
+        for (int c = 0; c < nrhs; c += VT_COLS)
+            launch_solve1<T>(P, F, B + (int64_t)c * ldb, ldb, std::min(VT_COLS, nrhs - c), (T*)f->xf, (T*)mv, H.mv_elems1,
+                             pl->V, (int)H.n, trace, (int64_t)H.ftask.size(), f->stream);
     });
 }
 
@@ -453,12 +476,12 @@ std::string hang_message(const mf_factor* f, const int32_t* h) {
         const void* base;
         size_t n;
     } bufs[] = {{"front flag/done", f->flags, nf1},
-                {"solve progress", f->prog, nf1},
                 {"tile counter", f->cnt, (size_t)H.dag_counters + 1},
                 {"extend-add counter", f->eacnt, nf1},
                 // (the single-column solves wait for the values themselves)
                 {"forward solution word", f->xf, 2 * VT_COLS * (size_t)(H.n + 1)},
                 {"solution word", f->Bws, f->Bws_bytes / 4},
+                {"blocked solution word", f->sw, f->sw_bytes / 4},
                 {"update vector word", f->Mv, f->Mv_bytes / 4}};
     std::string where = "an unknown counter";
     for (const Buf& b : bufs) {
@@ -526,15 +549,11 @@ static int plan_create(int64_t n, int64_t nfr, const int64_t* resptr, const int6
         (rc = upload(H.sgoff, (int32_t**)&D.sgoff, pl->allocs)) ||
         (rc = upload(H.gemm, (GemmTask**)&D.gemm, pl->allocs)) ||
         (rc = upload(H.diag, (DiagTask**)&D.diag, pl->allocs)) ||
-        (rc = upload(H.ftask, &pl->d_ftask, pl->allocs)) ||
-        (rc = upload(H.btask, &pl->d_btask, pl->allocs)) ||
         (rc = upload(H.vftask, (VTask**)&pl->V.ftask, pl->allocs)) ||
         (rc = upload(H.vbtask, (VTask**)&pl->V.btask, pl->allocs)) ||
         (rc = upload(H.vfunit, (int32_t**)&pl->V.funit, pl->allocs)) ||
         (rc = upload(H.vbunit, (int32_t**)&pl->V.bunit, pl->allocs)) ||
         (rc = upload(H.vchd, (VChild**)&pl->V.chd, pl->allocs)) ||
-        (rc = upload(H.ntf, &pl->d_ntf, pl->allocs)) ||
-        (rc = upload(H.ntb, &pl->d_ntb, pl->allocs)) ||
         (rc = upload(H.dag, &pl->d_dag, pl->allocs)) ||
         (rc = upload(H.dag_gmw, &pl->d_dag_gmw, pl->allocs)) ||
         (rc = upload(H.dagf, &pl->d_dagf, pl->allocs)) ||
@@ -643,7 +662,7 @@ static std::vector<std::pair<void**, size_t>> factor_buffers(mf_factor* f, const
     }
     const std::pair<void**, size_t> rest[] = {
         {(void**)&f->dref, 8 * n1},   {(void**)&f->adiag, 8 * n1},  {(void**)&f->signs, 8 * n1},
-        {(void**)&f->info, 64},       {(void**)&f->flags, 4 * nf},  {(void**)&f->prog, 4 * nf},
+        {(void**)&f->info, 64},       {(void**)&f->flags, 4 * nf},
         {(void**)&f->ticket, 64},     {(void**)&f->hang, 64},       {(void**)&f->gmw, 64},
         {(void**)&f->cnt, 4 * (size_t)(H.dag_counters + 1)},        {(void**)&f->eacnt, 4 * nf},
         {(void**)&f->perm_dev, 8 * n1}, {&f->xf, 8 * n1 * VT_COLS}};
@@ -983,7 +1002,7 @@ int mf_solve_natural(mf_factor* f, double* C, int64_t nrhs, int64_t ldc, int dev
     if (nrhs == 0 || H.n == 0) return MF_OK;
     if (solves64(f) && !f->sh_valid) return fail(MF_ESTATE, "FP64 solves of an FP32 factor: factorize after enabling them");
     size_t es = solve_elt(f);
-    if (ensure(&f->Mv, &f->Mv_bytes, es * (size_t)H.mv_elems1 * nrhs)) return MF_ENOMEM;
+    if (ensure_solve(f, es, (size_t)nrhs)) return MF_ENOMEM;
     if ((f->precision == MF_FP64 || solves64(f)) && device) {
         enqueue_solve<double>(f, C, ldc, (int)nrhs);
     } else {
@@ -1038,7 +1057,7 @@ int mf_solve(mf_factor* f, const int64_t* perm, double* B, int64_t nrhs, int64_t
     if (nrhs == 0 || H.n == 0) return MF_OK;
     if (solves64(f) && !f->sh_valid) return fail(MF_ESTATE, "FP64 solves of an FP32 factor: factorize after enabling them");
     size_t es = solve_elt(f);
-    if (ensure(&f->Mv, &f->Mv_bytes, es * (size_t)H.mv_elems1 * nrhs)) return MF_ENOMEM;
+    if (ensure_solve(f, es, (size_t)nrhs)) return MF_ENOMEM;
     if (ensure(&f->Bws, &f->Bws_bytes, es * (size_t)H.n * nrhs)) return MF_ENOMEM;
     if (f->perm_host.size() != (size_t)H.n ||
         std::memcmp(f->perm_host.data(), perm, 8 * H.n) != 0) {
@@ -1086,7 +1105,7 @@ int mf_solve_noalloc(mf_factor* f, const int64_t* perm, double* B, int64_t nrhs,
     if (nrhs == 0 || H.n == 0) return MF_OK;
     if (solves64(f) && !f->sh_valid) return fail(MF_ESTATE, "FP64 solves of an FP32 factor: factorize after enabling them");
     const size_t es = solve_elt(f);
-    const size_t mv_bytes = (es * (size_t)H.mv_elems1 * (size_t)nrhs + 255) & ~(size_t)255;
+    size_t mv_bytes = (es * (size_t)H.mv_elems1 * (size_t)nrhs + 255) & ~(size_t)255;
     const size_t need = mv_bytes + es * (size_t)H.n * (size_t)nrhs;
     if (need > MF_NOALLOC_SCRATCH_BYTES)
         return fail(MF_EARG, "mf_solve_noalloc: " + std::to_string(need) + " bytes of scratch needed, limit " +
@@ -1096,8 +1115,14 @@ int mf_solve_noalloc(mf_factor* f, const int64_t* perm, double* B, int64_t nrhs,
     if (dev != f->device) return fail(MF_EARG, "the factor's device is not the current device");
     void* base = nullptr;
     if (int rc = scratch_address(&base)) return rc;
+    // the blocked solves where their workspaces fit as well, else VT_COLS columns at a time
+    const size_t cols = padded((size_t)nrhs);
+    const size_t mvb = (es * (size_t)H.mv_elems1 * cols + 255) & ~(size_t)255, swb = (es * 2 * (size_t)H.n * cols + 255) & ~(size_t)255;
+    const bool blocked = nrhs > VT_COLS && mvb + swb + es * (size_t)H.n * (size_t)nrhs <= MF_NOALLOC_SCRATCH_BYTES;
+    if (blocked) mv_bytes = mvb;
     void* mv = base;
-    void* bws = (unsigned char*)base + mv_bytes;
+    void* sw = (unsigned char*)base + mv_bytes;
+    void* bws = blocked ? (unsigned char*)sw + swb : (unsigned char*)sw;
     if (f->perm_host.size() != (size_t)H.n ||
         std::memcmp(f->perm_host.data(), perm, 8 * H.n) != 0) {
         f->perm_host.assign(perm, perm + H.n);
@@ -1107,12 +1132,12 @@ int mf_solve_noalloc(mf_factor* f, const int64_t* perm, double* B, int64_t nrhs,
     if (f->precision == MF_FP32 && !solves64(f)) {
         launch_permute<float>(B, ldb, (float*)bws, H.n, f->perm_dev, (int)H.n, (int)nrhs, false,
                               f->stream);
-        enqueue_solve<float>(f, (float*)bws, H.n, (int)nrhs, mv);
+        enqueue_solve<float>(f, (float*)bws, H.n, (int)nrhs, mv, sw, blocked);
         launch_permute_back(bws, H.n, true, B, ldb, f->perm_dev, (int)H.n, (int)nrhs, f->stream);
     } else {
         launch_permute<double>(B, ldb, (double*)bws, H.n, f->perm_dev, (int)H.n, (int)nrhs, false,
                                f->stream);
-        enqueue_solve<double>(f, (double*)bws, H.n, (int)nrhs, mv);
+        enqueue_solve<double>(f, (double*)bws, H.n, (int)nrhs, mv, sw, blocked);
         launch_permute_back(bws, H.n, false, B, ldb, f->perm_dev, (int)H.n, (int)nrhs, f->stream);
     }
     HIPCHK(hipGetLastError());
@@ -1303,7 +1328,7 @@ int mf_div_impl(mf_plan* plan, const double* Dval, const double* Lval, const dou
 
 int mf_factor_bytes(const mf_factor* f, int64_t* bytes) {
     if (!f || !bytes) return fail(MF_EARG, "null argument");
-    size_t b = f->alloc_bytes + f->Mv_bytes + f->Bws_bytes + f->ir_ws_bytes + f->stage_bytes;
+    size_t b = f->alloc_bytes + f->Mv_bytes + f->sw_bytes + f->Bws_bytes + f->ir_ws_bytes + f->stage_bytes;
     if (f->A_n >= 0) b += 8 * (size_t)(f->A_n + 1) + 16 * (size_t)std::max<int64_t>(f->A_nnz, 1);
     if (f->nnz >= 0) b += 16 * (size_t)std::max<int64_t>(f->nnz, 2);
     *bytes = (int64_t)b;

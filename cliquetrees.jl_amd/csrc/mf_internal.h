@@ -29,7 +29,7 @@ constexpr int EA_ROWS = 16384;  // elements per extend-add task (at most, where 
 constexpr int WIDE_K = 128;     // update-matrix tiles are 128 x 128 when nn >= WIDE_K
 constexpr int UPD_GROUP = 8;    // panel steps applied by one trailing-update tile
 constexpr int SIM_WORKERS = 512;  // resident workgroups assumed when ordering the DAG tickets
-constexpr int VT_COLS = 4;                // right-hand sides solved column by column (more: blocked)
+constexpr int VT_COLS = 5;                // right-hand sides solved column by column (more: blocked)
 constexpr int VT_ROWBLOCKS = 4;           // row blocks of a one-task front of the single-column solves
 constexpr int VT_PANELS = 64 * 65;        // elements of the panels of their grouped small fronts
 constexpr int SEP_TILES = 8;    // separator tiles per backward partial-product task (fronts whose

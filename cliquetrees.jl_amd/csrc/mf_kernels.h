@@ -105,24 +105,9 @@ void launch_widen(const float* src, double* dst, int64_t count, hipStream_t s);
 template <typename T>
 void launch_gmw_beta(const DevPlan& P, const DevFactor<T>& F, double* gmw, int64_t n, hipStream_t s);
 
-// ---- solves (mf_solve.hip) ----
-template <typename T>
-struct DevSolve {
-    T* B;        // n x nrhs, permuted order
-    int64_t ldb;
-    T* Mv;       // update vectors, na_J x nrhs at mvoff1[J]*nrhs
-    int nrhs;
-};
-// Forward (children first) and backward (parents first) persistent solves,
-// the D^-1 scaling in between for LDLt.
-// trace: nullptr, or 2 (nf + nb) slots for per-ticket start / end ticks.
-template <typename T>
-void launch_solve(const DevPlan& P, const DevFactor<T>& F, const DevSolve<T>& S, int nJ,
-                  int32_t* done, int32_t* prog, const int32_t* ntf, const int32_t* ntb,
-                  const PTask* ftask, int nf, const PTask* btask, int nb, int n,
-                  unsigned long long* trace, hipStream_t s);
-// One right-hand side (mf_solve1.hip): task lists of the plan, and the
-// arguments of one direction.
+// ---- solves (mf_solve1.hip, mf_solve16.hip; permutations: mf_solve.hip) ----
+// Task lists of the plan, and the arguments of one direction of the solves
+// column by column (mf_solve1.hip).
 struct DevVPlan {
     const VTask* ftask = nullptr;
     const VTask* btask = nullptr;
@@ -151,6 +136,26 @@ struct DevVSolve {
 template <typename T>
 void launch_solve1(const DevPlan& P, const DevFactor<T>& F, T* B, int64_t ldb, int cols, T* X, T* Mv, int64_t mvs,
                    const DevVPlan& D, int n, unsigned long long* trace, int64_t ntrace_f, hipStream_t s);
+// Blocks of sixteen columns (mf_solve16.hip).  XZ: 2 x n x cols elements of
+// scratch, Mv: mvs x cols, cols = nrhs rounded up to a multiple of 16.
+template <typename T>
+struct DevBSolve {
+    T* B;                    // n x nrhs: right-hand sides, then solutions
+    T* X;                    // forward solution, per block n rows of sixteen
+    T* Z;                    // backward solution
+    T* Mv;
+    int64_t ldb, mvs;
+    int32_t nrhs, ncol;      // all columns; those of the current block
+    const VTask* task;
+    const int32_t* unit;
+    int32_t nunit;
+    const VChild* chd;
+    uint32_t* ticket;
+    unsigned long long* trace;
+};
+template <typename T>
+void launch_solve16(const DevPlan& P, const DevFactor<T>& F, T* B, int64_t ldb, int nrhs, T* XZ, T* Mv, int64_t mvs,
+                    const DevVPlan& D, unsigned long long* trace, int64_t ntrace_f, hipStream_t s);
 template <typename TB>
 void launch_permute(const double* src, int64_t lds, TB* dst, int64_t ldd, const int64_t* perm,
                     int n, int nrhs, bool inverse, hipStream_t s);

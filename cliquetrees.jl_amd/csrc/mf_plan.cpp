@@ -750,8 +750,6 @@ std::string Planner::solve_tasks() {
     // = diagonal blocks p-1..0 (a chain) after every task of its parent.
     P.ftask.clear();
     P.btask.clear();
-    P.ntf.assign(NJ, 0);
-    P.ntb.assign(NJ, 0);
     {
         auto nblk = [&](int32_t J) { return (P.fronts[J].nn + NB - 1) / NB; };
         auto nrow = [&](int32_t J) { return (P.fronts[J].na + NB - 1) / NB; };
@@ -874,7 +872,6 @@ std::string Planner::solve_tasks() {
                     const int32_t r0 = F.nn + (x.step - pk) * NB;
                     P.ftask.push_back(PTask{PT_ROWS, x.J, r0, std::min(F.nn + F.na, r0 + NB)});
                 }
-                P.ntf[x.J]++;
             }
         }
         // backward: the big region by depth (distance from the root): a
@@ -901,7 +898,6 @@ std::string Planner::solve_tasks() {
             for (int32_t d = 0; d <= maxd; ++d) {
                 for (int32_t J : small_at[d]) {
                     P.btask.push_back(PTask{PT_SMALL, J, 0, 0});
-                    P.ntb[J] = 1;
                 }
                 for (int32_t J : big_at[d]) {
                     if (P.sboff1[J] < 0) continue;
@@ -910,7 +906,6 @@ std::string Planner::solve_tasks() {
                     for (int32_t k = nblk(J) - 1; k >= 0; --k)
                         for (int32_t t0 = 0; t0 < nsep; t0 += SEP_TILES) {
                             P.btask.push_back(PTask{PT_SEPB, J, k * NB, t0, std::min(nsep, t0 + SEP_TILES)});
-                            P.ntb[J]++;
                         }
                 }
                 int32_t maxp = 0;
@@ -921,7 +916,6 @@ std::string Planner::solve_tasks() {
                         if (k >= 0) {
                             const Front& F = P.fronts[J];
                             P.btask.push_back(PTask{PT_DIAG, J, k * NB, std::min(NB, F.nn - k * NB)});
-                            P.ntb[J]++;
                         }
                     }
             }
@@ -934,7 +928,6 @@ std::string Planner::solve_tasks() {
         std::stable_sort(border.begin(), border.end(), [&](int32_t a, int32_t b) { return depth[a] < depth[b]; });
         for (int32_t J : border) {
             P.btask.push_back(PTask{PT_SMALL, J, 0, 0});
-            P.ntb[J] = 1;
         }
     }
 

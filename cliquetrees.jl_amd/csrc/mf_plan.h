@@ -116,7 +116,6 @@ struct HostPlan {
     std::vector<int32_t> init_hi, init_lo;  // tasks ready at the start, per queue
     int32_t n_hi = 0, n_lo = 0;             // tasks per queue
     double sim_makespan_us = 0;             // list-scheduled length of the DAG (estimate)
-    std::vector<int32_t> ntf, ntb;     // tasks per front (completion counts)
     std::vector<int64_t> mvoff1;       // per internal front: offset of Mv (na x 1)
     std::vector<int64_t> sboff1;       // per internal front: offset (per right-hand side) of its
                                        // backward separator partials (p x nch slots of 64 rows),

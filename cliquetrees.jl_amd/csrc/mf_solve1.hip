@@ -33,94 +33,23 @@
 // Several columns are independent solves that share the launch (the ticket
 // order is unit by unit, the columns of a unit side by side).
 //
-// Both directions with the permutations, blocked kernels -> these, us:
-//   56 x 60 x 52 grid, n 174720, 1 column     2237 -> 867, 4 columns 1650
-//   31 x 29 x 27 grid, n 24273, 1 / 3 columns  670 -> 179 / 241
-//   100 x 100 grid (minimum degree), 1 / 4     390 -> 120 / 191
-// The blocked kernels' times hardly depend on the columns up to 16, so the
-// line between them (VT_COLS = 4) lies below the crossing of the largest of
-// these (about 5.5 columns; 10 and 13 for the others).
+// Both directions with the permutations, us, 1 / 3 / 4 / 6 / 8 columns, and
+// mf_solve16.hip for up to 16 (its time hardly depends on the columns); with
+// per-front counters and matrix instructions for one column before:
+//   56 x 60 x 52 grid, n 174720   867 / 1350 / 1650 / 2290 / 2900   2030   (2237)
+//   31 x 29 x 27 grid, n 24273    179 /  241 /  278 /  360 /  439    415   (670)
+//   100 x 100 grid, n 10000       120 /  163 /  191 /  249 /  307    270   (390)
+// so the line (VT_COLS = 5) is where the largest of these crosses.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
-#include <type_traits>
 
 #include "mf_kernels.h"
-#include "mf_sync.h"
+#include "mf_vsolve.h"
 
 namespace mf {
 
 namespace {
-
-template <typename T>
-using bits_t = typename std::conditional<sizeof(T) == 8, unsigned long long, uint32_t>::type;
-// Signalling NaNs: every arithmetic instruction returns a quiet one.
-template <typename T>
-__device__ __forceinline__ constexpr bits_t<T> unset() {
-    if constexpr (sizeof(T) == 8) return 0x7FF4A5A5DEADBEE1ull;
-    else return 0x7FA5A5A5u;
-}
-template <typename T>
-__device__ __forceinline__ constexpr bits_t<T> quiet() {
-    if constexpr (sizeof(T) == 8) return 0x7FF8000000000000ull;
-    else return 0x7FC00000u;
-}
-
-template <typename T>
-__device__ __forceinline__ bits_t<T> peek(const T* p) {
-    return __hip_atomic_load(reinterpret_cast<const bits_t<T>*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ void publish(T* p, T v) {
-    bits_t<T> b = __builtin_bit_cast(bits_t<T>, v);
-    if (b == unset<T>()) b = quiet<T>();
-    __hip_atomic_store(reinterpret_cast<bits_t<T>*>(p), b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// A right-hand side entry that has been read (its owner is its only reader)
-// becomes the unset solution entry of the backward launch.
-template <typename T>
-__device__ __forceinline__ void wipe(T* p) {
-    *reinterpret_cast<bits_t<T>*>(p) = unset<T>();
-}
-
-// What a wait needs: the watchdog's record and the counter that shows progress.
-struct Ctl {
-    int32_t* hang;
-    const uint32_t* ticket;
-    unsigned long long stall;
-};
-
-// The value at p once it is set; v is an earlier peek at it.  Whole
-// wavefronts: lanes that want nothing pass on = false (with a valid p) and
-// get 0.
-template <typename T>
-__device__ __forceinline__ T settle(bits_t<T> v, const T* p, bool on, const Ctl& c) {
-    if (__any(on && v == unset<T>())) {
-        Watch w;
-        for (int spins = 1;; ++spins) {
-            v = peek(p);
-            if (!__any(on && v == unset<T>())) break;
-            if ((spins & 255) == 0) {
-                // once any wait has given up, every other wait returns at once
-                if (sync_ld(c.hang)) break;
-                if (w.expired(0, c.ticket, c.stall)) {
-                    if (on && v == unset<T>()) give_up(c.hang, reinterpret_cast<const int32_t*>(p), 1, 0, -1);
-                    break;
-                }
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-    }
-    return on ? __builtin_bit_cast(T, v) : (T)0;
-}
-
-// LDS traffic inside one wavefront completes in order; this keeps the
-// compiler from reordering it.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 
 // s0 + s1 += sum over j < 16 of a[j] * (lane j of each row of sixteen lanes of x).
 __device__ __forceinline__ void fma16(double& s0, double& s1, double x, const double (&a)[16]) {
@@ -166,73 +95,6 @@ __device__ __forceinline__ void fma16(float& s0, float& s1, float x, const float
         : "+v"(s0), "+v"(s1)
         : "v"(x), "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]),
           "v"(a[8]), "v"(a[9]), "v"(a[10]), "v"(a[11]), "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15]));
-}
-
-// Lane k of v, to every lane (k is uniform).
-__device__ __forceinline__ double lane_of(double v, int k) {
-    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)b, k), hi = __builtin_amdgcn_readlane((uint32_t)(b >> 32), k);
-    return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
-}
-__device__ __forceinline__ float lane_of(float v, int k) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(uint32_t, v), k));
-}
-__device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
-__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-
-// A front's record in scalar registers (the front is uniform).
-__device__ __forceinline__ int32_t uni(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ int64_t uni(int64_t v) {
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (int64_t)((unsigned long long)lo | ((unsigned long long)hi << 32));
-}
-__device__ __forceinline__ Front front_of(const DevPlan& P, int J) {
-    Front f = P.fronts[J];
-    f.poff = uni(f.poff);
-    f.woff = uni(f.woff);
-    f.c0 = uni(f.c0);
-    f.nn = uni(f.nn);
-    f.na = uni(f.na);
-    f.rowoff = uni(f.rowoff);
-    f.chd0 = uni(f.chd0);
-    f.chd1 = uni(f.chd1);
-    return f;
-}
-
-// y / d: the reciprocal of d is taken once, ahead of the substitution chain,
-// and one correction step gives the quotient its last bits (q + r (y - q d)).
-// `exact` (uniform): some reciprocal is not a normal number, divide instead.
-template <typename T>
-__device__ __forceinline__ T quot(T y, T d, T rd, bool exact) {
-    if (exact) return y / d;
-    const T q = y * rd, c = fma_(fma_(-q, d, y), rd, q);
-    return __builtin_isfinite(q) ? c : q;
-}
-template <typename T>
-__device__ __forceinline__ bool abnormal(T v) {
-    return !__builtin_isnormal(v);
-}
-
-// ---- small fronts (nJ <= 64), one wavefront each ------------------------------
-
-// The front's panel (contiguous, leading dimension nj) into Ps with leading
-// dimension nj | 1 (odd: rows and columns are both read without conflicts).
-template <typename T>
-__device__ __forceinline__ void stage_panel(const T* Pj, int nj, int nn, T* Ps) {
-    const int lane = threadIdx.x & 63, tot = nj * nn, ld = nj | 1;
-    // e / nj for e < 4096, nj <= 64: (e * ceil(2^20 / nj)) >> 20 (nj >= 2; nj = 1 has e = 0)
-    const uint32_t mul = nj > 1 ? ((1u << 20) / (uint32_t)nj + 1) : 0;
-    for (int e0 = 0; e0 < tot; e0 += 64 * 8) {
-        T v[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = Pj[min(e0 + 64 * i + lane, tot - 1)];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int e = e0 + 64 * i + lane;
-            const int c = (int)(((uint32_t)e * mul) >> 20);
-            if (e < tot) Ps[e - c * nj + c * ld] = v[i];
-        }
-    }
 }
 
 // Children's update vectors added into Yw (this wavefront's own rows), the
@@ -290,21 +152,18 @@ __device__ void small_fwd1(const DevPlan& P, const DevFactor<T>& F, const DevVSo
     Yw[r] = (T)0;
     stage_panel(F.panel + f.poff, nj, nn, Ps);
     wave_sync();
-    const int rd = min(r, nn - 1);
-    const T d = unit ? (T)1 : Ps[rd + rd * ld];
-    const T rcp = (T)1 / d;
-    const bool exact = __any(abnormal(rcp));
+    T d, rcp;
+    bool exact;
+    scale_panel(nj, nn, Ps, unit, d, rcp, exact);
     gather<T, false>(P, V, f, 0, 0, 0, 1, 0, Yw, ctl);
     wave_sync();
     T y = Yw[r] + (r < nn ? b : (T)0);
     const int rr = min(r, nj - 1);
     for (int k = 0; k < nn; ++k) {
-        const T l = Ps[rr + k * ld];
-        const T q = unit ? y : quot(y, d, rcp, exact);
-        const T x = lane_of(q, k);
-        const T z = fma_(-l, x, y);
-        y = r > k ? z : r == k ? x : y;
+        const T l = Ps[rr + k * ld], yk = lane_of(y, k);
+        if (r > k) y = fma_(-l, yk, y);
     }
+    if (!unit && r < nn) y = quot(y, d, rcp, exact);
     if (r < nn) {
         publish(V.out + f.c0 + r, y);
         wipe(V.wipe + f.c0 + r);
@@ -327,9 +186,10 @@ __device__ void small_bwd1(const DevPlan& P, const DevFactor<T>& F, const DevVSo
     if (unit) y /= F.d[f.c0 + rd];
     stage_panel(F.panel + f.poff, nj, nn, Ps);
     wave_sync();
-    const T d = unit ? (T)1 : Ps[rd + rd * ld];
-    const T rcp = (T)1 / d;
-    const bool exact = __any(abnormal(rcp));
+    T d, rcp;
+    bool exact;
+    scale_panel(nj, nn, Ps, unit, d, rcp, exact);
+    if (!unit) y = quot(y, d, rcp, exact);
     // separator part: the sixteen values of a group from LDS, broadcast by DPP
     const T x = settle(xv, px, r >= nn && r < nj, ctl);
     Yw[r] = x;
@@ -346,12 +206,9 @@ __device__ void small_bwd1(const DevPlan& P, const DevFactor<T>& F, const DevVSo
         fma16(s0, s1, xq, a);
     }
     y += s0 + s1;
-    for (int k = nn - 1; k >= 0; --k) {
-        const T l = Ps[k + rd * ld];
-        const T q = unit ? y : quot(y, d, rcp, exact);
-        const T xk = lane_of(q, k);
-        const T z = fma_(-l, xk, y);
-        y = r < k ? z : r == k ? xk : y;
+    for (int k = nn - 1; k > 0; --k) {
+        const T l = Ps[k + rd * ld], xk = lane_of(y, k);
+        if (r < k) y = fma_(-l, xk, y);
     }
     if (r < nn) publish(V.out + f.c0 + r, y);
 }

@@ -333,7 +333,8 @@ int mf_plan_gemm(const mf_plan* plan, int32_t* out, int64_t n);
  * then backward), as mf_dag_trace_read; n >= 2 x solve tasks.
  * mf_plan_solve_tasks: 5 int32 per ticket (kind 0 small front / 1 diagonal
  * block / 2 update rows / 3 up to four tiny fronts, front, a, b, c),
- * forward then backward.
+ * forward then backward.  Solves run these tickets merged: the times of a
+ * merged task stand at its first ticket, the others keep zero.
  * mf_plan_fronts: 5 int64 per internal front (first permuted column, nn, na,
  * parent or -1, 1 if in the small region). */
 int mf_solve_trace_read(mf_factor* f, unsigned long long* out, int64_t n);

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 # (block, separator): fronts of nn = block, na = separator, and a root of nn = separator
 SIZES = [(1, 1), (16, 16), (17, 47), (20, 44), (20, 45), (31, 33), (33, 31), (64, 1), (64, 64), (40, 65), (64, 255),
          (64, 256), (64, 257), (65, 256), (15, 512), (17, 513), (33, 576), (129, 520), (200, 1030)]
-COLS = [1, 2, 3, 4, 5, 15, 16, 17, 33]
+COLS = [1, 2, 3, 4, 5, 6, 15, 16, 17, 33]
 
 
 def _dense(nb, ns, blocks, seed, indefinite):
@@ -88,3 +88,41 @@ def test_nonfinite_columns_stay_apart(ct):
             X = ct.solve(F, D)
             assert not np.isfinite(X[:, 1]).all()
             assert np.array_equal(X[:, [0, 2, 3]], good[:, [0, 2, 3]])
+
+
+@pytest.mark.parametrize("cols", [5, 6, "half", "most"])
+def test_fixed_scratch(ct, cols):
+    """The solve without allocation from few columns up to as many as its fixed array takes: the
+    blocked form while its workspaces fit, a few columns at a time up to the limit, refused past it."""
+    import ctypes
+    import torch
+    from cliquetrees_amd import _native
+    lib = _native.hip()
+    pr = ct.problems
+    A = pr.laplacian3d_7pt(14, 12, 11, seed=3)
+    P, S = ct.symbolic(A, alg=ct.grid_nd(14, 12, 11))
+    F = ct.cholesky_(ct.ChordalCholesky(A, P, S))
+    n, h = A.shape[0], F._f.handle
+    perm = np.ascontiguousarray(P.perm, dtype=np.int64)
+    pp = perm.ctypes.data_as(_native.i64p)
+
+    def call(X, k):
+        return lib.mf_solve_noalloc(h, pp, ctypes.c_void_p(X.data_ptr() if X is not None else 16), k, n)
+
+    # the first column count that is refused (the call returns before anything is enqueued)
+    st = np.zeros(23, np.int64)
+    lib.mf_plan_stats(F._f.plan.handle, st.ctypes.data_as(_native.i64p), 23)
+    most = (64 << 20) // (8 * (n + int(st[22])))
+    while ((8 * int(st[22]) * most + 255) // 256 * 256) + 8 * n * most > 64 << 20:
+        most -= 1
+    k = {"half": most // 2, "most": most}.get(cols, cols)
+    print(cols, k, most, flush=True)
+    B = torch.tensor(np.random.default_rng(1).standard_normal((k, n)), device="cuda")
+    X = B.clone()
+    assert call(X, k) == 0, lib.mf_last_error()
+    assert lib.mf_factor_sync(h) == 0
+    torch.cuda.synchronize()
+    x, b = X.cpu().numpy().T, B.cpu().numpy().T
+    # n eps (condition number of the grid of order n): 1e-10
+    assert np.linalg.norm(A @ x - b) <= 1e-10 * np.linalg.norm(b)
+    assert call(None, most + 1) == -1 and b"scratch" in lib.mf_last_error()
