@@ -29,6 +29,12 @@ constexpr int EA_ROWS = 16384;  // elements per extend-add task (at most, where 
 constexpr int WIDE_K = 128;     // update-matrix tiles are 128 x 128 when nn >= WIDE_K
 constexpr int UPD_GROUP = 8;    // panel steps applied by one trailing-update tile
 constexpr int SIM_WORKERS = 512;  // resident workgroups assumed when ordering the DAG tickets
+// Phases of the selected inversion with at most this many 64 x 64 tiles run
+// them as 32 x 32 tiles: a phase is a step of a chain and its tiles alone do
+// not fill 256 CUs, so four times the tiles take a quarter of the time each
+// (selected inversion of a 28 x 30 x 26 grid: 1187 us at 32, 1192 at 128,
+// 1238 at 512, where larger phases become more tickets than workgroups).
+constexpr int SPLIT_TILES = 128;
 constexpr int VT_COLS = 5;                // right-hand sides solved column by column (more: blocked)
 constexpr int VT_ROWBLOCKS = 4;           // row blocks of a one-task front of the single-column solves
 constexpr int VT_PANELS = 64 * 65;        // elements of the panels of their grouped small fronts
@@ -156,8 +162,8 @@ struct SelTask {
     int8_t arrC, np, lower, pad;  // lower: store r >= c only (diagonal tile)
     int32_t kind;
     int32_t front;
-    int32_t a;        // ST_XDIAG: diagonal tile; ST_GATHER: column tile of M
-    int32_t b;
+    int32_t a;        // ST_XDIAG: diagonal tile; ST_GATHER: column tile of M,
+    int32_t b;        //   row tile (>= a)
     int32_t wait[2];  // counters that must reach target (-1: none): the front's
     int32_t target[2];//   own earlier phases, the parent's completion
 };

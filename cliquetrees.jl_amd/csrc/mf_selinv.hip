@@ -5,13 +5,13 @@
 //              mf_selinv_plan.cpp (root first) and run one task each:
 //              ST_XDIAG   X(K, K) = W_K, a diagonal tile of L11^-1 from the
 //                         factor's inverted 64 x 64 tiles
-//              ST_GEMM    one 64 x 64 tile C = sum of up to two products
+//              ST_GEMM    one tile of at most 64 x 64, C = sum of up to two products
 //                         sgn A B' (operands plain or transposed), on MFMA:
 //                         the recursion of X = L11^-1, Lt = L21 X,
 //                         Sigma21 = -M Lt, Sigma11 = X' X - Lt' Sigma21
-//              ST_GATHER  a column tile of M = Sigma(sep, sep) from the
-//                         parent's frontal matrix (selinv_send!,
-//                         copygathertri!, utils.jl:529-553), both triangles
+//              ST_GATHER  a tile of M = Sigma(sep, sep) from the parent's
+//                         frontal matrix and its mirror image (selinv_send!,
+//                         copygathertri!, utils.jl:529-553)
 //              ST_SMALL   a whole front with nJ <= 64 in LDS
 //              (selinv_loop_snd!/nod!, selinv.jl:122-379).
 // Synchronization is the tile-DAG factorization's: a task waits (bounded,
@@ -27,6 +27,7 @@
 #include "mf_kernels.h"
 #include "mf_mfma.h"
 #include "mf_sync.h"
+#include "mf_vsolve.h"
 
 namespace mf {
 
@@ -42,92 +43,104 @@ __device__ __forceinline__ void stc(T* p, T v) {
 }
 __device__ __forceinline__ void drain_stores() { __builtin_amdgcn_s_waitcnt(0); }
 
-constexpr int SKC = 32;      // k-chunk of the tile product
-constexpr int SLD = 64 + 4;  // leading dimension of its LDS stages
 constexpr int FLD = 64 + 1;  // leading dimension of LDS fronts and tiles
 
-// One element of the parent's frontal matrix [Sigma11, .; Sigma21, M]
-// (lower triangle, p >= q, positions in the parent's row list).
-template <typename T>
-__device__ __forceinline__ T parent_entry(const DevSel<T>& S, const Front& pf, int64_t pm, int p, int q) {
-    const int nJ = pf.nn + pf.na;
-    if (q < pf.nn) return ldc(S.base[SP_SIG] + pf.poff + p + (int64_t)q * nJ);
-    return ldc(S.base[SP_M] + pm + (p - pf.nn) + (int64_t)(q - pf.nn) * pf.na);
-}
-
-// One output tile: acc = sum over the task's products of sgn A B' (wave w
-// owns the 32 x 32 quarter (w & 1, w >> 1) as 2 x 2 MFMA blocks), then
-// C = acc (lower triangle only for a diagonal tile).  Each k-chunk of A and
-// B goes through LDS; the next chunk is fetched into registers while the
-// current one is multiplied.  A plain operand is fetched down its columns
-// (lane = row), a transposed one along its rows (lane = k), so both are
-// coalesced.
-template <typename T>
-__device__ void sel_tile(const DevSel<T>& S, const SelTask& t, T* As, T* Bs, const int tid) {
+// One output tile of at most E x E: acc = sum over the task's products of
+// sgn A B', then C = acc (lower triangle only for a diagonal tile).  Wave w
+// owns the quarter (w & 1, w >> 1), E/32 x E/32 MFMA blocks.  Each chunk of
+// KC inner columns of A and B goes through LDS; the next chunk is fetched
+// into registers while the current one is multiplied.  A plain operand is
+// fetched down its columns (lane = row), a transposed one along its rows
+// (lane = k), so both are coalesced; the loads are unconditional (clamped)
+// and the predicates applied when they go to LDS.
+//
+// E = 64, KC = 32 and E = 32, KC = 128 hold the same 2048 and 4096 values an
+// operand; both spend 32 matrix instructions a wavefront (0.9 us in FP64) on
+// a chunk, so a 32-wide tile runs its inner dimension four times as fast.
+// The tiles of one front's phase rarely fill the chip and the phases down the
+// tree are a chain, so phases of few tiles take the small one (28 x 30 x 26
+// grid, with the gathers a task per tile: 2553 -> 1192 us).
+template <typename T, int E, int KC>
+__device__ __forceinline__ void sel_tile(const DevSel<T>& S, const SelTask& t, const SelPart* parts, T* As, T* Bs,
+                                         const int tid) {
     typedef typename Mfma<T>::v4 v4;
-    constexpr int PER = SKC * 64 / 256;
+    constexpr int PER = KC * E / 256, LD = E + 1, Q = E / 32, RS = 256 / KC, KS = 256 / E;
     const int wave = tid >> 6, lane = tid & 63;
-    const int wr = (wave & 1) * 32, wc = (wave >> 1) * 32;
+    const int wr = (wave & 1) * (E / 2), wc = (wave >> 1) * (E / 2);
     const int li = lane & 15, lk = lane >> 4;
-    v4 acc[2][2];
+    v4 acc[Q][Q];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < Q; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = v4{0, 0, 0, 0};
+        for (int j = 0; j < Q; ++j) acc[i][j] = v4{0, 0, 0, 0};
+    // element i of this thread in a chunk: plain (row tid % E, k tid / E + KS i),
+    // transposed (row tid / KC + RS i, k tid % KC)
+    // (A, lda uniform: one base in scalar registers and a lane offset a load)
+    auto fetch = [&](const T* A, int lda, bool tr, int rows, int k0, int k1, T (&v)[PER]) {
+        const T* q = A + (tr ? (int64_t)k0 : (int64_t)k0 * lda);
+        const int kn = k1 - k0;
+        if (tr) {
+            const uint32_t k = min(tid % KC, kn - 1);
+#pragma unroll
+            for (int i = 0; i < PER; ++i) v[i] = ldc(q + (k + (uint32_t)min(tid / KC + RS * i, rows - 1) * (uint32_t)lda));
+        } else {
+            const uint32_t r = min(tid % E, rows - 1);
+#pragma unroll
+            for (int i = 0; i < PER; ++i) v[i] = ldc(q + (r + (uint32_t)min(tid / E + KS * i, kn - 1) * (uint32_t)lda));
+        }
+    };
+    auto put = [&](const T (&v)[PER], bool tr, int rows, int k0, int k1, T sg, T* X) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int r = tr ? tid / KC + RS * i : tid % E, k = tr ? tid % KC : tid / E + KS * i;
+            X[k * LD + r] = (r < rows && k0 + k < k1) ? sg * v[i] : (T)0;
+        }
+    };
     for (int q = 0; q < t.np; ++q) {
-        const SelPart p = t.p[q];
+        SelPart p = parts[q];
+        p.a_off = uni(p.a_off);
+        p.b_off = uni(p.b_off);
+        p.lda = uni(p.lda);
+        p.ldb = uni(p.ldb);
+        p.k = uni(p.k);
+        p.ta = (int8_t)uni((int32_t)p.ta);
+        p.tb = (int8_t)uni((int32_t)p.tb);
+        p.arrA = (int8_t)uni((int32_t)p.arrA);
+        p.arrB = (int8_t)uni((int32_t)p.arrB);
         const T* A = S.base[p.arrA] + p.a_off;
         const T* B = S.base[p.arrB] + p.b_off;
-        const T sg = (T)p.sgn;
         T ra[PER], rb[PER];
-        // element i of this thread in a chunk: plain (row tid & 63, k (tid >> 6) + 4 i),
-        // transposed (row (tid >> 5) + 8 i, k tid & 31)
-        auto fetch = [&](int k0) {
-#pragma unroll
-            for (int i = 0; i < PER; ++i) {
-                int r, gk;
-                if (p.ta) { r = (tid >> 5) + 8 * i; gk = k0 + (tid & 31); }
-                else { r = tid & 63; gk = k0 + (tid >> 6) + 4 * i; }
-                T v = (T)0;
-                if (r < t.m && gk < p.k) v = ldc(p.ta ? A + gk + (int64_t)r * p.lda : A + r + (int64_t)gk * p.lda);
-                ra[i] = v;
-                if (p.tb) { r = (tid >> 5) + 8 * i; gk = k0 + (tid & 31); }
-                else { r = tid & 63; gk = k0 + (tid >> 6) + 4 * i; }
-                v = (T)0;
-                if (r < t.n && gk < p.k) v = ldc(p.tb ? B + gk + (int64_t)r * p.ldb : B + r + (int64_t)gk * p.ldb);
-                rb[i] = v;
-            }
-        };
-        fetch(0);
-        for (int k0 = 0; k0 < p.k; k0 += SKC) {
-#pragma unroll
-            for (int i = 0; i < PER; ++i) {
-                const int ai = p.ta ? (tid & 31) * SLD + (tid >> 5) + 8 * i : ((tid >> 6) + 4 * i) * SLD + (tid & 63);
-                const int bi = p.tb ? (tid & 31) * SLD + (tid >> 5) + 8 * i : ((tid >> 6) + 4 * i) * SLD + (tid & 63);
-                As[ai] = sg * ra[i];
-                Bs[bi] = rb[i];
-            }
+        fetch(A, p.lda, p.ta, t.m, 0, p.k, ra);
+        fetch(B, p.ldb, p.tb, t.n, 0, p.k, rb);
+        for (int k0 = 0; k0 < p.k; k0 += KC) {
+            put(ra, p.ta, t.m, k0, p.k, (T)p.sgn, As);
+            put(rb, p.tb, t.n, k0, p.k, (T)1, Bs);
             __syncthreads();
-            if (k0 + SKC < p.k) fetch(k0 + SKC);
+            if (k0 + KC < p.k) {
+                fetch(A, p.lda, p.ta, t.m, k0 + KC, p.k, ra);
+                fetch(B, p.ldb, p.tb, t.n, k0 + KC, p.k, rb);
+            }
+            const int ke = min(KC, (p.k - k0 + 3) & ~3);
+#pragma unroll 8
+            for (int kk = 0; kk < ke; kk += 4) {
+                T a[Q], b[Q];
 #pragma unroll
-            for (int kk = 0; kk < SKC; kk += 4) {
-                const T a0 = As[(kk + lk) * SLD + wr + li];
-                const T a1 = As[(kk + lk) * SLD + wr + 16 + li];
-                const T b0 = Bs[(kk + lk) * SLD + wc + li];
-                const T b1 = Bs[(kk + lk) * SLD + wc + 16 + li];
-                acc[0][0] = Mfma<T>::op(a0, b0, acc[0][0]);
-                acc[0][1] = Mfma<T>::op(a0, b1, acc[0][1]);
-                acc[1][0] = Mfma<T>::op(a1, b0, acc[1][0]);
-                acc[1][1] = Mfma<T>::op(a1, b1, acc[1][1]);
+                for (int i = 0; i < Q; ++i) a[i] = As[(kk + lk) * LD + wr + 16 * i + li];
+#pragma unroll
+                for (int j = 0; j < Q; ++j) b[j] = Bs[(kk + lk) * LD + wc + 16 * j + li];
+#pragma unroll
+                for (int i = 0; i < Q; ++i)
+#pragma unroll
+                    for (int j = 0; j < Q; ++j) acc[i][j] = Mfma<T>::op(a[i], b[j], acc[i][j]);
             }
             __syncthreads();
         }
     }
     T* C = S.base[t.arrC] + t.c_off;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < Q; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < Q; ++j)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int row = wr + i * 16 + Mfma<T>::row(lk, v), col = wc + j * 16 + li;
@@ -148,37 +161,48 @@ __device__ void sel_xdiag(const DevPlan& P, const DevSel<T>& S, int J, int K, co
         if (r < kb) stc(X + r + (int64_t)c * f.nn, ldc(W + r + (int64_t)c * f.nn));
 }
 
-// Column tile jb of M (rows jb*64 .. na-1 and, by symmetry, the same tiles
-// above the diagonal): M(a, b) = F_parent(rel[max(a, b)], rel[min(a, b)]).
+// Address of an element of the parent's frontal matrix [Sigma11, .; Sigma21, M]
+// (lower triangle, p >= q, positions in the parent's row list).
 template <typename T>
-__device__ void sel_gather(const DevPlan& P, const DevSel<T>& S, int J, int jb, T* Ts, const int tid) {
+__device__ __forceinline__ const T* parent_addr(const T* sig, const T* M, int nn, int na, int p, int q) {
+    return q < nn ? sig + p + (int64_t)q * (nn + na) : M + (p - nn) + (int64_t)(q - nn) * na;
+}
+
+// Tile (ib, jb), ib >= jb, of M and its mirror image above the diagonal:
+// M(a, b) = F_parent(rel[max(a, b)], rel[min(a, b)]).  All of a thread's
+// sixteen elements load at once (one at a time, with a store after each, a
+// tile took sixteen trips to memory).
+template <typename T>
+__device__ void sel_gather(const DevPlan& P, const DevSel<T>& S, int J, int jb, int ib, T* Ts, const int tid) {
     const Front f = P.fronts[J];
     const Front pf = P.fronts[f.parent];
-    const int64_t pm = S.moff[f.parent];
     const int32_t* rel = P.rel + f.reloff;
     T* M = S.base[SP_M] + S.moff[J];
-    const int na = f.na, b0 = NB * jb, cb = min(NB, na - b0);
-    for (int a0 = b0; a0 < na; a0 += NB) {
-        const int rb = min(NB, na - a0);
-        for (int e = tid; e < NB * NB; e += 256) {
-            const int r = e & 63, c = e >> 6;
-            if (r < rb && c < cb) {
-                const int a = a0 + r, b = b0 + c;
-                const int pa = rel[max(a, b)], pb = rel[min(a, b)];
-                const T v = parent_entry(S, pf, pm, pa, pb);
-                stc(M + a + (int64_t)b * na, v);
-                Ts[r + c * FLD] = v;
-            }
-        }
-        __syncthreads();
-        if (a0 != b0) {  // the mirrored tile, written down its columns
-            for (int e = tid; e < NB * NB; e += 256) {
-                const int x = e & 63, y = e >> 6;
-                if (x < cb && y < rb) stc(M + (b0 + x) + (int64_t)(a0 + y) * na, Ts[y + x * FLD]);
-            }
-        }
-        __syncthreads();
+    const T* sig = S.base[SP_SIG] + pf.poff;
+    const T* pM = S.base[SP_M] + S.moff[f.parent];
+    const int na = f.na, b0 = NB * jb, cb = min(NB, na - b0), a0 = NB * ib, rb = min(NB, na - a0);
+    const int r = tid & 63, g = tid >> 6;
+    const int ra = rel[min(a0 + r, na - 1)];
+    T v[NB / 4];
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) {
+        const int rc = rel[min(b0 + g + 4 * i, na - 1)];  // rel is increasing
+        v[i] = ldc(parent_addr(sig, pM, pf.nn, pf.na, max(ra, rc), min(ra, rc)));
     }
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) {
+        const int c = g + 4 * i;
+        if (r < rb && c < cb) stc(M + (a0 + r) + (int64_t)(b0 + c) * na, v[i]);
+        Ts[r + c * FLD] = v[i];
+    }
+    if (ib == jb) return;
+    __syncthreads();
+    // the mirrored tile, written down its columns
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) v[i] = Ts[(g + 4 * i) + r * FLD];
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i)
+        if (r < cb && g + 4 * i < rb) stc(M + (b0 + r) + (int64_t)(a0 + g + 4 * i) * na, v[i]);
 }
 
 // A whole front with nJ <= 64 in LDS: L = [L11; L21] in Lf (ld FLD), M in
@@ -189,21 +213,38 @@ __device__ void sel_small(const DevPlan& P, const DevSel<T>& S, int J, T* Lf, T*
     const Front f = P.fronts[J];
     const int nn = f.nn, na = f.na, nJ = nn + na;
     const T* Lp = S.base[SP_PANEL] + f.poff;
-    for (int e = tid; e < nJ * nn; e += 256) {
-        const int r = e % nJ, c = e / nJ;
-        Lf[r + c * FLD] = Lp[r + (int64_t)c * nJ];
+    const int r = tid & 63, g = tid >> 6;
+    for (int c0 = g; c0 < nn; c0 += 32) {
+        T v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = Lp[min(r, nJ - 1) + (int64_t)min(c0 + 4 * i, nn - 1) * nJ];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (r < nJ && c0 + 4 * i < nn) Lf[r + (c0 + 4 * i) * FLD] = v[i];
     }
     if (na > 0) {
         const Front pf = P.fronts[f.parent];
-        const int64_t pm = S.moff[f.parent];
+        const T* sig = S.base[SP_SIG] + pf.poff;
+        const T* pM = S.base[SP_M] + S.moff[f.parent];
         const int32_t* rel = P.rel + f.reloff;
         T* Mo = S.base[SP_M] + S.moff[J];
         const bool keep = f.chd1 > f.chd0;  // the children gather from it
-        for (int e = tid; e < na * na; e += 256) {
-            const int a = e % na, b = e / na;
-            const T v = parent_entry(S, pf, pm, rel[max(a, b)], rel[min(a, b)]);
-            Mf[a + b * FLD] = v;
-            if (keep) stc(Mo + a + (int64_t)b * na, v);
+        const int ra = rel[min(r, na - 1)];
+        for (int c0 = g; c0 < na; c0 += 32) {
+            T v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int rc = rel[min(c0 + 4 * i, na - 1)];
+                v[i] = ldc(parent_addr(sig, pM, pf.nn, pf.na, max(ra, rc), min(ra, rc)));
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int c = c0 + 4 * i;
+                if (r < na && c < na) {
+                    Mf[r + c * FLD] = v[i];
+                    if (keep) stc(Mo + r + (int64_t)c * na, v[i]);
+                }
+            }
         }
     }
     __syncthreads();
@@ -211,12 +252,10 @@ __device__ void sel_small(const DevPlan& P, const DevSel<T>& S, int J, T* Lf, T*
     // L21'(:, j) -= Lt(:, c) L(c, j) for j < c
     for (int c = nn - 1; c >= 0 && na > 0; --c) {
         const T inv = (T)1 / Lf[c + c * FLD];
-        for (int r = tid; r < na; r += 256) Lf[nn + r + c * FLD] *= inv;
+        if (tid < na) Lf[nn + tid + c * FLD] *= inv;
         __syncthreads();
-        for (int e = tid; e < na * c; e += 256) {
-            const int r = e % na, j = e / na;
-            Lf[nn + r + j * FLD] -= Lf[nn + r + c * FLD] * Lf[c + j * FLD];
-        }
+        if (r < na)
+            for (int j = g; j < c; j += 4) Lf[nn + r + j * FLD] -= Lf[nn + r + c * FLD] * Lf[c + j * FLD];
         __syncthreads();
     }
     // X = L11^-1 in place, last column first: X(i, j) = -X(j, j) sum_{k=j+1}^{i} X(i, k) L(k, j)
@@ -271,7 +310,7 @@ __device__ void sel_small(const DevPlan& P, const DevSel<T>& S, int J, T* Lf, T*
 
 template <typename T>
 __global__ __launch_bounds__(256, 2) void k_selinv(DevPlan P, DevSel<T> S) {
-    constexpr int SM1 = 2 * 64 * FLD, SM2 = 2 * SKC * SLD;
+    constexpr int SM1 = 2 * 64 * FLD, SM2 = 2 * 128 * 33;
     __shared__ T smem[SM1 > SM2 ? SM1 : SM2];
     __shared__ int s_t;
     for (;;) {
@@ -289,8 +328,11 @@ __global__ __launch_bounds__(256, 2) void k_selinv(DevPlan P, DevSel<T> S) {
         __syncthreads();
         switch (tk.kind) {
             case ST_XDIAG: sel_xdiag<T>(P, S, tk.front, tk.a, tid); break;
-            case ST_GEMM: sel_tile<T>(S, tk, smem, smem + SKC * SLD, tid); break;
-            case ST_GATHER: sel_gather<T>(P, S, tk.front, tk.a, smem, tid); break;
+            case ST_GEMM:
+                if (tk.m <= 32 && tk.n <= 32) sel_tile<T, 32, 128>(S, tk, S.task[t].p, smem, smem + 128 * 33, tid);
+                else sel_tile<T, 64, 32>(S, tk, S.task[t].p, smem, smem + 32 * 65, tid);
+                break;
+            case ST_GATHER: sel_gather<T>(P, S, tk.front, tk.a, tk.b, smem, tid); break;
             default: sel_small<T>(P, S, tk.front, smem, smem + 64 * FLD, tid); break;
         }
         drain_stores();

@@ -84,6 +84,39 @@ SelTask plain_task(int kind, int J, int a) {
     return t;
 }
 
+// The phase's products as 32 x 32 tiles, where it has at most SPLIT_TILES
+// tiles: the four quarters of each (two rows of quarters by two columns, a
+// diagonal tile's upper one left out).
+void split_phase(std::vector<SelTask>& v, size_t first) {
+    constexpr int H = NB / 2;
+    const size_t n = v.size() - first;
+    if (n > (size_t)SPLIT_TILES) return;
+    std::vector<SelTask> out;
+    for (size_t i = first; i < v.size(); ++i) {
+        const SelTask& t = v[i];
+        if (t.kind != ST_GEMM) {
+            out.push_back(t);
+            continue;
+        }
+        for (int c0 = 0; c0 < t.n; c0 += H)
+            for (int r0 = 0; r0 < t.m; r0 += H) {
+                if (t.lower && r0 < c0) continue;
+                SelTask q = t;
+                q.m = std::min(H, t.m - r0);
+                q.n = std::min(H, t.n - c0);
+                q.c_off += r0 + (int64_t)c0 * t.ldc;
+                q.lower = t.lower && r0 == c0;
+                for (int k = 0; k < q.np; ++k) {
+                    q.p[k].a_off += q.p[k].ta ? (int64_t)r0 * q.p[k].lda : r0;
+                    q.p[k].b_off += q.p[k].tb ? (int64_t)c0 * q.p[k].ldb : c0;
+                }
+                out.push_back(q);
+            }
+    }
+    v.resize(first);
+    v.insert(v.end(), out.begin(), out.end());
+}
+
 }  // namespace
 
 std::string build_selinv(const HostPlan& H, SelPlan& S) {
@@ -123,6 +156,7 @@ std::string build_selinv(const HostPlan& H, SelPlan& S) {
         const int nn = F.nn, na = F.na, nJ = F.nn + F.na;
         int32_t done = 0;  // tasks of J in finished phases
         auto close_phase = [&](std::vector<SelTask>& v, size_t first) {
+            split_phase(v, first);
             for (size_t i = first; i < v.size(); ++i) {
                 v[i].wait[0] = done > 0 ? J : -1;
                 v[i].target[0] = done;
@@ -196,9 +230,13 @@ std::string build_selinv(const HostPlan& H, SelPlan& S) {
                         A[J].push_back(t);
                     }
                 close_phase(A[J], f0);
-                // gather M from the parent, one column tile per task
+                // gather M from the parent, one tile and its mirror image per task
                 f0 = B[J].size();
-                for (int jb = 0; jb < nr; ++jb) B[J].push_back(plain_task(ST_GATHER, J, jb));
+                for (int jb = 0; jb < nr; ++jb)
+                    for (int ib = jb; ib < nr; ++ib) {
+                        B[J].push_back(plain_task(ST_GATHER, J, jb));
+                        B[J].back().b = ib;
+                    }
                 // the B list continues the phase count of the A list
                 close_phase(B[J], f0);
                 // Sigma21(i, j) = -sum_k M(i, k) Lt(k, j)
@@ -449,12 +487,12 @@ struct HostSel {
         return pool[SP_M][S.moff[P] + (p - F.nn) + (int64_t)(q - F.nn) * F.na];
     }
 
-    void gather(int32_t J, int b0, int b1) {
+    void gather(int32_t J, int b0, int b1, int a0, int a1) {
         const Front& F = H.fronts[J];
         const int32_t* rel = H.rel.data() + F.reloff;
         double* M = pool[SP_M].data() + S.moff[J];
         for (int b = b0; b < b1; ++b)
-            for (int a = b; a < F.na; ++a) {
+            for (int a = std::max(a0, b); a < a1; ++a) {
                 const double v = fp(F.parent, rel[a], rel[b]);
                 M[a + (int64_t)b * F.na] = v;
                 M[b + (int64_t)a * F.na] = v;
@@ -491,7 +529,7 @@ struct HostSel {
         const double* Lp = pool[SP_PANEL].data() + F.poff;
         std::vector<double> L(Lp, Lp + (size_t)nJ * nn), M((size_t)na * na), S21((size_t)na * nn);
         if (na > 0) {
-            gather(J, 0, na);
+            gather(J, 0, na, 0, na);
             std::copy(pool[SP_M].begin() + S.moff[J], pool[SP_M].begin() + S.moff[J] + (int64_t)na * na,
                       M.begin());
         }
@@ -556,7 +594,9 @@ struct HostSel {
                     break;
                 }
                 case ST_GEMM: gemm(t); break;
-                case ST_GATHER: gather(t.front, NB * t.a, std::min(F.na, NB * t.a + NB)); break;
+                case ST_GATHER:
+                    gather(t.front, NB * t.a, std::min(F.na, NB * t.a + NB), NB * t.b, std::min(F.na, NB * t.b + NB));
+                    break;
                 case ST_SMALL: small(t.front); break;
                 default: return "selinv task kind";
             }
