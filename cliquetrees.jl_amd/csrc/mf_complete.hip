@@ -38,10 +38,12 @@ namespace {
 // front (nn + na > 64).
 __device__ __forceinline__ int cpl_sep_rows(int nn, int na) { return nn + na > 64 ? (na + 63) & ~63 : na; }
 
-constexpr int CPL_SEP_LDS = 12288;  // separator rows staged in LDS (ints)
+constexpr int CPL_SEP_LDS = 4096;   // separator rows staged in LDS (ints); 16 KB, so that eight
+                                    // workgroups share a CU (with 48 KB three did)
+constexpr int CPL_COLS = 16;        // columns of K a workgroup takes at least
 
-// Workgroups (u, y) for root u (reference front fr[u]): columns c = y,
-// y + gridDim.y, ... of its K (nJ' x nJ' column-major at K + koff[u]; the
+// Workgroups (u, y) for root u (reference front fr[u]), y < ny = at most one
+// per CPL_COLS columns (the others end at once): columns c = y, y + ny, ... of its K (nJ' x nJ' column-major at K + koff[u]; the
 // lower triangle, which is all the factorization reads).  M(r, c) =
 // Sigma(a, b) with a = sep[r] >= b = sep[c]: column b's front o holds it in
 // its diagonal block (a in o's residual) or at a's position among o's
@@ -56,13 +58,15 @@ __global__ __launch_bounds__(256) void k_cpl_gather(DevPlan P, const int32_t* fr
     const int u = blockIdx.x, tid = threadIdx.x;
     const OutFront o = P.out[fr[u]];
     const int nn = o.nn, na = o.na, np = cpl_sep_rows(nn, na), nj = nn + np;
+    const int ny = min((int)gridDim.y, (nj + CPL_COLS - 1) / CPL_COLS);
+    if ((int)blockIdx.y >= ny) return;
     double* Kj = K + koff[u];
     const double* D11 = Dval + o.Dp;
     const double* L21 = Lval + o.Lp;
     const int32_t* sep = septgt + o.sepoff;
     if (tid == 0) s_owner = -1;
     __syncthreads();
-    for (int c = blockIdx.y; c < nj; c += gridDim.y) {
+    for (int c = blockIdx.y; c < nj; c += ny) {
         double* col = Kj + (int64_t)c * nj;
         if (c < na) {
             // M's column c, rows r >= c (uniform per workgroup)
