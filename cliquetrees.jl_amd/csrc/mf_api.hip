@@ -376,7 +376,7 @@ void enqueue_factor(mf_factor* f) {
         else launch_fill<double>(f->gmw + 2, 1, f->eps, s);
     }
     timed(f, MF_KC_SMALL, pl->ref_flops_small, H.n_small_region, [&] {
-        launch_small<T>(P, F, P.small_order, P.small_units, (int)H.small_units.size(), s);
+        launch_small<T>(P, F, (int)H.small_units.size(), s);
     });
     if (!H.dag.empty()) {
         launch_copy_i32(pl->d_cnt0, f->cnt, H.dag_counters, s);
@@ -553,7 +553,7 @@ static int plan_create(int64_t n, int64_t nfr, const int64_t* resptr, const int6
         (rc = upload(H.vbtask, (VTask**)&pl->V.btask, pl->allocs)) ||
         (rc = upload(H.vfunit, (int32_t**)&pl->V.funit, pl->allocs)) ||
         (rc = upload(H.vbunit, (int32_t**)&pl->V.bunit, pl->allocs)) ||
-        (rc = upload(H.vchd, (VChild**)&pl->V.chd, pl->allocs)) ||
+        (rc = upload(H.vchd, (VChild**)&D.vchd, pl->allocs)) ||
         (rc = upload(H.dag, &pl->d_dag, pl->allocs)) ||
         (rc = upload(H.dag_gmw, &pl->d_dag_gmw, pl->allocs)) ||
         (rc = upload(H.dagf, &pl->d_dagf, pl->allocs)) ||
@@ -568,6 +568,7 @@ static int plan_create(int64_t n, int64_t nfr, const int64_t* resptr, const int6
         delete pl;
         return rc;
     }
+    pl->V.chd = D.vchd;
     D.nJ = (int32_t)H.fronts.size();
     pl->V.nfu = std::max<int32_t>(0, (int32_t)H.vfunit.size() - 1);
     pl->V.nbu = std::max<int32_t>(0, (int32_t)H.vbunit.size() - 1);

@@ -22,6 +22,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "mf_kernels.h"
 #include "mf_mfma.h"
@@ -124,206 +125,321 @@ __device__ __forceinline__ void pin(T (&v)[N]) {
     for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
 }
 
-// Right-looking partial factorization of the first nn columns of the
-// nj x nj front M (lower triangle, leading dimension LDS) in LDS.
-// Returns after a failed pivot (recorded in F.info).
+// 1 / sqrt(d) and 1 / d to full double precision: the hardware estimate
+// (about 24 bits) and one step of third order, a chain of five and three
+// operations.
+__device__ __forceinline__ double rsqrt_full(double d) {
+    const double y = __builtin_amdgcn_rsq(d);
+    const double e = __builtin_fma(-(d * y), y, 1.0);
+    return __builtin_fma(y, e * __builtin_fma(e, 0.375, 0.5), y);
+}
+__device__ __forceinline__ double rcp_full(double d) {
+    const double y = __builtin_amdgcn_rcp(d);
+    const double e = __builtin_fma(-d, y, 1.0);
+    return __builtin_fma(y, __builtin_fma(e, e, e), y);
+}
+// Lane k of v, to every lane (k is uniform).
+__device__ __forceinline__ double lane_of(double v, int k) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)b, k), hi = __builtin_amdgcn_readlane((uint32_t)(b >> 32), k);
+    return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
+}
+__device__ __forceinline__ float lane_of(float v, int k) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(uint32_t, v), k));
+}
+
+// The children of a front final: one lane a child, by a whole wavefront.
 template <typename T>
-__device__ __forceinline__ void factor_lds(T* M, int nn, int nj, int gc0, const DevFactor<T>& F,
-                           T* s_piv, T* s_inv, int* s_fail, const int tid) {
+__device__ __forceinline__ void wait_children(const DevPlan& P, const DevFactor<T>& F, int q0, int q1, int lane) {
+    for (int b = q0; b < q1; b += 64) {
+        const bool on = b + lane < q1;
+        const int32_t* w = F.flags + P.vchd[min(b + lane, q1 - 1)].front;
+        Watch watch;
+        for (int spins = 1;; ++spins) {
+            const bool ok = !on || ld_rel(w) >= 1;
+            if (__all(ok)) break;
+            if ((spins & 255) == 0) {
+                // once any wait has given up, every other wait returns at once
+                if (ld_rel(F.hang)) return;
+                if (watch.expired((int32_t)__popcll(__ballot(ok)), F.ticket, F.stall)) {
+                    if (!ok) give_up(F.hang, w, 1, 0, -1);
+                    return;
+                }
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+    }
+}
+
+// The pivot of column k from its diagonal entry and (GMW81) the magnitudes
+// below it: the pivot (0: failed), and its scale (1 / sqrt or 1 /).
+template <typename T>
+__device__ __forceinline__ double small_pivot(const DevFactor<T>& F, int gcol, double akk, double below, double* scale) {
+    const double piv = F.reg_kind == 2 ? regularize_gmw(F, sign_of(F, gcol), akk, wave_max(below))
+                                       : regularize(F, sign_of(F, gcol), akk);
+    *scale = F.diag == 0 ? rsqrt_full(piv) : rcp_full(piv);
+    return piv;
+}
+
+// One small front (nJ <= 64) by a workgroup: the panel's A entries and the
+// children's update matrices meet in LDS (M), then wavefront g keeps columns
+// c = g mod 4, row r in lane r, in registers for the partial factorization:
+// the wavefront that owns column k scales it and leaves it in LDS, and after
+// one barrier every wavefront subtracts it from its later columns.  The
+// owned columns shift down by one register every four columns, so the pivot
+// is always in the first.  Both small-front kernels on a 100 x 100 grid: 199
+// -> 156 us of the small region.  WAIT: the children are waited for here, after the
+// loads that do not depend on them.  Returns after a failed pivot (recorded
+// in F.info).
+// Bound: the chain of pivots (square root, LDS, barrier and the update) and
+// the loads' round trips.  A front of the DAG took 28 us with the columns in
+// LDS, one thread's square root and division and three barriers a pivot, and
+// the children's records read one by one.
+template <typename T, bool WAIT>
+__device__ __forceinline__ void small_front(const DevPlan& P, const DevFactor<T>& F, int J, T* M, T* s_piv, int* s_fail,
+                                            const int tid) {
+    const Front f = uniform(P.fronts[J]);
+    const int nn = f.nn, na = f.na, nj = nn + na;
+    const int r = tid & 63, g = __builtin_amdgcn_readfirstlane(tid >> 6);
+    T* Pj = F.panel + f.poff;
+    T a[NB / 4];
+    for (int c0 = 0; c0 < nj; c0 += 32) {
+        T v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = Pj[min(r, nj - 1) + (int64_t)min(c0 + 4 * i + g, nn - 1) * nj];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int c = c0 + 4 * i + g;
+            if (c < nj) M[r + c * LDS] = (c < nn && c <= r && r < nj) ? v[i] : (T)0;
+        }
+    }
+    if (WAIT && g == 0) wait_children(P, F, f.chd0, f.chd1, r);
+    __syncthreads();
+    for (int qb = f.chd0; qb < f.chd1; qb += 64) {
+        const int ns = min(64, f.chd1 - qb);
+        const VChild x = P.vchd[qb + min(r, ns - 1)];  // one child a lane
+        auto get = [&](int32_t v, int q) { return __builtin_amdgcn_readlane(v, q); };
+        // wavefront g: columns c = g mod 4 of the child, row in the lane, all in flight
+        auto load = [&](int q, T (&v)[NB / 4], int& rr) {
+            const int ma = get(x.ma, q);
+            const uint64_t uo = (uint32_t)get((int32_t)(uint64_t)x.u, q) |
+                                (uint64_t)(uint32_t)get((int32_t)((uint64_t)x.u >> 32), q) << 32;
+            const uint32_t row = min(r, ma - 1);
+            rr = (P.rel + get(x.rel, q))[row];
+            const T* u = F.U + uo;
+#pragma unroll
+            for (int h = 0; h < NB / 4; h += 4) {
+                if (4 * h >= ma) break;  // uniform
+#pragma unroll
+                for (int i = h; i < h + 4; ++i) v[i] = ldc(u + (int64_t)min(4 * i + g, ma - 1) * ma + row);
+            }
+        };
+        auto add = [&](int q, const T (&v)[NB / 4], int rr) {
+            const int ma = get(x.ma, q);
+#pragma unroll
+            for (int h = 0; h < NB / 4; h += 4) {
+                if (4 * h >= ma) break;  // uniform
+#pragma unroll
+                for (int i = h; i < h + 4; ++i) {
+                    const int c = 4 * i + g;
+                    const int cc = get(rr, min(c, ma - 1));
+                    if (c <= r && r < ma) M[rr + cc * LDS] += v[i];
+                }
+            }
+        };
+        T v0[NB / 4], v1[NB / 4];
+        int r0 = 0, r1 = 0;
+        load(0, v0, r0);
+        for (int q = 0; q < ns; q += 2) {
+            if (q + 1 < ns) load(q + 1, v1, r1);
+            add(q, v0, r0);
+            __syncthreads();
+            if (q + 1 >= ns) break;
+            if (q + 2 < ns) load(q + 2, v0, r0);
+            add(q + 1, v1, r1);
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) a[i] = 4 * i + g < nj && r < nj ? M[r + (4 * i + g) * LDS] : (T)0;
+    __syncthreads();
+    const bool chol = F.diag == 0;
+    int k4 = 0;  // first column of the wavefronts' first registers
     for (int k = 0; k < nn; ++k) {
-        double amax = 0.0;
-        if (F.reg_kind == 2 && tid < 64)  // GMW81: the column below the pivot (nj <= 64 rows)
-            amax = wave_max((tid > k && tid < nj) ? fabs((double)M[tid + k * LDS]) : 0.0);
-        if (tid == 0) {
-            double akk = (double)M[k + k * LDS];
-            double piv = F.reg_kind == 2 ? regularize_gmw(F, sign_of(F, gc0 + k), akk, amax)
-                                         : regularize(F, sign_of(F, gc0 + k), akk);
+        const int o = k & 3;
+        if (g == o) {
+            double sc;
+            const double piv = small_pivot(F, f.c0 + k, (double)lane_of(a[0], k),
+                                           (r > k && r < nj) ? fabs((double)a[0]) : 0.0, &sc);
             if (piv == 0.0) {
-                *s_fail = 1;
-                atomicMin(F.info, (unsigned long long)(gc0 + k + 1));
-            } else if (F.diag == 0) {
-                T r = (T)sqrt(piv);
-                M[k + k * LDS] = r;
-                *s_piv = (T)1;
-                *s_inv = (T)1 / r;
+                if (r == 0) {
+                    *s_fail = 1;
+                    atomicMin(F.info, (unsigned long long)(f.c0 + k + 1));
+                }
             } else {
-                stc(F.d + gc0 + k, (T)piv);
-                *s_piv = (T)piv;
-                *s_inv = (T)1 / (T)piv;
+                if (r == 0) {
+                    *s_piv = chol ? (T)1 : (T)piv;
+                    if (!chol) stc(F.d + f.c0 + k, (T)piv);
+                }
+                M[r + k * LDS] = r > k ? a[0] * (T)sc : (r == k && chol) ? (T)(piv * sc) : a[0];
             }
         }
         __syncthreads();
         if (*s_fail) return;
-        const T inv = *s_inv;
-        const int r = tid & 63, cg = tid >> 6;
-        if (tid < 64 && r > k && r < nj) M[r + k * LDS] *= inv;
-        __syncthreads();
-        const T piv = *s_piv;
-        if (r < nj) {
-            const T lr = M[r + k * LDS] * piv;
-            for (int c = k + 1 + cg; c <= r; c += 4) M[r + c * LDS] -= lr * M[c + k * LDS];
+        const T lr = -M[r + k * LDS] * *s_piv;
+#pragma unroll
+        for (int h = 0; h < NB / 4; h += 4) {
+            if (k4 + 4 * h >= nj) break;  // uniform
+#pragma unroll
+            for (int i = h; i < h + 4; ++i)
+                if (i > 0 || g > o) a[i] += lr * M[min(k4 + 4 * i + g, NB - 1) + k * LDS];
         }
-        __syncthreads();
-    }
-}
-
-// One small front (nJ <= 64) in LDS: extend-add of the children's update
-// matrices, assembly with the panel's A entries, partial factorization,
-// write-out of the panel and of U.  The caller has made the children final.
-template <typename T>
-__device__ __forceinline__ void small_front(const DevPlan& P, const DevFactor<T>& F, int J, T* M, T* s_piv,
-                            T* s_inv, int* s_fail, const int tid) {
-    const Front f = P.fronts[J];
-    const int nn = f.nn, na = f.na, nj = nn + na;
-    const int r = tid & 63, cg = tid >> 6;
-    for (int c = cg; c < nj; c += 4) M[r + c * LDS] = (T)0;
-    __syncthreads();
-    for (int q = f.chd0; q < f.chd1; ++q) {
-        const Front kf = P.fronts[P.chd[q]];
-        const int ma = kf.na;
-        const int32_t* relK = P.rel + kf.reloff;
-        const T* UK = F.U + kf.uoff;
-        if (r < ma) {
-            // all loads first (fixed count, clamped in-bounds addresses), then
-            // the adds: loads under a per-lane loop bound would each be waited
-            // for inside the loop
-            const int rr = relK[r];
-            for (int i0 = 0; i0 < SMALL_NJ / 4; i0 += 8) {
-                if (cg + 4 * i0 > r) break;
-                int cc[8];
-                T v[8];
+        if (o == 3) {
+            k4 += 4;
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int c = cg + 4 * (i0 + i), cs = c <= r ? c : 0;
-                    cc[i] = relK[cs];
-                    v[i] = ldc(UK + r + cs * ma);
-                }
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    if (cg + 4 * (i0 + i) <= r) M[rr + cc[i] * LDS] += v[i];
-            }
+            for (int i = 0; i + 1 < NB / 4; ++i) a[i] = a[i + 1];
         }
-        __syncthreads();
+        // s_piv is one column's: the next owner writes it after every
+        // wavefront has read it
+        if (!chol) __syncthreads();
     }
-    T* Pj = F.panel + f.poff;
-    if (r < nj) {
-        for (int i0 = 0; i0 < SMALL_NJ / 4; i0 += 8) {
-            if (cg + 4 * i0 > r || cg + 4 * i0 >= nn) break;
-            T v[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int c = cg + 4 * (i0 + i);
-                v[i] = (c <= r && c < nn) ? Pj[r + c * nj] : (T)0;
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int c = cg + 4 * (i0 + i);
-                if (c <= r && c < nn) M[r + c * LDS] += v[i];
-            }
-        }
-    }
-    __syncthreads();
-    factor_lds<T>(M, nn, nj, f.c0, F, s_piv, s_inv, s_fail, tid);
-    if (r < nj)
-        for (int c = cg; c <= r && c < nn; c += 4) stc(Pj + r + c * nj, M[r + c * LDS]);
-    if (na > 0 && r < na) {
+    // the update matrix's columns (c >= nn) and the panel
+    pin(a);
+    if (na > 0) {
         T* Uj = F.U + f.uoff;
-        for (int c = cg; c <= r; c += 4) stc(Uj + r + c * na, M[(nn + r) + (nn + c) * LDS]);
+#pragma unroll
+        for (int i = 0; i < NB / 4; ++i) {
+            const int c = k4 + 4 * i + g;
+            if (c >= nn && c < nj && r >= c && r < nj) stc(Uj + (r - nn) + (int64_t)(c - nn) * na, a[i]);
+        }
     }
+    for (int c = g; c < nn; c += 4)
+        if (r >= c && r < nj) stc(Pj + r + (int64_t)c * nj, M[r + c * LDS]);
 }
 
 constexpr int LDT1 = TINY_NJ + 1;     // leading dimension of a wavefront's LDS front
 
-// One tiny front (nJ <= TINY_NJ) by one wavefront in its own LDS slab Mw:
-// the same extend-add, assembly, right-looking partial factorization and
-// write-out as small_front, lane r keeping row r.  A wavefront's LDS
-// operations complete in order, so no barrier is needed.
+// One tiny front (nJ <= TINY_NJ) by one wavefront: as small_front, with the
+// whole front in the wavefront's registers (row in the lane, one register a
+// column, four columns to a step of the loop) and its own LDS slab Mw for
+// the sums and the finished columns.  A wavefront's LDS operations complete
+// in order, so no barrier is needed.  Children are added two at a time, even
+// columns by lanes 0..31 and odd ones by lanes 32..63.
 template <typename T>
-__device__ __forceinline__ void wave_front(const DevPlan& P, const DevFactor<T>& F, int J, T* Mw,
-                                           const int lane) {
-    const Front f = P.fronts[J];
-    const int nn = f.nn, na = f.na, nj = nn + na, gc0 = f.c0;
-    const int r = lane;
-    if (r < nj)
-        for (int c = 0; c <= r; ++c) Mw[r + c * LDT1] = (T)0;
-    for (int q = f.chd0; q < f.chd1; ++q) {
-        const Front kf = P.fronts[P.chd[q]];
-        const int ma = kf.na;
-        const int32_t* relK = P.rel + kf.reloff;
-        const T* UK = F.U + kf.uoff;
-        if (r < ma) {
-            // loads first, eight at a time (fixed count, clamped in-bounds
-            // addresses), then the adds
-            const int rr = relK[r];
-#pragma unroll
-            for (int c0 = 0; c0 < TINY_NJ; c0 += 8) {
-                if (c0 > r) break;
-                int cc[8];
-                T v[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int c = c0 + i, cs = c <= r ? c : 0;
-                    cc[i] = relK[cs];
-                    v[i] = ldc(UK + r + cs * ma);
-                }
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    if (c0 + i <= r) Mw[rr + cc[i] * LDT1] += v[i];
-            }
-        }
-    }
+__device__ __forceinline__ void wave_front(const DevPlan& P, const DevFactor<T>& F, int J, T* Mw, const int lane) {
+    const Front f = uniform(P.fronts[J]);
+    const int nn = f.nn, na = f.na, nj = nn + na;
+    const int r = lane & (TINY_NJ - 1), half = lane >> 5;
     T* Pj = F.panel + f.poff;
-    if (r < nj) {
+    auto sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
 #pragma unroll
-        for (int c0 = 0; c0 < TINY_NJ; c0 += 8) {
-            if (c0 > r || c0 >= nn) break;
-            T v[8];
+    for (int c0 = 0; c0 < TINY_NJ; c0 += 16) {
+        if (c0 >= nj) break;  // uniform
+        T v[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int c = c0 + i;
-                v[i] = (c <= r && c < nn) ? Pj[r + c * nj] : (T)0;
+        for (int i = 0; i < 8; ++i) v[i] = Pj[min(r, nj - 1) + (int64_t)min(c0 + 2 * i + half, nn - 1) * nj];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int c = c0 + 2 * i + half;
+            Mw[r + c * LDT1] = (c < nn && c <= r && r < nj) ? v[i] : (T)0;
+        }
+    }
+    wait_children(P, F, f.chd0, f.chd1, lane);
+    sync();
+    for (int qb = f.chd0; qb < f.chd1; qb += 64) {
+        const int ns = min(64, f.chd1 - qb);
+        const VChild x = P.vchd[qb + min(lane, ns - 1)];
+        auto get = [&](int32_t v, int q) { return __builtin_amdgcn_readlane(v, q); };
+        auto load = [&](int q, T (&v)[TINY_NJ / 2], int& rr) {
+            const int ma = get(x.ma, q);
+            const uint64_t uo = (uint32_t)get((int32_t)(uint64_t)x.u, q) |
+                                (uint64_t)(uint32_t)get((int32_t)((uint64_t)x.u >> 32), q) << 32;
+            const uint32_t row = min(r, ma - 1);
+            rr = (P.rel + get(x.rel, q))[row];
+            const T* u = F.U + uo;
+#pragma unroll
+            for (int h = 0; h < TINY_NJ / 2; h += 4) {
+                if (2 * h >= ma) break;  // uniform
+#pragma unroll
+                for (int i = h; i < h + 4; ++i) v[i] = ldc(u + (row + (uint32_t)(min(2 * i + half, ma - 1) * ma)));
             }
+        };
+        auto add = [&](int q, const T (&v)[TINY_NJ / 2], int rr) {
+            const int ma = get(x.ma, q);
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-                if (c0 + i <= r && c0 + i < nn) Mw[r + (c0 + i) * LDT1] += v[i];
+            for (int h = 0; h < TINY_NJ / 2; h += 4) {
+                if (2 * h >= ma) break;  // uniform
+#pragma unroll
+                for (int i = h; i < h + 4; ++i) {
+                    const int c = 2 * i + half;
+                    const int c0 = get(rr, min(2 * i, ma - 1)), c1 = get(rr, min(2 * i + 1, ma - 1));
+                    if (c <= r && r < ma) Mw[rr + (half ? c1 : c0) * LDT1] += v[i];
+                }
+            }
+            sync();
+        };
+        T v0[TINY_NJ / 2], v1[TINY_NJ / 2];
+        int r0 = 0, r1 = 0;
+        for (int q = 0; q < ns; q += 2) {
+            load(q, v0, r0);
+            if (q + 1 < ns) load(q + 1, v1, r1);
+            add(q, v0, r0);
+            if (q + 1 < ns) add(q + 1, v1, r1);
         }
     }
-    for (int k = 0; k < nn; ++k) {
-        const T akk = Mw[k + k * LDT1];
-        double piv;
-        if (F.reg_kind == 2) {  // GMW81: the column below the pivot, one row per lane
-            const double amax = wave_max((r > k && r < nj) ? fabs((double)Mw[r + k * LDT1]) : 0.0);
-            piv = regularize_gmw(F, sign_of(F, gc0 + k), (double)akk, amax);
-        } else {
-            piv = regularize(F, sign_of(F, gc0 + k), (double)akk);
-        }
+    T a[TINY_NJ];
+#pragma unroll
+    for (int c = 0; c < TINY_NJ; ++c) a[c] = (c & ~3) < nj ? Mw[r + c * LDT1] : (T)0;
+    const bool chol = F.diag == 0;
+    int k4 = 0;
+    bool failed = false;
+    // column k = k4 + O, held in register O
+    auto pivot = [&](auto O) {
+        constexpr int o = decltype(O)::value;
+        const int k = k4 + o;
+        if (k >= nn || failed) return;  // uniform
+        double sc;
+        const double piv = small_pivot(F, f.c0 + k, (double)lane_of(a[o], k), (r > k && r < nj) ? fabs((double)a[o]) : 0.0, &sc);
         if (piv == 0.0) {
-            if (lane == 0) atomicMin(F.info, (unsigned long long)(gc0 + k + 1));
-            return;  // the front stays unfinished; info reports the column
+            if (lane == 0) atomicMin(F.info, (unsigned long long)(f.c0 + k + 1));
+            failed = true;
+            return;
         }
-        T inv, spv;
-        if (F.diag == 0) {
-            const T rt = (T)sqrt(piv);
-            if (lane == 0) Mw[k + k * LDT1] = rt;
-            inv = (T)1 / rt;
-            spv = (T)1;
-        } else {
-            if (lane == 0) stc(F.d + gc0 + k, (T)piv);
-            inv = (T)1 / (T)piv;
-            spv = (T)piv;
-        }
-        if (r > k && r < nj) Mw[r + k * LDT1] *= inv;
-        if (r > k && r < nj) {
-            const T lr = Mw[r + k * LDT1] * spv;
-            for (int c = k + 1; c <= r; ++c) Mw[r + c * LDT1] -= lr * Mw[c + k * LDT1];
-        }
+        if (!chol && lane == 0) stc(F.d + f.c0 + k, (T)piv);
+        const T l = r > k ? a[o] * (T)sc : (r == k && chol) ? (T)(piv * sc) : a[o];
+        Mw[r + k * LDT1] = l;
+        const T lr = chol ? -l : -l * (T)piv;
+#pragma unroll
+        for (int i = o + 1; i < TINY_NJ; ++i)
+            if (k4 + (i & ~3) < nj) a[i] += lr * lane_of(l, min(k4 + i, TINY_NJ - 1));
+    };
+    for (;;) {
+        pivot(std::integral_constant<int, 0>());
+        pivot(std::integral_constant<int, 1>());
+        pivot(std::integral_constant<int, 2>());
+        pivot(std::integral_constant<int, 3>());
+        if (failed) return;  // the front stays unfinished; info reports the column
+        if (k4 + 4 > nn) break;
+        k4 += 4;
+#pragma unroll
+        for (int i = 0; i + 4 < TINY_NJ; ++i) a[i] = a[i + 4];
     }
-    if (r < nj)
-        for (int c = 0; c <= r && c < nn; ++c) stc(Pj + r + c * nj, Mw[r + c * LDT1]);
-    if (na > 0 && r < na) {
+    pin(a);
+    sync();
+    // the update matrix's columns, odd and even in the two halves' lanes
+    if (na > 0) {
         T* Uj = F.U + f.uoff;
-        for (int c = 0; c <= r; ++c) stc(Uj + r + c * na, Mw[(nn + r) + (nn + c) * LDT1]);
+#pragma unroll
+        for (int i = 0; i < TINY_NJ; ++i) {
+            const int c = k4 + i;
+            if ((i & 1) == half && c >= nn && c < nj && r >= c && r < nj) stc(Uj + (r - nn) + (c - nn) * na, a[i]);
+        }
     }
+    for (int c = half; c < nn; c += 2)
+        if (r >= c && r < nj) stc(Pj + r + (int64_t)c * nj, Mw[r + c * LDT1]);
 }
 
 // Persistent walk of the small region.  Tickets are units of the planner's
@@ -332,13 +448,13 @@ __device__ __forceinline__ void wave_front(const DevPlan& P, const DevFactor<T>&
 // its own children; a child in the same unit belongs to another wavefront,
 // which progresses on its own).  Update matrices go through device-coherent
 // accesses, so a front is published by draining its stores and setting its
-// flag; no cache-wide write-back or invalidate.
+// flag; no cache-wide write-back or invalidate.  (Several units a ticket, as
+// the solves take their tasks, were slower: 600 systems 655 -> 706 us.)
 template <typename T>
-__global__ __launch_bounds__(256, 4) void k_small(DevPlan P, DevFactor<T> F, const int32_t* list,
-                                               const int32_t* units, int count) {
+__global__ __launch_bounds__(256, 4) void k_small(DevPlan P, DevFactor<T> F, int tickets) {
     constexpr int MS = SMALL_NJ * LDS > 4 * TINY_NJ * LDT1 ? SMALL_NJ * LDS : 4 * TINY_NJ * LDT1;
     __shared__ T M[MS];
-    __shared__ T s_piv, s_inv;
+    __shared__ T s_piv;
     __shared__ int s_fail, s_t;
     for (;;) {
         int tid = (int)threadIdx.x;
@@ -347,30 +463,19 @@ __global__ __launch_bounds__(256, 4) void k_small(DevPlan P, DevFactor<T> F, con
         __syncthreads();
         const int t = s_t;
         __syncthreads();
-        if (t >= count) break;
-        const int u = units[t], start = u >> 3, cnt = u & 7;
+        if (t >= tickets) break;
+        const int u = P.small_units[t], start = u >> 3, cnt = u & 7;
         if (cnt == 0) {  // one front, the whole workgroup
-            const int J = list[start];
-            if (tid == 0) {
-                s_fail = 0;
-                const Front f = P.fronts[J];
-                for (int q = f.chd0; q < f.chd1; ++q) wait_ge(F.flags + P.chd[q], 1, F);
-            }
-            __syncthreads();
-            small_front<T>(P, F, J, M, &s_piv, &s_inv, &s_fail, tid);
+            const int J = P.small_order[start];
+            if (tid == 0) s_fail = 0;
+            small_front<T, true>(P, F, J, M, &s_piv, &s_fail, tid);
             drain_stores();
             __syncthreads();
             if (tid == 0) __hip_atomic_store(F.flags + J, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
-            const int wave = tid >> 6, lane = tid & 63;
+            const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
             if (wave < cnt) {
-                const int J = list[start + wave];
-                const Front f = P.fronts[J];
-                if (lane == 0)
-                    for (int q = f.chd0; q < f.chd1; ++q) wait_ge(F.flags + P.chd[q], 1, F);
-                // the children's data is read after the wait (device-coherent loads)
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                const int J = P.small_order[start + wave];
                 wave_front<T>(P, F, J, M + wave * TINY_NJ * LDT1, lane);
                 drain_stores();
                 __builtin_amdgcn_wave_barrier();
@@ -564,19 +669,6 @@ __device__ __forceinline__ float dpp_bcast(float s) {
         float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0x150 + K, 0xf, 0xf, true));
 }
 
-// 1 / sqrt(d) and 1 / d to full double precision: the hardware estimate
-// (about 24 bits) and one step of third order, a chain of five and three
-// operations.
-__device__ __forceinline__ double rsqrt_full(double d) {
-    const double y = __builtin_amdgcn_rsq(d);
-    const double e = __builtin_fma(-(d * y), y, 1.0);
-    return __builtin_fma(y, e * __builtin_fma(e, 0.375, 0.5), y);
-}
-__device__ __forceinline__ double rcp_full(double d) {
-    const double y = __builtin_amdgcn_rcp(d);
-    const double e = __builtin_fma(-d, y, 1.0);
-    return __builtin_fma(y, __builtin_fma(e, e, e), y);
-}
 
 // Pivot rules of the diagonal tile.  PR_RULE: signs and regularization, one
 // call of regularize per pivot; PR_CHOL / PR_LDLT: the default signs (fails
@@ -1369,7 +1461,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
     static_assert(SMALL_NJ * LDS <= SMEM && 4 * EA_LDS <= SMEM && 32 * 129 <= SMEM, "LDS");
     static_assert(SMEM >= 2 * NB * LDS + NB + 6 * (int)(sizeof(double) / sizeof(T)), "potrf_gmw LDS");
     __shared__ __align__(16) T smem[SMEM];
-    __shared__ T s_piv, s_inv;
+    __shared__ T s_piv;
     __shared__ int s_fail, s_sel;
     __shared__ int s_win[WIN];
     if (threadIdx.x == 0)
@@ -1475,7 +1567,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
                 break;
             }
             case DT_SMALL:
-                small_front<T>(P, F, J, smem, &s_piv, &s_inv, &s_fail, tid);
+                small_front<T, false>(P, F, J, smem, &s_piv, &s_fail, tid);
                 break;
             case DT_POTRF:
                 if constexpr (GMW) potrf_gmw<T>(F, uniform(P.fronts[J]), d.a * NB, smem, tid);
@@ -1704,11 +1796,10 @@ void launch_refresh(const DevFactor<T>& F, const int64_t* tp, const int64_t* td,
 }
 
 template <typename T>
-void launch_small(const DevPlan& P, const DevFactor<T>& F, const int32_t* list, const int32_t* units,
-                  int count, hipStream_t s) {
-    if (count <= 0) return;
-    const int grid = count < 2048 ? count : 2048;
-    hipLaunchKernelGGL(k_small<T>, dim3(grid), dim3(256), 0, s, P, F, list, units, count);
+void launch_small(const DevPlan& P, const DevFactor<T>& F, int tickets, hipStream_t s) {
+    if (tickets <= 0) return;
+    const int grid = tickets < 2048 ? tickets : 2048;
+    hipLaunchKernelGGL(k_small<T>, dim3(grid), dim3(256), 0, s, P, F, tickets);
 }
 
 template <typename T>
@@ -1797,8 +1888,7 @@ void launch_copyout(const DevPlan& P, const DevFactor<T>& F, double* Dval, doubl
                                          const double*, int, double*, hipStream_t);             \
     template void launch_refresh<T>(const DevFactor<T>&, const int64_t*, const int64_t*,        \
                                     const double*, int64_t, double*, hipStream_t);              \
-    template void launch_small<T>(const DevPlan&, const DevFactor<T>&, const int32_t*,          \
-                                  const int32_t*, int, hipStream_t);                            \
+    template void launch_small<T>(const DevPlan&, const DevFactor<T>&, int, hipStream_t);                            \
     template void launch_diag<T>(const DevPlan&, const DevFactor<T>&, int, int, bool,           \
                                  hipStream_t);                                                 \
     template void launch_copyout<T>(const DevPlan&, const DevFactor<T>&, double*, double*,      \

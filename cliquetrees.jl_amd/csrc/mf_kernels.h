@@ -16,6 +16,7 @@ struct DevPlan {
     const Front* fronts;
     const int32_t* rows;
     const int32_t* chd;
+    const VChild* vchd;          // per entry of chd
     const int32_t* rel;
     const int32_t* small_order;
     const int32_t* small_units;  // tickets of the small region: start << 3 | tiny count (0: one front)
@@ -88,8 +89,7 @@ template <typename T>
 void launch_refresh(const DevFactor<T>& F, const int64_t* tgt_panel, const int64_t* tgt_diag,
                     const double* nzval, int64_t nnz, double* adiag, hipStream_t s);
 template <typename T>
-void launch_small(const DevPlan& P, const DevFactor<T>& F, const int32_t* list, const int32_t* units,
-                  int count, hipStream_t s);
+void launch_small(const DevPlan& P, const DevFactor<T>& F, int tickets, hipStream_t s);
 // invert_only: the block already holds the factor; only W is produced.
 template <typename T>
 void launch_diag(const DevPlan& P, const DevFactor<T>& F, int t0, int t1, bool invert_only,

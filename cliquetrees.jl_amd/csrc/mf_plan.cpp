@@ -27,6 +27,21 @@ namespace mf {
 
 namespace {
 
+// Runs of consecutive short tasks that one ticket covers, in order: run u is
+// [r[u], r[u + 1]).  A ticket costs 11.5 ns of the one counter whatever runs,
+// so a list of short tasks is paced by it (workgroups x 11.5 ns is 6 to 12 us
+// a task).  One task near both ends of the list (the leaves' first tickets,
+// the root path), up to four in between, where many more tasks are ready
+// than workgroups run.
+std::vector<int32_t> ticket_runs(int32_t n) {
+    std::vector<int32_t> r(1, 0);
+    for (int32_t i = 0; i < n;) {
+        i = std::min(n, i + std::min(4, 1 + std::min(i, n - i) / 2048));
+        r.push_back(i);
+    }
+    return r;
+}
+
 // First-fit allocator over a linear address space with coalescing.
 struct Allocator {
     std::map<int64_t, int64_t> free_;  // offset -> size
@@ -472,6 +487,12 @@ std::string Planner::gather_tables() {
         }
     }
 
+    P.vchd.resize(P.chd.size());
+    for (size_t q = 0; q < P.chd.size(); ++q) {
+        const int32_t K = P.chd[q];
+        const Front& F = P.fronts[K];
+        P.vchd[q] = VChild{P.mvoff1[K], F.uoff, F.na, F.reloff, P.sgoff[K], K};
+    }
     for (int32_t J = 0; J < NJ; ++J) {
         if (P.is_small[J]) continue;
         const Front& F = P.fronts[J];
@@ -974,11 +995,6 @@ std::string Planner::solve_tasks() {
 // task.  Every wait still points to an earlier task or an earlier member of
 // the same group (another wavefront of the same workgroup).
 std::string Planner::vector_tasks() {
-    P.vchd.resize(P.chd.size());
-    for (size_t q = 0; q < P.chd.size(); ++q) {
-        const int32_t K = P.chd[q];
-        P.vchd[q] = VChild{P.mvoff1[K], P.fronts[K].na, P.fronts[K].reloff, P.sgoff[K], 0};
-    }
     for (int dir = 0; dir < 2; ++dir) {
         const std::vector<PTask>& in = dir ? P.btask : P.ftask;
         std::vector<VTask>& out = dir ? P.vbtask : P.vftask;
@@ -1018,16 +1034,8 @@ std::string Planner::vector_tasks() {
             else out.push_back(VTask{VT_SEPB, J, t.a, t.b, t.c, 0, 0, t0});
             pos[J] = (int32_t)out.size() - 1;
         }
-        // tasks per ticket: one near both ends of the list (the root path),
-        // up to four in between, where many more tasks are ready than
-        // workgroups run and the ticket counter would set the pace
-        std::vector<int32_t>& unit = dir ? P.vbunit : P.vfunit;
-        unit.assign(1, 0);
+        (dir ? P.vbunit : P.vfunit) = ticket_runs((int32_t)out.size());
         const int32_t N = (int32_t)out.size();
-        for (int32_t i = 0; i < N;) {
-            i = std::min(N, i + std::min(4, 1 + std::min(i, N - i) / 2048));
-            unit.push_back(i);
-        }
         // every wait points to an earlier task, or an earlier member of a group
         std::vector<int64_t> first(NJ, -1), last(NJ, -1);
         std::vector<int32_t> done(NJ, 0);  // diagonal blocks seen, in chain order

@@ -54,11 +54,11 @@ struct VTask {
     int32_t o12, o3;
     int32_t t0;
 };
-// A child in chd[] order: update vector, rel map and gather table.
+// A child in chd[] order.
 struct VChild {
-    int64_t mv;
-    int32_t ma, rel, sg;
-    int32_t pad;
+    int64_t mv, u;           // update vector, update matrix
+    int32_t ma, rel, sg;     // rows, rel map, gather table
+    int32_t front;
 };
 
 struct Level {
