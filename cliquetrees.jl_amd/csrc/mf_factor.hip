@@ -757,10 +757,11 @@ __device__ __forceinline__ void pivot_cols(T (&x)[PB], T (&y)[PB], const DevFact
 // block; 40 us with the rows below and the inverse in passes of their own).
 // W = L^-1 (ld = nn, zeros above the diagonal) goes to the W pool; L stays in
 // LDS for store_diag.  invert_only: the tile already holds L and only W is
-// formed.  LDS: PTILE elements.
+// formed.  resident: the tile is in LDS already (chain_step left it there).
+// LDS: PTILE elements.
 template <typename T>
 __device__ __forceinline__ void potrf_blocked(const DevFactor<T>& F, const Front f, int k0, bool invert_only,
-                              T* lds, const int tid) {
+                              bool resident, T* lds, const int tid) {
     typedef typename Mfma<T>::v4 v4;
     constexpr int NBLK = NB / PB;
     T* A = lds;                          // 64 x LDS, column-major
@@ -772,7 +773,11 @@ __device__ __forceinline__ void potrf_blocked(const DevFactor<T>& F, const Front
     const int r = tid & 63, cg = tid >> 6, lane = tid & 63, wave = tid >> 6;
     const int li = lane & 15, lk = lane >> 4;
     const bool chol = F.diag == 0;
-    {
+    // the identity's diagonal blocks: block = wave, four elements per thread
+#pragma unroll
+    for (int q = 0; q < 4; ++q) WD[wave * PB * LDP + li + (lk + 4 * q) * LDP] = li == lk + 4 * q ? (T)1 : (T)0;
+    if (tid < NB) sc[tid] = (T)1;
+    if (!resident) {
         // all sixteen loads in flight (outside the tile: the tile's first
         // element stands in), then the LDS writes
         T tv[NB / 4];
@@ -781,10 +786,6 @@ __device__ __forceinline__ void potrf_blocked(const DevFactor<T>& F, const Front
             const int c = cg + 4 * i;
             tv[i] = ldc(blk + ((r < kb && c < kb && c <= r) ? r + (int64_t)c * nj : 0));
         }
-        // the identity's diagonal blocks: block = wave, four elements per thread
-#pragma unroll
-        for (int q = 0; q < 4; ++q) WD[wave * PB * LDP + li + (lk + 4 * q) * LDP] = li == lk + 4 * q ? (T)1 : (T)0;
-        if (tid < NB) sc[tid] = (T)1;
 #pragma unroll
         for (int i = 0; i < NB / 4; ++i) {
             const int c = cg + 4 * i;
@@ -933,10 +934,12 @@ __device__ __forceinline__ void write_c(T* C, int64_t ldc_, int m, int n, bool l
 // the matrix cores' operand registers, and L1 takes the diagonal tile's place
 // in LDS for the update.  The diagonal tile's own L leaves here, behind the
 // loads, since no task waits for it.  The caller has seen A1 and C final
-// through the previous block column.  LDS: PTILE + NB * LDS elements.
+// through the previous block column.  keep: the next diagonal tile stays in
+// LDS, where potrf_blocked's tile goes, instead of going to memory.  LDS:
+// PTILE + NB * LDS elements.
 template <typename T>
 __device__ __forceinline__ void chain_step(const DevFactor<T>& F, const Front f, int k0, const GemmTask t,
-                                           const GemmTask u, T* lds, const int tid) {
+                                           const GemmTask u, bool keep, T* lds, const int tid) {
     typedef typename Mfma<T>::v4 v4;
     constexpr int NBLK = NB / PB;
     T* A = lds;
@@ -1014,7 +1017,17 @@ __device__ __forceinline__ void chain_step(const DevFactor<T>& F, const Front f,
 #pragma unroll
             for (int v = 0; v < 4; ++v) Cs[dst[q] + Mfma<T>::row(lk, v)] = acc[q][v];
     __syncthreads();
-    write_c<T, true>(C, nj, m, m, true, c, Cs, tid);
+    if (!keep) {
+        write_c<T, true>(C, nj, m, m, true, c, Cs, tid);
+        return;
+    }
+    const int r = tid & 63, g = tid >> 6;
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) {
+        const int col = g + 4 * i;
+        const T x = c[i] - Cs[r + col * LDS];
+        A[r + col * LDS] = (r < m && col < m && col <= r) ? x : (r == col ? (T)1 : (T)0);
+    }
 }
 
 // Diagonal tile under GMW81 (chol_factor! GMW81 specialization,
@@ -1136,7 +1149,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_diag(DevPlan P, DevFactor<T> F, int t0, int invert_only) {
     __shared__ T lds[PTILE];
     const DiagTask dt = P.diag[t0 + blockIdx.x];
-    potrf_blocked<T>(F, P.fronts[dt.front], dt.k0, invert_only != 0, lds, (int)threadIdx.x);
+    potrf_blocked<T>(F, P.fronts[dt.front], dt.k0, invert_only != 0, false, lds, (int)threadIdx.x);
     if (!invert_only) store_diag<T>(F, P.fronts[dt.front], dt.k0, lds, (int)threadIdx.x);
 }
 
@@ -1431,6 +1444,20 @@ constexpr int WIN = 1;
 constexpr int WDEP = 64;
 constexpr unsigned long long WMASK = WDEP == 64 ? ~0ull : (1ull << (WDEP & 63)) - 1;
 
+// Thread 0's clocks of a finished task.
+__device__ __forceinline__ void dag_clock(const DevDag& D, int kind, int t, unsigned long long& mark,
+                                          unsigned long long begin) {
+    const unsigned long long now = wall_clock64();
+    if (D.trace) {
+        D.trace[2 * t] = begin | ((unsigned long long)blockIdx.x << 48);
+        D.trace[2 * t + 1] = now;
+    }
+    atomicAdd(D.prof + 3 * kind, begin - mark);
+    atomicAdd(D.prof + 3 * kind + 1, now - begin);
+    atomicAdd(D.prof + 3 * kind + 2, 1ull);
+    mark = now;
+}
+
 // Persistent tile-DAG factorization of the big region.  Tickets are handed
 // out in the planner's order (a list schedule, critical path first); a task
 // depends only on tasks with smaller tickets.  Each workgroup holds WIN
@@ -1462,8 +1489,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
     static_assert(SMEM >= 2 * NB * LDS + NB + 6 * (int)(sizeof(double) / sizeof(T)), "potrf_gmw LDS");
     __shared__ __align__(16) T smem[SMEM];
     __shared__ T s_piv;
-    __shared__ int s_fail, s_sel;
+    __shared__ int s_fail, s_sel, s_drop;
     __shared__ int s_win[WIN];
+    if (threadIdx.x == 0) s_drop = 0;
     if (threadIdx.x == 0)
         for (int i = 0; i < WIN; ++i) {
             const int t = (int)atomicAdd(F.ticket, 1u);
@@ -1471,7 +1499,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
         }
     __syncthreads();
     // wave 0, lane (slot, q): dependency q of the ticket held in slot
-    int my_t = -3, my_tgt = 0, my_extra = 0;
+    int my_t = -3, my_tgt = 0, my_extra = 0, my_drop = 0;
     bool my_has = false;
     int32_t* my_w = nullptr;
     unsigned long long t_mark = 0;
@@ -1496,10 +1524,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
                         const DagTask dd = D.task[t];
                         int nw = 0;
                         my_has = dag_dep<T, GMW>(P, F, D, dd, q, &my_w, &my_tgt, &nw);
+                        my_drop = dd.kind == DT_POTRF ? dd.a + 2 : 0;
                         if (q == 0 && nw > WDEP) my_extra = nw;
                     }
                 }
-                bool ok = !my_has || ld_rel(my_w) >= my_tgt;
+                const int seen = my_has ? ld_rel(my_w) : my_tgt;
+                bool ok = seen >= my_tgt;
                 if (my_extra) {  // more dependencies than lanes (many children): checked here
                     const DagTask dd = D.task[my_t];
                     for (int k = WDEP; k < my_extra && ok; ++k) {
@@ -1533,6 +1563,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
                         }
                     }
                 }
+                // a diagonal tile that the workgroup before it in the chain has
+                // factored already: drop the ticket
+                if (!GMW && tid == 0) s_drop = sel >= 0 && my_drop > 0 && seen >= my_drop;
                 sel = __shfl(sel, 0);
                 if (sel != -1) break;
                 __builtin_amdgcn_s_sleep(1);
@@ -1549,8 +1582,17 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
         __syncthreads();
         const int sel = s_sel;
         if (sel < 0) break;
-        const int t = __builtin_amdgcn_readfirstlane(s_win[sel]);
-        const DagTask d = uniform(D.task[t]);
+        if (s_drop) {
+            __syncthreads();
+            if (tid == 0) {
+                const int nt = (int)atomicAdd(F.ticket, 1u);
+                s_win[sel] = nt < D.ntask ? nt : -1;
+            }
+            __syncthreads();
+            continue;
+        }
+        int t = __builtin_amdgcn_readfirstlane(s_win[sel]);
+        DagTask d = uniform(D.task[t]);
         const int J = d.front;
         const DagFront g = uniform(D.df[J]);
         int32_t* cnt = D.cnt + g.toff;
@@ -1570,26 +1612,39 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
                 small_front<T, false>(P, F, J, smem, &s_piv, &s_fail, tid);
                 break;
             case DT_POTRF:
-                if constexpr (GMW) potrf_gmw<T>(F, uniform(P.fronts[J]), d.a * NB, smem, tid);
-                else potrf_blocked<T>(F, uniform(P.fronts[J]), d.a * NB, false, smem, tid);
-                if (d.b < 0) {
-                    if constexpr (!GMW) store_diag<T>(F, uniform(P.fronts[J]), d.a * NB, smem, tid);
-                } else {
+                for (bool resident = false;;) {
+                    int tid = (int)threadIdx.x;  // opaque again: nothing derived is kept across steps
+                    asm volatile("" : "+v"(tid));
+                    if constexpr (GMW) potrf_gmw<T>(F, uniform(P.fronts[J]), d.a * NB, smem, tid);
+                    else potrf_blocked<T>(F, uniform(P.fronts[J]), d.a * NB, false, resident, smem, tid);
+                    if (d.b < 0) {
+                        if constexpr (!GMW) store_diag<T>(F, uniform(P.fronts[J]), d.a * NB, smem, tid);
+                        break;
+                    }
                     // publish the diagonal tile (the other panel solves of column a
                     // need only it), then the fused panel solve of tile (a+1, a) and
                     // the update of the next diagonal tile, once both tiles are
                     // updated through column a - 1: set by tasks with smaller tickets
-                    // (the planner checks), so the waits end
+                    // (the planner checks), so the waits end.
+                    // The next diagonal tile is then final through column a, and if
+                    // its ticket d.d has been handed out, this workgroup factors it
+                    // as well, from LDS: its holder waits for nothing else, finds
+                    // the tile already final and drops the ticket.  (Every ticket
+                    // before d.d has a holder then, so the fused step's waits end.)
+                    // Otherwise the tile goes to memory for whoever takes it.
                     drain_stores();
                     __syncthreads();
                     if (tid == 0) {
                         __builtin_amdgcn_s_waitcnt(0);
                         __hip_atomic_store(cnt + d.a * g.R + d.a, d.a + 2, __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
+                        const uint32_t taken = sync_ld(F.ticket);
                         (void)bounded_wait(cnt + d.a * g.R + d.a + 1, d.a + 1, F.hang, F.ticket, F.stall, 1);
                         (void)bounded_wait(cnt + (d.a + 1) * g.R + d.a + 1, d.a + 1, F.hang, F.ticket, F.stall, 1);
+                        s_sel = (!GMW && taken > (uint32_t)d.d) ? 1 : 0;
                     }
                     __syncthreads();
+                    const bool keep = __builtin_amdgcn_readfirstlane(s_sel) != 0;
                     if constexpr (GMW) {
                         gemm_tile64<T, true>(F, uniform(P.gemm[d.b]), smem, smem + NB * LDT, tid);
                         // the update reads the panel solve's tile back from memory
@@ -1598,8 +1653,19 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
                         gemm_tile64<T, false>(F, uniform(P.gemm[d.c]), smem, smem + NB * LDT, tid);
                     } else {
                         chain_step<T>(F, uniform(P.fronts[J]), d.a * NB, uniform(P.gemm[d.b]),
-                                      uniform(P.gemm[d.c]), smem, tid);
+                                      uniform(P.gemm[d.c]), keep, smem, tid);
                     }
+                    if (!keep) break;
+                    drain_stores();
+                    __syncthreads();
+                    if (tid == 0) {
+                        __hip_atomic_store(cnt + d.a * g.R + d.a + 1, d.a + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        if (D.prof) dag_clock(D, d.kind, t, t_mark, t_begin);
+                        if (D.prof) t_begin = t_mark;
+                    }
+                    t = d.d;
+                    d = uniform(D.task[t]);
+                    resident = true;
                 }
                 break;
             default: {
@@ -1615,17 +1681,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2) void k_dag(DevPlan P, 
         drain_stores();
         __syncthreads();
         if (tid == 0) {
-            if (D.prof) {
-                const unsigned long long now = wall_clock64();
-                if (D.trace) {
-                    D.trace[2 * t] = t_begin | ((unsigned long long)blockIdx.x << 48);
-                    D.trace[2 * t + 1] = now;
-                }
-                atomicAdd(D.prof + 3 * d.kind, t_begin - t_mark);
-                atomicAdd(D.prof + 3 * d.kind + 1, now - t_begin);
-                atomicAdd(D.prof + 3 * d.kind + 2, 1ull);
-                t_mark = now;
-            }
+            if (D.prof) dag_clock(D, d.kind, t, t_mark, t_begin);
             const unsigned long long r0 = D.prof ? wall_clock64() : 0;
             // every task output is written through (device-coherent stores), and
             // every wave drained its stores before the barrier: no L2 write-back

@@ -111,7 +111,8 @@ struct DagTask {
     int32_t c;   // DT_EA: 1 for panel columns, 0 for update-matrix columns;
                  // DT_TRSM: panel block K; DT_UPD/SYRK: column block Jc
     int32_t d;   // DT_UPD: panel blocks [K0, K1) as K0 | K1 << 16; DT_SYRK: bit 0 /
-                 // bit 1: the tile also covers row block I+1 / column block Jc+1
+                 // bit 1: the tile also covers row block I+1 / column block Jc+1;
+                 // DT_POTRF with fused products: the ticket of block K + 1
 };
 
 // Per-front constants of the DAG.

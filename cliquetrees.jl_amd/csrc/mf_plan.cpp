@@ -1614,6 +1614,14 @@ std::string Planner::schedule() {
         for (size_t i = 0; i < order_gmw.size(); ++i) dag3[i] = P.dag[order_gmw[i]];
         P.dag.swap(dag2);
         P.dag_gmw.swap(dag3);
+        // a diagonal task's successor in its front's chain
+        std::vector<int32_t> next(NJ, -1);
+        for (int32_t t = NT - 1; t >= 0; --t) {
+            DagTask& d = P.dag[t];
+            if (d.kind != DT_POTRF) continue;
+            if (d.c >= 0) d.d = next[d.front];
+            next[d.front] = t;
+        }
     }
     return std::string();
 }
@@ -1692,6 +1700,9 @@ std::string Planner::check_order() {
             if ((d.kind == DT_TRSM || d.kind == DT_UPD) && !ea_done(d.b, d.c)) return "dag: panel task before extend-add";
             if (d.kind == DT_SYRK && last_ea[d.front] >= t) return "dag: update-matrix tile before extend-add";
             auto need = [&](int32_t I, int32_t K) { return setter[cnt_id(d.front, I, K)]; };
+            if (d.kind == DT_POTRF && d.c >= 0 && !gmw &&
+                (d.d <= t || d.d >= NT || dg[d.d].kind != DT_POTRF || dg[d.d].front != d.front || dg[d.d].a != d.a + 1))
+                return "dag: chain successor";
             if (d.kind == DT_POTRF && d.a > 0) {
                 auto it = upd_at.find(cnt_id(d.front, d.a, d.a) * 4096 + d.a - 1);
                 if (it == upd_at.end() || it->second >= t) return "dag: potrf before its update";

@@ -85,3 +85,38 @@ def test_extend_add_many_children(ct, oracle, kids, rows, ns):
     D, L, d, info = oracle.chol_impl(S, Dv, Lv)
     F = ct.cholesky_(ct.ChordalCholesky(A, P, S))
     assert info == 0 and _rel(F.Dval, D) <= 1e-12 and _rel(F.Lval, L) <= 1e-12
+
+
+@pytest.mark.parametrize("sizes", [[65], [150], [700], [1500], [200] * 12])
+@pytest.mark.parametrize("wg_per_cu", [0, 1])
+@pytest.mark.parametrize("kind", ["chol", "ldlt", "chol_f32"])
+def test_diagonal_chain(ct, sizes, wg_per_cu, kind):
+    """Chains of two to twenty-four diagonal tiles, one of them or several at once: a workgroup
+    goes on to the next tile where its ticket has been handed out (short lists, all at once) and
+    leaves it to the ticket's holder where it has not (long lists, fewer workgroups)."""
+    rng = np.random.default_rng(len(sizes) + sizes[0])
+    n = sum(sizes)
+    A = np.zeros((n, n))
+    at = 0
+    for m in sizes:
+        A[at:at + m, at:at + m] = rng.uniform(-1, 1, (m, m))
+        at += m
+    A = np.tril(A, -1)
+    A = A + A.T
+    d = np.abs(A).sum(1) + rng.uniform(0.5, 1.5, n)
+    if kind == "ldlt":
+        d *= np.where(rng.random(n) < 0.3, -1.0, 1.0)
+    A += np.diag(d)
+    C = sp.csc_matrix(A)
+    P, S = ct.symbolic(C)
+    print(kind, sizes, wg_per_cu, S.nfr, flush=True)
+    prec = ct.MF_FP32 if kind == "chol_f32" else ct.MF_FP64
+    tuning = [0, 0, 0, 0, 0, 0, 1, wg_per_cu]  # 0: the default
+    make = ct.ChordalLDLt if kind == "ldlt" else ct.ChordalCholesky
+    F = make(C, P, S, precision=prec, tuning=tuning)
+    F = ct.ldlt_(F) if kind == "ldlt" else ct.cholesky_(F)
+    assert ct.issuccess(F)
+    B = rng.standard_normal((n, 2))
+    X = ct.solve(F, B)
+    # diagonally dominant: n eps with the margin of the other tile tests
+    assert np.linalg.norm(A @ X - B) <= (1e-4 if kind == "chol_f32" else 1e-12) * np.linalg.norm(B)
