@@ -1,7 +1,7 @@
 """Autotuner of the tile-DAG planner parameters, per pattern and precision.
 
 The shape of the big-front schedule is set by seven planner parameters
-(``TUNING_NAMES``: panel steps per trailing-update tile, parent rows per
+(``TUNING_NAMES``: panel steps per trailing-update tile, elements per
 extend-add task, the front width from which update-matrix tiles are
 128 x 128, the workgroups the ticket order is simulated with, and the
 explicit zeros a chain merge may add, the task kinds run at raised wave

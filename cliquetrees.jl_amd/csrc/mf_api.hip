@@ -534,6 +534,11 @@ static int plan_create(int64_t n, int64_t nfr, const int64_t* resptr, const int6
     for (int64_t j = 0; j < H.nfr; ++j)
         for (int64_t g = H.resptr[j]; g < H.resptr[j + 1]; ++g) pl->col2ref[g] = (int32_t)j;
     for (int32_t J : H.small_order) pl->in_small[J] = 1;
+    // both directions' solve tasks and ticket runs in one buffer each
+    std::vector<VTask> vtask(H.vftask);
+    vtask.insert(vtask.end(), H.vbtask.begin(), H.vbtask.end());
+    std::vector<int32_t> vunit(H.vfunit);
+    vunit.insert(vunit.end(), H.vbunit.begin(), H.vbunit.end());
     if ((rc = upload(H.fronts, (Front**)&D.fronts, pl->allocs)) ||
         (rc = upload(H.rows, (int32_t**)&D.rows, pl->allocs)) ||
         (rc = upload(H.chd, (int32_t**)&D.chd, pl->allocs)) ||
@@ -549,10 +554,8 @@ static int plan_create(int64_t n, int64_t nfr, const int64_t* resptr, const int6
         (rc = upload(H.sgoff, (int32_t**)&D.sgoff, pl->allocs)) ||
         (rc = upload(H.gemm, (GemmTask**)&D.gemm, pl->allocs)) ||
         (rc = upload(H.diag, (DiagTask**)&D.diag, pl->allocs)) ||
-        (rc = upload(H.vftask, (VTask**)&pl->V.ftask, pl->allocs)) ||
-        (rc = upload(H.vbtask, (VTask**)&pl->V.btask, pl->allocs)) ||
-        (rc = upload(H.vfunit, (int32_t**)&pl->V.funit, pl->allocs)) ||
-        (rc = upload(H.vbunit, (int32_t**)&pl->V.bunit, pl->allocs)) ||
+        (rc = upload(vtask, (VTask**)&pl->V.ftask, pl->allocs)) ||
+        (rc = upload(vunit, (int32_t**)&pl->V.funit, pl->allocs)) ||
         (rc = upload(H.vchd, (VChild**)&D.vchd, pl->allocs)) ||
         (rc = upload(H.dag, &pl->d_dag, pl->allocs)) ||
         (rc = upload(H.dag_gmw, &pl->d_dag_gmw, pl->allocs)) ||
@@ -568,6 +571,8 @@ static int plan_create(int64_t n, int64_t nfr, const int64_t* resptr, const int6
         delete pl;
         return rc;
     }
+    pl->V.btask = pl->V.ftask + H.vftask.size();
+    pl->V.bunit = pl->V.funit + H.vfunit.size();
     pl->V.chd = D.vchd;
     D.nJ = (int32_t)H.fronts.size();
     pl->V.nfu = std::max<int32_t>(0, (int32_t)H.vfunit.size() - 1);

@@ -4,7 +4,8 @@
 // src/Multifrontal.jl/src/chordal_symbolic.jl:15-28).  Output: HostPlan.
 //   1. internal fronts: chains j -> pnt(j) with pnt(j) = j + 1 (j is the last
 //      child, so columns are contiguous) merged while the explicit zeros stay
-//      under `zero_frac` of the merged panel (or the panel is tiny);
+//      under `zero_frac` of the merged panel (MERGE_FRAC of a small front's, or
+//      the panel is tiny);
 //   2. small region (whole subtree with nJ <= SMALL_NJ): one persistent
 //      launch in ticket order; big region: levels by height;
 //   3. memory: panel pool (all fronts), U pool (small region: private slots;
@@ -203,7 +204,8 @@ std::string Planner::amalgamate() {
         int64_t C = c1 + c2;
         int64_t total = C * (C + 1) / 2 + C * nap;
         int64_t z = gzeros[G] + extra;
-        if ((double)z <= zero_frac * (double)total || C <= 8) {
+        const double frac = C + nap <= MERGE_NJ ? std::max(zero_frac, MERGE_FRAC) : zero_frac;
+        if ((double)z <= frac * (double)total || C <= 8) {
             gowner[p] = G;
             gcols[G] = C;
             gzeros[G] = z;

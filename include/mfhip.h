@@ -63,17 +63,19 @@ int mf_plan_destroy(mf_plan* plan);
 /*
  * mf_plan_create with planner parameters (no counterpart in the reference:
  * the autotuner's entry).  tuning[0..4]: panel steps per trailing-update
- * tile (1..64, default 8), parent rows per extend-add task (default 16384),
+ * tile (1..64, default 8), elements per extend-add task (at least one 64 x 64
+ * tile, 4096 elements; default 16384),
  * the front width from which update-matrix tiles are 128 x 128 (default
  * 128), workgroups assumed resident when ordering the tile-DAG's tickets
  * (default 512), explicit zeros allowed by a chain merge in parts per
- * million (default 50000), and tuning[5] a bit mask of tile-DAG task kinds
+ * million (default 50000; a merged front of at most 256 rows may hold 30 %),
+ * and tuning[5] a bit mask of tile-DAG task kinds
  * run at raised wave priority (bits 0..5: extend-add, small front, diagonal
  * tile, panel solve, trailing update, update matrix; bit 6: the look-ahead
  * trailing update of the panel chain; default 0; negative keeps it),
  * tuning[6] 1 to let each diagonal-tile task also run the panel solve of
- * the tile below it and the look-ahead update of the next diagonal tile, 0
- * (default) for separate tasks (negative keeps it), tuning[7] the resident
+ * the tile below it and the look-ahead update of the next diagonal tile
+ * (default), 0 for separate tasks (negative keeps it), tuning[7] the resident
  * tile-DAG workgroups per CU (0, the default: as many as fit).  Entries
  * 0..4 <= 0 or beyond ntuning keep the default.  mf_plan_tuning reads back
  * the eight values and, as a ninth, the scheduler's estimate of the
