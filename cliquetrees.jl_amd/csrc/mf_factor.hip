@@ -1182,9 +1182,10 @@ __device__ __forceinline__ void load_lds16(const void* g, void* lds) {
 // (the panel pool has 2 NB elements of slack behind its end) and only reach
 // rows and columns of C that are not stored.  C leaves through LDS in rounds
 // (fetch_c's reason).  Bound: the matrix cores, which reach 75 TFLOP/s from
-// LDS alone; FP64, 1,176 tiles of 128 x 128 x 512 on 512 workgroups: 52.7
-// TFLOP/s (34.9 with the chunks staged through registers), 4,656 tiles of
-// 64 x 64 x 512: 45.8 (39.4).
+// LDS alone; FP64, 1,176 tiles of 128 x 128 x 512 on 512 workgroups in step:
+// 43.9 TFLOP/s (52.7 before pin() ordered the stores of C, which left the
+// DAG's task times as they were; 34.9 with the chunks staged through
+// registers), 4,656 tiles of 64 x 64 x 512: 45.8 (39.4).
 template <typename T, int E>
 __device__ __forceinline__ void gemm_tile(const DevFactor<T>& F, const GemmTask g, T* S, const int tid) {
     typedef typename Mfma<T>::v4 v4;
