@@ -26,6 +26,7 @@
 
 #include "mf_kernels.h"
 #include "mf_mfma.h"
+#include "mf_pivots.h"
 #include "mf_sync.h"
 
 namespace mf {
@@ -265,27 +266,32 @@ __device__ __forceinline__ void small_front(const DevPlan& P, const DevFactor<T>
     __syncthreads();
     const bool chol = F.diag == 0;
     int k4 = 0;  // first column of the wavefronts' first registers
-    for (int k = 0; k < nn; ++k) {
-        const int o = k & 3;
-        if (g == o) {
-            double sc;
-            const double piv = small_pivot(F, f.c0 + k, (double)lane_of(a[0], k),
-                                           (r > k && r < nj) ? fabs((double)a[0]) : 0.0, &sc);
-            if (piv == 0.0) {
-                if (r == 0) {
-                    *s_fail = 1;
-                    atomicMin(F.info, (unsigned long long)(f.c0 + k + 1));
-                }
-            } else {
-                if (r == 0) {
-                    *s_piv = chol ? (T)1 : (T)piv;
-                    if (!chol) stc(F.d + f.c0 + k, (T)piv);
-                }
-                M[r + k * LDS] = r > k ? a[0] * (T)sc : (r == k && chol) ? (T)(piv * sc) : a[0];
-            }
+    struct Fail {
+        int* p;
+        bool writer;  // one lane of the owner
+        __device__ __forceinline__ void set(int v) const {
+            if (writer) *p = v;
         }
-        __syncthreads();
-        if (*s_fail) return;
+        __device__ __forceinline__ int get() const { return *p; }
+    };
+    // column k, held in the owner's first register
+    auto own = [&](int k) {
+        double sc;
+        const double piv = small_pivot(F, f.c0 + k, (double)lane_of(a[0], k),
+                                       (r > k && r < nj) ? fabs((double)a[0]) : 0.0, &sc);
+        if (piv == 0.0) {
+            if (r == 0) atomicMin(F.info, (unsigned long long)(f.c0 + k + 1));
+            return false;
+        }
+        if (r == 0) {
+            *s_piv = chol ? (T)1 : (T)piv;
+            if (!chol) stc(F.d + f.c0 + k, (T)piv);
+        }
+        M[r + k * LDS] = r > k ? a[0] * (T)sc : (r == k && chol) ? (T)(piv * sc) : a[0];
+        return true;
+    };
+    auto update = [&](int k) {
+        const int o = k & 3;
         const T lr = -M[r + k * LDS] * *s_piv;
 #pragma unroll
         for (int h = 0; h < NB / 4; h += 4) {
@@ -299,10 +305,9 @@ __device__ __forceinline__ void small_front(const DevPlan& P, const DevFactor<T>
 #pragma unroll
             for (int i = 0; i + 1 < NB / 4; ++i) a[i] = a[i + 1];
         }
-        // s_piv is one column's: the next owner writes it after every
-        // wavefront has read it
-        if (!chol) __syncthreads();
-    }
+    };
+    // (closed for LDLt: s_piv is one column's)
+    if (!pivot_columns(nn, g, !chol, own, Fail{s_fail, r == 0}, [] { __syncthreads(); }, update)) return;
     // the update matrix's columns (c >= nn) and the panel
     pin(a);
     if (na > 0) {
