@@ -173,12 +173,24 @@ __device__ __forceinline__ void wait_children(const DevPlan& P, const DevFactor<
 }
 
 // The pivot of column k from its diagonal entry and (GMW81) the magnitudes
-// below it: the pivot (0: failed), and its scale (1 / sqrt or 1 /).
+// below it: the pivot (0: failed), its scale (1 / sqrt or 1 /) and, for
+// Cholesky, its root.  The estimates of rsqrt_full and rcp_full hold where the
+// pivot and its reciprocal are normal numbers (exponents 1 to 2044); any other
+// takes the square root and the division, so that an infinite diagonal entry
+// (a pinned unknown) scales its column to zero and a subnormal one is as
+// accurate as the rest.
 template <typename T>
-__device__ __forceinline__ double small_pivot(const DevFactor<T>& F, int gcol, double akk, double below, double* scale) {
+__device__ __forceinline__ double small_pivot(const DevFactor<T>& F, int gcol, double akk, double below, double* scale,
+                                              double* root) {
     const double piv = F.reg_kind == 2 ? regularize_gmw(F, sign_of(F, gcol), akk, wave_max(below))
                                        : regularize(F, sign_of(F, gcol), akk);
     *scale = F.diag == 0 ? rsqrt_full(piv) : rcp_full(piv);
+    *root = piv * *scale;
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(__builtin_bit_cast(unsigned long long, piv) >> 32));
+    if (__builtin_expect(((hi >> 20) & 0x7ff) - 1 >= 2044, 0)) {
+        *root = sqrt(piv);
+        *scale = 1.0 / (F.diag == 0 ? *root : piv);
+    }
     return piv;
 }
 
@@ -276,9 +288,9 @@ __device__ __forceinline__ void small_front(const DevPlan& P, const DevFactor<T>
     };
     // column k, held in the owner's first register
     auto own = [&](int k) {
-        double sc;
+        double sc, rt;
         const double piv = small_pivot(F, f.c0 + k, (double)lane_of(a[0], k),
-                                       (r > k && r < nj) ? fabs((double)a[0]) : 0.0, &sc);
+                                       (r > k && r < nj) ? fabs((double)a[0]) : 0.0, &sc, &rt);
         if (piv == 0.0) {
             if (r == 0) atomicMin(F.info, (unsigned long long)(f.c0 + k + 1));
             return false;
@@ -287,7 +299,7 @@ __device__ __forceinline__ void small_front(const DevPlan& P, const DevFactor<T>
             *s_piv = chol ? (T)1 : (T)piv;
             if (!chol) stc(F.d + f.c0 + k, (T)piv);
         }
-        M[r + k * LDS] = r > k ? a[0] * (T)sc : (r == k && chol) ? (T)(piv * sc) : a[0];
+        M[r + k * LDS] = r > k ? a[0] * (T)sc : (r == k && chol) ? (T)rt : a[0];
         return true;
     };
     auto update = [&](int k) {
@@ -406,15 +418,15 @@ __device__ __forceinline__ void wave_front(const DevPlan& P, const DevFactor<T>&
         constexpr int o = decltype(O)::value;
         const int k = k4 + o;
         if (k >= nn || failed) return;  // uniform
-        double sc;
-        const double piv = small_pivot(F, f.c0 + k, (double)lane_of(a[o], k), (r > k && r < nj) ? fabs((double)a[o]) : 0.0, &sc);
+        double sc, rt;
+        const double piv = small_pivot(F, f.c0 + k, (double)lane_of(a[o], k), (r > k && r < nj) ? fabs((double)a[o]) : 0.0, &sc, &rt);
         if (piv == 0.0) {
             if (lane == 0) atomicMin(F.info, (unsigned long long)(f.c0 + k + 1));
             failed = true;
             return;
         }
         if (!chol && lane == 0) stc(F.d + f.c0 + k, (T)piv);
-        const T l = r > k ? a[o] * (T)sc : (r == k && chol) ? (T)(piv * sc) : a[o];
+        const T l = r > k ? a[o] * (T)sc : (r == k && chol) ? (T)rt : a[o];
         Mw[r + k * LDT1] = l;
         const T lr = chol ? -l : -l * (T)piv;
 #pragma unroll
