@@ -195,7 +195,9 @@ __device__ void small_bwd1(const DevPlan& P, const DevFactor<T>& F, const DevVSo
     Yw[r] = x;
     wave_sync();
     T s0 = (T)0, s1 = (T)0;
-    for (int q = nn & ~15; q < nj; q += 16) {
+    // (without separator rows the stand-in row would be the last diagonal
+    // entry's, and an infinite one times 0 is not 0)
+    for (int q = nj > nn ? nn & ~15 : nj; q < nj; q += 16) {
         T a[16];
         const T xq = Yw[q + (r & 15)];
 #pragma unroll

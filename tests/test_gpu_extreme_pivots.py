@@ -70,3 +70,27 @@ def test_subnormal_pivots(ct, oracle, n, kind):
         if b.size:
             a, b = a * big, b * big
             assert np.isfinite(a).all() and np.linalg.norm(a - b) <= 1e-12 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("n", [12, 16, 21, 32, 33, 47, 64])
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_solves_with_infinite_pivots(ct, n, prec):
+    """Finite solutions with a zero at every pinned unknown, column by column and in blocks."""
+    M = _matrix(n, 3, n)
+    pins = [0, 3, n - 9, n + 2, M.shape[0] - 8, M.shape[0] - 1]
+    A = M.copy()
+    A[pins, pins] = np.inf
+    A = sp.csc_matrix(A)
+    P, S = ct.symbolic(A)
+    print(n, prec, S.nfr, flush=True)
+    F = ct.cholesky_(ct.ChordalCholesky(A, P, S, precision=ct.MF_FP32 if prec == "f32" else ct.MF_FP64))
+    assert ct.issuccess(F)
+    free = np.setdiff1d(np.arange(M.shape[0]), pins)
+    for nrhs in (1, 5, 7, 17):
+        B = np.random.default_rng(nrhs).standard_normal((M.shape[0], nrhs))
+        X = ct.solve(F, B)
+        X0 = np.zeros_like(B)
+        X0[free] = np.linalg.solve(M[np.ix_(free, free)], B[free])
+        assert np.all(X[pins] == 0.0), nrhs
+        # the suite's bars for solutions
+        assert np.linalg.norm(X - X0) <= (1e-4 if prec == "f32" else 1e-11) * np.linalg.norm(X0), nrhs
