@@ -91,8 +91,8 @@ struct mf_plan {
     DagTask* d_dag = nullptr;
     DagTask* d_dag_gmw = nullptr;  // the same tasks in creation order (GMW81 factorizations)
     DagFront* d_dagf = nullptr;
-    int32_t* d_uwait_ptr = nullptr;
-    int32_t* d_uwait = nullptr;
+    int32_t* d_gate_ptr = nullptr;
+    int32_t* d_gate = nullptr;
     int32_t* d_cnt0 = nullptr;     // initial tile counters
     double ea_bytes = 0, small_flops = 0, diag_flops = 0;
     // reference flops (sum nn^3/3 + na nn^2 + na^2 nn over the reference's own
@@ -383,7 +383,7 @@ void enqueue_factor(mf_factor* f) {
         launch_fill<int32_t>(f->eacnt, (int64_t)H.fronts.size() + 1, 0, s);
         launch_fill<uint32_t>(f->ticket, 1, 0u, s);
         // GMW81: the ticket order where a diagonal tile follows every update of its block column
-        DevDag D{f->reg_kind == MF_REG_GMW81 ? pl->d_dag_gmw : pl->d_dag, pl->d_dagf, pl->d_uwait_ptr, pl->d_uwait, f->cnt, f->eacnt,
+        DevDag D{f->reg_kind == MF_REG_GMW81 ? pl->d_dag_gmw : pl->d_dag, pl->d_dagf, pl->d_gate_ptr, pl->d_gate, f->cnt, f->eacnt,
                  f->prof, f->prof ? f->trace_buf : nullptr,
                  (int32_t)H.dag.size(), H.tune.prio, H.tune.wg_per_cu};
         timed(f, MF_KC_DAG, pl->ref_flops_dag, 1, [&] { launch_dag<T>(P, F, D, s); });
@@ -534,6 +534,17 @@ static int plan_create(int64_t n, int64_t nfr, const int64_t* resptr, const int6
     for (int64_t j = 0; j < H.nfr; ++j)
         for (int64_t g = H.resptr[j]; g < H.resptr[j + 1]; ++g) pl->col2ref[g] = (int32_t)j;
     for (int32_t J : H.small_order) pl->in_small[J] = 1;
+    // What a front of the tile-DAG waits for before its extend-add: its children
+    // in the same launch (those of the small region are final before it starts,
+    // and a front may have tens of thousands of them) and the fronts whose U
+    // slot it takes.
+    std::vector<int32_t> gate_ptr(1, 0), gate;
+    for (size_t J = 0; J < H.fronts.size(); ++J) {
+        for (int32_t q = H.fronts[J].chd0; q < H.fronts[J].chd1 && !pl->in_small[J]; ++q)
+            if (!pl->in_small[H.chd[q]]) gate.push_back(~H.chd[q]);
+        gate.insert(gate.end(), H.uwait.begin() + H.uwait_ptr[J], H.uwait.begin() + H.uwait_ptr[J + 1]);
+        gate_ptr.push_back((int32_t)gate.size());
+    }
     // both directions' solve tasks and ticket runs in one buffer each
     std::vector<VTask> vtask(H.vftask);
     vtask.insert(vtask.end(), H.vbtask.begin(), H.vbtask.end());
@@ -560,8 +571,8 @@ static int plan_create(int64_t n, int64_t nfr, const int64_t* resptr, const int6
         (rc = upload(H.dag, &pl->d_dag, pl->allocs)) ||
         (rc = upload(H.dag_gmw, &pl->d_dag_gmw, pl->allocs)) ||
         (rc = upload(H.dagf, &pl->d_dagf, pl->allocs)) ||
-        (rc = upload(H.uwait_ptr, &pl->d_uwait_ptr, pl->allocs)) ||
-        (rc = upload(H.uwait, &pl->d_uwait, pl->allocs)) ||
+        (rc = upload(gate_ptr, &pl->d_gate_ptr, pl->allocs)) ||
+        (rc = upload(gate, &pl->d_gate, pl->allocs)) ||
         (rc = upload(H.out, (OutFront**)&D.out, pl->allocs)) ||
         (rc = upload(H.septpos, (int32_t**)&D.septpos, pl->allocs)) ||
         (rc = upload(H.mvoff1, (int64_t**)&D.mvoff1, pl->allocs)) ||

@@ -546,7 +546,93 @@ __device__ __forceinline__ void ea_tile(const DevPlan& P, const DevFactor<T>& F,
         int rr, rc, i, rb, t0, t1, ta;
         T v[16];
     };
-    for (int sb = e.src0; sb < e.src1; sb += 64) {
+    // Thin sources (the planner's choice: many, and few of them more than
+    // sixteen rows high in the tile), eight at a time: lane (i, j) =
+    // (l mod 16, l / 16) is row i of columns j, j + 4, ... of the source's in
+    // this wavefront's strip, so a source is a load and an LDS addition per
+    // four columns, and eight sources' round trips are one.  20000 children of
+    // 20 rows in a front of 500: 20.7 -> 7.3 ms a factorization, of 60 rows in
+    // 4000: 57.5 -> 15.0.  A group with a higher source goes one by one.
+    for (int sb = e.src0; e.thin && sb < e.src1; sb += 64) {
+        const int ns = min(64, e.src1 - sb);
+        const EaSrc x = P.ea_src[sb + min(lane, ns - 1)];
+        const unsigned long long high = __ballot(x.rb - x.ra > 16);
+        auto get = [&](int32_t v, int q) { return __builtin_amdgcn_readlane(v, q); };
+        const int li = lane & 15, lj = lane >> 4;
+        // the source's columns in the strip: the first, their number, this lane's column's place
+        struct Cols {
+            int t0, nt, rc;
+        };
+        auto cols = [&](int q, int rc, bool valid) {
+            const bool has = valid && lane < get(x.tb, q) - get(x.ta, q);
+            const int t0 = (int)__popcll(__ballot(has && rc < cw));
+            return Cols{t0, (int)__popcll(__ballot(has && rc < cw + 16)) - t0, rc};
+        };
+        // columns j + 4 h, row `row` (at place pr of the tile): value and place (a spare one if there is none)
+        auto fetch = [&](int q, const Cols& c, int h, int row, int pr, T& v, int& at) {
+            const int ta = get(x.ta, q), rb = get(x.rb, q);
+            const uint64_t uo = (uint32_t)get((int32_t)(uint64_t)x.u_off, q) |
+                                (uint64_t)(uint32_t)get((int32_t)((uint64_t)x.u_off >> 32), q) << 32;
+            const int j = lj + 4 * h, t = min(c.t0 + j, get(x.tb, q) - ta - 1);
+            const bool on = j < c.nt && row < rb && (!diag || row >= ta + t);
+            const int col = __shfl(c.rc, t) - cw;  // (by every lane)
+            at = on ? col * LDS + pr : 16 * LDS + lane;
+            const T u = ldc(F.U + uo + min(row, rb - 1) + (int64_t)(ta + t) * get(x.ma, q));
+            v = on ? u : (T)0;
+        };
+        constexpr int G = 8;
+        for (int q0 = 0; q0 < ns; q0 += G) {
+            if (((high >> q0) & ((1u << G) - 1)) != 0) {
+#pragma unroll 1
+                for (int q = q0; q < min(q0 + G, ns); ++q) {
+                    const int32_t* rel = P.rel + get(x.rel_off, q);
+                    const Cols c = cols(q, rel[min(get(x.ta, q) + lane, get(x.tb, q) - 1)] - c0, true);
+                    for (int row = get(x.ra, q) + li, r1 = get(x.rb, q), g = 0; 16 * g < r1 - get(x.ra, q); ++g, row += 16) {
+                        const int pr = rel[min(row, r1 - 1)] - r0;
+                        for (int h = 0; 4 * h < c.nt; ++h) {
+                            T v;
+                            int at;
+                            fetch(q, c, h, row, pr, v, at);
+                            acc[at] += v;
+                        }
+                    }
+                }
+                continue;
+            }
+            int pr[G], most = 0;
+            Cols c[G];
+#pragma unroll
+            for (int i = 0; i < G; ++i) {
+                const int q = min(q0 + i, ns - 1);
+                const int32_t* rel = P.rel + get(x.rel_off, q);
+                pr[i] = rel[min(get(x.ra, q) + li, get(x.rb, q) - 1)];
+                c[i].rc = rel[min(get(x.ta, q) + lane, get(x.tb, q) - 1)];
+            }
+#pragma unroll
+            for (int i = 0; i < G; ++i) {
+                pr[i] -= r0;
+                c[i] = cols(min(q0 + i, ns - 1), c[i].rc - c0, q0 + i < ns);
+                most = max(most, c[i].nt);
+            }
+            T v[4][G];
+            int at[4][G];
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                if (4 * h >= most) break;  // uniform
+#pragma unroll
+                for (int i = 0; i < G; ++i) {
+                    const int q = min(q0 + i, ns - 1);
+                    fetch(q, c[i], h, get(x.ra, q) + li, pr[i], v[h][i], at[h][i]);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < G; ++i)
+#pragma unroll
+                for (int h = 0; h < 4; ++h)
+                    if (4 * h < c[i].nt) acc[at[h][i]] += v[h][i];
+        }
+    }
+    for (int sb = e.src0; !e.thin && sb < e.src1; sb += 64) {
         const int ns = min(64, e.src1 - sb);
         // the source records, one per lane
         const EaSrc x = P.ea_src[sb + min(lane, ns - 1)];
@@ -1398,19 +1484,12 @@ __device__ __forceinline__ bool dag_dep(const DevPlan& P, const DevFactor<T>& F,
     switch (d.kind) {
         case DT_EA:
         case DT_SMALL: {  // children complete, earlier users of the U slot consumed
-            const Front f = P.fronts[J];
-            const int nchd = f.chd1 - f.chd0, u0 = D.uwait_ptr[J];
-            *nw = nchd + D.uwait_ptr[J + 1] - u0;
+            const int g0 = D.gate_ptr[J];
+            *nw = D.gate_ptr[J + 1] - g0;
             if (q >= *nw) return false;
-            if (q < nchd) {
-                const int K = P.chd[f.chd0 + q];
-                *w = F.flags + K;
-                *target = D.df[K].n_done;
-            } else {
-                const int c = D.uwait[u0 + q - nchd];
-                *w = D.eacnt + c;
-                *target = D.df[c].n_ea;
-            }
+            const int c = D.gate[g0 + q];
+            *w = c < 0 ? F.flags + ~c : D.eacnt + c;
+            *target = c < 0 ? D.df[~c].n_done : D.df[c].n_ea;
             return true;
         }
         case DT_POTRF:

@@ -26,6 +26,10 @@ constexpr int SMALL_NJ = 64;    // fronts with nJ <= SMALL_NJ use the fused LDS 
 constexpr int TINY_NJ = 32;     // small fronts that one wavefront factors (four per ticket)
 constexpr int EA_TILE = 4096;   // elements of an extend-add tile (64 x 64)
 constexpr int EA_ROWS = 16384;  // elements per extend-add task (at most, where that fills the chip)
+// An extend-add tile takes its sources eight at a time from this many of them
+// on, if at most one in eight times as many is more than sixteen rows high
+// there (such a one takes itself and its seven neighbours one by one).
+constexpr int EA_THIN = 8;
 constexpr int WIDE_K = 128;     // update-matrix tiles are 128 x 128 when nn >= WIDE_K
 constexpr int UPD_GROUP = 8;    // panel steps applied by one trailing-update tile
 constexpr int SIM_WORKERS = 512;  // resident workgroups assumed when ordering the DAG tickets
@@ -76,6 +80,7 @@ struct EaTask {
     int32_t I, J;
     int32_t src0;   // sources [src0, src1) in ea_src
     int32_t src1;
+    int32_t thin;   // 1: many thin sources (EA_THIN)
 };
 struct EaSrc {
     int64_t u_off;    // the child's U

@@ -64,8 +64,8 @@ struct DevFactor {
 struct DevDag {
     const DagTask* task;
     const DagFront* df;
-    const int32_t* uwait_ptr;
-    const int32_t* uwait;
+    const int32_t* gate_ptr;  // per front, what its extend-add waits for:
+    const int32_t* gate;      // ~child of this launch (its flag), or a front whose U slot it takes
     int32_t* cnt;      // tile counters
     int32_t* eacnt;    // finished extend-add tasks per front
     unsigned long long* prof;  // NULL, or per task kind: wait, body (wall-clock ticks), count

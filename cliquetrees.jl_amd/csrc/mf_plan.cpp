@@ -581,12 +581,15 @@ std::string Planner::factor_tasks() {
                     e.I = I;
                     e.J = Jc;
                     e.src0 = (int32_t)P.ea_src.size();
+                    size_t high = 0;  // sources of more than sixteen rows
                     for (int32_t K : src[I - Jc]) {
                         const Front& Kf = P.fronts[K];
                         const int32_t* tb = P.sgstart.data() + P.sgoff[K];
+                        high += tb[I + 1] - tb[I] > 16;
                         P.ea_src.push_back(EaSrc{Kf.uoff, Kf.reloff, Kf.na, tb[I], tb[I + 1], tb[Jc], tb[Jc + 1]});
                     }
                     e.src1 = (int32_t)P.ea_src.size();
+                    e.thin = src[I - Jc].size() >= EA_THIN * (1 + 8 * high);
                     P.ea.push_back(e);
                 }
             }
