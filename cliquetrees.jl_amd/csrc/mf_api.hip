@@ -415,26 +415,27 @@ void sync_ref(mf_factor* f) {
 // Columns of the blocked solves: blocks of sixteen.
 size_t padded(size_t nrhs) { return (nrhs + 15) & ~(size_t)15; }
 
-// Workspaces of the solves of nrhs columns: update vectors, and for the
-// blocked solves the solutions in their row-by-row form.  Without memory for
-// these the columns are solved VT_COLS at a time.
+// Workspaces of the solves of nrhs columns: update vectors, and past VT_COLS
+// columns or for the blocked form the solutions (of the blocked form twice,
+// row by row).  Without memory for these the columns are solved VT_COLS at a
+// time.
 int ensure_solve(mf_factor* f, size_t es, size_t nrhs) {
     const HostPlan& H = f->plan->H;
-    if (nrhs > (size_t)VT_COLS) {
+    if (nrhs > (size_t)std::min(VT_COLS, H.vcols)) {
         const size_t c = padded(nrhs);
         if (ensure(&f->Mv, &f->Mv_bytes, es * (size_t)H.mv_elems1 * c) == MF_OK &&
             ensure(&f->sw, &f->sw_bytes, es * 2 * (size_t)H.n * c) == MF_OK)
             return MF_OK;
         (void)hipGetLastError();
-        nrhs = VT_COLS;
+        nrhs = std::min<size_t>(nrhs, VT_COLS);
     }
     return ensure(&f->Mv, &f->Mv_bytes, es * (size_t)H.mv_elems1 * nrhs);
 }
 
 // mv, sw: the update-vector and solution workspaces (ensure_solve) instead of
-// the factor's own; blocked: they hold the blocked form.
+// the factor's own; room: sw is there, both for padded(nrhs) columns.
 template <typename T>
-void enqueue_solve(mf_factor* f, T* B, int64_t ldb, int nrhs, void* mv = nullptr, void* sw = nullptr, bool blocked = false) {
+void enqueue_solve(mf_factor* f, T* B, int64_t ldb, int nrhs, void* mv = nullptr, void* sw = nullptr, bool room = false) {
     mf_plan* pl = f->plan;
     const HostPlan& H = pl->H;
     const DevPlan& P = pl->D;
@@ -446,19 +447,20 @@ void enqueue_solve(mf_factor* f, T* B, int64_t ldb, int nrhs, void* mv = nullptr
         mv = f->Mv;
         sw = f->sw;
         const size_t c = padded(nrhs);
-        blocked = f->Mv_bytes >= sizeof(T) * (size_t)H.mv_elems1 * c && f->sw_bytes >= sizeof(T) * 2 * (size_t)H.n * c;
+        room = f->Mv_bytes >= sizeof(T) * (size_t)H.mv_elems1 * c && f->sw_bytes >= sizeof(T) * 2 * (size_t)H.n * c;
     }
     double bytes = (double)sizeof(T) * (2.0 * (double)(H.ndz + H.nlz) + 4.0 * H.n * nrhs);
     timed(f, MF_KC_SOLVE, bytes, 1, [&] {
         unsigned long long* trace = f->prof ? f->strace_buf : nullptr;
-        if (nrhs > VT_COLS && blocked) {
+        if (nrhs > H.vcols && room) {
             launch_solve16<T>(P, F, B, ldb, nrhs, (T*)sw, (T*)mv, H.mv_elems1, pl->V, trace, (int64_t)H.ftask.size(),
                               f->stream);
             return;
         }
-        for (int c = 0; c < nrhs; c += VT_COLS)
-            launch_solve1<T>(P, F, B + (int64_t)c * ldb, ldb, std::min(VT_COLS, nrhs - c), (T*)f->xf, (T*)mv, H.mv_elems1,
-                             pl->V, (int)H.n, trace, (int64_t)H.ftask.size(), f->stream);
+        const int step = nrhs > VT_COLS && room ? nrhs : VT_COLS;
+        for (int c = 0; c < nrhs; c += step)
+            launch_solve1<T>(P, F, B + (int64_t)c * ldb, ldb, std::min(step, nrhs - c), (T*)(step > VT_COLS ? sw : f->xf), (T*)mv,
+                             H.mv_elems1, pl->V, (int)H.n, trace, (int64_t)H.ftask.size(), f->stream);
     });
 }
 
@@ -1132,14 +1134,14 @@ int mf_solve_noalloc(mf_factor* f, const int64_t* perm, double* B, int64_t nrhs,
     if (dev != f->device) return fail(MF_EARG, "the factor's device is not the current device");
     void* base = nullptr;
     if (int rc = scratch_address(&base)) return rc;
-    // the blocked solves where their workspaces fit as well, else VT_COLS columns at a time
+    // room for any form where the workspaces fit as well, else VT_COLS columns at a time
     const size_t cols = padded((size_t)nrhs);
     const size_t mvb = (es * (size_t)H.mv_elems1 * cols + 255) & ~(size_t)255, swb = (es * 2 * (size_t)H.n * cols + 255) & ~(size_t)255;
-    const bool blocked = nrhs > VT_COLS && mvb + swb + es * (size_t)H.n * (size_t)nrhs <= MF_NOALLOC_SCRATCH_BYTES;
-    if (blocked) mv_bytes = mvb;
+    const bool room = nrhs > std::min(VT_COLS, H.vcols) && mvb + swb + es * (size_t)H.n * (size_t)nrhs <= MF_NOALLOC_SCRATCH_BYTES;
+    if (room) mv_bytes = mvb;
     void* mv = base;
     void* sw = (unsigned char*)base + mv_bytes;
-    void* bws = blocked ? (unsigned char*)sw + swb : (unsigned char*)sw;
+    void* bws = room ? (unsigned char*)sw + swb : (unsigned char*)sw;
     if (f->perm_host.size() != (size_t)H.n ||
         std::memcmp(f->perm_host.data(), perm, 8 * H.n) != 0) {
         f->perm_host.assign(perm, perm + H.n);
@@ -1149,12 +1151,12 @@ int mf_solve_noalloc(mf_factor* f, const int64_t* perm, double* B, int64_t nrhs,
     if (f->precision == MF_FP32 && !solves64(f)) {
         launch_permute<float>(B, ldb, (float*)bws, H.n, f->perm_dev, (int)H.n, (int)nrhs, false,
                               f->stream);
-        enqueue_solve<float>(f, (float*)bws, H.n, (int)nrhs, mv, sw, blocked);
+        enqueue_solve<float>(f, (float*)bws, H.n, (int)nrhs, mv, sw, room);
         launch_permute_back(bws, H.n, true, B, ldb, f->perm_dev, (int)H.n, (int)nrhs, f->stream);
     } else {
         launch_permute<double>(B, ldb, (double*)bws, H.n, f->perm_dev, (int)H.n, (int)nrhs, false,
                                f->stream);
-        enqueue_solve<double>(f, (double*)bws, H.n, (int)nrhs, mv, sw, blocked);
+        enqueue_solve<double>(f, (double*)bws, H.n, (int)nrhs, mv, sw, room);
         launch_permute_back(bws, H.n, false, B, ldb, f->perm_dev, (int)H.n, (int)nrhs, f->stream);
     }
     HIPCHK(hipGetLastError());

@@ -111,7 +111,8 @@ class Planner {
     std::string gather_tables();  // children's rows per row block of a big front
     std::string factor_tasks();   // 4. extend-add, diagonal and tile-DAG tasks
     std::string solve_tasks();    // persistent solve task lists
-    std::string vector_tasks();   // those of one right-hand side
+    std::string vector_tasks();   // those the solve kernels run
+    void solve_columns();         // columns up to which they run column by column
     std::string check_bounds();   // every task's accesses inside its pools
     std::string dataflow();       // predecessor counts and successor lists of the DAG
     std::string schedule();       // tickets by list scheduling (and the GMW81 order)
@@ -959,6 +960,7 @@ std::string Planner::solve_tasks() {
 
     std::string err = vector_tasks();
     if (!err.empty()) return err;
+    solve_columns();
 
     // consecutive tickets of tiny fronts share one ticket, one wavefront each
     // (a front may wait for another front of the same ticket: that one runs
@@ -1086,6 +1088,60 @@ std::string Planner::vector_tasks() {
         }
     }
     return std::string();
+}
+
+// How many columns the column kernels (mf_solve1.hip) solve faster than one
+// block of sixteen (mf_solve16.hip), both directions.  c columns take the
+// longest path of the tree plus c times the tasks' time over all workgroups;
+// a block takes its own, longer path plus its tasks' time once.  Measured on
+// MI355X with every column count either way (us, columns 1 / 2 / 3 / 4 / 8
+// and a block, columns chosen):
+//   forest of 2000 small grids   195 /  330 /  460 /  593 / 1118    271   1
+//   100000 systems of order 1    372 /  680 /  986 / 1290 / 2496    533   1
+//   700 x 700 grid               704 / 1125 / 1572 / 2017 / 3827   1500   2
+//   56 x 60 x 52 grid            861 / 1036 / 1314 / 1608 / 2782   1920   4
+//   31 x 29 x 27 grid            178 /  204 /  235 /  269 /  414    395   6
+//   20 x 20 x 20 grid            114 /  122 /  125 /  131 /  158    246  13
+//   path of 50000, min. degree  8517 / 8487 / 8528 / 8596 / 8719  25700  16
+// (the line at five columns for every plan had cost the forest 726 against
+// 271 at five columns, and the path 25700 against 8700 at six).
+// The terms, in us: a small front of nn columns 1.76 + 0.118 nn on the path
+// (blocked 3.86 + 0.545 nn), a 64-column block 2.5 (5), a child past the
+// eighth 0.35 in a small front and 0.12 in a big one (0.8, 0.5), 40 for the
+// launches; per task, in ns over all workgroups, a group of small fronts 4 +
+// 0.5 a column (7 + 0.8), any other 12.5 (25 + 14 a tile).
+void Planner::solve_columns() {
+    std::vector<double> lc(NJ, 0.0), lb(NJ, 0.0);
+    double pc = 0, pb = 0, cols = 0, tiles = 0;
+    for (int32_t J = NJ - 1; J >= 0; --J) {
+        const Front& F = P.fronts[J];
+        const double extra = std::max(0, F.chd1 - F.chd0 - 8);
+        const int32_t p = (F.nn + NB - 1) / NB, R = p + (F.na + NB - 1) / NB;
+        if (F.parent >= 0) {
+            lc[J] = lc[F.parent];
+            lb[J] = lb[F.parent];
+        }
+        if (P.is_small[J]) {
+            lc[J] += 1.76 + 0.118 * F.nn + 0.35 * extra;
+            lb[J] += 3.86 + 0.545 * F.nn + 0.8 * extra;
+            cols += 2.0 * F.nn;
+        } else {
+            lc[J] += 2.5 * p + 0.12 * extra;
+            lb[J] += 5.0 * p + 0.5 * extra;
+            tiles += 2.0 * (p * (double)R - 0.5 * p * (p - 1.0));
+        }
+        pc = std::max(pc, lc[J]);
+        pb = std::max(pb, lb[J]);
+    }
+    double small = 0;
+    for (const std::vector<VTask>* l : {&P.vftask, &P.vbtask})
+        for (const VTask& t : *l) small += t.kind == VT_SMALL;
+    const double other = (double)(P.vftask.size() + P.vbtask.size()) - small;
+    const double column = (4.0 * small + 0.5 * cols + 12.5 * other) * 1e-3;
+    const double block = 40.0 + pb + (7.0 * small + 0.8 * cols + 25.0 * other + 14.0 * tiles) * 1e-3;
+    // (0.85: a block too early costs less than columns too long)
+    const double c = 0.85 * (block - 40.0 - pc) / std::max(column, 1e-3);
+    P.vcols = (int32_t)std::min<double>(VT_MAX, std::max(1.0, std::floor(c)));
 }
 
 std::string Planner::check_bounds() {
@@ -1847,7 +1903,7 @@ extern "C" int mf_plan_check(int64_t n, int64_t nfr, const int64_t* resptr, cons
                    P.panel_elems, P.u_elems, P.w_elems, (int64_t)P.gemm.size(),
                    (int64_t)P.ea.size(), (int64_t)(P.ftask.size() + P.btask.size()), (int64_t)P.ref_flops,
                    (int64_t)P.engine_flops, P.max_nj, (int64_t)P.dag.size(), P.dag_counters,
-                   (int64_t)P.sim_makespan_us, ea_u, ea_p, ea_src_rows};
+                   (int64_t)P.sim_makespan_us, ea_u, ea_p, ea_src_rows, P.vcols};
     for (int64_t i = 0; stats && i < nstats && i < (int64_t)(sizeof(v) / sizeof(v[0])); ++i)
         stats[i] = v[i];
     return err.empty() ? 0 : -1;

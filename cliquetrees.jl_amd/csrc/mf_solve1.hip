@@ -1,9 +1,9 @@
-// mf_solve1.hip — gfx950 kernels of the supernodal triangular solves for FEW
-// right-hand sides, column by column (the blocked solves of mf_solve.hip take
-// more than VT_COLS).
+// mf_solve1.hip — gfx950 kernels of the supernodal triangular solves for few
+// right-hand sides, column by column (mf_solve16.hip takes more than the plan
+// says, HostPlan::vcols).
 //
-// Same per-front recurrences as mf_solve.hip (divide.jl:417-659, 864-1038),
-// one persistent launch per direction.  With one column the solves are bound
+// Per-front recurrences of divide.jl:417-659, 864-1038, one persistent launch
+// per direction.  With one column the solves are bound
 // by latency: the chain of diagonal blocks up the root path and the hand-off
 // between workgroups at each of its links.  Three things differ from the
 // blocked kernels because of that:
@@ -39,7 +39,7 @@
 //   56 x 60 x 52 grid, n 174720   867 / 1350 / 1650 / 2290 / 2900   2030   (2237)
 //   31 x 29 x 27 grid, n 24273    179 /  241 /  278 /  360 /  439    415   (670)
 //   100 x 100 grid, n 10000       120 /  163 /  191 /  249 /  307    270   (390)
-// so the line (VT_COLS = 5) is where the largest of these crosses.
+// The planner places the line between the two by the plan (solve_columns).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

@@ -1,5 +1,6 @@
 // mf_solve16.hip — gfx950 kernels of the supernodal triangular solves for more
-// than VT_COLS right-hand sides, in blocks of sixteen on the matrix cores.
+// right-hand sides than go column by column (HostPlan::vcols), in blocks of
+// sixteen on the matrix cores.
 //
 // The tasks, the tickets and the hand-off are those of mf_solve1.hip: an
 // element that another workgroup waits for starts as a signalling NaN and is

@@ -101,7 +101,8 @@ int mfs_grid_nd(int64_t nx, int64_t ny, int64_t nz, int64_t leaf, int64_t* order
  * ChordalSymbolic arrays of mfs_export.  No counterpart in the reference: it
  * lets the planner be checked without a GPU.  stats (optional): internal
  * fronts, small-region fronts, big fronts, levels, panel/U/W elements, GEMM,
- * extend-add and solve tasks, reference and engine flops, max front size.
+ * extend-add and solve tasks, reference and engine flops, max front size, ...;
+ * the twentieth: right-hand sides up to which a solve goes column by column.
  * Returns 0, or -1 with the reason in msg.
  */
 int mf_plan_check(int64_t n, int64_t nfr, const int64_t* resptr, const int64_t* sepptr,
