@@ -174,16 +174,17 @@ __device__ __forceinline__ void wait_children(const DevPlan& P, const DevFactor<
 
 // The pivot of column k from its diagonal entry and (GMW81) the magnitudes
 // below it: the pivot (0: failed), its scale (1 / sqrt or 1 /) and, for
-// Cholesky, its root.  The estimates of rsqrt_full and rcp_full hold where the
+// Cholesky, its root.  sgn: the signs of the front's columns, one a lane (read
+// where there are any).  The estimates of rsqrt_full and rcp_full hold where the
 // pivot and its reciprocal are normal numbers (exponents 1 to 2044); any other
 // takes the square root and the division, so that an infinite diagonal entry
 // (a pinned unknown) scales its column to zero and a subnormal one is as
 // accurate as the rest.
 template <typename T>
-__device__ __forceinline__ double small_pivot(const DevFactor<T>& F, int gcol, double akk, double below, double* scale,
+__device__ __forceinline__ double small_pivot(const DevFactor<T>& F, double sgn, int k, double akk, double below, double* scale,
                                               double* root) {
-    const double piv = F.reg_kind == 2 ? regularize_gmw(F, sign_of(F, gcol), akk, wave_max(below))
-                                       : regularize(F, sign_of(F, gcol), akk);
+    const double sg = F.signs ? lane_of(sgn, k) : F.diag == 0 ? 1.0 : 0.0;
+    const double piv = F.reg_kind == 2 ? regularize_gmw(F, sg, akk, wave_max(below)) : regularize(F, sg, akk);
     *scale = F.diag == 0 ? rsqrt_full(piv) : rcp_full(piv);
     *root = piv * *scale;
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(__builtin_bit_cast(unsigned long long, piv) >> 32));
@@ -278,6 +279,7 @@ __device__ __forceinline__ void small_front(const DevPlan& P, const DevFactor<T>
     __syncthreads();
     const bool chol = F.diag == 0;
     int k4 = 0;  // first column of the wavefronts' first registers
+    const double sgn = F.signs ? F.signs[f.c0 + min(r, nn - 1)] : 0.0;
     struct Fail {
         int* p;
         bool writer;  // one lane of the owner
@@ -289,7 +291,7 @@ __device__ __forceinline__ void small_front(const DevPlan& P, const DevFactor<T>
     // column k, held in the owner's first register
     auto own = [&](int k) {
         double sc, rt;
-        const double piv = small_pivot(F, f.c0 + k, (double)lane_of(a[0], k),
+        const double piv = small_pivot(F, sgn, k, (double)lane_of(a[0], k),
                                        (r > k && r < nj) ? fabs((double)a[0]) : 0.0, &sc, &rt);
         if (piv == 0.0) {
             if (r == 0) atomicMin(F.info, (unsigned long long)(f.c0 + k + 1));
@@ -364,6 +366,7 @@ __device__ __forceinline__ void wave_front(const DevPlan& P, const DevFactor<T>&
             Mw[r + c * LDT1] = (c < nn && c <= r && r < nj) ? v[i] : (T)0;
         }
     }
+    const double sgn = F.signs ? F.signs[f.c0 + min(r, nn - 1)] : 0.0;
     wait_children(P, F, f.chd0, f.chd1, lane);
     sync();
     for (int qb = f.chd0; qb < f.chd1; qb += 64) {
@@ -419,7 +422,7 @@ __device__ __forceinline__ void wave_front(const DevPlan& P, const DevFactor<T>&
         const int k = k4 + o;
         if (k >= nn || failed) return;  // uniform
         double sc, rt;
-        const double piv = small_pivot(F, f.c0 + k, (double)lane_of(a[o], k), (r > k && r < nj) ? fabs((double)a[o]) : 0.0, &sc, &rt);
+        const double piv = small_pivot(F, sgn, k, (double)lane_of(a[o], k), (r > k && r < nj) ? fabs((double)a[o]) : 0.0, &sc, &rt);
         if (piv == 0.0) {
             if (lane == 0) atomicMin(F.info, (unsigned long long)(f.c0 + k + 1));
             failed = true;
@@ -429,9 +432,16 @@ __device__ __forceinline__ void wave_front(const DevPlan& P, const DevFactor<T>&
         const T l = r > k ? a[o] * (T)sc : (r == k && chol) ? (T)rt : a[o];
         Mw[r + k * LDT1] = l;
         const T lr = chol ? -l : -l * (T)piv;
+        // (out of the loop at the first group past the front: a test of every
+        // group is an execution mask each, 10 us a front of nine columns on a
+        // path of 50000 unknowns against 8.7)
 #pragma unroll
-        for (int i = o + 1; i < TINY_NJ; ++i)
-            if (k4 + (i & ~3) < nj) a[i] += lr * lane_of(l, min(k4 + i, TINY_NJ - 1));
+        for (int h = 0; h < TINY_NJ; h += 4) {
+            if (k4 + h >= nj) break;
+#pragma unroll
+            for (int i = h; i < h + 4; ++i)
+                if (i > o) a[i] += lr * lane_of(l, min(k4 + i, TINY_NJ - 1));
+        }
     };
     for (;;) {
         pivot(std::integral_constant<int, 0>());
