@@ -1185,12 +1185,13 @@ __device__ __forceinline__ void potrf_gmw(const DevFactor<T>& F, const Front& f,
         // (2) the largest magnitude below the pivot: tile rows from LDS, rows
         // below the tile from the block column
         double m = (r > j && r < kb && cg == 0) ? fabs((double)A[r + j * LDS]) : 0.0;
-        // RB rows per thread and QB columns per step: RB * QB independent
-        // loads in flight (the rows are device-coherent loads from far
-        // memory); out-of-range rows and columns read row kb / column 0 and
-        // are dropped
-        constexpr int RB = 4, QB = 4;
-        for (int i0 = kb; i0 < nbelow; i0 += 256 * RB) {
+        // RB rows per thread and QB columns per step, as many independent loads
+        // in flight (the rows are device-coherent loads from far memory, a
+        // round trip a step: with 4 x 4 for every height a column of a band of
+        // 100 took 6.7 us, 5.0 now); out-of-range rows and columns read row kb /
+        // column 0 and are dropped
+        auto below = [&](int i0, auto rows, auto cols) {
+            constexpr int RB = decltype(rows)::value, QB = decltype(cols)::value;
             T acc[RB];
             int64_t ro[RB];
 #pragma unroll
@@ -1216,6 +1217,11 @@ __device__ __forceinline__ void potrf_gmw(const DevFactor<T>& F, const Front& f,
 #pragma unroll
             for (int u = 0; u < RB; ++u)
                 if (i0 + tid + 256 * u < nbelow) m = jmax(m, fabs((double)acc[u]));
+        };
+        for (int i0 = kb; i0 < nbelow; i0 += 1024) {
+            if (nbelow - i0 > 512) below(i0, std::integral_constant<int, 4>(), std::integral_constant<int, 4>());
+            else if (nbelow - i0 > 256) below(i0, std::integral_constant<int, 2>(), std::integral_constant<int, 8>());
+            else below(i0, std::integral_constant<int, 1>(), std::integral_constant<int, 16>());
         }
         m = wave_max(m);
         if (lane == 0) s_red[wave] = m;
