@@ -40,14 +40,16 @@ constexpr int SIM_WORKERS = 512;  // resident workgroups assumed when ordering t
 // 1238 at 512, where larger phases become more tickets than workgroups).
 constexpr int SPLIT_TILES = 128;
 // A chain merge whose front stays within MERGE_NJ rows may hold this share of
-// explicit zeros (a larger one the planner's zero_frac): a front of that size
+// explicit zeros (a larger one the planner's zero_frac, which bounds both when
+// the caller sets it): a front of that size
 // costs 20 to 35 us of task latency on the critical path and a handful of
 // tasks, its products almost nothing.  us per pass, 5 % everywhere -> this:
 // 31 x 29 x 27 step 1709 -> 1578, 27-point 48^3 7037 -> 6737, 64^3 20034 ->
 // 19370, batch of 600 3184 -> 2667, 40^3 solve of 75 columns 1536 -> 1429.
 // (128 rows 1622, 6982, 19479, 2677, 1432; half zeros up to 256 rows takes 64^3
-// to 19067 and the batch to 2406, but kkt_7000 from 2066 to 2104; 10 % at
-// every size slows the 27-point grid.)
+// to 19067 and the batch to 2406, but kkt_7000 from 2066 to 2104; 40 % up to
+// 320 rows takes them to 19126 and 2417 and the 27-point grid to 6590, but the
+// 100 x 100 grid from 546 to 589; 10 % at every size slows the 27-point grid.)
 constexpr int MERGE_NJ = 256;
 constexpr double MERGE_FRAC = 0.3;
 constexpr int VT_COLS = 5;                // right-hand sides whose forward solutions a factor always has room for

@@ -97,7 +97,7 @@ inline int64_t rup(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 class Planner {
   public:
     Planner(HostPlan& plan, const PlanTuning& tune)
-        : P(plan), zero_frac(tune.zero_frac), UPD_GROUP(tune.upd_group), EA_ROWS(tune.ea_rows),
+        : P(plan), zero_frac(tune.zero_frac), small_zero_frac(tune.small_zero_frac), UPD_GROUP(tune.upd_group), EA_ROWS(tune.ea_rows),
           WIDE_K(tune.wide_k), SIM_WORKERS(tune.sim_workers), FUSE(tune.fuse != 0) {
         P.tune = tune;
     }
@@ -121,7 +121,7 @@ class Planner {
 
   private:
     HostPlan& P;
-    const double zero_frac;
+    const double zero_frac, small_zero_frac;
     const int32_t UPD_GROUP, EA_ROWS, WIDE_K, SIM_WORKERS;
     const bool FUSE;
     int64_t n = 0, nfr = 0, nsep = 0;  // matrix order, reference fronts, separator entries
@@ -205,7 +205,7 @@ std::string Planner::amalgamate() {
         int64_t C = c1 + c2;
         int64_t total = C * (C + 1) / 2 + C * nap;
         int64_t z = gzeros[G] + extra;
-        const double frac = C + nap <= MERGE_NJ ? std::max(zero_frac, MERGE_FRAC) : zero_frac;
+        const double frac = C + nap <= MERGE_NJ ? small_zero_frac : zero_frac;
         if ((double)z <= frac * (double)total || C <= 8) {
             gowner[p] = G;
             gcols[G] = C;
@@ -1871,7 +1871,9 @@ std::string tuning_from(const int64_t* v, int64_t nv, PlanTuning* t) {
     t->ea_rows = (int32_t)er;
     t->wide_k = (int32_t)wk;
     t->sim_workers = (int32_t)sw;
-    t->zero_frac = (double)zf * 1e-6;
+    // the default value stands for the default rule (plans read back their
+    // parameters and are made again from them)
+    if (zf != (int64_t)llround(t->zero_frac * 1e6)) t->zero_frac = t->small_zero_frac = (double)zf * 1e-6;
     t->prio = (int32_t)pr;
     t->fuse = (int32_t)fu;
     t->wg_per_cu = (int32_t)wc;

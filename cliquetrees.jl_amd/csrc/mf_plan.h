@@ -19,6 +19,8 @@ struct PlanTuning {
     int32_t wide_k = WIDE_K;            // 128 x 128 update-matrix tiles when nn >= wide_k
     int32_t sim_workers = SIM_WORKERS;  // resident workgroups of the ticket simulation
     double zero_frac = 0.05;            // explicit zeros allowed by a chain merge
+    double small_zero_frac = MERGE_FRAC;  // the same up to MERGE_NJ rows (a zero_frac of the caller's
+                                        // own bounds these as well)
     int32_t prio = 0;                   // tile-DAG task kinds at raised wave priority (bit mask)
     int32_t fuse = 1;                   // diagonal tasks run the next panel solve and look-ahead update
     int32_t wg_per_cu = 0;              // resident tile-DAG workgroups per CU (0: as many as fit)

@@ -68,7 +68,8 @@ int mf_plan_destroy(mf_plan* plan);
  * the front width from which update-matrix tiles are 128 x 128 (default
  * 128), workgroups assumed resident when ordering the tile-DAG's tickets
  * (default 512), explicit zeros allowed by a chain merge in parts per
- * million (default 50000; a merged front of at most 256 rows may hold 30 %),
+ * million (default 50000, with 30 % for a merged front of at most 256 rows;
+ * any other value holds at every size),
  * and tuning[5] a bit mask of tile-DAG task kinds
  * run at raised wave priority (bits 0..5: extend-add, small front, diagonal
  * tile, panel solve, trailing update, update matrix; bit 6: the look-ahead
