@@ -14,6 +14,7 @@
 
 #include "../../include/mfhip.h"
 #include "mf_kernels.h"
+#include "mf_room.h"
 #include "mf_plan.h"
 
 using namespace mf;
@@ -412,30 +413,50 @@ void sync_ref(mf_factor* f) {
     f->ref_stale = false;
 }
 
-// Columns of the blocked solves: blocks of sixteen.
-size_t padded(size_t nrhs) { return (nrhs + 15) & ~(size_t)15; }
-
-// Workspaces of the solves of nrhs columns: update vectors, and past VT_COLS
-// columns or for the blocked form the solutions (of the blocked form twice,
-// row by row).  Without memory for these the columns are solved VT_COLS at a
-// time.
-int ensure_solve(mf_factor* f, size_t es, size_t nrhs) {
+// Workspaces of a solve of nrhs columns: Bws for the permuted columns, stage
+// for a staging copy, the update vectors, and past VT_COLS columns or for the
+// blocked form the solutions (of the blocked form twice, row by row).
+int ensure_solve(mf_factor* f, size_t es, size_t nrhs, bool bws, bool stage) {
     const HostPlan& H = f->plan->H;
-    if (nrhs > (size_t)std::min(VT_COLS, H.vcols)) {
-        const size_t c = padded(nrhs);
-        if (ensure(&f->Mv, &f->Mv_bytes, es * (size_t)H.mv_elems1 * c) == MF_OK &&
-            ensure(&f->sw, &f->sw_bytes, es * 2 * (size_t)H.n * c) == MF_OK)
-            return MF_OK;
-        (void)hipGetLastError();
-        nrhs = std::min<size_t>(nrhs, VT_COLS);
-    }
-    return ensure(&f->Mv, &f->Mv_bytes, es * (size_t)H.mv_elems1 * nrhs);
+    const size_t n = (size_t)H.n, mv = (size_t)H.mv_elems1;
+    const int64_t few = std::min(VT_COLS, H.vcols);
+    auto got = [](int rc) {
+        if (rc != MF_OK) (void)hipGetLastError();
+        return rc == MF_OK;
+    };
+    auto drop = [&](void** p, size_t* have) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+        *have = 0;
+    };
+    const bool ok = take_room(
+        (int64_t)nrhs, few,
+        [&] {
+            return (!bws || got(ensure(&f->Bws, &f->Bws_bytes, es * n * nrhs))) &&
+                   (!stage || got(ensure((void**)&f->stage, &f->stage_bytes, 8 * n * nrhs)));
+        },
+        [&](int64_t c) {
+            return got(ensure(&f->Mv, &f->Mv_bytes, es * mv * (size_t)c)) && got(ensure(&f->sw, &f->sw_bytes, es * 2 * n * (size_t)c));
+        },
+        [&] { return got(ensure(&f->Mv, &f->Mv_bytes, es * mv * std::min<size_t>(nrhs, VT_COLS))); },
+        [&] {
+            drop(&f->Mv, &f->Mv_bytes);
+            drop(&f->sw, &f->sw_bytes);
+        });
+    return ok ? MF_OK : fail(MF_ENOMEM, "hipMalloc failed (workspace)");
+}
+
+// Columns, in whole blocks, that mv_bytes of update vectors and sw_bytes of solutions hold.
+int64_t room_for(const HostPlan& H, size_t es, size_t mv_bytes, size_t sw_bytes) {
+    const int64_t s = (int64_t)(sw_bytes / (es * 2 * (size_t)H.n));
+    const int64_t m = H.mv_elems1 > 0 ? (int64_t)(mv_bytes / (es * (size_t)H.mv_elems1)) : s;
+    return std::min(m, s) / ROOM_BLOCK * ROOM_BLOCK;
 }
 
 // mv, sw: the update-vector and solution workspaces (ensure_solve) instead of
-// the factor's own; room: sw is there, both for padded(nrhs) columns.
+// the factor's own, for `room` columns (a multiple of sixteen; 0: no sw).
 template <typename T>
-void enqueue_solve(mf_factor* f, T* B, int64_t ldb, int nrhs, void* mv = nullptr, void* sw = nullptr, bool room = false) {
+void enqueue_solve(mf_factor* f, T* B, int64_t ldb, int nrhs, void* mv = nullptr, void* sw = nullptr, int64_t room = 0) {
     mf_plan* pl = f->plan;
     const HostPlan& H = pl->H;
     const DevPlan& P = pl->D;
@@ -446,21 +467,22 @@ void enqueue_solve(mf_factor* f, T* B, int64_t ldb, int nrhs, void* mv = nullptr
     if (!mv) {
         mv = f->Mv;
         sw = f->sw;
-        const size_t c = padded(nrhs);
-        room = f->Mv_bytes >= sizeof(T) * (size_t)H.mv_elems1 * c && f->sw_bytes >= sizeof(T) * 2 * (size_t)H.n * c;
+        room = room_for(H, sizeof(T), f->Mv_bytes, f->sw_bytes);
     }
     double bytes = (double)sizeof(T) * (2.0 * (double)(H.ndz + H.nlz) + 4.0 * H.n * nrhs);
     timed(f, MF_KC_SOLVE, bytes, 1, [&] {
         unsigned long long* trace = f->prof ? f->strace_buf : nullptr;
-        if (nrhs > H.vcols && room) {
-            launch_solve16<T>(P, F, B, ldb, nrhs, (T*)sw, (T*)mv, H.mv_elems1, pl->V, trace, (int64_t)H.ftask.size(),
-                              f->stream);
-            return;
+        const int step = room >= ROOM_BLOCK ? (int)std::min<int64_t>(nrhs, room) : VT_COLS;
+        for (int c = 0; c < nrhs; c += step) {
+            const int k = std::min(step, nrhs - c);
+            T* b = B + (int64_t)c * ldb;
+            if (k > H.vcols && room >= ROOM_BLOCK)
+                launch_solve16<T>(P, F, b, ldb, k, (T*)sw, (T*)mv, H.mv_elems1, pl->V, trace, (int64_t)H.ftask.size(),
+                                  f->stream);
+            else
+                launch_solve1<T>(P, F, b, ldb, k, (T*)(k > VT_COLS ? sw : f->xf), (T*)mv, H.mv_elems1, pl->V, (int)H.n,
+                                 trace, (int64_t)H.ftask.size(), f->stream);
         }
-        const int step = nrhs > VT_COLS && room ? nrhs : VT_COLS;
-        for (int c = 0; c < nrhs; c += step)
-            launch_solve1<T>(P, F, B + (int64_t)c * ldb, ldb, std::min(step, nrhs - c), (T*)(step > VT_COLS ? sw : f->xf), (T*)mv,
-                             H.mv_elems1, pl->V, (int)H.n, trace, (int64_t)H.ftask.size(), f->stream);
     });
 }
 
@@ -1021,17 +1043,16 @@ int mf_solve_natural(mf_factor* f, double* C, int64_t nrhs, int64_t ldc, int dev
     if (nrhs == 0 || H.n == 0) return MF_OK;
     if (solves64(f) && !f->sh_valid) return fail(MF_ESTATE, "FP64 solves of an FP32 factor: factorize after enabling them");
     size_t es = solve_elt(f);
-    if (ensure_solve(f, es, (size_t)nrhs)) return MF_ENOMEM;
-    if ((f->precision == MF_FP64 || solves64(f)) && device) {
+    const bool direct = (f->precision == MF_FP64 || solves64(f)) && device;
+    if (ensure_solve(f, es, (size_t)nrhs, !direct, !device)) return MF_ENOMEM;
+    if (direct) {
         enqueue_solve<double>(f, C, ldc, (int)nrhs);
     } else {
-        if (ensure(&f->Bws, &f->Bws_bytes, es * (size_t)H.n * nrhs)) return MF_ENOMEM;
         // identity permutation copies through the workspace
         std::vector<int64_t> id;
         const double* src = C;
         double* stage = nullptr;
         if (!device) {
-            if (ensure((void**)&f->stage, &f->stage_bytes, 8 * (size_t)H.n * nrhs)) return MF_ENOMEM;
             for (int64_t c = 0; c < nrhs; ++c)
                 HIPCHK(hipMemcpyAsync(f->stage + c * H.n, C + c * ldc, 8 * H.n, hipMemcpyHostToDevice,
                                       f->stream));
@@ -1076,8 +1097,7 @@ int mf_solve(mf_factor* f, const int64_t* perm, double* B, int64_t nrhs, int64_t
     if (nrhs == 0 || H.n == 0) return MF_OK;
     if (solves64(f) && !f->sh_valid) return fail(MF_ESTATE, "FP64 solves of an FP32 factor: factorize after enabling them");
     size_t es = solve_elt(f);
-    if (ensure_solve(f, es, (size_t)nrhs)) return MF_ENOMEM;
-    if (ensure(&f->Bws, &f->Bws_bytes, es * (size_t)H.n * nrhs)) return MF_ENOMEM;
+    if (ensure_solve(f, es, (size_t)nrhs, true, !device)) return MF_ENOMEM;
     if (f->perm_host.size() != (size_t)H.n ||
         std::memcmp(f->perm_host.data(), perm, 8 * H.n) != 0) {
         f->perm_host.assign(perm, perm + H.n);
@@ -1087,7 +1107,6 @@ int mf_solve(mf_factor* f, const int64_t* perm, double* B, int64_t nrhs, int64_t
     double* src = B;
     int64_t lds = ldb;
     if (!device) {
-        if (ensure((void**)&f->stage, &f->stage_bytes, 8 * (size_t)H.n * nrhs)) return MF_ENOMEM;
         for (int64_t c = 0; c < nrhs; ++c)
             HIPCHK(hipMemcpyAsync(f->stage + c * H.n, B + c * ldb, 8 * H.n, hipMemcpyHostToDevice,
                                   f->stream));
@@ -1124,7 +1143,7 @@ int mf_solve_noalloc(mf_factor* f, const int64_t* perm, double* B, int64_t nrhs,
     if (nrhs == 0 || H.n == 0) return MF_OK;
     if (solves64(f) && !f->sh_valid) return fail(MF_ESTATE, "FP64 solves of an FP32 factor: factorize after enabling them");
     const size_t es = solve_elt(f);
-    size_t mv_bytes = (es * (size_t)H.mv_elems1 * (size_t)nrhs + 255) & ~(size_t)255;
+    const size_t mv_bytes = (es * (size_t)H.mv_elems1 * (size_t)nrhs + 255) & ~(size_t)255;
     const size_t need = mv_bytes + es * (size_t)H.n * (size_t)nrhs;
     if (need > MF_NOALLOC_SCRATCH_BYTES)
         return fail(MF_EARG, "mf_solve_noalloc: " + std::to_string(need) + " bytes of scratch needed, limit " +
@@ -1134,14 +1153,24 @@ int mf_solve_noalloc(mf_factor* f, const int64_t* perm, double* B, int64_t nrhs,
     if (dev != f->device) return fail(MF_EARG, "the factor's device is not the current device");
     void* base = nullptr;
     if (int rc = scratch_address(&base)) return rc;
-    // room for any form where the workspaces fit as well, else VT_COLS columns at a time
-    const size_t cols = padded((size_t)nrhs);
-    const size_t mvb = (es * (size_t)H.mv_elems1 * cols + 255) & ~(size_t)255, swb = (es * 2 * (size_t)H.n * cols + 255) & ~(size_t)255;
-    const bool room = nrhs > std::min(VT_COLS, H.vcols) && mvb + swb + es * (size_t)H.n * (size_t)nrhs <= MF_NOALLOC_SCRATCH_BYTES;
-    if (room) mv_bytes = mvb;
-    void* mv = base;
-    void* sw = (unsigned char*)base + mv_bytes;
-    void* bws = room ? (unsigned char*)sw + swb : (unsigned char*)sw;
+    // in the scratch: the permuted columns, then room for as many columns as
+    // fit beside them (as ensure_solve takes them), else update vectors for VT_COLS
+    const size_t bws_bytes = (es * (size_t)H.n * (size_t)nrhs + 255) & ~(size_t)255;
+    const size_t left = MF_NOALLOC_SCRATCH_BYTES - std::min<size_t>(bws_bytes, MF_NOALLOC_SCRATCH_BYTES);
+    int64_t room = 0;
+    size_t mvb = 0;
+    (void)take_room(
+        nrhs, std::min(VT_COLS, H.vcols), [] { return true; },
+        [&](int64_t c) {
+            mvb = (es * (size_t)H.mv_elems1 * (size_t)c + 255) & ~(size_t)255;
+            const bool fits = mvb + es * 2 * (size_t)H.n * (size_t)c <= left;
+            room = fits ? c : 0;
+            return fits;
+        },
+        [] { return true; }, [] {});
+    void* bws = base;
+    void* mv = (unsigned char*)base + bws_bytes;
+    void* sw = room ? (void*)((unsigned char*)mv + mvb) : nullptr;
     if (f->perm_host.size() != (size_t)H.n ||
         std::memcmp(f->perm_host.data(), perm, 8 * H.n) != 0) {
         f->perm_host.assign(perm, perm + H.n);
