@@ -127,6 +127,7 @@ __device__ __forceinline__ void zero(v4_t<T> (&acc)[4]) {
 // counts the 18 wait states such a result needs (FP64, 16 passes) along the
 // longest way through the branches only, and on the short way (one group) the
 // next instruction read the last register early: its low word was still 0.
+// (tests/test_matrix_waits.py looks for such paths in the built library.)
 template <typename T>
 __device__ __forceinline__ void mma_done(v4_t<T> (&acc)[4]) {
     asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
