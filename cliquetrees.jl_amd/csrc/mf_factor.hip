@@ -812,7 +812,7 @@ __device__ __forceinline__ void pivot_cols(T (&x)[PB], T (&y)[PB], const DevFact
             my = y[K];
         } else if constexpr (RULE == PR_INV) {
             l = x[K];
-            my = y[K] * (T)rcp_full((double)dpp_bcast<K>(x[K]));
+            my = y[K] * ((T)1 / dpp_bcast<K>(x[K]));  // (a factor from elsewhere: any number)
         } else {
             double piv = (double)dpp_bcast<K>(x[K]);
             const bool ch = RULE == PR_CHOL || (RULE == PR_RULE && chol);

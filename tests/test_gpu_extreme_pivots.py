@@ -94,3 +94,25 @@ def test_solves_with_infinite_pivots(ct, n, prec):
         assert np.all(X[pins] == 0.0), nrhs
         # the suite's bars for solutions
         assert np.linalg.norm(X - X0) <= (1e-4 if prec == "f32" else 1e-11) * np.linalg.norm(X0), nrhs
+
+
+@pytest.mark.parametrize("n", [64, 65, 100, 150, 200])
+def test_given_factor_with_infinite_pivots(ct, oracle, n):
+    """div_impl! on a factor from elsewhere whose big fronts have infinite diagonal entries."""
+    M = _matrix(n, 3, n)
+    pins = [0, 3, 40, n - 9, n + 2, M.shape[0] - 8, M.shape[0] - 1]
+    A = M.copy()
+    A[pins, pins] = np.inf
+    P, S = ct.symbolic(sp.csc_matrix(A))
+    print(n, S.nfr, flush=True)
+    D, L, d, info = oracle.chol_impl(S, *oracle.assemble(S, P, sp.csc_matrix(A)))
+    assert info == 0 and np.isinf(D).sum() == len(set(pins))
+    perm = P.perm - 1
+    free = np.setdiff1d(np.arange(M.shape[0]), pins)
+    for nrhs in (1, 5, 17):
+        B = np.random.default_rng(nrhs).standard_normal((M.shape[0], nrhs))
+        X0 = np.zeros_like(B)
+        X0[free] = np.linalg.solve(M[np.ix_(free, free)], B[free])
+        X = ct.div_impl(S, D, L, None, B[perm], diag=ct.MF_CHOLESKY)
+        assert np.all(X[np.isin(perm, pins)] == 0.0), nrhs
+        assert np.linalg.norm(X - X0[perm]) <= 1e-11 * np.linalg.norm(X0), nrhs
