@@ -355,7 +355,7 @@ void enqueue_widen(mf_factor* f) {
     hipStream_t s = f->stream;
     launch_widen((const float*)f->panel, (double*)f->sh_panel, H.panel_elems, s);
     launch_widen((const float*)f->d, (double*)f->sh_d, H.n, s);
-    launch_diag<double>(f->plan->D, dev_factor_solve64(f), 0, (int)H.diag.size(), true, s);
+    launch_diag<double>(f->plan->D, dev_factor_solve64(f), 0, (int)H.diag.size(), s);
     f->sh_valid = true;
 }
 
@@ -502,7 +502,7 @@ std::string hang_message(const mf_factor* f, const int32_t* h) {
     } bufs[] = {{"front flag/done", f->flags, nf1},
                 {"tile counter", f->cnt, (size_t)H.dag_counters + 1},
                 {"extend-add counter", f->eacnt, nf1},
-                // (the single-column solves wait for the values themselves)
+                // (the solves wait for the values themselves)
                 {"forward solution word", f->xf, 2 * VT_COLS * (size_t)(H.n + 1)},
                 {"solution word", f->Bws, f->Bws_bytes / 4},
                 {"blocked solution word", f->sw, f->sw_bytes / 4},
@@ -868,7 +868,7 @@ int mf_factor_load(mf_factor* f, const double* Dval, const double* Lval, const d
     }
     launch_fill<unsigned long long>(f->info, 1, ~0ull, f->stream);
     // W = inverses of the 64 x 64 diagonal blocks, as the factorization leaves them
-    launch_diag<double>(f->plan->D, dev_factor<double>(f), 0, (int)H.diag.size(), true, f->stream);
+    launch_diag<double>(f->plan->D, dev_factor<double>(f), 0, (int)H.diag.size(), f->stream);
     HIPCHK(hipGetLastError());
     if (!device) HIPCHK(hipStreamSynchronize(f->stream));
     f->factored = true;
@@ -1367,7 +1367,7 @@ int mf_div_impl(mf_plan* plan, const double* Dval, const double* Lval, const dou
     if (diag == MF_LDLT && plan->H.n)
         HIPCHK(hipMemcpyAsync(f->d, d, 8 * plan->H.n, hipMemcpyHostToDevice, f->stream));
     // the big-front solves use the inverted 64x64 diagonal blocks
-    launch_diag<double>(plan->D, dev_factor<double>(f), 0, (int)plan->H.diag.size(), true, f->stream);
+    launch_diag<double>(plan->D, dev_factor<double>(f), 0, (int)plan->H.diag.size(), f->stream);
     f->factored = true;
     f->sel_valid = false;
     f->ref_stale = false;

@@ -74,12 +74,6 @@ __device__ __forceinline__ double wave_max(double v) {
 // follows all of the task's data.
 __device__ __forceinline__ void drain_stores() { __builtin_amdgcn_s_waitcnt(0); }
 
-// Bounded wait until *flag >= target (the watchdog of mf_sync.h).
-template <typename T>
-__device__ __forceinline__ void wait_ge(int32_t* flag, int32_t target, const DevFactor<T>& F) {
-    (void)bounded_wait(flag, target, F.hang, F.ticket, F.stall, 2);
-}
-
 __device__ __forceinline__ int ld_rel(const int32_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1265,11 +1259,10 @@ __device__ __forceinline__ void potrf_gmw(const DevFactor<T>& F, const Front& f,
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_diag(DevPlan P, DevFactor<T> F, int t0, int invert_only) {
+__global__ __launch_bounds__(256) void k_diag(DevPlan P, DevFactor<T> F, int t0) {
     __shared__ T lds[PTILE];
     const DiagTask dt = P.diag[t0 + blockIdx.x];
-    potrf_blocked<T>(F, P.fronts[dt.front], dt.k0, invert_only != 0, false, lds, (int)threadIdx.x);
-    if (!invert_only) store_diag<T>(F, P.fronts[dt.front], dt.k0, lds, (int)threadIdx.x);
+    potrf_blocked<T>(F, P.fronts[dt.front], dt.k0, true, false, lds, (int)threadIdx.x);
 }
 
 template <typename T>
@@ -1972,10 +1965,9 @@ void launch_small(const DevPlan& P, const DevFactor<T>& F, int tickets, hipStrea
 }
 
 template <typename T>
-void launch_diag(const DevPlan& P, const DevFactor<T>& F, int t0, int t1, bool invert_only,
-                 hipStream_t s) {
+void launch_diag(const DevPlan& P, const DevFactor<T>& F, int t0, int t1, hipStream_t s) {
     if (t1 <= t0) return;
-    hipLaunchKernelGGL(k_diag<T>, dim3(t1 - t0), dim3(256), 0, s, P, F, t0, invert_only ? 1 : 0);
+    hipLaunchKernelGGL(k_diag<T>, dim3(t1 - t0), dim3(256), 0, s, P, F, t0);
 }
 
 template <typename T>
@@ -2058,14 +2050,13 @@ void launch_copyout(const DevPlan& P, const DevFactor<T>& F, double* Dval, doubl
     template void launch_refresh<T>(const DevFactor<T>&, const int64_t*, const int64_t*,        \
                                     const double*, int64_t, double*, hipStream_t);              \
     template void launch_small<T>(const DevPlan&, const DevFactor<T>&, int, hipStream_t);                            \
-    template void launch_diag<T>(const DevPlan&, const DevFactor<T>&, int, int, bool,           \
-                                 hipStream_t);                                                 \
     template void launch_copyout<T>(const DevPlan&, const DevFactor<T>&, double*, double*,      \
                                     double*, int, const double*, hipStream_t);                  \
     template void launch_dag<T>(const DevPlan&, const DevFactor<T>&, const DevDag&, hipStream_t); \
     template void launch_gmw_beta<T>(const DevPlan&, const DevFactor<T>&, double*, int64_t, hipStream_t);
 MF_INST(double)
 MF_INST(float)
+template void launch_diag<double>(const DevPlan&, const DevFactor<double>&, int, int, hipStream_t);
 template void launch_fill<int32_t>(int32_t*, int64_t, int32_t, hipStream_t);
 template void launch_fill<uint32_t>(uint32_t*, int64_t, uint32_t, hipStream_t);
 template void launch_fill<unsigned long long>(unsigned long long*, int64_t, unsigned long long,

@@ -54,7 +54,7 @@ constexpr int MERGE_NJ = 256;
 constexpr double MERGE_FRAC = 0.3;
 constexpr int VT_COLS = 5;                // right-hand sides whose forward solutions a factor always has room for
 constexpr int VT_MAX = 16;                // right-hand sides solved column by column at most (one block)
-constexpr int VT_ROWBLOCKS = 4;           // row blocks of a one-task front of the single-column solves
+constexpr int VT_ROWBLOCKS = 4;           // row blocks of a one-task front of the forward solves
 constexpr int VT_PANELS = 64 * 65;        // elements of the panels of their grouped small fronts
 constexpr int SEP_TILES = 8;    // separator tiles per backward partial-product task (fronts whose
                                 // separator has more are split over several tasks)

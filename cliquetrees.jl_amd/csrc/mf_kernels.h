@@ -90,10 +90,9 @@ void launch_refresh(const DevFactor<T>& F, const int64_t* tgt_panel, const int64
                     const double* nzval, int64_t nnz, double* adiag, hipStream_t s);
 template <typename T>
 void launch_small(const DevPlan& P, const DevFactor<T>& F, int tickets, hipStream_t s);
-// invert_only: the block already holds the factor; only W is produced.
+// W of the diagonal tiles [t0, t1) of a factor that the panels hold.
 template <typename T>
-void launch_diag(const DevPlan& P, const DevFactor<T>& F, int t0, int t1, bool invert_only,
-                 hipStream_t s);
+void launch_diag(const DevPlan& P, const DevFactor<T>& F, int t0, int t1, hipStream_t s);
 template <typename T>
 void launch_dag(const DevPlan& P, const DevFactor<T>& F, const DevDag& D, hipStream_t s);
 template <typename T>

@@ -995,7 +995,7 @@ std::string Planner::solve_tasks() {
     return std::string();
 }
 
-// The task lists of the single-column solves, from the ungrouped ftask and
+// The task lists of both solve kernels, from the ungrouped ftask and
 // btask: small fronts in groups of up to four (a front joins the open group,
 // which keeps the place of its first member, when what it waits for is at or
 // before that place), one-block fronts with few row blocks in one forward

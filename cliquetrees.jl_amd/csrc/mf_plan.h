@@ -42,7 +42,7 @@ struct PTask {
     int32_t c;
 };
 
-// Task of the solves of one right-hand side, and the runs of tasks that one
+// Task of the solve kernels (column by column and blocked), and the runs of tasks that one
 // ticket covers.  VT_SMALL: up to four small fronts a, b, c, d (-1: absent),
 // one wavefront each, their panels (leading dimension nJ | 1) in LDS from 0,
 // o12 & 0xffff, o12 >> 16 and o3; VT_FRONT (forward): the front a, one
@@ -93,7 +93,7 @@ struct HostPlan {
     std::vector<GemmTask> gemm;
     std::vector<DiagTask> diag;
     std::vector<PTask> ftask, btask;   // forward / backward solve tasks, ticket order
-    std::vector<VTask> vftask, vbtask; // the same for one right-hand side
+    std::vector<VTask> vftask, vbtask; // the same merged, as the solve kernels run them
     std::vector<int32_t> vfunit, vbunit;  // ticket u covers tasks [unit[u], unit[u + 1])
     std::vector<VChild> vchd;          // per entry of chd
     int32_t vcols = 1;                 // solves of up to this many columns go column by column
