@@ -609,6 +609,7 @@ static int plan_create(int64_t n, int64_t nfr, const int64_t* resptr, const int6
     pl->V.btask = pl->V.ftask + H.vftask.size();
     pl->V.bunit = pl->V.funit + H.vfunit.size();
     pl->V.chd = D.vchd;
+    pl->V.group = H.vgroup;
     D.nJ = (int32_t)H.fronts.size();
     pl->V.nfu = std::max<int32_t>(0, (int32_t)H.vfunit.size() - 1);
     pl->V.nbu = std::max<int32_t>(0, (int32_t)H.vbunit.size() - 1);

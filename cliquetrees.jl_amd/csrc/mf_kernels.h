@@ -114,6 +114,7 @@ struct DevVPlan {
     const int32_t* bunit = nullptr;
     const VChild* chd = nullptr;
     int32_t nfu = 0, nbu = 0;
+    bool group = false;      // several blocks of columns a ticket (HostPlan::vgroup)
 };
 template <typename T>
 struct DevVSolve {
@@ -145,6 +146,7 @@ struct DevBSolve {
     T* Mv;
     int64_t ldb, mvs;
     int32_t nrhs, ncol;      // all columns; those of the current block
+    int32_t group;           // blocks that a ticket covers
     const VTask* task;
     const int32_t* unit;
     int32_t nunit;

@@ -97,6 +97,7 @@ struct HostPlan {
     std::vector<int32_t> vfunit, vbunit;  // ticket u covers tasks [unit[u], unit[u + 1])
     std::vector<VChild> vchd;          // per entry of chd
     int32_t vcols = 1;                 // solves of up to this many columns go column by column
+    bool vgroup = false;               // small fronts only, whose tasks outweigh the longest path
     std::vector<DagTask> dag;          // tile-DAG factorization of the big region
     std::vector<DagTask> dag_gmw;      // the same tasks in creation order (GMW81: a diagonal
                                        // tile waits for its whole block column)

@@ -29,6 +29,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "mf_kernels.h"
 #include "mf_mfma.h"
@@ -213,6 +214,16 @@ __device__ __forceinline__ void gather(const DevPlan& P, const DevBSolve<T>& V, 
 // Lane r keeps row r's sixteen values; the slab Y (64 rows) carries them to
 // and from the row-by-row layout.
 
+// What scale_panel returns, of a panel that it has scaled already (the
+// diagonal keeps D).
+template <typename T>
+__device__ __forceinline__ void scaled_diagonal(int nn, int nj, const T* Ps, bool unit, T& d, T& rd, bool& exact) {
+    const int rr = min((int)(threadIdx.x & 63), nn - 1);
+    d = unit ? (T)1 : Ps[rr + rr * (nj | 1)];
+    rd = (T)1 / d;
+    exact = __any(abnormal(rd));
+}
+
 template <typename T>
 __device__ __forceinline__ void store_rows(const T* Y, int r0, int rows, T* dst) {
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
@@ -220,7 +231,7 @@ __device__ __forceinline__ void store_rows(const T* Y, int r0, int rows, T* dst)
 }
 
 template <typename T>
-__device__ void small_fwd16(const DevPlan& P, const DevFactor<T>& F, const DevBSolve<T>& V, int J, T* Ps, T* Y,
+__device__ void small_fwd16(const DevPlan& P, const DevFactor<T>& F, const DevBSolve<T>& V, int J, bool staged, T* Ps, T* Y,
                             const Ctl& ctl) {
     const int r = threadIdx.x & 63;
     const Front f = front_of(P, J);
@@ -238,11 +249,12 @@ __device__ void small_fwd16(const DevPlan& P, const DevFactor<T>& F, const DevBS
         if (r >= nn || c >= V.ncol) y[c] = (T)0;
         Y[r * LR + c] = (T)0;
     }
-    stage_panel(F.panel + f.poff, nj, nn, Ps);
+    if (!staged) stage_panel(F.panel + f.poff, nj, nn, Ps);
     wave_sync();
     T d, rcp;
     bool exact;
-    scale_panel(nj, nn, Ps, unit, d, rcp, exact);
+    scale_panel(nj, nn, Ps, unit || staged, d, rcp, exact);
+    if (staged) scaled_diagonal(nn, nj, Ps, unit, d, rcp, exact);
     gather<T, false, 4>(P, V, f, 0, 0, Y, 0, ctl);
     wave_sync();
 #pragma unroll
@@ -266,7 +278,7 @@ __device__ void small_fwd16(const DevPlan& P, const DevFactor<T>& F, const DevBS
 }
 
 template <typename T>
-__device__ void small_bwd16(const DevPlan& P, const DevFactor<T>& F, const DevBSolve<T>& V, int J, T* Ps, T* Y,
+__device__ void small_bwd16(const DevPlan& P, const DevFactor<T>& F, const DevBSolve<T>& V, int J, bool staged, T* Ps, T* Y,
                             const Ctl& ctl) {
     const int r = threadIdx.x & 63, li = r & 15, lk = r >> 4;
     const Front f = front_of(P, J);
@@ -280,11 +292,12 @@ __device__ void small_bwd16(const DevPlan& P, const DevFactor<T>& F, const DevBS
 #pragma unroll
     for (int c = 0; c < RB; ++c) b[c] = in[(uint32_t)(rd * RB + c)];
     const T dd = unit ? F.d[f.c0 + rd] : (T)1;
-    stage_panel(F.panel + f.poff, nj, nn, Ps);
+    if (!staged) stage_panel(F.panel + f.poff, nj, nn, Ps);
     wave_sync();
     T d, rcp;
     bool exact;
-    scale_panel(nj, nn, Ps, unit, d, rcp, exact);
+    scale_panel(nj, nn, Ps, unit || staged, d, rcp, exact);
+    if (staged) scaled_diagonal(nn, nj, Ps, unit, d, rcp, exact);
     // separator part: -L21' x_sep, sixteen separator rows at a time
     v4_t<T> acc[4];
     zero<T>(acc);
@@ -692,49 +705,65 @@ union BLds {
     } b;
 };
 
-template <typename T, bool FWD>
+// GROUP: a ticket covers V0.group blocks of a unit's tasks, one after the
+// other (a small front's panel is staged and scaled for the first of them).
+// One block a ticket / groups of up to four, us: 30000 systems of order 3, 33
+// and 100 columns 616 / 475 and 1387 / 1036, 1500 of order 60 572 / 440 and
+// 1306 / 1002, 2000 small grids, 33 and 75 columns 699 / 580 and 1148 / 974.
+template <typename T, bool FWD, bool GROUP>
 __global__ __launch_bounds__(256, 2) void k_bsolve16(DevPlan P, DevFactor<T> F, DevBSolve<T> V0) {
     static_assert(VROWS >= 4 * NB, "the second set of partial sums in Y");
     __shared__ BLds<T> S;
     __shared__ uint32_t s_tick;
     const int tid = threadIdx.x, g = uni(tid >> 6);
     const Ctl ctl{F.hang, V0.ticket, F.stall};
-    const uint32_t nblk = (V0.nrhs + RB - 1) / RB, tickets = (uint32_t)V0.nunit * nblk;
+    const int nblk = (V0.nrhs + RB - 1) / RB, per = GROUP ? V0.group : 1;
+    const uint32_t ngrp = (nblk + per - 1) / per, tickets = (uint32_t)V0.nunit * ngrp;
     for (;;) {
         if (tid == 0) s_tick = atomicAdd(V0.ticket, 1u);
         __syncthreads();
         const uint32_t tick = uni((int32_t)s_tick);
         if (tick >= tickets) break;
-        const uint32_t u = tick / nblk;
-        const int64_t blk = tick - u * nblk;
-        DevBSolve<T> V = V0;
-        V.B += blk * RB * V.ldb;
-        V.ncol = min(RB, V.nrhs - (int)blk * RB);
-        V.X += blk * RB * P.n;
-        V.Z += blk * RB * P.n;
-        V.Mv += blk * RB * V.mvs;
-        const int t1 = V.unit[u + 1];
-        for (int t = V.unit[u]; t < t1; ++t) {
-            const unsigned long long t_begin = (V.trace && tid == 0) ? wall_clock64() : 0;
-            const VTask tk = V.task[t];
+        const uint32_t u = tick / ngrp;
+        const int blk0 = (int)(tick - u * ngrp) * per, blk1 = GROUP ? min(nblk, blk0 + per) : blk0 + 1;
+        auto block = [&](int blk) {
+            DevBSolve<T> V = V0;
+            V.B += (int64_t)blk * RB * V.ldb;
+            V.ncol = min(RB, V.nrhs - blk * RB);
+            V.X += (int64_t)blk * RB * P.n;
+            V.Z += (int64_t)blk * RB * P.n;
+            V.Mv += (int64_t)blk * RB * V.mvs;
+            return V;
+        };
+        const int t1 = V0.unit[u + 1];
+        for (int t = V0.unit[u]; t < t1; ++t) {
+            const unsigned long long t_begin = (V0.trace && tid == 0) ? wall_clock64() : 0;
+            const VTask tk = V0.task[t];
             if (tk.kind == VT_SMALL) {
                 const int J = uni(g == 0 ? tk.a : g == 1 ? tk.b : g == 2 ? tk.c : tk.d);
                 const int o = uni(g == 0 ? 0 : g == 1 ? (tk.o12 & 0xffff) : g == 2 ? (int)((uint32_t)tk.o12 >> 16) : tk.o3);
-                if (J >= 0) {
-                    if (FWD) small_fwd16(P, F, V, J, S.s.panel + o, S.s.slab + g * NB * LR, ctl);
-                    else small_bwd16(P, F, V, J, S.s.panel + o, S.s.slab + g * NB * LR, ctl);
+                for (int blk = blk0; blk < blk1 && J >= 0; ++blk) {
+                    const DevBSolve<T> V = block(blk);
+                    if (FWD) small_fwd16(P, F, V, J, GROUP && blk > blk0, S.s.panel + o, S.s.slab + g * NB * LR, ctl);
+                    else small_bwd16(P, F, V, J, GROUP && blk > blk0, S.s.panel + o, S.s.slab + g * NB * LR, ctl);
                 }
-            } else if (FWD) {
-                if (tk.kind == VT_FRONT) front_fwd16(P, F, V, uni(tk.a), S.b.Y, S.b.Red, ctl);
-                else if (tk.kind == VT_DIAG) diag_fwd16(P, F, V, uni(tk.a), uni(tk.b), uni(tk.c), S.b.Y, S.b.Red, ctl);
-                else rows_fwd16(P, F, V, uni(tk.a), uni(tk.b), uni(tk.c), S.b.Y, S.b.Red, ctl);
             } else {
-                if (tk.kind == VT_SEPB) sep_bwd16(P, F, V, uni(tk.a), uni(tk.b), uni(tk.c), uni(tk.d), S.b.Red, ctl);
-                else diag_bwd16(P, F, V, uni(tk.a), uni(tk.b), uni(tk.c), S.b.Red, S.b.Y, ctl);
+                for (int blk = blk0; blk < blk1; ++blk) {
+                    const DevBSolve<T> V = block(blk);
+                    if (GROUP && blk > blk0) __syncthreads();  // the LDS of the block before is free
+                    if (FWD) {
+                        if (tk.kind == VT_FRONT) front_fwd16(P, F, V, uni(tk.a), S.b.Y, S.b.Red, ctl);
+                        else if (tk.kind == VT_DIAG) diag_fwd16(P, F, V, uni(tk.a), uni(tk.b), uni(tk.c), S.b.Y, S.b.Red, ctl);
+                        else rows_fwd16(P, F, V, uni(tk.a), uni(tk.b), uni(tk.c), S.b.Y, S.b.Red, ctl);
+                    } else {
+                        if (tk.kind == VT_SEPB) sep_bwd16(P, F, V, uni(tk.a), uni(tk.b), uni(tk.c), uni(tk.d), S.b.Red, ctl);
+                        else diag_bwd16(P, F, V, uni(tk.a), uni(tk.b), uni(tk.c), S.b.Red, S.b.Y, ctl);
+                    }
+                }
             }
-            if (V.trace && tid == 0) {  // (the last block's clocks stay)
-                V.trace[2 * tk.t0] = t_begin | ((unsigned long long)blockIdx.x << 48);
-                V.trace[2 * tk.t0 + 1] = wall_clock64();
+            if (V0.trace && tid == 0) {  // (the last block's clocks stay)
+                V0.trace[2 * tk.t0] = t_begin | ((unsigned long long)blockIdx.x << 48);
+                V0.trace[2 * tk.t0 + 1] = wall_clock64();
             }
             __syncthreads();  // the LDS of this task is free; every thread has read s_tick
         }
@@ -760,15 +789,23 @@ void launch_solve16(const DevPlan& P, const DevFactor<T>& F, T* B, int64_t ldb, 
     const int64_t blocks = (std::max<int64_t>(mvs, 2 * (int64_t)P.n) * cols + 1023) / 1024;
     hipLaunchKernelGGL((k_binit<T>), dim3((unsigned)std::min<int64_t>(blocks, 4096)), dim3(256), 0, s, (bits_t<T>*)XZ, 2 * half,
                        (bits_t<T>*)Mv, mvs * cols, F.ticket);
-    DevBSolve<T> V{B, XZ, XZ + half, Mv, ldb, mvs, nrhs, 0, D.ftask, D.funit, D.nfu, D.chd, F.ticket, trace};
-    auto grid = [&](int64_t units) { return dim3((unsigned)std::min<int64_t>(units * nblk, 512)); };
-    hipLaunchKernelGGL((k_bsolve16<T, true>), grid(D.nfu), dim3(256), 0, s, P, F, V);
+    // blocks a ticket: several where the plan's tasks fill the chip by themselves
+    // (HostPlan::vgroup) and many tickets are left all the same
+    const int64_t group = D.group ? std::max<int64_t>(1, std::min<int64_t>({nblk, 4, nblk * D.nfu / 1024})) : 1;
+    DevBSolve<T> V{B, XZ, XZ + half, Mv, ldb, mvs, nrhs, 0, (int32_t)group, D.ftask, D.funit, D.nfu, D.chd, F.ticket, trace};
+    auto grid = [&](int64_t units) { return dim3((unsigned)std::min<int64_t>(units * ((nblk + group - 1) / group), 512)); };
+    auto run = [&](auto fwd, int64_t units) {
+        constexpr bool FWD = decltype(fwd)::value;
+        if (group > 1) hipLaunchKernelGGL((k_bsolve16<T, FWD, true>), grid(units), dim3(256), 0, s, P, F, V);
+        else hipLaunchKernelGGL((k_bsolve16<T, FWD, false>), grid(units), dim3(256), 0, s, P, F, V);
+    };
+    run(std::true_type(), D.nfu);
     V.task = D.btask;
     V.unit = D.bunit;
     V.nunit = D.nbu;
     V.ticket = F.ticket + 1;
     V.trace = trace ? trace + 2 * ntrace_f : nullptr;
-    hipLaunchKernelGGL((k_bsolve16<T, false>), grid(D.nbu), dim3(256), 0, s, P, F, V);
+    run(std::false_type(), D.nbu);
 }
 
 template void launch_solve16<double>(const DevPlan&, const DevFactor<double>&, double*, int64_t, int, double*, double*,

@@ -50,3 +50,24 @@ def test_columns(ct, what, prec):
                                               ctypes.c_void_p(T.data_ptr()), nrhs, n) == 0
         assert _native.hip().mf_factor_sync(F._f.handle) == 0
         assert np.linalg.norm(T.cpu().numpy().T - X0) <= tol * np.linalg.norm(X0)
+
+
+@pytest.mark.parametrize("k,m", [(9000, 2), (2500, 40)])
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_groups_of_blocks(ct, k, m, prec):
+    """Many small systems: one to four blocks of columns to a ticket, the last one short."""
+    rng = np.random.default_rng(m)
+    L = np.tril(rng.uniform(-1, 1, (k, m, m)), -1)
+    M = L + L.transpose(0, 2, 1)
+    M[:, np.arange(m), np.arange(m)] = np.abs(M).sum(2) + rng.uniform(0.5, 1.5, (k, m))
+    i = np.arange(k)[:, None, None] * m + np.arange(m)[None, :, None] + np.zeros((1, 1, m), int)
+    A = sp.csc_matrix((M.ravel(), (i.ravel(), i.transpose(0, 2, 1).ravel())), shape=(k * m, k * m))
+    A.sort_indices()
+    P, S = ct.symbolic(A)
+    F = ct.cholesky_(ct.ChordalCholesky(A, P, S, precision=ct.MF_FP32 if prec == "f32" else ct.MF_FP64))
+    for nrhs in (17, 50, 70):
+        print(k, m, prec, nrhs, flush=True)
+        B = rng.standard_normal((k * m, nrhs))
+        X0 = np.linalg.solve(M, B.reshape(k, m, nrhs)).reshape(k * m, nrhs)
+        X = ct.solve(F, B)
+        assert np.linalg.norm(X - X0) <= (1e-4 if prec == "f32" else 1e-11) * np.linalg.norm(X0)
