@@ -62,9 +62,11 @@ __device__ __forceinline__ double regularize_gmw(const DevFactor<T>& F, double s
     return s * jmax(jmax(fabs(Djj), amax * amax / F.gmw[2]), F.delta);
 }
 
-// Largest value over the wavefront (NaN-propagating), in every lane.
+// Largest value over the wavefront (NaN-propagating), in every lane; over
+// each half of it with LANES = 32.
+template <int LANES = 64>
 __device__ __forceinline__ double wave_max(double v) {
-    for (int o = 32; o > 0; o >>= 1) v = jmax(v, __shfl_xor(v, o));
+    for (int o = LANES / 2; o > 0; o >>= 1) v = jmax(v, __shfl_xor(v, o));
     return v;
 }
 
@@ -174,11 +176,12 @@ __device__ __forceinline__ void wait_children(const DevPlan& P, const DevFactor<
 // takes the square root and the division, so that an infinite diagonal entry
 // (a pinned unknown) scales its column to zero and a subnormal one is as
 // accurate as the rest.
-template <typename T>
+// LANES: rows that differ (32: the wavefront's halves hold the same ones).
+template <int LANES, typename T>
 __device__ __forceinline__ double small_pivot(const DevFactor<T>& F, double sgn, int k, double akk, double below, double* scale,
                                               double* root) {
     const double sg = F.signs ? lane_of(sgn, k) : F.diag == 0 ? 1.0 : 0.0;
-    const double piv = F.reg_kind == 2 ? regularize_gmw(F, sg, akk, wave_max(below)) : regularize(F, sg, akk);
+    const double piv = F.reg_kind == 2 ? regularize_gmw(F, sg, akk, wave_max<LANES>(below)) : regularize(F, sg, akk);
     *scale = F.diag == 0 ? rsqrt_full(piv) : rcp_full(piv);
     *root = piv * *scale;
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(__builtin_bit_cast(unsigned long long, piv) >> 32));
@@ -285,7 +288,7 @@ __device__ __forceinline__ void small_front(const DevPlan& P, const DevFactor<T>
     // column k, held in the owner's first register
     auto own = [&](int k) {
         double sc, rt;
-        const double piv = small_pivot(F, sgn, k, (double)lane_of(a[0], k),
+        const double piv = small_pivot<64>(F, sgn, k, (double)lane_of(a[0], k),
                                        (r > k && r < nj) ? fabs((double)a[0]) : 0.0, &sc, &rt);
         if (piv == 0.0) {
             if (r == 0) atomicMin(F.info, (unsigned long long)(f.c0 + k + 1));
@@ -331,6 +334,7 @@ __device__ __forceinline__ void small_front(const DevPlan& P, const DevFactor<T>
 }
 
 constexpr int LDT1 = TINY_NJ + 1;     // leading dimension of a wavefront's LDS front
+static_assert(TINY_NJ == 32, "both halves of a wavefront hold the rows of a tiny front");
 
 // One tiny front (nJ <= TINY_NJ) by one wavefront: as small_front, with the
 // whole front in the wavefront's registers (row in the lane, one register a
@@ -416,7 +420,7 @@ __device__ __forceinline__ void wave_front(const DevPlan& P, const DevFactor<T>&
         const int k = k4 + o;
         if (k >= nn || failed) return;  // uniform
         double sc, rt;
-        const double piv = small_pivot(F, sgn, k, (double)lane_of(a[o], k), (r > k && r < nj) ? fabs((double)a[o]) : 0.0, &sc, &rt);
+        const double piv = small_pivot<TINY_NJ>(F, sgn, k, (double)lane_of(a[o], k), (r > k && r < nj) ? fabs((double)a[o]) : 0.0, &sc, &rt);
         if (piv == 0.0) {
             if (lane == 0) atomicMin(F.info, (unsigned long long)(f.c0 + k + 1));
             failed = true;
