@@ -561,14 +561,18 @@ std::string Planner::factor_tasks() {
             const int32_t p = (F.nn + NB - 1) / NB, R = p + (F.na + NB - 1) / NB;
             std::vector<std::vector<std::pair<int32_t, int32_t>>> hit(R);  // per row block: (child's place, child)
             std::vector<std::vector<int32_t>> blocks;                      // per child: its row blocks
+            size_t pairs = 0;                                              // sources of J's tiles
             for (int32_t q = F.chd0; q < F.chd1; ++q) {
                 const int32_t* tb = P.sgstart.data() + P.sgoff[P.chd[q]];
                 std::vector<int32_t> bl;
                 for (int32_t b = 0; b < R; ++b)
                     if (tb[b + 1] > tb[b]) bl.push_back(b);
                 for (int32_t b : bl) hit[b].push_back({q - F.chd0, P.chd[q]});
+                pairs += bl.size() * (bl.size() + 1) / 2;
                 blocks.push_back(std::move(bl));
             }
+            // (tens of thousands of children: hundreds of megabytes, taken once)
+            if (pairs > P.ea_src.size()) P.ea_src.reserve(P.ea_src.size() + pairs);
             for (int32_t Jc = 0; Jc < R; ++Jc) {
                 // sources per row block I >= Jc, children in accumulation order
                 std::vector<std::vector<int32_t>> src(R - Jc);
