@@ -207,17 +207,23 @@ __device__ void sel_gather(const DevPlan& P, const DevSel<T>& S, int J, int jb, 
 
 // A whole front with nJ <= 64 in LDS: L = [L11; L21] in Lf (ld FLD), M in
 // Mf; Lt = L21 L11^-1 and X = L11^-1 in place, Sigma21 = -M Lt into Mf,
-// Sigma11 = X' X - Lt' Sigma21 straight to the output panel.
+// Sigma11 = X' X - Lt' Sigma21 straight to the output panel.  Up to eight
+// columns a wavefront load at once, in pairs that stop at the front's last (a
+// chain of fronts of nine columns, 8.3 us a front; 9.3 with all eight always).
 template <typename T>
 __device__ void sel_small(const DevPlan& P, const DevSel<T>& S, int J, T* Lf, T* Mf, const int tid) {
     const Front f = P.fronts[J];
     const int nn = f.nn, na = f.na, nJ = nn + na;
     const T* Lp = S.base[SP_PANEL] + f.poff;
-    const int r = tid & 63, g = tid >> 6;
+    const int r = tid & 63, g = uni(tid >> 6);
     for (int c0 = g; c0 < nn; c0 += 32) {
         T v[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = Lp[min(r, nJ - 1) + (int64_t)min(c0 + 4 * i, nn - 1) * nJ];
+        for (int h = 0; h < 8; h += 2) {
+            if (c0 + 4 * h >= nn) break;  // uniform
+#pragma unroll
+            for (int i = h; i < h + 2; ++i) v[i] = Lp[min(r, nJ - 1) + (int64_t)min(c0 + 4 * i, nn - 1) * nJ];
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             if (r < nJ && c0 + 4 * i < nn) Lf[r + (c0 + 4 * i) * FLD] = v[i];
@@ -233,9 +239,13 @@ __device__ void sel_small(const DevPlan& P, const DevSel<T>& S, int J, T* Lf, T*
         for (int c0 = g; c0 < na; c0 += 32) {
             T v[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int rc = rel[min(c0 + 4 * i, na - 1)];
-                v[i] = ldc(parent_addr(sig, pM, pf.nn, pf.na, max(ra, rc), min(ra, rc)));
+            for (int h = 0; h < 8; h += 2) {
+                if (c0 + 4 * h >= na) break;  // uniform
+#pragma unroll
+                for (int i = h; i < h + 2; ++i) {
+                    const int rc = rel[min(c0 + 4 * i, na - 1)];
+                    v[i] = ldc(parent_addr(sig, pM, pf.nn, pf.na, max(ra, rc), min(ra, rc)));
+                }
             }
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
